@@ -22,6 +22,7 @@ POL = {"Ez": 0, "Hz": 1}
 PREC = {"fp64": 0, "c64": 1}
 FACTOR_PIVOT = 0x100     # FDFD_FACTOR_PIVOT
 FACTOR_STEPWISE = 0x200  # FDFD_FACTOR_STEPWISE
+FACTOR_ND = 0x400        # FDFD_FACTOR_ND
 
 
 class FdfdGrid(ctypes.Structure):
@@ -89,6 +90,8 @@ SIGNATURES = {
     "fdfd_set_step_symmetry": (c_int, [c_int]),
     "fdfd_set_twist": (c_int, [c_int]),
     "fdfd_twist_block": (c_int, [_G]),
+    "fdfd_nd_supported": (c_int, [_G]),
+    "fdfd_nd_front": (c_int, [_G, c_int, c_int, POINTER(c_int32), POINTER(ctypes.c_int64), POINTER(c_int32)]),
 }
 
 _lib = None

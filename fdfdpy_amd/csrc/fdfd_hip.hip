@@ -2818,9 +2818,16 @@ int check_grid(const fdfd_grid *g) {
 int check_prec(int precision) {
   const int base = precision & 0xff, flags = precision & ~0xff;
   if ((base != FDFD_PREC_FP64 && base != FDFD_PREC_C64) ||
-      (flags & ~(FDFD_FACTOR_PIVOT | FDFD_FACTOR_STEPWISE)))
+      (flags & ~(FDFD_FACTOR_PIVOT | FDFD_FACTOR_STEPWISE | FDFD_FACTOR_ND)) ||
+      ((flags & FDFD_FACTOR_ND) && flags != FDFD_FACTOR_ND))
     return fail(FDFD_ERR_ARG, "precision must be FDFD_PREC_FP64 or FDFD_PREC_C64 (optionally | "
-                "FDFD_FACTOR_PIVOT), got %d", precision);
+                "FDFD_FACTOR_PIVOT, or | FDFD_FACTOR_ND alone), got %d", precision);
+  return FDFD_OK;
+}
+// for entry points of the block factorization alone
+int check_prec_block(int precision) {
+  if (int rc = check_prec(precision)) return rc;
+  if (precision & FDFD_FACTOR_ND) return fail(FDFD_ERR_ARG, "this entry point has no nested-dissection form");
   return FDFD_OK;
 }
 inline int base_prec(int precision) { return precision & 0xff; }
@@ -2949,6 +2956,8 @@ inline void *wrap_sigma_last(const fdfd_grid *g, int precision, const void *fact
   const size_t np = pad_n(g->ny);
   return (char *)wrap_sigma(g, precision, factor) + 2 * np * np * elem_size(precision);
 }
+
+#include "fdfd_nd.h"
 
 template <typename T, bool PIV>
 int launch_step(const FBatch<T> &b, hipStream_t s) {
@@ -3598,6 +3607,22 @@ __global__ void __launch_bounds__(NT) k_flux(int ny, double dl, int kind, const 
   if (threadIdx.x == 0) out[0] = dl * part[0];
 }
 
+namespace {
+// The kind of a factor handed to a solve: as the caller says (FDFD_FACTOR_ND,
+// or FDFD_FACTOR_STEPWISE / FDFD_FACTOR_PIVOT for a block factor), else by
+// its tag.
+int factor_is_nd(const fdfd_grid *g, const void *factor, int precision, hipStream_t s, bool *nd, NdPlan *P) {
+  *nd = false;
+  if (precision & (FDFD_FACTOR_STEPWISE | FDFD_FACTOR_PIVOT)) return FDFD_OK;
+  if (!nd_fits(g, P)) {
+    if (precision & FDFD_FACTOR_ND) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
+    return FDFD_OK;
+  }
+  if (precision & FDFD_FACTOR_ND) { *nd = true; return FDFD_OK; }
+  return nd_is_factor(factor, s, nd);
+}
+}  // namespace
+
 // =================================================================== C ABI
 extern "C" {
 
@@ -3611,10 +3636,20 @@ size_t fdfd_op_bytes(const fdfd_grid *g) {
 }
 size_t fdfd_factor_bytes(const fdfd_grid *g, int precision) {
   if (check_grid(g) || check_prec(precision)) return 0;
+  if (precision & FDFD_FACTOR_ND) {
+    NdPlan P;
+    if (!nd_fits(g, &P)) { fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range"); return 0; }
+    return nd_factor_bytes(g, P, precision);
+  }
   return factor_total_bytes(g, precision);
 }
 size_t fdfd_factor_workspace_bytes(const fdfd_grid *g, int precision) {
   if (check_grid(g) || check_prec(precision)) return 0;
+  if (precision & FDFD_FACTOR_ND) {
+    NdPlan P;
+    if (!nd_fits(g, &P)) { fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range"); return 0; }
+    return nd_work_layout(P, precision).total;
+  }
   return factor_work_bytes(g, precision);
 }
 size_t fdfd_solve_workspace_bytes(const fdfd_grid *g, int precision, int nrhs) {
@@ -3694,6 +3729,8 @@ int fdfd_factor(const fdfd_grid *g, const double *op, void *factor, int precisio
   if (!op || !factor || !work) return fail(FDFD_ERR_ARG, "bad arguments to fdfd_factor");
   const bool piv = precision & FDFD_FACTOR_PIVOT;
   const bool fp64 = base_prec(precision) == FDFD_PREC_FP64;
+  if (precision & FDFD_FACTOR_ND)
+    return fp64 ? nd_factor<double>(g, op, factor, work, stream) : nd_factor<float>(g, op, factor, work, stream);
   bool ran = false;
   // the persistent kernel factors one chain; a twisted factorization is stepwise
   if (!(precision & FDFD_FACTOR_STEPWISE) && twist_block(g) == g->nx - 1) {
@@ -3717,7 +3754,7 @@ int fdfd_factor(const fdfd_grid *g, const double *op, void *factor, int precisio
 int fdfd_factor_batch(const fdfd_grid *g, const double *const *ops, void *const *factors, int njobs,
                       int precision, void *const *works, hipStream_t stream) {
   if (int rc = check_grid(g)) return rc;
-  if (int rc = check_prec(precision)) return rc;
+  if (int rc = check_prec_block(precision)) return rc;
   if (!ops || !factors || !works || njobs < 1 || njobs > MAX_BATCH)
     return fail(FDFD_ERR_ARG, "bad arguments to fdfd_factor_batch (1 <= njobs <= %d)", MAX_BATCH);
   for (int j = 0; j < njobs; ++j)
@@ -3739,7 +3776,7 @@ int fdfd_factor_batch(const fdfd_grid *g, const double *const *ops, void *const 
 int fdfd_factor_wrap(const fdfd_grid *g, const double *op, void *factor, int precision, void *work,
                      hipStream_t stream) {
   if (int rc = check_grid(g)) return rc;
-  if (int rc = check_prec(precision)) return rc;
+  if (int rc = check_prec_block(precision)) return rc;
   if (!op || !factor || !work) return fail(FDFD_ERR_ARG, "bad arguments to fdfd_factor_wrap");
   const bool piv = precision & FDFD_FACTOR_PIVOT;
   return base_prec(precision) == FDFD_PREC_FP64 ? wrap_setup<double>(g, op, factor, work, piv, stream)
@@ -3763,6 +3800,18 @@ int fdfd_sweep(const fdfd_grid *g, const double *op, const void *factor, int pre
   if (int rc = check_grid(g)) return rc;
   if (int rc = check_prec(precision)) return rc;
   if (!op || !factor || !r || !x || !work || nrhs < 1) return fail(FDFD_ERR_ARG, "bad arguments to fdfd_sweep");
+  bool nd = false;
+  NdPlan P;
+  if (int rc = factor_is_nd(g, factor, precision, stream, &nd, &P)) return rc;
+  if (nd) {
+    const NdSolveWork w = nd_solve_layout(P, precision, nrhs);
+    int rc = base_prec(precision) == FDFD_PREC_FP64
+                 ? nd_sweep<double>(P, g, factor, r, x, nrhs, 1, (char *)work, w, stream)
+                 : nd_sweep<float>(P, g, factor, r, x, nrhs, 1, (char *)work, w, stream);
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(stream));
+    return FDFD_OK;
+  }
   SolveWork sw = solve_work_layout(g, precision, nrhs, work);
   HIP_TRY(hipMemsetAsync(sw.sync, 0, sizeof(SweepSync), stream));
   int rc = base_prec(precision) == FDFD_PREC_FP64
@@ -3805,6 +3854,13 @@ namespace {
 int solve_impl(const fdfd_grid *g, const double *op, const void *factor, int precision, const double *b,
                double *x, int nrhs, int transpose, double tol, int max_iter, void *work,
                fdfd_solve_stats *stats, double *rel_res, hipStream_t stream, double *host) {
+  bool nd = false;
+  NdPlan P;
+  if (int rc = factor_is_nd(g, factor, precision, stream, &nd, &P)) return rc;
+  if (nd)
+    return base_prec(precision) == FDFD_PREC_FP64
+               ? nd_solve<double>(g, op, factor, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res, stream, host)
+               : nd_solve<float>(g, op, factor, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res, stream, host);
   SolveWork sw = solve_work_layout(g, precision, nrhs, work);
   const size_t M = (size_t)g->nx * g->ny;
   const dim3 sgrid((g->ny + NT - 1) / NT, g->nx);
@@ -4053,7 +4109,7 @@ int fdfd_engine_submit(fdfd_engine *E, const fdfd_grid *g, const double *op, voi
                        void *work, uint64_t *ticket) {
   if (!E || !ticket) return fail(FDFD_ERR_ARG, "bad arguments to fdfd_engine_submit");
   if (int rc = check_grid(g)) return rc;
-  if (int rc = check_prec(precision)) return rc;
+  if (int rc = check_prec_block(precision)) return rc;
   if (!op || !factor || !work) return fail(FDFD_ERR_ARG, "bad arguments to fdfd_engine_submit");
   auto e = std::make_shared<EngineJob>();
   e->g = *g; e->op = op; e->factor = factor; e->work = work;
@@ -4117,6 +4173,45 @@ int fdfd_set_twist(int on) { return g_twist.exchange(on ? 1 : 0); }
 int fdfd_twist_block(const fdfd_grid *g) {
   if (check_grid(g)) return -1;
   return twist_block(g);
+}
+
+int fdfd_nd_supported(const fdfd_grid *g) {
+  NdPlan P;
+  if (check_grid(g)) return -1;
+  return g_twist.load() && nd_fits(g, &P) ? 1 : 0;
+}
+
+int fdfd_nd_front(const fdfd_grid *g, int level, int box, int32_t *info, int64_t *cells, int32_t *map) {
+  if (int rc = check_grid(g)) return rc;
+  NdPlan P;
+  if (!info || !nd_fits(g, &P)) return fail(FDFD_ERR_ARG, "fdfd_nd_front: bad arguments, or a grid outside its range");
+  NdLevel L;
+  memset(&L, 0, sizeof L);
+  if (level == -1) {
+    L.nx = P.nx; L.ny = P.ny; L.dx = P.Dx; L.dy = P.Dy; L.nbox = P.nleaf;
+  } else if (level >= 0 && level <= P.nlev) {
+    L = P.lev[level];
+  } else {
+    return fail(FDFD_ERR_ARG, "fdfd_nd_front: level %d outside -1..%d", level, P.nlev);
+  }
+  if (box < 0 || box >= L.nbox) return fail(FDFD_ERR_ARG, "fdfd_nd_front: box %d outside 0..%d", box, L.nbox - 1);
+  NdBox B = nd_box(L, box);
+  if (level == -1) B.s = B.w * B.h;
+  const int v[8] = {P.nlev, L.nbox, L.ax, B.s, B.b, B.k0, B.k1, level == -1 ? B.h : 0};
+  memcpy(info, v, sizeof v);
+  for (int j = 0; cells && j < B.s + B.b; ++j) {
+    if (j >= B.s) cells[j] = (int64_t)nd_border_cell(P.nx, P.ny, L.dx, L.dy, B, j - B.s);
+    else if (level == -1) cells[j] = (int64_t)(B.x0 + j / B.h) * P.ny + B.y0 + j % B.h;
+    else cells[j] = (int64_t)nd_sep_cell(L, B, j);
+  }
+  for (int j = 0; map && level >= 0 && j < B.s + B.b; ++j) {
+    int m0, m1;
+    if (j < B.s) nd_sep_map(L, B, j, m0, m1);
+    else nd_border_map(L, B, j - B.s, m0, m1);
+    map[2 * j] = m0;
+    map[2 * j + 1] = m1;
+  }
+  return FDFD_OK;
 }
 
 int fdfd_selftest_mfma(int precision, const double *a, const double *b, double *d, hipStream_t stream) {

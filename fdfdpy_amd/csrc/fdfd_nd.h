@@ -1,0 +1,1546 @@
+// fdfd_nd.h -- nested-dissection (multifrontal) direct solver of the whole
+// periodic operator, included by fdfd_hip.hip after its tile helpers.
+//
+// The block sweep of fdfd_hip.hip is serial in the long axis: m n/32 dependent
+// pivot steps to factor, m dependent blocks per sweep, 8 m n^3 flops. Here the
+// cells are ordered by nested dissection on a regular tree: about 5n/32
+// dependent pivot steps on an n x n grid, two launches per tree level per
+// sweep, and O(n^3) flops.
+//
+// Tree. Cell column 0 and cell row 0 (the cross) are the root separator, so
+// what is left, cells 1..nx-1 x 1..ny-1, is not periodic. A box is split by
+// its middle column or row (across its longer side) until it has at most
+// ND_LEAF cells. All boxes of one depth come from halving both axes the same
+// number of times, so their sides differ by at most one and every index
+// below is computed, not stored. The separator of a box and the ring of cells
+// around it (its border) form its front; the five-point stencil needs no
+// corners. At the top the two ends of an axis that has not been cut are the
+// same cells (the cross), and the border holds them once.
+//
+// Elimination. With E = diag(sqrt(sxf_i syf_j)) the matrix M = a E A E^-1 is
+// complex symmetric (a: a power of two that brings its entries near one).
+// For a box with front [[F_ss, F_sb], [F_sb^T, F_bb]] summed from its two
+// children's updates and its separator's own entries:
+//   X = F_ss^-1,  W = X F_sb,  C = F_bb - F_sb^T X F_sb  (to the parent).
+// X comes from the tiled Gauss-Jordan steps of the block factorization on
+// the upper tiles of [F_ss | F_sb]; C is one MFMA product per level.
+//
+// Solve. Upwards f_s = r_s + (children), z = X f_s, u = (children) - W^T f_s;
+// downwards x_s = z - W x_b. Everything is gathered by the reader in a fixed
+// order: no atomics, the same bits on every run.
+
+constexpr int ND_LEAF = 32;        // most cells of a leaf box: one pivot tile
+constexpr int ND_MIN_SIDE = 64;    // shorter grid side the path takes
+constexpr int ND_MAX_LEVELS = 40;
+constexpr size_t ND_HEADER = 256;  // the tag, at the start of the factor
+__host__ __device__ inline unsigned long long nd_tag(int i) {
+  return 0x6664666400000000ull + 0x9e3779b97f4a7c15ull * (unsigned long long)(i + 1);
+}
+
+// Segment idx of the interior 1..N-1 of an axis of N cells halved d times:
+// [a, a + len); the middle cell of a segment separates its halves.
+__host__ __device__ inline void nd_seg(int N, int d, int idx, int &a, int &len) {
+  a = 1;
+  len = N - 1;
+  for (int t = d - 1; t >= 0; --t) {
+    const int l = (len - 1) >> 1;
+    if ((idx >> t) & 1) { a += l + 1; len -= l + 1; }
+    else len = l;
+  }
+}
+inline int nd_longest(int N, int d) {
+  int len = N - 1;
+  for (int t = 0; t < d; ++t) len -= 1 + ((len - 1) >> 1);
+  return len;
+}
+
+// One merge level: boxes of depth (dx, dy), split along axis ax (0: by a
+// column, into halves of depth dx + 1). s, b: the largest separator and
+// border; sp, bp: padded to tiles; cbp: the children's bp.
+struct NdLevel {
+  int nx, ny, dx, dy, ax, root;
+  int s, b, sp, bp, nbox;
+  int cb, cbp;         // the children's b and bp
+  size_t xoff, woff;   // X [nbox][2][sp][sp] and W [nbox][2][sp][bp] in the factor's data (elements)
+};
+struct NdPlan {
+  int nx, ny, nlev, Dx, Dy, nleaf, leaf_b, leaf_bp;
+  NdLevel lev[ND_MAX_LEVELS];   // from the leaves' parents to the top box, then the root (lev[nlev])
+  size_t leaf_off, leafc_off, elems;
+};
+
+// false: the grid is outside the path's range
+bool nd_plan(const fdfd_grid *g, NdPlan *P) {
+  memset(P, 0, sizeof *P);
+  const int nx = g->nx, ny = g->ny;
+  if (std::min(nx, ny) < ND_MIN_SIDE) return false;
+  P->nx = nx;
+  P->ny = ny;
+  NdLevel down[ND_MAX_LEVELS];
+  int dx = 0, dy = 0, n = 0;
+  for (;;) {
+    const int w = nd_longest(nx, dx), h = nd_longest(ny, dy);
+    if (w * (long)h <= ND_LEAF) break;
+    if (n >= ND_MAX_LEVELS - 1) return false;
+    NdLevel &L = down[n++];
+    memset(&L, 0, sizeof L);
+    L.nx = nx; L.ny = ny; L.dx = dx; L.dy = dy;
+    L.ax = w >= h ? 0 : 1;
+    L.s = L.ax == 0 ? h : w;
+    L.b = (dx ? 2 : 1) * h + (dy ? 2 : 1) * w;
+    L.sp = pad_n(L.s);
+    L.bp = pad_n(L.b);
+    L.nbox = 1 << (dx + dy);
+    if (L.ax == 0) ++dx;
+    else ++dy;
+  }
+  if (!dx || !dy || dx + dy > 26) return false;
+  P->Dx = dx;
+  P->Dy = dy;
+  P->nleaf = 1 << (dx + dy);
+  P->leaf_b = 2 * (nd_longest(nx, dx) + nd_longest(ny, dy));
+  P->leaf_bp = TB;
+  if (P->leaf_b > TB) return false;
+  P->nlev = n;
+  // leaves: X [nleaf][2][TB][TB], then the border couplings [nleaf][TB] complex
+  size_t off = 0;
+  P->leaf_off = off;  off += (size_t)P->nleaf * 2 * TB * TB;
+  P->leafc_off = off; off += (size_t)P->nleaf * TB * 2;
+  for (int i = 0; i < n; ++i) {
+    NdLevel &L = P->lev[i] = down[n - 1 - i];
+    L.cb = i == 0 ? P->leaf_b : P->lev[i - 1].b;
+    L.cbp = i == 0 ? P->leaf_bp : P->lev[i - 1].bp;
+    L.xoff = off; off += (size_t)L.nbox * 2 * L.sp * L.sp;
+    L.woff = off; off += (size_t)L.nbox * 2 * L.sp * L.bp;
+  }
+  NdLevel &R = P->lev[n];
+  R.nx = nx; R.ny = ny; R.root = 1; R.nbox = 1;
+  R.s = nx + ny - 1;
+  R.sp = pad_n(R.s);
+  R.cb = P->lev[n - 1].b;
+  R.cbp = P->lev[n - 1].bp;
+  R.xoff = R.woff = off;
+  off += 2 * (size_t)R.sp * R.sp;
+  P->elems = off;
+  return true;
+}
+
+// Factor buffer: the tag, the tables E_x, 1/E_x [nx], E_y, 1/E_y [ny]
+// (complex FP64), then the data of the plan.
+inline size_t nd_data_off(const NdPlan &P) { return ND_HEADER + align_up(32 * (size_t)(P.nx + P.ny), 256); }
+// Never the size of a block factor of the grid: a buffer's size names its kind.
+inline size_t nd_factor_bytes(const fdfd_grid *g, const NdPlan &P, int precision) {
+  const size_t n = nd_data_off(P) + align_up(P.elems * elem_size(precision), 256);
+  return n == factor_total_bytes(g, base_prec(precision)) ? n + 256 : n;
+}
+// Factor workspace (after the status header): the scaled bands, the pivot
+// inverses of two steps, the ping-pong pairs of [F_ss] and [F_sb], the panels
+// U and R of the elimination (k_nd_step), the updates C of two levels.
+struct NdWork {
+  size_t bands, pinv[2], S[2], B[2], U, R, C[2], total;
+};
+NdWork nd_work_layout(const NdPlan &P, int precision) {
+  const size_t es = elem_size(precision), M = (size_t)P.nx * P.ny;
+  size_t boxes = 0, ss = 0, sb = 0, sb1 = 0, cc = (size_t)P.nleaf * P.leaf_bp * P.leaf_bp;
+  for (int i = 0; i <= P.nlev; ++i) {
+    const NdLevel &L = P.lev[i];
+    boxes = std::max(boxes, (size_t)L.nbox);
+    if (L.sp > TB) ss = std::max(ss, (size_t)L.nbox * L.sp * L.sp);
+    sb = std::max(sb, (size_t)L.nbox * L.sp * L.bp);
+    if (L.sp > TB) sb1 = std::max(sb1, (size_t)L.nbox * L.sp * L.bp);
+    cc = std::max(cc, (size_t)L.nbox * L.bp * L.bp);
+  }
+  NdWork w;
+  size_t off = WORK_HEADER;
+  auto take = [&](size_t bytes) { const size_t at = off; off += align_up(bytes, 256); return at; };
+  w.bands = take(3 * 2 * M * es);
+  for (int i = 0; i < 2; ++i) w.pinv[i] = take(boxes * 2 * TB * TB * es);
+  for (int i = 0; i < 2; ++i) w.S[i] = take(2 * ss * es);
+  for (int i = 0; i < 2; ++i) w.B[i] = take(2 * sb1 * es);
+  w.U = take(2 * sb * es);
+  w.R = take(2 * sb1 * es);
+  for (int i = 0; i < 2; ++i) w.C[i] = take(2 * cc * es);
+  w.total = off;
+  return w;
+}
+// Scale of M: 2^-e with the stencil's size 4 / (mu0' h^2) (Ez) or 4 /
+// (eps0' h^2) (Hz) brought to [0.5, 1)
+inline double nd_alpha(const fdfd_grid *g) {
+  const double h = g->dl, c = 4.0 / ((g->pol == FDFD_POL_EZ ? MU_0 : EPSILON_0) * g->L0 * h * h);
+  int e = 0;
+  (void)frexp(c, &e);
+  return ldexp(1.0, -e);
+}
+
+// -------------------------------------------------------- box geometry
+struct NdBox {
+  int x0, w, y0, h;   // interior
+  int k0, k1;         // the children's numbers
+  int c0, c1;         // the children's lengths along the split axis
+  int s, b;           // separator and border
+  int oB, oT;         // where the border's row sections start (L at 0, R at h)
+};
+__host__ __device__ inline NdBox nd_box(const NdLevel &L, int k) {
+  NdBox B;
+  if (L.root) {
+    B.x0 = 1; B.w = L.nx - 1; B.y0 = 1; B.h = L.ny - 1;
+    B.k0 = 0; B.k1 = 0; B.c0 = B.c1 = 0;
+    B.s = L.s; B.b = 0; B.oB = B.oT = 0;
+    return B;
+  }
+  const int ix = k >> L.dy, iy = k & ((1 << L.dy) - 1);
+  nd_seg(L.nx, L.dx, ix, B.x0, B.w);
+  nd_seg(L.ny, L.dy, iy, B.y0, B.h);
+  const int len = L.ax == 0 ? B.w : B.h;
+  B.c0 = (len - 1) >> 1;
+  B.c1 = len - 1 - B.c0;
+  if (L.ax == 0) {
+    B.k0 = ((2 * ix) << L.dy) + iy;
+    B.k1 = B.k0 + (1 << L.dy);
+    B.s = B.h;
+  } else {
+    B.k0 = (ix << (L.dy + 1)) + 2 * iy;
+    B.k1 = B.k0 + 1;
+    B.s = B.w;
+  }
+  B.oB = (L.dx ? 2 : 1) * B.h;
+  B.oT = B.oB + B.w;
+  B.b = B.oB + (L.dy ? 2 : 1) * B.w;
+  return B;
+}
+// cell of separator entry j
+__host__ __device__ inline size_t nd_sep_cell(const NdLevel &L, const NdBox &B, int j) {
+  if (L.root) {
+    const int h = L.ny - 1, w = L.nx - 1;
+    return j < h ? (size_t)(j + 1) : (j < h + w ? (size_t)(j - h + 1) * L.ny : (size_t)0);
+  }
+  return L.ax == 0 ? (size_t)(B.x0 + B.c0) * L.ny + B.y0 + j : (size_t)(B.x0 + j) * L.ny + B.y0 + B.c0;
+}
+// cell of border entry j of a box of depth (dx, dy)
+__host__ __device__ inline size_t nd_border_cell(int nx, int ny, int dx, int dy, const NdBox &B, int j) {
+  if (j < B.h) return (size_t)(B.x0 - 1) * ny + B.y0 + j;
+  j -= B.h;
+  if (dx) {
+    if (j < B.h) return (size_t)(B.x0 + B.w == nx ? 0 : B.x0 + B.w) * ny + B.y0 + j;
+    j -= B.h;
+  }
+  if (j < B.w) return (size_t)(B.x0 + j) * ny + B.y0 - 1;
+  return (size_t)(B.x0 + j - B.w) * ny + (B.y0 + B.h == ny ? 0 : B.y0 + B.h);
+}
+// entry of each child's border (-1: none) for separator entry j
+__host__ __device__ inline void nd_sep_map(const NdLevel &L, const NdBox &B, int j, int &m0, int &m1) {
+  if (L.root) {   // the top box's border is the cross in the root's order, without the corner
+    m0 = j < L.s - 1 ? j : -1;
+    m1 = -1;
+  } else if (L.ax == 0) {
+    m0 = B.h + j;
+    m1 = j;
+  } else {
+    const int sides = L.dx ? 2 : 1;
+    m0 = sides * B.c0 + B.w + j;
+    m1 = sides * B.c1 + j;
+  }
+}
+// ... for border entry j
+__host__ __device__ inline void nd_border_map(const NdLevel &L, const NdBox &B, int j, int &m0, int &m1) {
+  const int h = B.h, w = B.w;
+  if (L.ax == 0) {
+    if (j < h) { m0 = j; m1 = L.dx ? -1 : h + j; return; }
+    if (L.dx && j < 2 * h) { m0 = -1; m1 = j; return; }
+    const int t = j >= B.oT ? 1 : 0, i = j - (t ? B.oT : B.oB);
+    m0 = i < B.c0 ? 2 * h + (t ? B.c0 : 0) + i : -1;
+    m1 = i > B.c0 ? 2 * h + (t ? B.c1 : 0) + i - B.c0 - 1 : -1;
+  } else {
+    if (j < B.oB) {
+      const int r = j >= h ? 1 : 0, i = j - (r ? h : 0);
+      m0 = i < B.c0 ? (r ? B.c0 : 0) + i : -1;
+      m1 = i > B.c0 ? (r ? B.c1 : 0) + i - B.c0 - 1 : -1;
+      return;
+    }
+    const int sides = L.dx ? 2 : 1, o0 = sides * B.c0, o1 = sides * B.c1;
+    if (j < B.oT) { m0 = o0 + j - B.oB; m1 = L.dy ? -1 : o1 + w + j - B.oB; return; }
+    m0 = -1;
+    m1 = o1 + w + j - B.oT;
+  }
+}
+
+// ------------------------------------------------------------- factor
+// Scaled bands: planes [3][nx ny] of complex T, the diagonal and the
+// couplings to (i+1, j) and (i, j+1).
+template <typename T> struct NdBands {
+  const T *c, *x, *y;
+};
+template <typename T>
+__device__ inline void nd_ld(const T *p, size_t at, T &re, T &im) {
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  const t2 v = *reinterpret_cast<const t2 *>(p + 2 * at);
+  re = v.x;
+  im = v.y;
+}
+template <typename T>
+__device__ inline void nd_st(T *p, size_t at, T re, T im) {
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  *reinterpret_cast<t2 *>(p + 2 * at) = t2{re, im};
+}
+
+// Square root of s = 1 - i sigma
+__device__ inline cd nd_sqrt(cd s) {
+  const double re = sqrt(0.5 * (sqrt(s.r * s.r + s.i * s.i) + s.r));
+  return {re, s.i / (2 * re)};
+}
+// The factor's tag and tables; clears the status word and the bytes [gap0,
+// data) and [gap1, end) of the factor that hold nothing (its bits are a
+// function of the operator).
+__global__ void __launch_bounds__(NT) k_nd_tables(fdfd_grid g, unsigned long long *head, double *tab, int *status,
+                                                  size_t gap0, size_t data, size_t gap1, size_t end) {
+  const int t = blockIdx.x * NT + threadIdx.x, nx = g.nx, ny = g.ny;
+  if (t < (int)(ND_HEADER / 8)) head[t] = nd_tag(t);
+  if (t == 0) *status = 0;
+  unsigned char *bytes = reinterpret_cast<unsigned char *>(head);
+  if (t < 512) {
+    if (gap0 + t < data) bytes[gap0 + t] = 0;
+    if (gap1 + t < end) bytes[gap1 + t] = 0;
+  }
+  if (t >= nx + ny) return;
+  const bool xa = t < nx;
+  const int i = xa ? t : t - nx, n = xa ? nx : ny;
+  const double h = ((double)n * g.dl) / n;
+  const cd e = nd_sqrt(sfactor(0, i, n, xa ? g.npml_x : g.npml_y, h, g.omega, g.L0));
+  double *ex = tab, *iex = tab + 2 * (size_t)nx, *ey = tab + 4 * (size_t)nx, *iey = ey + 2 * (size_t)ny;
+  st_c(xa ? ex : ey, i, e);
+  st_c(xa ? iex : iey, i, cinv(e));
+}
+struct NdTab {
+  const double *ex, *iex, *ey, *iey;
+};
+__host__ __device__ inline NdTab nd_tables(const double *tab, int nx, int ny) {
+  return NdTab{tab, tab + 2 * (size_t)nx, tab + 4 * (size_t)nx, tab + 4 * (size_t)nx + 2 * (size_t)ny};
+}
+
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_bands(int nx, int ny, double alpha, const double *__restrict__ op, NdTab tb,
+                                                 T *__restrict__ bands) {
+  const int j = blockIdx.x * NT + threadIdx.x, i = blockIdx.y;
+  if (j >= ny) return;
+  const size_t M = (size_t)nx * ny, p = (size_t)i * ny + j;
+  const int ip = i + 1 == nx ? 0 : i + 1, jp = j + 1 == ny ? 0 : j + 1;
+  const cd c = cscale(ld_c(op, FDFD_OP_C * M + p), alpha);
+  const cd x = cscale(cmul(ld_c(op, FDFD_OP_XP * M + p), cmul(ld_c(tb.ex, i), ld_c(tb.iex, ip))), alpha);
+  const cd y = cscale(cmul(ld_c(op, FDFD_OP_YP * M + p), cmul(ld_c(tb.ey, j), ld_c(tb.iey, jp))), alpha);
+  nd_st<T>(bands, p, (T)c.r, (T)c.i);
+  nd_st<T>(bands + 2 * M, p, (T)x.r, (T)x.i);
+  nd_st<T>(bands + 4 * M, p, (T)y.r, (T)y.i);
+}
+
+// Inverse of the TB x TB tile in (Ar, Ai), in place, by Gauss-Jordan with
+// 2 x 2 diagonal block pivots taken in the order of their size: each step
+// picks, of the adjacent pairs not yet taken, the block P with the largest
+// |det P| / max |P_ij| (about 1 / ||P^-1||). The fronts of interior boxes are
+// real and indefinite, and a fixed order meets small leading minors: on the
+// request stream's 512 x 512 grid the complex64 factor of seed 7 then does not
+// refine at all, against a contraction of 2e-4 per sweep with the picked
+// order (2e-4 too for row pivoting inside the tile). Diagonal pivots move no
+// rows, so the order costs only the choice: lane l of every wave forms det and
+// inverse of pair l % 16 while the others do, a maximum over 16 lanes (row
+// rotations) names the pair, and its inverse comes by readlane. Only the
+// upper triangle is read: the fronts stay symmetric to the last bit, without
+// which the rounding of a nearly resonant box (|X| ~ 10^3) grows by another
+// two digits on the way up.
+// Layout and exchange as in tile_inverse_diag.
+__device__ inline float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ inline double lane_value(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+__device__ inline unsigned row16_max(unsigned v) {
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));   // row_ror:8
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
+  return v;
+}
+template <typename T, typename LT>
+__device__ void tile_inverse_pairs(LT &L, int *status) {
+  static_assert(TB * TB == 4 * NT, "4 elements per thread");
+  static_assert(2 * sizeof(InvX<T>) <= offsetof(LT, mag), "exchange buffers overlay the tiles only");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int i = tid >> 3, c0 = (tid & 7) * 4;
+  T ar[4], ai[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {   // the upper triangle
+    const int x = min(i, c0 + q), y = max(i, c0 + q);
+    ar[q] = L.Ar[x][y];
+    ai[q] = L.Ai[x][y];
+  }
+  __syncthreads();   // every row is in registers before the exchange buffers cover Ar, Ai
+  InvX<T> *X = reinterpret_cast<InvX<T> *>(&L);
+  const int mine = lane & 15, d = 2 * mine;
+  bool bad = false, taken = false;
+#pragma unroll 2
+  for (int st = 0; st < TB / 2; ++st) {
+    InvX<T> &B = X[st & 1];
+    lds_st4(&B.r[i][c0], ar);
+    lds_st4(&B.i[i][c0], ai);
+    __syncthreads();
+    // this lane's pair: P, scaled by an exact power of two near 1 / max |P_ij|,
+    // and Q = P^-1 = adj(P') sc / det(P')
+    T p00r, p01r, p00i, p01i, p10r, p11r, p10i, p11i;
+    lds_ld2(&B.r[d][d], p00r, p01r);
+    lds_ld2(&B.i[d][d], p00i, p01i);
+    lds_ld2(&B.r[d + 1][d], p10r, p11r);
+    lds_ld2(&B.i[d + 1][d], p10i, p11i);
+    const T mx = fmax(fmax(fmax(fabs(p00r), fabs(p00i)), fmax(fabs(p01r), fabs(p01i))),
+                      fmax(fmax(fabs(p10r), fabs(p10i)), fmax(fabs(p11r), fabs(p11i))));
+    const T sc = exp_scale(mx);
+    const T a00r = p00r * sc, a00i = p00i * sc, a01r = p01r * sc, a01i = p01i * sc;
+    const T a10r = p10r * sc, a10i = p10i * sc, a11r = p11r * sc, a11i = p11i * sc;
+    const T dr = (a00r * a11r - a00i * a11i) - (a01r * a10r - a01i * a10i);
+    const T di = (a00r * a11i + a00i * a11r) - (a01r * a10i + a01i * a10r);
+    const T da = fabs(dr) + fabs(di);
+    const bool ok = da > T(0) && isfinite(da) && mx > T(0) && isfinite(mx);
+    const unsigned size = __float_as_uint(fabsf((float)(da * exp_scale(sc)))) & ~15u;
+    const unsigned key = row16_max(taken ? 0u : size + 16u + (unsigned)mine);
+    const int pick = __builtin_amdgcn_readfirstlane((int)(key & 15u)), j = 2 * pick;
+    T f0r, f1r, f0i, f1i, h0r[4], h0i[4], h1r[4], h1i[4];
+    lds_ld2(&B.r[i][j], f0r, f1r);
+    lds_ld2(&B.i[i][j], f0i, f1i);
+    lds_ld4(&B.r[j][c0], h0r);
+    lds_ld4(&B.i[j][c0], h0i);
+    lds_ld4(&B.r[j + 1][c0], h1r);
+    lds_ld4(&B.i[j + 1][c0], h1i);
+    // 1 / det: (dr - i di) / |det|^2 with det brought to [0.5, 1) by an exact scale
+    const T ds = exp_scale(fmax(fabs(dr), fabs(di)));
+    const T br = dr * ds, bi = di * ds;
+    const T rm = rcp_nr(br * br + bi * bi) * ds * sc;
+    const T er = br * rm, ei = -bi * rm;
+    const T q00r = lane_value(a11r * er - a11i * ei, pick), q00i = lane_value(a11r * ei + a11i * er, pick);
+    const T q01r = lane_value(-(a01r * er - a01i * ei), pick), q01i = lane_value(-(a01r * ei + a01i * er), pick);
+    const T q10r = lane_value(-(a10r * er - a10i * ei), pick), q10i = lane_value(-(a10r * ei + a10i * er), pick);
+    const T q11r = lane_value(a00r * er - a00i * ei, pick), q11i = lane_value(a00r * ei + a00i * er, pick);
+    if (!__builtin_amdgcn_readlane((int)ok, pick)) bad = true;
+    taken = taken || mine == pick;
+    // new row = base - g0 h0 - g1 h1: off the pivot rows base = row and
+    // g = [f0 f1] Q; on them base = 0 and g = -(row of Q)
+    T g0r = f0r * q00r - f0i * q00i + f1r * q10r - f1i * q10i;
+    T g0i = f0r * q00i + f0i * q00r + f1r * q10i + f1i * q10r;
+    T g1r = f0r * q01r - f0i * q01i + f1r * q11r - f1i * q11i;
+    T g1i = f0r * q01i + f0i * q01r + f1r * q11i + f1i * q11r;
+    const bool r0 = i == j, r1 = i == j + 1, prow = r0 || r1;
+    g0r = r0 ? -q00r : (r1 ? -q10r : g0r);
+    g0i = r0 ? -q00i : (r1 ? -q10i : g0i);
+    g1r = r0 ? -q01r : (r1 ? -q11r : g1r);
+    g1i = r0 ? -q01i : (r1 ? -q11i : g1i);
+    // the pivot columns: Q on the pivot rows, -g elsewhere
+    const T cjr = -g0r, cji = -g0i, ckr = -g1r, cki = -g1i;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const T xr0 = prow ? T(0) : ar[q], xi0 = prow ? T(0) : ai[q];
+      const T xr = xr0 - (g0r * h0r[q] - g0i * h0i[q]) - (g1r * h1r[q] - g1i * h1i[q]);
+      const T xi = xi0 - (g0r * h0i[q] + g0i * h0r[q]) - (g1r * h1i[q] + g1i * h1r[q]);
+      const int c = c0 + q;
+      ar[q] = c == j ? cjr : (c == j + 1 ? ckr : xr);
+      ai[q] = c == j ? cji : (c == j + 1 ? cki : xi);
+    }
+  }
+  __syncthreads();   // the last step's reads are done before Ar, Ai are written
+#pragma unroll
+  for (int q = 0; q < 4; ++q) { L.Ar[i][c0 + q] = ar[q]; L.Ai[i][c0 + q] = ai[q]; }
+  if (bad) *status = 1;
+  __syncthreads();
+}
+
+// A leaf box per workgroup: its five-point matrix (cells in (x, y) order,
+// identity beyond) inverted as one pivot tile; X, the border couplings c and
+// the update C[a][b] = -c_a X[p_a][p_b] c_b, p_a the cell inside border cell a.
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_leaf(int nx, int ny, int Dx, int Dy, NdBands<T> bd, T *__restrict__ X,
+                                                T *__restrict__ cpl, T *__restrict__ C, int *status) {
+  __shared__ Lds<T> L;
+  __shared__ T cr[TB], ci[TB];
+  __shared__ int cp[TB];
+  const int tid = threadIdx.x, k = blockIdx.x;
+  const int ix = k >> Dy, iy = k & ((1 << Dy) - 1);
+  int x0, w, y0, h;
+  nd_seg(nx, Dx, ix, x0, w);
+  nd_seg(ny, Dy, iy, y0, h);
+  const int s = w * h, b = 2 * (w + h);
+  const int a = tid >> 3, b0 = (tid & 7) * 4;
+  const int ai = a / h, aj = a % h;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int c = b0 + u;
+    T re = a == c ? T(1) : T(0), im = 0;
+    if (a < s && c < s) {
+      const int qi = c / h, qj = c % h;
+      const size_t pa = (size_t)(x0 + ai) * ny + y0 + aj, pc = (size_t)(x0 + qi) * ny + y0 + qj;
+      re = 0;
+      if (a == c) nd_ld(bd.c, pa, re, im);
+      else if (aj == qj && (ai + 1 == qi || qi + 1 == ai)) nd_ld(bd.x, ai < qi ? pa : pc, re, im);
+      else if (ai == qi && (aj + 1 == qj || qj + 1 == aj)) nd_ld(bd.y, aj < qj ? pa : pc, re, im);
+    }
+    L.Ar[a][c] = re;
+    L.Ai[a][c] = im;
+  }
+  if (tid < TB) {
+    T re = 0, im = 0;
+    int p = 0;
+    if (tid < h) {
+      p = tid;
+      nd_ld(bd.x, (size_t)(x0 - 1) * ny + y0 + tid, re, im);
+    } else if (tid < 2 * h) {
+      p = (w - 1) * h + tid - h;
+      nd_ld(bd.x, (size_t)(x0 + w - 1) * ny + y0 + tid - h, re, im);
+    } else if (tid < 2 * h + w) {
+      p = (tid - 2 * h) * h;
+      nd_ld(bd.y, (size_t)(x0 + tid - 2 * h) * ny + y0 - 1, re, im);
+    } else if (tid < b) {
+      p = (tid - 2 * h - w) * h + h - 1;
+      nd_ld(bd.y, (size_t)(x0 + tid - 2 * h - w) * ny + y0 + h - 1, re, im);
+    }
+    cr[tid] = re;
+    ci[tid] = im;
+    cp[tid] = p;
+    nd_st<T>(cpl, (size_t)k * TB + tid, re, im);
+  }
+  __syncthreads();
+  tile_inverse_pairs<T>(L, status);
+  T *Xk = X + (size_t)k * 2 * TB * TB, *Ck = C + (size_t)k * 2 * TB * TB;
+  store4(Xk + a * TB + b0, &L.Ar[a][b0]);
+  store4(Xk + TB * TB + a * TB + b0, &L.Ai[a][b0]);
+  T vr[4], vi[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int x = min(a, b0 + u), y = max(a, b0 + u);   // symmetric to the last bit
+    const T xr = L.Ar[cp[x]][cp[y]], xi = L.Ai[cp[x]][cp[y]];
+    const T tr = cr[x] * xr - ci[x] * xi, ti = cr[x] * xi + ci[x] * xr;
+    vr[u] = -(tr * cr[y] - ti * ci[y]);
+    vi[u] = -(tr * ci[y] + ti * cr[y]);
+  }
+  store4(Ck + a * TB + b0, vr);
+  store4(Ck + TB * TB + a * TB + b0, vi);
+}
+
+// Four consecutive entries (row i of the front, columns given by their
+// children's entries) summed from the children's updates.
+template <typename T>
+__device__ inline void nd_children(const NdLevel &L, const NdBox &B, const T *__restrict__ C, int r0, int r1,
+                                   const int (&c0)[4], const int (&c1)[4], T (&re)[4], T (&im)[4]) {
+  const size_t pl = (size_t)L.cbp * L.cbp;
+  const T *A0 = C + (size_t)B.k0 * 2 * pl + (size_t)(r0 < 0 ? 0 : r0) * L.cbp;
+  const T *A1 = C + (size_t)B.k1 * 2 * pl + (size_t)(r1 < 0 ? 0 : r1) * L.cbp;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    re[u] = 0;
+    im[u] = 0;
+    if (r0 >= 0 && c0[u] >= 0) { re[u] = A0[c0[u]]; im[u] = A0[pl + c0[u]]; }
+    if (r1 >= 0 && c1[u] >= 0) { re[u] += A1[c1[u]]; im[u] += A1[pl + c1[u]]; }
+  }
+}
+// The entries of M itself between separator entries i and j
+template <typename T>
+__device__ inline void nd_own_ss(const NdLevel &L, const NdBox &B, const NdBands<T> &bd, int i, int j, T &re, T &im) {
+  re = 0;
+  im = 0;
+  if (i == j) { nd_ld(bd.c, nd_sep_cell(L, B, i), re, im); return; }
+  const int lo = min(i, j), hi = max(i, j);
+  if (!L.root) {
+    if (hi == lo + 1) nd_ld(L.ax == 0 ? bd.y : bd.x, nd_sep_cell(L, B, lo), re, im);
+    return;
+  }
+  // the cross: rows 1.. of column 0, columns 1.. of row 0, cell (0, 0)
+  const int h = L.ny - 1, n = L.s;
+  if (hi == n - 1) {
+    if (lo == 0) nd_ld(bd.y, 0, re, im);
+    else if (lo == h - 1) nd_ld(bd.y, (size_t)(L.ny - 1), re, im);
+    else if (lo == h) nd_ld(bd.x, 0, re, im);
+    else if (lo == n - 2) nd_ld(bd.x, (size_t)(L.nx - 1) * L.ny, re, im);
+  } else if (hi == lo + 1 && hi != h) {
+    nd_ld(lo < h ? bd.y : bd.x, nd_sep_cell(L, B, lo), re, im);
+  }
+}
+// ... between separator entry i and border entry j (the separator's ends)
+template <typename T>
+__device__ inline void nd_own_sb(const NdLevel &L, const NdBox &B, const NdBands<T> &bd, int i, int j, T &re, T &im) {
+  const int o = L.ax == 0 ? B.oB : 0, far = L.ax == 0 ? (L.dy ? B.w : 0) : (L.dx ? B.h : 0);
+  const T *p = L.ax == 0 ? bd.y : bd.x;
+  const size_t step = L.ax == 0 ? 1 : (size_t)L.ny;
+  if (i == 0 && j == o + B.c0) {
+    T r, m;
+    nd_ld(p, nd_sep_cell(L, B, 0) - step, r, m);
+    re += r;
+    im += m;
+  }
+  if (i == B.s - 1 && j == o + far + B.c0) {
+    T r, m;
+    nd_ld(p, nd_sep_cell(L, B, B.s - 1), r, m);
+    re += r;
+    im += m;
+  }
+}
+
+// Workgroup g of total items cut into XCDS equal ranges, one per XCD (the
+// dispatcher places workgroup b on XCD b % XCDS): neighbouring items, which
+// read the same rows and panels, share an L2. -1: past the end.
+__device__ inline int nd_item(int g, int total) {
+  const int x = g % XCDS, i = (int)((long)total * x / XCDS) + g / XCDS;
+  return i < (int)((long)total * (x + 1) / XCDS) ? i : -1;
+}
+inline int nd_grid(int total) { return XCDS * ((total + XCDS - 1) / XCDS); }
+
+template <typename T> struct NdStep {
+  NdLevel L;
+  NdBands<T> bd;
+  const T *C;              // the children's updates
+  const T *Ss, *Sb;        // [F_ss], [F_sb] before the step
+  T *Ds, *Db;              // after it
+  T *P0, *P1;              // pivot inverses of this step and the next
+  T *U, *R;                // rows of the border part as they are eliminated, before and after P
+  int *status;
+  int p;
+};
+
+// The front's [F_ss | F_sb] (tiles I <= J and the border's) from the
+// children, and the inverse of the first pivot tile.
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_front(NdStep<T> A) {
+  __shared__ Lds<T> S;
+  const NdLevel &L = A.L;
+  const int ns = L.sp / TB, nb = L.bp / TB, tri = ns * (ns + 1) / 2, per = tri + ns * nb;
+  int box, t;
+  if ((int)blockIdx.x < L.nbox) {       // the tiles inverted here go first
+    box = blockIdx.x;
+    t = 0;
+  } else {
+    const int first = (L.nbox + XCDS - 1) / XCDS * XCDS;
+    if ((int)blockIdx.x < first) return;
+    const int it = nd_item(blockIdx.x - first, L.nbox * (per - 1));
+    if (it < 0) return;
+    box = it / (per - 1);
+    t = 1 + it % (per - 1);
+  }
+  const NdBox B = nd_box(L, box);
+  int I, J;
+  if (t < tri) { const int e = upper_tile(ns, t); I = e / ns; J = e % ns; }
+  else { I = (t - tri) / nb; J = ns + (t - tri) % nb; }
+  const int tid = threadIdx.x, a = tid >> 3, b0 = (tid & 7) * 4;
+  const int i = I * TB + a;
+  T re[4], im[4];
+  int c0[4], c1[4], r0 = -1, r1 = -1;
+  if (i < B.s) nd_sep_map(L, B, i, r0, r1);
+  if (J < ns) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = J * TB + b0 + u;
+      c0[u] = c1[u] = -1;
+      if (j < B.s) nd_sep_map(L, B, j, c0[u], c1[u]);
+    }
+    nd_children(L, B, A.C, r0, r1, c0, c1, re, im);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = J * TB + b0 + u;
+      T mr = i == j ? T(1) : T(0), mi = 0;
+      if (i < B.s && j < B.s) nd_own_ss(L, B, A.bd, i, j, mr, mi);
+      re[u] += mr;
+      im[u] += mi;
+    }
+    if (t == 0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { S.Ar[a][b0 + u] = re[u]; S.Ai[a][b0 + u] = im[u]; }
+      __syncthreads();
+      tile_inverse_pairs<T>(S, A.status);
+      store_pinv(S, A.P0 + (size_t)box * 2 * TB * TB);
+      return;
+    }
+    T *D = A.Ds + (size_t)box * 2 * L.sp * L.sp + (size_t)i * L.sp + J * TB + b0;
+    store4(D, re);
+    store4(D + (size_t)L.sp * L.sp, im);
+  } else {
+    const int j0 = (J - ns) * TB + b0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      c0[u] = c1[u] = -1;
+      if (j0 + u < B.b) nd_border_map(L, B, j0 + u, c0[u], c1[u]);
+    }
+    nd_children(L, B, A.C, r0, r1, c0, c1, re, im);
+    if (i == 0 || i == B.s - 1)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) nd_own_sb(L, B, A.bd, i, j0 + u, re[u], im[u]);
+    T *D = A.U + (size_t)box * 2 * L.sp * L.bp + (size_t)i * L.bp + j0;
+    store4(D, re);
+    store4(D + (size_t)L.sp * L.bp, im);
+  }
+}
+
+// Gauss-Jordan step p on the tiles (I, J), I <= J < ns, and (I, J) of the
+// border (J >= ns), of every box, as in k_gj_step with D = 1:
+//   I == p == J: P;  I == p: P X[p,J];  J == p: -X[I,p] P;
+//   else X[I,J] - X[I,p] (P X[p,J]),
+// X[p,J] = -X[J,p]^T for J < p and X[I,p] = X[p,I]^T for I > p. The workgroup
+// of tile (p+1, p+1) inverts it for the next step; these start first. The
+// last step writes X and W into the factor, X with both triangles. The border
+// tiles of row p leave X[p,J] (U) and P X[p,J] (R) behind: the update is
+// C = F_bb - sum_p U_p^T R_p, as elimination forms it. (F_sb^T W with the
+// finished W loses the digits that a nearly resonant box costs twice: the
+// complex64 factor of a 512 x 512 stream grid with |X| = 550 in one box then
+// contracts by 0.03-0.2 per sweep instead of 2e-4.)
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
+  __shared__ Lds<T> S;
+  const NdLevel &L = A.L;
+  const int ns = L.sp / TB, nb = L.bp / TB, tri = ns * (ns + 1) / 2, per = tri + ns * nb, p = A.p;
+  const bool last = p == ns - 1;
+  const int ncrit = last ? 0 : L.nbox, first = (ncrit + XCDS - 1) / XCDS * XCDS;
+  int box, I, J;
+  bool crit = false;
+  if ((int)blockIdx.x < ncrit) {
+    box = blockIdx.x;
+    I = J = p + 1;
+    crit = true;
+    __builtin_amdgcn_s_setprio(3);
+  } else {
+    if ((int)blockIdx.x < first) return;
+    const int it = nd_item(blockIdx.x - first, L.nbox * per);
+    if (it < 0) return;
+    box = it / per;
+    const int t = it % per;
+    if (t < tri) { const int e = upper_tile(ns, t); I = e / ns; J = e % ns; }
+    else { I = (t - tri) / nb; J = ns + (t - tri) % nb; }
+    if (!last && I == p + 1 && J == p + 1) return;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, qi = wv >> 1, qj = wv & 1;
+  const int a = tid >> 3, b0 = (tid & 7) * 4;
+  const size_t sp = L.sp, bp = L.bp, ps = sp * sp, pb = sp * bp;
+  const T *Ss = A.Ss + (size_t)box * 2 * ps, *Sb = A.Sb + (size_t)box * 2 * pb;
+  const T *P = A.P0 + (size_t)box * 2 * TB * TB;
+  const bool row = I == p, col = J == p, mirA = J < p, mirB = I > p;
+  // every global read first: P, X[p,J], X[I,p] and the tile itself
+  T pr[4], pi[4], ar[4], ai[4], br[4], bi[4];
+  typename Mfma<T>::v4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+  ld_row4(P + a * TB + b0, pr);
+  ld_row4(P + TB * TB + a * TB + b0, pi);
+  if (!col) {
+    const T *q = J >= ns ? Sb + (p * TB + a) * bp + (size_t)(J - ns) * TB + b0
+                         : (mirA ? Ss + ((size_t)J * TB + a) * sp + p * TB + b0
+                                 : Ss + ((size_t)p * TB + a) * sp + J * TB + b0);
+    const size_t pl = J >= ns ? pb : ps;
+    ld_row4(q, ar);
+    ld_row4(q + pl, ai);
+  }
+  if (!row) {
+    const T *q = mirB ? Ss + ((size_t)p * TB + a) * sp + I * TB + b0 : Ss + ((size_t)I * TB + a) * sp + p * TB + b0;
+    ld_row4(q, br);
+    ld_row4(q + ps, bi);
+  }
+  if (!row && !col) {
+    const T *q = J >= ns ? Sb + (size_t)(J - ns) * TB : Ss + (size_t)J * TB;
+    const size_t pitch = J >= ns ? bp : sp, pl = J >= ns ? pb : ps;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const size_t e = (size_t)(I * TB + qi * 16 + Mfma<T>::crow(lane, t)) * pitch + qj * 16 + (lane & 15);
+      cr[t] = q[e];
+      ci[t] = q[pl + e];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int c = b0 + u;
+    S.Pr[a][c] = pr[u];
+    S.Pi[a][c] = pi[u];
+    if (!col) {
+      if (mirA) { S.Ar[c][a] = -ar[u]; S.Ai[c][a] = -ai[u]; }
+      else { S.Ar[a][c] = ar[u]; S.Ai[a][c] = ai[u]; }
+    }
+    if (!row) {
+      if (mirB) { S.Br[c][a] = br[u]; S.Bi[c][a] = bi[u]; }
+      else { S.Br[a][c] = br[u]; S.Bi[a][c] = bi[u]; }
+    }
+  }
+  __syncthreads();
+  if (row && col) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int x = qi * 16 + Mfma<T>::crow(lane, t), y = qj * 16 + (lane & 15);
+      cr[t] = S.Pr[x][y];
+      ci[t] = S.Pi[x][y];
+    }
+  } else if (col) {
+    cgemm_quad<T>(cr, ci, S.Br, S.Bi, S.Pr, S.Pi, qi, qj, lane, T(-1));
+  } else {
+    typename Mfma<T>::v4 rr = {0, 0, 0, 0}, ri = {0, 0, 0, 0};
+    cgemm_quad<T>(rr, ri, S.Pr, S.Pi, S.Ar, S.Ai, qi, qj, lane, T(1));
+    if (row) {
+      cr = rr;
+      ci = ri;
+    } else {
+      __syncthreads();   // every wave has read X[p,J]
+      acc_to_lds<T>(rr, ri, S.Ar, S.Ai, qi, qj, lane);
+      __syncthreads();
+      cgemm_quad<T>(cr, ci, S.Br, S.Bi, S.Ar, S.Ai, qi, qj, lane, T(-1));
+    }
+  }
+  // out through LDS as whole rows
+  __syncthreads();
+  acc_to_lds<T>(cr, ci, S.Ar, S.Ai, qi, qj, lane);
+  __syncthreads();
+  if (crit) {   // replaced by its inverse at the next step and read by nobody before
+    tile_inverse_pairs<T>(S, A.status);
+    store_pinv(S, A.P1 + (size_t)box * 2 * TB * TB);
+    return;
+  }
+  if (J >= ns) {
+    const size_t o = (size_t)box * 2 * pb + ((size_t)I * TB + a) * bp + (size_t)(J - ns) * TB + b0;
+    store4(A.Db + o, &S.Ar[a][b0]);
+    store4(A.Db + o + pb, &S.Ai[a][b0]);
+    if (row && ns > 1) {
+      store4(A.R + o, &S.Ar[a][b0]);
+      store4(A.R + o + pb, &S.Ai[a][b0]);
+      if (p > 0) {   // at p = 0 U holds F_sb itself
+        store4(A.U + o, ar);
+        store4(A.U + o + pb, ai);
+      }
+    }
+    return;
+  }
+  T *D = A.Ds + (size_t)box * 2 * ps;
+  store4(D + ((size_t)I * TB + a) * sp + J * TB + b0, &S.Ar[a][b0]);
+  store4(D + ps + ((size_t)I * TB + a) * sp + J * TB + b0, &S.Ai[a][b0]);
+  if (last && I != J) {
+    T mr[4], mi[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { mr[u] = S.Ar[b0 + u][a]; mi[u] = S.Ai[b0 + u][a]; }
+    store4(D + ((size_t)J * TB + a) * sp + I * TB + b0, mr);
+    store4(D + ps + ((size_t)J * TB + a) * sp + I * TB + b0, mi);
+  }
+}
+
+// c += sign * A^T[quadrant rows, :] * B[:, quadrant cols], both tiles stored
+// with the inner index as rows.
+template <typename T>
+__device__ inline void cgemm_quad_tn(typename Mfma<T>::v4 &cr, typename Mfma<T>::v4 &ci, const T (*Ar)[TBP],
+                                     const T (*Ai)[TBP], const T (*Br)[TBP], const T (*Bi)[TBP], int qi, int qj,
+                                     int lane, T sign) {
+  const int r = lane & 15, kq = lane >> 4;
+  const int k0 = (kq >> 1) + 16 * (kq & 1);
+#pragma unroll
+  for (int s = 0; s < TB / 4; ++s) {
+    const int k = 2 * s + k0;
+    const T ar = sign * Ar[k][qi * 16 + r], ai = sign * Ai[k][qi * 16 + r];
+    const T br = Br[k][qj * 16 + r], bi = Bi[k][qj * 16 + r];
+    cr = Mfma<T>::mac(ar, br, cr);
+    cr = Mfma<T>::mac(-ai, bi, cr);
+    ci = Mfma<T>::mac(ar, bi, ci);
+    ci = Mfma<T>::mac(ai, br, ci);
+  }
+}
+
+// C = F_bb - U^T R: one tile I <= J of one box per workgroup, stored with
+// its mirror image; F_bb is summed from the children as the tile is stored.
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_update(NdLevel L, const T *__restrict__ Cin, const T *__restrict__ U,
+                                                  const T *__restrict__ R, T *__restrict__ Cout) {
+  __shared__ T Ar[TB][TBP], Ai[TB][TBP], Br[TB][TBP], Bi[TB][TBP];
+  const int ns = L.sp / TB, nb = L.bp / TB, per = nb * (nb + 1) / 2;
+  const int it = nd_item(blockIdx.x, L.nbox * per);
+  if (it < 0) return;
+  const int box = it / per, e = upper_tile(nb, it % per), I = e / nb, J = e % nb;
+  const NdBox B = nd_box(L, box);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, qi = wv >> 1, qj = wv & 1;
+  const int a = tid >> 3, b0 = (tid & 7) * 4;
+  const size_t bp = L.bp, pb = (size_t)L.sp * bp;
+  const T *F = U + (size_t)box * 2 * pb + (size_t)a * bp + I * TB + b0;
+  const T *V = R + (size_t)box * 2 * pb + (size_t)a * bp + J * TB + b0;
+  T ar[4], ai[4], br[4], bi[4];
+  typename Mfma<T>::v4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+  ld_row4(F, ar);
+  ld_row4(F + pb, ai);
+  ld_row4(V, br);
+  ld_row4(V + pb, bi);
+  for (int k = 0; k < ns; ++k) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      Ar[a][b0 + u] = ar[u];
+      Ai[a][b0 + u] = ai[u];
+      Br[a][b0 + u] = br[u];
+      Bi[a][b0 + u] = bi[u];
+    }
+    __syncthreads();
+    if (k + 1 < ns) {
+      const size_t o = (size_t)(k + 1) * TB * bp;
+      ld_row4(F + o, ar);
+      ld_row4(F + o + pb, ai);
+      ld_row4(V + o, br);
+      ld_row4(V + o + pb, bi);
+    }
+    cgemm_quad_tn<T>(cr, ci, Ar, Ai, Br, Bi, qi, qj, lane, T(-1));
+    __syncthreads();
+  }
+  acc_to_lds<T>(cr, ci, Ar, Ai, qi, qj, lane);
+  int c0[4], c1[4], r0 = -1, r1 = -1;
+  if (I * TB + a < B.b) nd_border_map(L, B, I * TB + a, r0, r1);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    c0[u] = c1[u] = -1;
+    if (J * TB + b0 + u < B.b) nd_border_map(L, B, J * TB + b0 + u, c0[u], c1[u]);
+  }
+  T re[4], im[4];
+  nd_children(L, B, Cin, r0, r1, c0, c1, re, im);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    re[u] += Ar[a][b0 + u];
+    im[u] += Ai[a][b0 + u];
+  }
+  T *D = Cout + (size_t)box * 2 * bp * bp;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) { Ar[a][b0 + u] = re[u]; Ai[a][b0 + u] = im[u]; }
+  __syncthreads();
+  if (I == J) {   // a diagonal tile's lower triangle mirrors its upper one
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (b0 + u < a) { re[u] = Ar[b0 + u][a]; im[u] = Ai[b0 + u][a]; }
+  }
+  store4(D + ((size_t)I * TB + a) * bp + J * TB + b0, re);
+  store4(D + bp * bp + ((size_t)I * TB + a) * bp + J * TB + b0, im);
+  if (I == J) return;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) { re[u] = Ar[b0 + u][a]; im[u] = Ai[b0 + u][a]; }
+  store4(D + ((size_t)J * TB + a) * bp + I * TB + b0, re);
+  store4(D + bp * bp + ((size_t)J * TB + a) * bp + I * TB + b0, im);
+}
+
+template <typename T>
+int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hipStream_t s) {
+  const int prec = sizeof(T) == 8 ? FDFD_PREC_FP64 : FDFD_PREC_C64;
+  NdPlan P;
+  if (!nd_plan(g, &P)) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
+  const NdWork w = nd_work_layout(P, prec);
+  char *base = (char *)work;
+  double *tab = (double *)((char *)factor + ND_HEADER);
+  T *data = (T *)((char *)factor + nd_data_off(P));
+  int *status = (int *)base;
+  const size_t M = (size_t)P.nx * P.ny;
+  T *bands = (T *)(base + w.bands);
+  NdStep<T> A;
+  memset(&A, 0, sizeof A);
+  A.bd = NdBands<T>{bands, bands + 2 * M, bands + 4 * M};
+  A.U = (T *)(base + w.U);
+  A.R = (T *)(base + w.R);
+  A.status = status;
+  T *C[2] = {(T *)(base + w.C[0]), (T *)(base + w.C[1])};
+  T *S[2] = {(T *)(base + w.S[0]), (T *)(base + w.S[1])}, *Bf[2] = {(T *)(base + w.B[0]), (T *)(base + w.B[1])};
+  T *pv[2] = {(T *)(base + w.pinv[0]), (T *)(base + w.pinv[1])};
+  hipLaunchKernelGGL(k_nd_tables, dim3((std::max(P.nx + P.ny, 512) + NT - 1) / NT), dim3(NT), 0, s, *g,
+                     (unsigned long long *)factor, tab, status, ND_HEADER + 32 * (size_t)(P.nx + P.ny),
+                     nd_data_off(P), nd_data_off(P) + P.elems * sizeof(T), nd_factor_bytes(g, P, prec));
+  hipLaunchKernelGGL(k_nd_bands<T>, dim3((P.ny + NT - 1) / NT, P.nx), dim3(NT), 0, s, P.nx, P.ny, nd_alpha(g), op,
+                     nd_tables(tab, P.nx, P.ny), bands);
+  hipLaunchKernelGGL(k_nd_leaf<T>, dim3(P.nleaf), dim3(NT), 0, s, P.nx, P.ny, P.Dx, P.Dy, A.bd, data + P.leaf_off,
+                     data + P.leafc_off, C[0], status);
+  int cin = 0;
+  for (int l = 0; l <= P.nlev; ++l) {
+    const NdLevel &L = P.lev[l];
+    const int ns = L.sp / TB, nb = L.bp / TB, per = ns * (ns + 1) / 2 + ns * nb;
+    const int first = (L.nbox + XCDS - 1) / XCDS * XCDS;
+    A.L = L;
+    A.C = C[cin];
+    A.Ds = S[1];
+    A.P0 = pv[0];
+    hipLaunchKernelGGL(k_nd_front<T>, dim3(first + nd_grid(L.nbox * (per - 1))), dim3(NT), 0, s, A);
+    for (int p = 0; p < ns; ++p) {
+      const bool last = p == ns - 1;
+      A.p = p;
+      A.Ss = S[(p + 1) & 1];
+      A.Sb = p == 0 ? A.U : Bf[(p + 1) & 1];
+      A.Ds = last ? data + L.xoff : S[p & 1];
+      A.Db = last ? data + L.woff : Bf[p & 1];
+      A.P0 = pv[p & 1];
+      A.P1 = pv[(p + 1) & 1];
+      hipLaunchKernelGGL(k_nd_step<T>, dim3((last ? 0 : first) + nd_grid(L.nbox * per)), dim3(NT), 0, s, A);
+    }
+    if (L.root) break;
+    hipLaunchKernelGGL(k_nd_update<T>, dim3(nd_grid(L.nbox * (nb * (nb + 1) / 2))), dim3(NT), 0, s, L,
+                       (const T *)C[cin], (const T *)A.U, (const T *)(ns > 1 ? A.R : data + L.woff), C[cin ^ 1]);
+    cin ^= 1;
+  }
+  HIP_TRY(hipGetLastError());
+  return FDFD_OK;
+}
+
+// -------------------------------------------------------------- solve
+// Vectors of one pass of R right-hand sides: r and x (complex FP64, caller's
+// planes of nx ny), v (complex T, the same planes: z, then x, on the
+// separators), u (complex T, [box][R][pitch]: a level's updates).
+template <typename T> struct NdSolve {
+  NdLevel L;
+  NdTab tb;
+  double alpha;
+  const T *X, *W;       // this level's
+  const double *r;      // [q][M]
+  double *x;            // [q][M]
+  T *v;                 // [q][M]
+  const T *uin;         // the children's updates
+  T *uout;
+  int nq, add;          // right-hand sides of this pass; x += (else x =)
+};
+
+template <typename T>
+__device__ inline void nd_rhs(const NdSolve<T> &A, size_t cell, int q, T &re, T &im) {
+  const size_t M = (size_t)A.L.nx * A.L.ny;
+  const int i = (int)(cell / A.L.ny), j = (int)(cell % A.L.ny);
+  const cd e = cscale(cmul(ld_c(A.tb.ex, i), ld_c(A.tb.ey, j)), A.alpha);
+  const cd f = cmul(e, ld_c(A.r + 2 * M * q, cell));
+  re = (T)f.r;
+  im = (T)f.i;
+}
+template <typename T>
+__device__ inline void nd_out(const NdSolve<T> &A, size_t cell, int q, T re, T im) {
+  const size_t M = (size_t)A.L.nx * A.L.ny;
+  const int i = (int)(cell / A.L.ny), j = (int)(cell % A.L.ny);
+  const cd o = cmul(cmul(ld_c(A.tb.iex, i), ld_c(A.tb.iey, j)), cd{(double)re, (double)im});
+  double *x = A.x + 2 * M * q;
+  st_c(x, cell, A.add ? cadd(ld_c(x, cell), o) : o);
+}
+// separator entry j of the children's updates plus r, right-hand side q
+template <typename T>
+__device__ inline void nd_fs(const NdSolve<T> &A, const NdBox &B, int j, int q, T &re, T &im) {
+  nd_rhs(A, nd_sep_cell(A.L, B, j), q, re, im);
+  int m0, m1;
+  nd_sep_map(A.L, B, j, m0, m1);
+  T a, b;
+  if (m0 >= 0) { nd_ld(A.uin, ((size_t)B.k0 * A.nq + q) * A.L.cb + m0, a, b); re += a; im += b; }
+  if (m1 >= 0) { nd_ld(A.uin, ((size_t)B.k1 * A.nq + q) * A.L.cb + m1, a, b); re += a; im += b; }
+}
+
+// Upwards, one level (and the root, whose z is x): columns [64 c, 64 c + 64)
+// of [X | W] of one box per NW waves, which split the separator's rows.
+template <typename T, int R, int NW> struct NdUp {
+  static constexpr int TASKS = NW == 1 ? 4 : 1, THREADS = 64 * NW * TASKS;
+  static constexpr int JC = NW == 1 ? TB : 64 * NW;   // rows staged at a time
+  union Mem {
+    T f[TASKS][R][2][JC];
+    T red[NW][2 * R][64];
+  };
+};
+template <typename T, int R, int NW>
+__global__ void __launch_bounds__(64 * NW * (NW == 1 ? 4 : 1)) k_nd_up(NdSolve<T> A) {
+  typedef NdUp<T, R, NW> Cfg;
+  __shared__ typename Cfg::Mem S;
+  const NdLevel &L = A.L;
+  const int tid = threadIdx.x, lane = tid & 63, task = tid / (64 * NW), wv = (tid >> 6) % NW;
+  const int chunks = (L.sp + L.bp + 63) / 64;
+  const int id = blockIdx.x * Cfg::TASKS + task;
+  const bool live = id < L.nbox * chunks;
+  const int box = live ? id / chunks : 0, c = (live ? id % chunks : 0) * 64 + lane;
+  const NdBox B = nd_box(L, box);
+  const bool inX = c < L.sp, inW = !inX && c < L.sp + L.bp;
+  const size_t pitch = inX ? L.sp : L.bp, plane = (size_t)L.sp * pitch;
+  const T *m = inX ? A.X + (size_t)box * 2 * plane + c : A.W + (size_t)box * 2 * plane + (c - L.sp);
+  T ar[R], ai[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
+  for (int j0 = 0; j0 < B.s; j0 += Cfg::JC) {
+    const int nj = min(Cfg::JC, B.s - j0);
+    if (j0) __syncthreads();
+    for (int e = wv * 64 + lane; e < Cfg::JC * R; e += 64 * NW) {
+      const int q = e / Cfg::JC, j = e % Cfg::JC;
+      T fr = 0, fi = 0;
+      if (live && j < nj && q < A.nq) nd_fs(A, B, j0 + j, q, fr, fi);
+      S.f[task][q][0][j] = fr;
+      S.f[task][q][1][j] = fi;
+    }
+    __syncthreads();
+    if (inX || inW) {
+      const int per = (nj + NW - 1) / NW, ja = wv * per, jb = min(nj, ja + per);
+#pragma unroll 4
+      for (int j = ja; j < jb; ++j) {
+        const T gr = m[(size_t)(j0 + j) * pitch], gi = m[plane + (size_t)(j0 + j) * pitch];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const T fr = S.f[task][q][0][j], fi = S.f[task][q][1][j];
+          ar[q] += gr * fr - gi * fi;
+          ai[q] += gr * fi + gi * fr;
+        }
+      }
+    }
+  }
+  if (NW > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      S.red[wv][2 * q][lane] = ar[q];
+      S.red[wv][2 * q + 1][lane] = ai[q];
+    }
+    __syncthreads();
+  }
+  // wave w finishes right-hand sides w, w + NW, ...
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    if (q % NW != wv || q >= A.nq || !live) continue;
+    T sr = ar[q], si = ai[q];
+    if (NW > 1) {
+      sr = si = 0;
+      for (int t = 0; t < NW; ++t) { sr += S.red[t][2 * q][lane]; si += S.red[t][2 * q + 1][lane]; }
+    }
+    if (c < B.s) {
+      const size_t cell = nd_sep_cell(L, B, c);
+      nd_st<T>(A.v, (size_t)q * L.nx * L.ny + cell, sr, si);
+      if (L.root) nd_out(A, cell, q, sr, si);
+    } else if (inW && c - L.sp < B.b) {
+      const int j = c - L.sp;
+      int m0, m1;
+      nd_border_map(L, B, j, m0, m1);
+      T ur = 0, ui = 0, a, b;
+      if (m0 >= 0) { nd_ld(A.uin, ((size_t)B.k0 * A.nq + q) * L.cb + m0, a, b); ur += a; ui += b; }
+      if (m1 >= 0) { nd_ld(A.uin, ((size_t)B.k1 * A.nq + q) * L.cb + m1, a, b); ur += a; ui += b; }
+      nd_st<T>(A.uout, ((size_t)box * A.nq + q) * L.b + j, ur - sr, ui - si);
+    }
+  }
+}
+
+// Downwards, one level: x_s = z - W x_b. LPR lanes share a row: 64 (a box's
+// rows in groups of eight per workgroup) or 8 (separators of one tile: a box
+// per wave).
+template <typename T, int R, int LPR> struct NdDown {
+  static constexpr int RW = LPR == 64 ? 2 : 1;              // rows per LPR lanes
+  static constexpr int TASKS = LPR == 64 ? 1 : 4;           // boxes per workgroup
+  static constexpr int CC = LPR == 64 ? 256 : 96;           // border entries staged at a time
+  static constexpr int ROWS = LPR == 64 ? 8 : TB;           // rows of a task
+};
+template <typename T, int R, int LPR>
+__global__ void __launch_bounds__(NT) k_nd_down(NdSolve<T> A) {
+  typedef NdDown<T, R, LPR> Cfg;
+  __shared__ T S[Cfg::TASKS][R][2][Cfg::CC];
+  const NdLevel &L = A.L;
+  const size_t M = (size_t)L.nx * L.ny;
+  const int tid = threadIdx.x, task = LPR == 64 ? 0 : tid >> 6, tl = LPR == 64 ? tid : tid & 63;
+  constexpr int TT = NT / Cfg::TASKS;                        // threads of a task
+  const int groups = (L.s + Cfg::ROWS - 1) / Cfg::ROWS;
+  const int id = blockIdx.x * Cfg::TASKS + task;
+  const bool live = id < L.nbox * groups;
+  const int box = live ? id / groups : 0, g = live ? id % groups : 0;
+  const NdBox B = nd_box(L, box);
+  const size_t plane = (size_t)L.sp * L.bp;
+  const T *W = A.W + (size_t)box * 2 * plane;
+  constexpr int RPP = TT / LPR * Cfg::RW;                    // rows at a time
+  const int l = tl % LPR;
+  for (int q0 = 0; q0 < Cfg::ROWS && q0 < L.s; q0 += RPP) {
+    const int row = g * Cfg::ROWS + q0 + tl / LPR * Cfg::RW;
+    T ar[Cfg::RW][R], ai[Cfg::RW][R];
+#pragma unroll
+    for (int w = 0; w < Cfg::RW; ++w)
+#pragma unroll
+      for (int q = 0; q < R; ++q) { ar[w][q] = 0; ai[w][q] = 0; }
+    for (int b0 = 0; b0 < L.b; b0 += Cfg::CC) {
+      const bool restage = q0 == 0 || L.b > Cfg::CC;
+      if (restage) {
+        __syncthreads();
+        for (int e = tl; e < Cfg::CC * R; e += TT) {
+          const int q = e / Cfg::CC, c = e % Cfg::CC;
+          T xr = 0, xi = 0;
+          if (live && b0 + c < B.b && q < A.nq)
+            nd_ld(A.v, (size_t)q * M + nd_border_cell(L.nx, L.ny, L.dx, L.dy, B, b0 + c), xr, xi);
+          S[task][q][0][c] = xr;
+          S[task][q][1][c] = xi;
+        }
+        __syncthreads();
+      }
+      const int nc = min(Cfg::CC, L.bp - b0);   // W is zero beyond the border
+      const T *w0 = W + (size_t)min(row, L.sp - Cfg::RW) * L.bp + b0;
+#pragma unroll 4
+      for (int c = l; c < nc; c += LPR) {
+        T gr[Cfg::RW], gi[Cfg::RW];
+#pragma unroll
+        for (int w = 0; w < Cfg::RW; ++w) {
+          gr[w] = w0[(size_t)w * L.bp + c];
+          gi[w] = w0[plane + (size_t)w * L.bp + c];
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const T xr = S[task][q][0][c], xi = S[task][q][1][c];
+#pragma unroll
+          for (int w = 0; w < Cfg::RW; ++w) {
+            ar[w][q] += gr[w] * xr - gi[w] * xi;
+            ai[w][q] += gr[w] * xi + gi[w] * xr;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int w = 0; w < Cfg::RW; ++w)
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+#pragma unroll
+        for (int off = LPR / 2; off >= 1; off >>= 1) {
+          ar[w][q] += __shfl_xor(ar[w][q], off);
+          ai[w][q] += __shfl_xor(ai[w][q], off);
+        }
+        // lane (w R + q) % LPR of the row finishes this sum
+        if (l == (w * R + q) % LPR && live && row + w < B.s && q < A.nq) {
+          const size_t cell = nd_sep_cell(L, B, row + w);
+          T zr, zi;
+          nd_ld(A.v, (size_t)q * M + cell, zr, zi);
+          zr -= ar[w][q];
+          zi -= ai[w][q];
+          nd_st<T>(A.v, (size_t)q * M + cell, zr, zi);
+          nd_out(A, cell, q, zr, zi);
+        }
+      }
+  }
+}
+
+// The leaves, a box per wave: X is symmetric, so lane c of each half wave
+// sums its column over half of the rows. Upwards z = X r and the updates
+// -c_a z[p_a]; downwards x = X (r - F_sb x_b).
+template <typename T, int R, bool DOWN>
+__global__ void __launch_bounds__(NT) k_nd_leaf_solve(NdSolve<T> A, const T *__restrict__ cpl) {
+  __shared__ T S[4][R][2][TB], Z[4][R][2][TB];
+  const NdLevel &L = A.L;   // dx, dy: the leaves' depth
+  const size_t M = (size_t)L.nx * L.ny;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 31, half = lane >> 5;
+  const int k = blockIdx.x * 4 + wv;
+  const bool live = k < L.nbox;
+  const int kk = live ? k : 0, ix = kk >> L.dy, iy = kk & ((1 << L.dy) - 1);
+  int x0, w, y0, h;
+  nd_seg(L.nx, L.dx, ix, x0, w);
+  nd_seg(L.ny, L.dy, iy, y0, h);
+  const int s = w * h, b = 2 * (w + h);
+  const int ci = c / h, cj = c % h;
+  const size_t cell = (size_t)(x0 + ci) * L.ny + y0 + cj;
+  const T *cp = cpl + (size_t)kk * TB * 2;
+  for (int q = half; q < R; q += 2) {
+    T fr = 0, fi = 0;
+    if (live && c < s && q < A.nq) {
+      nd_rhs(A, cell, q, fr, fi);
+      if (DOWN) {
+        // the four border neighbours of an edge cell (entry order L, R, B, T)
+        const T *v = A.v + 2 * M * q;
+        T cr, cim, xr, xi;
+        auto take = [&](int e, size_t nb) {
+          nd_ld(cp, e, cr, cim);
+          nd_ld(v, nb, xr, xi);
+          fr -= cr * xr - cim * xi;
+          fi -= cr * xi + cim * xr;
+        };
+        if (ci == 0) take(cj, cell - L.ny);
+        if (ci == w - 1) take(h + cj, x0 + w == L.nx ? (size_t)(y0 + cj) : cell + L.ny);
+        if (cj == 0) take(2 * h + ci, cell - 1);
+        if (cj == h - 1) take(2 * h + w + ci, y0 + h == L.ny ? (size_t)(x0 + ci) * L.ny : cell + 1);
+      }
+    }
+    S[wv][q][0][c] = fr;
+    S[wv][q][1][c] = fi;
+  }
+  __syncthreads();
+  T ar[R], ai[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
+  const T *X = A.X + (size_t)kk * 2 * TB * TB + c;
+  const int sh = (s + 1) / 2, ja = half * sh, jb = half ? s : sh;
+#pragma unroll 4
+  for (int j = ja; j < jb; ++j) {
+    const T gr = X[j * TB], gi = X[TB * TB + j * TB];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const T fr = S[wv][q][0][j], fi = S[wv][q][1][j];
+      ar[q] += gr * fr - gi * fi;
+      ai[q] += gr * fi + gi * fr;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    ar[q] += __shfl_xor(ar[q], 32);
+    ai[q] += __shfl_xor(ai[q], 32);
+    if (DOWN) {
+      if (half == (q & 1) && live && c < s && q < A.nq) nd_out(A, cell, q, ar[q], ai[q]);
+    } else if (half == 0) {
+      Z[wv][q][0][c] = ar[q];
+      Z[wv][q][1][c] = ai[q];
+    }
+  }
+  if (DOWN) return;
+  __syncthreads();
+  for (int q = half; q < A.nq; q += 2) {
+    if (!live || c >= b) continue;
+    const int p = c < h ? c : c < 2 * h ? (w - 1) * h + c - h : c < 2 * h + w ? (c - 2 * h) * h : (c - 2 * h - w) * h + h - 1;
+    T cr, cim;
+    nd_ld(cp, c, cr, cim);
+    const T zr = Z[wv][q][0][p], zi = Z[wv][q][1][p];
+    nd_st<T>(A.uout, ((size_t)k * A.nq + q) * L.b + c, -(cr * zr - cim * zi), -(cr * zi + cim * zr));
+  }
+}
+
+// r = b' - A x with b' = b, or D^-1 b in the transposed solve, and per
+// right-hand side the partial sums of |r|^2 (weighted by |D|^2 in the
+// transposed solve). A null x: r = b' and the partial sums of |b|^2. Blocks
+// take every gridDim.x-th piece of a row.
+constexpr int ND_RES_RHS = 4;     // right-hand sides per thread (grid.y passes)
+__global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, const double *__restrict__ op,
+                                                    const double *__restrict__ b, const double *__restrict__ x,
+                                                    double *__restrict__ r, int nrhs, int transpose,
+                                                    double *__restrict__ part) {
+  __shared__ double red[ND_RES_RHS][NT];
+  const int nx = g.nx, ny = g.ny, tid = threadIdx.x, q0 = blockIdx.y * ND_RES_RHS;
+  const int nq = min(ND_RES_RHS, nrhs - q0), cpr = (ny + NT - 1) / NT;
+  const size_t M = (size_t)nx * ny;
+  double acc[ND_RES_RHS] = {0, 0, 0, 0};
+  for (int piece = blockIdx.x; piece < nx * cpr; piece += gridDim.x) {
+    const int i = piece / cpr, j = (piece % cpr) * NT + tid;
+    if (j >= ny) continue;
+    const size_t p = (size_t)i * ny + j;
+    cd dinv = {1, 0};
+    double w2 = 1;
+    if (transpose) {
+      const double hx = ((double)nx * g.dl) / nx, hy = ((double)ny * g.dl) / ny;
+      const cd d = cmul(sfactor(0, i, nx, g.npml_x, hx, g.omega, g.L0), sfactor(0, j, ny, g.npml_y, hy, g.omega, g.L0));
+      dinv = cinv(d);
+      w2 = d.r * d.r + d.i * d.i;
+    }
+    if (!x) {
+#pragma unroll
+      for (int q = 0; q < ND_RES_RHS; ++q)
+        if (q < nq) {
+          cd v = ld_c(b + 2 * M * (q0 + q), p);
+          acc[q] += v.r * v.r + v.i * v.i;
+          if (transpose) v = cmul(v, dinv);
+          st_c(r + 2 * M * (q0 + q), p, v);
+        }
+      continue;
+    }
+    const size_t pxm = (i == 0 ? p + M - ny : p - ny), pxp = (i + 1 == nx ? p + ny - M : p + ny);
+    const size_t pym = (j == 0 ? p + ny - 1 : p - 1), pyp = (j + 1 == ny ? p + 1 - ny : p + 1);
+    const cd c0 = ld_c(op, FDFD_OP_C * M + p), cxm = ld_c(op, FDFD_OP_XM * M + p), cxp = ld_c(op, FDFD_OP_XP * M + p);
+    const cd cym = ld_c(op, FDFD_OP_YM * M + p), cyp = ld_c(op, FDFD_OP_YP * M + p);
+#pragma unroll
+    for (int q = 0; q < ND_RES_RHS; ++q)
+      if (q < nq) {
+        const double *xq = x + 2 * M * (q0 + q);
+        cd a = cmul(c0, ld_c(xq, p));
+        a = cadd(a, cmul(cxm, ld_c(xq, pxm)));
+        a = cadd(a, cmul(cxp, ld_c(xq, pxp)));
+        a = cadd(a, cmul(cym, ld_c(xq, pym)));
+        a = cadd(a, cmul(cyp, ld_c(xq, pyp)));
+        cd v = ld_c(b + 2 * M * (q0 + q), p);
+        if (transpose) v = cmul(v, dinv);
+        v = csub(v, a);
+        acc[q] += w2 * (v.r * v.r + v.i * v.i);
+        st_c(r + 2 * M * (q0 + q), p, v);
+      }
+  }
+#pragma unroll
+  for (int q = 0; q < ND_RES_RHS; ++q) red[q][tid] = acc[q];
+  __syncthreads();
+  for (int st = NT / 2; st > 0; st >>= 1) {
+    if (tid < st)
+#pragma unroll
+      for (int q = 0; q < ND_RES_RHS; ++q) red[q][tid] += red[q][tid + st];
+    __syncthreads();
+  }
+  if (tid < nq) part[(size_t)(q0 + tid) * gridDim.x + blockIdx.x] = red[tid][0];
+}
+
+// right-hand sides of one pass over the factor
+template <typename T> constexpr int nd_rhs_per_pass() { return sizeof(T) == 8 ? 4 : 8; }
+// u of one right-hand side: the largest level's, complex T
+inline size_t nd_u_entries(const NdPlan &P) {
+  size_t n = (size_t)P.nleaf * P.leaf_b;
+  for (int i = 0; i < P.nlev; ++i) n = std::max(n, (size_t)P.lev[i].nbox * P.lev[i].b);
+  return n;
+}
+// Solve workspace: r, v and two u buffers of one pass, norm partials, norms.
+struct NdSolveWork {
+  size_t r, v, u[2], part, norms, total;
+};
+inline NdSolveWork nd_solve_layout(const NdPlan &P, int precision, int nrhs) {
+  const size_t M = (size_t)P.nx * P.ny, es = elem_size(precision);
+  const size_t R = std::min(nrhs, es == 8 ? nd_rhs_per_pass<double>() : nd_rhs_per_pass<float>());
+  NdSolveWork w;
+  size_t off = 0;
+  auto take = [&](size_t bytes) { const size_t at = off; off += align_up(bytes, 256); return at; };
+  w.r = take(16 * M * nrhs);
+  w.v = take(2 * es * M * R);
+  for (int i = 0; i < 2; ++i) w.u[i] = take(2 * es * nd_u_entries(P) * R);
+  w.part = take(8 * (size_t)2 * NORM_PARTS * nrhs);
+  w.norms = take(8 * 2 * (size_t)nrhs);
+  w.total = off;
+  return w;
+}
+
+// x (+)= A^-1 r for nq <= R right-hand sides
+template <typename T, int R>
+int nd_pass(const NdPlan &P, const NdTab &tb, double alpha, const T *data, const double *r, double *x, int nq, int add,
+            T *v, T *u0, T *u1, hipStream_t s) {
+  NdSolve<T> A;
+  memset(&A, 0, sizeof A);
+  A.tb = tb;
+  A.alpha = alpha;
+  A.r = r;
+  A.x = x;
+  A.v = v;
+  A.nq = nq;
+  A.add = add;
+  T *u[2] = {u0, u1};
+  NdLevel leaf;
+  memset(&leaf, 0, sizeof leaf);
+  leaf.nx = P.nx; leaf.ny = P.ny; leaf.dx = P.Dx; leaf.dy = P.Dy; leaf.nbox = P.nleaf; leaf.b = P.leaf_b;
+  A.L = leaf;
+  A.X = data + P.leaf_off;
+  A.uout = u[0];
+  hipLaunchKernelGGL((k_nd_leaf_solve<T, R, false>), dim3((P.nleaf + 3) / 4), dim3(NT), 0, s, A, data + P.leafc_off);
+  for (int l = 0; l <= P.nlev; ++l) {
+    const NdLevel &L = P.lev[l];
+    A.L = L;
+    A.X = data + L.xoff;
+    A.W = data + L.woff;
+    A.uin = u[l & 1];
+    A.uout = u[(l + 1) & 1];
+    const int tasks = L.nbox * ((L.sp + L.bp + 63) / 64);
+    if (L.sp <= TB)
+      hipLaunchKernelGGL((k_nd_up<T, R, 1>), dim3((tasks + 3) / 4), dim3(NdUp<T, R, 1>::THREADS), 0, s, A);
+    else if (L.sp <= 128)
+      hipLaunchKernelGGL((k_nd_up<T, R, 4>), dim3(tasks), dim3(NdUp<T, R, 4>::THREADS), 0, s, A);
+    else
+      hipLaunchKernelGGL((k_nd_up<T, R, 8>), dim3(tasks), dim3(NdUp<T, R, 8>::THREADS), 0, s, A);
+  }
+  for (int l = P.nlev - 1; l >= 0; --l) {
+    const NdLevel &L = P.lev[l];
+    A.L = L;
+    A.W = data + L.woff;
+    if (L.sp <= TB)
+      hipLaunchKernelGGL((k_nd_down<T, R, 8>), dim3((L.nbox + 3) / 4), dim3(NT), 0, s, A);
+    else
+      hipLaunchKernelGGL((k_nd_down<T, R, 64>), dim3(L.nbox * ((L.s + 7) / 8)), dim3(NT), 0, s, A);
+  }
+  A.L = leaf;
+  A.X = data + P.leaf_off;
+  hipLaunchKernelGGL((k_nd_leaf_solve<T, R, true>), dim3((P.nleaf + 3) / 4), dim3(NT), 0, s, A, data + P.leafc_off);
+  HIP_TRY(hipGetLastError());
+  return FDFD_OK;
+}
+template <typename T>
+int nd_sweep(const NdPlan &P, const fdfd_grid *g, const void *factor, const double *r, double *x, int nrhs, int add,
+             char *work, const NdSolveWork &w, hipStream_t s) {
+  const double *tab = (const double *)((const char *)factor + ND_HEADER);
+  const T *data = (const T *)((const char *)factor + nd_data_off(P));
+  const NdTab tb = nd_tables(tab, P.nx, P.ny);
+  const size_t M = (size_t)P.nx * P.ny;
+  T *v = (T *)(work + w.v), *u0 = (T *)(work + w.u[0]), *u1 = (T *)(work + w.u[1]);
+  const double alpha = nd_alpha(g);
+  constexpr int most = nd_rhs_per_pass<T>();
+  for (int q0 = 0; q0 < nrhs; q0 += most) {
+    const int nq = std::min(most, nrhs - q0);
+    const double *rq = r + 2 * M * q0;
+    double *xq = x + 2 * M * q0;
+    int rc = FDFD_OK;
+    if (nq == 1) rc = nd_pass<T, 1>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
+    else if (nq == 2) rc = nd_pass<T, 2>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
+    else if (nq <= 4) rc = nd_pass<T, 4>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
+    else if constexpr (most >= 8) rc = nd_pass<T, 8>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
+    if (rc) return rc;
+  }
+  return FDFD_OK;
+}
+
+// The path's range: a plan exists and its solve fits the workspace that
+// fdfd_solve_workspace_bytes reports without knowing the factor's kind
+inline bool nd_fits(const fdfd_grid *g, NdPlan *P) {
+  if (!nd_plan(g, P)) return false;
+  for (int prec = 0; prec < 2; ++prec)
+    for (int k = 1; k <= 8; ++k)
+      if (nd_solve_layout(*P, prec, k).total > solve_work_bytes(g, prec, k)) return false;
+  return true;
+}
+
+// The refinement of fdfd_solve with a nested-dissection factor: x = A^-1 b,
+// then x += A^-1 (b - A x) until every right-hand side meets the tolerance.
+// With a periodic axis a step is two sweeps, as on the block path. The first
+// sweep starts before ||b|| is known on the host; a zero b gives x = 0.
+template <typename T>
+int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const double *b, double *x, int nrhs,
+             int transpose, double tol, int max_iter, void *work, fdfd_solve_stats *stats, double *rel_res,
+             hipStream_t s, double *host) {
+  const int prec = sizeof(T) == 8 ? FDFD_PREC_FP64 : FDFD_PREC_C64;
+  NdPlan P;
+  if (!nd_fits(g, &P)) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
+  const NdSolveWork w = nd_solve_layout(P, prec, nrhs);
+  char *base = (char *)work;
+  double *r = (double *)(base + w.r), *part = (double *)(base + w.part), *norms = (double *)(base + w.norms);
+  const int cpr = (P.ny + NT - 1) / NT, parts = std::min(2 * NORM_PARTS, P.nx * cpr);
+  const dim3 rgrid(parts, (nrhs + ND_RES_RHS - 1) / ND_RES_RHS);
+  auto residual = [&](const double *xi) {
+    hipLaunchKernelGGL(k_nd_residual, rgrid, dim3(NT), 0, s, *g, op, b, xi, r, nrhs, transpose, part);
+  };
+  fdfd_solve_stats st;
+  memset(&st, 0, sizeof st);
+  double *nr = host, *nb = host + nrhs, *rel = host + 2 * nrhs, *prev = host + 3 * nrhs;
+  for (int q = 0; q < nrhs; ++q) { rel[q] = 0.0; prev[q] = INFINITY; }
+  residual(nullptr);
+  hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts, norms + nrhs);
+  const int sweeps = wrap_exact(g) ? 2 : 1;
+  int stall_count = 0;
+  for (int it = 1; it <= max_iter; ++it) {
+    for (int k = 0; k < sweeps; ++k) {
+      const bool first = it == 1 && k == 0;
+      if (int rc = nd_sweep<T>(P, g, factor, r, x, nrhs, first ? 0 : 1, base, w, s)) return rc;
+      residual(x);
+    }
+    hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts, norms);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(nr, norms, sizeof(double) * (it == 1 ? 2 : 1) * nrhs, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if (it == 1) {
+      bool all_zero = true;
+      for (int q = 0; q < nrhs; ++q) all_zero = all_zero && nb[q] == 0.0;
+      if (all_zero) {   // linalg.py:128-129
+        HIP_TRY(hipMemsetAsync(x, 0, 16 * (size_t)P.nx * P.ny * nrhs, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        st.zero_rhs = 1;
+        st.converged = 1;
+        if (stats) *stats = st;
+        if (rel_res) for (int q = 0; q < nrhs; ++q) rel_res[q] = 0;
+        return FDFD_OK;
+      }
+    }
+    st.iterations = it;
+    st.sweeps += sweeps;
+    double worst = 0;
+    bool contracting = false;
+    for (int q = 0; q < nrhs; ++q) {
+      rel[q] = nb[q] > 0 ? sqrt(nr[q] / nb[q]) : 0.0;
+      if (!std::isfinite(rel[q])) rel[q] = INFINITY;
+      worst = std::max(worst, rel[q]);
+      if (rel[q] > tol && rel[q] < 0.7 * prev[q]) contracting = true;
+    }
+    st.max_rel_residual = worst;
+    if (worst <= tol) { st.converged = 1; break; }
+    if (!std::isfinite(worst)) { st.stalled = 1; break; }
+    stall_count = contracting ? 0 : stall_count + 1;
+    if (stall_count >= 2) { st.stalled = 1; break; }
+    for (int q = 0; q < nrhs; ++q) prev[q] = rel[q];
+  }
+  if (transpose) {   // x = D x'
+    hipLaunchKernelGGL(k_stretch_scale, dim3((P.ny + NT - 1) / NT, P.nx, nrhs), dim3(NT), 0, s, *g, x, 0);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(s));
+  }
+  if (stats) *stats = st;
+  if (rel_res) for (int q = 0; q < nrhs; ++q) rel_res[q] = rel[q];
+  if (!st.converged)
+    return fail(FDFD_ERR_NOT_CONVERGED, "refinement reached %.3e after %d sweeps (tol %.1e)%s",
+                st.max_rel_residual, st.iterations, tol, st.stalled ? ", stalled" : "");
+  return FDFD_OK;
+}
+
+// Whether a factor buffer of unknown kind (on a grid of the path's range)
+// holds a nested-dissection factor: its tag; waits for the stream.
+int nd_is_factor(const void *factor, hipStream_t s, bool *nd) {
+  unsigned long long head[4];
+  HIP_TRY(hipMemcpyAsync(head, factor, sizeof head, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  *nd = true;
+  for (int i = 0; i < 4; ++i) *nd = *nd && head[i] == nd_tag(i);
+  return FDFD_OK;
+}

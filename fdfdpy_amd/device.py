@@ -146,6 +146,9 @@ class DeviceOperator:
         nbytes = self.lib.fdfd_op_bytes(ctypes.byref(self.grid))
         if nbytes == 0:
             raise ValueError(self.lib.fdfd_last_error().decode())
+        # the nested-dissection factor's bytes by precision (0: the grid is outside its range)
+        gp = ctypes.byref(self.grid)
+        self.nd_bytes = {k: int(self.lib.fdfd_factor_bytes(gp, v | L.FACTOR_ND)) for k, v in L.PREC.items()}
         self.op = torch.empty(nbytes // 8, dtype=torch.float64, device=self.device)
         self.eps = None          # complex128, solver orientation
         self.eps_user = None     # complex128, caller orientation
@@ -156,7 +159,14 @@ class DeviceOperator:
         self.engine = None       # FactorEngine shared with other operators, if any
 
     # -- sizes ----------------------------------------------------------
+    @property
+    def nested(self):
+        """The next factor is a nested-dissection one (unless it pivots or an engine builds it)."""
+        return self.lib.fdfd_nd_supported(ctypes.byref(self.grid)) == 1
+
     def factor_bytes(self, precision):
+        if self.nested:
+            return self.nd_bytes[precision]
         return int(self.lib.fdfd_factor_bytes(ctypes.byref(self.grid), L.PREC[precision]))
 
     def op_bytes(self):
@@ -201,18 +211,22 @@ class DeviceOperator:
         when absent, or when refresh is set and the resident one belongs to
         an older operator or another pivoting mode. pivot=True pivots inside
         each 32x32 pivot tile (the fallback when the diagonal-pivot factor
-        does not refine). stepwise=True forces one launch per Gauss-Jordan
-        step instead of the persistent launch."""
+        does not refine). The factor is the nested-dissection one where the
+        grid is in its range; pivot, stepwise=True (one launch per
+        Gauss-Jordan step of the block chains) and an engine take the block
+        factorization."""
         if precision in self.factors:
             fac, ver, piv = self.factors[precision]
-            if not refresh or (ver == self.version and piv == pivot):
+            blocks = stepwise and fac.numel() == self.nd_bytes[precision]   # a block factor is asked for
+            if not refresh or (ver == self.version and piv == pivot and not blocks):
                 return fac
         g = ctypes.byref(self.grid)
-        p = L.PREC[precision] | (L.FACTOR_PIVOT if pivot else 0) | (L.FACTOR_STEPWISE if stepwise else 0)
-        fac = torch.empty(self.lib.fdfd_factor_bytes(g, L.PREC[precision]), dtype=torch.uint8,
-                          device=self.device)
-        work = torch.empty(self.lib.fdfd_factor_workspace_bytes(g, L.PREC[precision]), dtype=torch.uint8,
-                           device=self.device)
+        if self.nested and not pivot and not stepwise and self.engine is None:
+            p = L.PREC[precision] | L.FACTOR_ND
+        else:
+            p = L.PREC[precision] | (L.FACTOR_PIVOT if pivot else 0) | (L.FACTOR_STEPWISE if stepwise else 0)
+        fac = torch.empty(self.lib.fdfd_factor_bytes(g, p), dtype=torch.uint8, device=self.device)
+        work = torch.empty(self.lib.fdfd_factor_workspace_bytes(g, p), dtype=torch.uint8, device=self.device)
         s = _stream(self.device)
         t0 = time.perf_counter()
         if self.engine is not None:
@@ -240,31 +254,36 @@ class DeviceOperator:
 
         precision 'c64' factors in complex64 and refines in FP64. When the
         refinement stalls the solve falls back to the FP64 factor, and then
-        to the FP64 factor with pivoting inside the pivot tiles.
+        to the FP64 block factor with pivoting inside the pivot tiles;
+        without fallback, from a nested-dissection factor to the block factor
+        of the same precision (a box of the tree near resonance costs a
+        complex64 factor its digits in about 1% of random designs).
         """
         squeeze = b.dim() == 2
         bb = b.reshape((1,) + self.shape) if squeeze else b
         nrhs = bb.shape[0]
         bs = self.to_solver(bb.to(device=self.device, dtype=torch.complex128))
         x = torch.empty_like(bs)
-        # attempts in order: (precision, pivoted, refactor first)
-        plan = [(precision, False, False)]
+        # attempts in order: (precision, pivoted, refactor first, as a block factor)
+        plan = [(precision, False, False, False)]
         if precision in self.factors and self.factors[precision][1] != self.version:
             # the resident factor belongs to an earlier diagonal (Born steps):
             # it preconditions the refinement first, then is rebuilt
-            plan.append((precision, False, True))
+            plan.append((precision, False, True, False))
         if precision == "c64" and fallback:
-            plan.append(("fp64", False, True))
+            plan.append(("fp64", False, True, False))
         if fallback:
             # last resort: partial pivoting inside the 32x32 pivot tiles
-            plan.append(("fp64", True, True))
+            plan.append(("fp64", True, True, False))
+        elif self.nested:
+            plan.append((precision, False, True, True))
         rep, failed, spent = None, [], [0.0, 0.0, 0]
-        for prec, piv, refresh in plan:
+        for prec, piv, refresh, blocks in plan:
             if rep is not None and rep.converged:
                 break
             try:
                 if refresh:
-                    self.factor(prec, refresh=True, pivot=piv)
+                    self.factor(prec, refresh=True, pivot=piv, stepwise=blocks)
                 rep2 = self._solve_one(bs, x, nrhs, prec, tol, max_iter, transpose)
             except L.FdfdError as e:
                 if e.code != L.FDFD_ERR_NUMERIC:
@@ -294,7 +313,8 @@ class DeviceOperator:
         fac = self.factor(precision)
         tf = time.perf_counter() - t0 if precision not in self.factor_seconds else self.factor_seconds[precision]
         g = ctypes.byref(self.grid)
-        p = L.PREC[precision]
+        # the two kinds of factor never have the same size
+        p = L.PREC[precision] | (L.FACTOR_ND if fac.numel() == self.nd_bytes[precision] else L.FACTOR_STEPWISE)
         work = torch.empty(self.lib.fdfd_solve_workspace_bytes(g, p, nrhs), dtype=torch.uint8,
                            device=self.device)
         st = L.FdfdSolveStats()

@@ -64,7 +64,9 @@ def operator_key(p):
 
 
 def request_bytes(p, precision, nrhs=None):
-    """Device bytes a request holds while it runs (operator, factor, workspaces, vectors)."""
+    """Device bytes a request may hold while it runs (operator, factor,
+    workspaces, vectors), with a block factor of its precision, the larger
+    kind, which a solve without its nested-dissection factor falls back to."""
     lib = L.lib()
     Nx, Ny = p.shape
     g = L.FdfdGrid(Nx, Ny, p.npml[0], p.npml[1], L.POL[p.pol], 0, p.omega, p.dl, p.L0)
@@ -168,7 +170,8 @@ class ServingEngine:
                 reused = True
             else:
                 op = DeviceOperator(p.shape, p.omega, p.dl, p.npml, p.pol, p.L0, self.device)
-                op.engine = self._engine_for(stream)
+                if not op.nested:   # block factorizations share step launches
+                    op.engine = self._engine_for(stream)
                 op.set_eps(p.eps)
             b = torch.as_tensor(p.rhs(), device=self.device)
             x, rep = op.solve(b, precision=self.precision, tol=self.tol, max_iter=self.max_iter)

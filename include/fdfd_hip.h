@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define FDFD_ABI_VERSION 4
+#define FDFD_ABI_VERSION 5
 
 enum {
   FDFD_OK = 0,
@@ -56,6 +56,14 @@ enum { FDFD_PREC_FP64 = 0, FDFD_PREC_C64 = 1 };      /* factor precision  */
  * Gauss-Jordan step instead of the single persistent launch (which
  * fdfd_factor uses, synchronously, when the tile grid fits the device). */
 #define FDFD_FACTOR_STEPWISE 0x200
+/* OR'ed, alone, into the precision argument of fdfd_factor and of the size
+ * functions: the nested-dissection factor of the whole periodic operator
+ * (grids that fdfd_nd_supported accepts) instead of the block factorization.
+ * Its buffers have sizes of their own. fdfd_solve, fdfd_solve_static and
+ * fdfd_sweep recognise it by a tag at its start, which costs a read of the
+ * device; with FDFD_FACTOR_ND (or, for a block factor, FDFD_FACTOR_STEPWISE)
+ * in their precision they take the caller's word. */
+#define FDFD_FACTOR_ND 0x400
 enum { FDFD_OP_C = 0, FDFD_OP_XM = 1, FDFD_OP_XP = 2, FDFD_OP_YM = 3, FDFD_OP_YP = 4 };
 
 /* Grid and physics parameters; the fields of Simulation.__init__
@@ -165,7 +173,8 @@ int fdfd_factor_wrap(const fdfd_grid *g, const double *op, void *factor, int pre
 int fdfd_factor_status(const fdfd_grid *g, int precision, void *work, hipStream_t stream);
 
 /* One block sweep with the factor: x += T^-1 r (nrhs vectors), without the
- * x-wrap correction that fdfd_solve applies. */
+ * x-wrap correction that fdfd_solve applies. A nested-dissection factor
+ * holds the wrap: x += A^-1 r. */
 int fdfd_sweep(const fdfd_grid *g, const double *op, const void *factor, int precision,
                const double *r, double *x, int nrhs, void *work, hipStream_t stream);
 
@@ -281,6 +290,21 @@ int fdfd_set_twist(int on);
 /* The twist block c for g under the current setting (m - 1: one chain);
  * -1 for an invalid grid. */
 int fdfd_twist_block(const fdfd_grid *g);
+
+/* 1 when FDFD_FACTOR_ND is the factor of choice for this grid (its shorter
+ * side has 64 cells or more), 0 when not (also while fdfd_set_twist(0) asks
+ * for the one-chain order), -1 for an invalid grid. No reference
+ * counterpart. */
+int fdfd_nd_supported(const fdfd_grid *g);
+
+/* One front of the nested-dissection tree of g, on the host (no GPU; no
+ * reference counterpart): level -1 the leaves, 0 .. nlev - 1 the merges
+ * upwards, nlev the root. info[8] = {nlev, boxes of the level, split axis,
+ * separator entries s, border entries b, the children's numbers, a leaf's
+ * height}; cells (optional, s + b) the cell i * ny + j of each separator
+ * (a leaf: interior) and border entry; map (optional, 2 (s + b)) the entry
+ * of each child's border that is added to it, or -1. */
+int fdfd_nd_front(const fdfd_grid *g, int level, int box, int32_t *info, int64_t *cells, int32_t *map);
 
 /* Check of the MFMA operand layouts the factor kernels rely on (no reference
  * counterpart): D = A (16x4) * B (4x16) with the 16x16x4 f64 (precision 0)

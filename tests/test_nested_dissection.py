@@ -1,0 +1,216 @@
+"""The nested-dissection factor: its tree and index maps on the CPU, the factor
+and solve on the GPU against the oracle.
+
+The CPU half eliminates the oracle's operator front by front with numpy, in
+the library's own tree and maps (fdfd_nd_front), and compares the solution
+with SuperLU: every cell is eliminated once, every index lies inside its
+array, and the fronts add up to the whole periodic operator.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from fdfdpy_amd import _lib as L
+from fdfdpy_amd import configs as C
+from oracle import construct_A, solver_direct
+
+OMEGA = C.omega_of(1.55e-6)
+DEV = "cuda:0"
+
+
+def relerr(a, b):
+    return float(np.linalg.norm(np.asarray(a) - np.asarray(b)) / np.linalg.norm(np.asarray(b)))
+
+
+def _eps(rng, N):
+    return 1 + 11.25 * (rng.random(N) < 0.5)
+
+
+def _front(g, level, box):
+    lib = L.lib()
+    info = (ctypes.c_int32 * 8)()
+    L.check(lib.fdfd_nd_front(ctypes.byref(g), level, box, info, None, None))
+    n = info[3] + info[4]
+    cells, maps = np.zeros(n, np.int64), np.zeros((n, 2), np.int32)
+    L.check(lib.fdfd_nd_front(ctypes.byref(g), level, box, info, cells.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)),
+                              maps.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))))
+    return list(info), cells, maps
+
+
+def _multifrontal(nx, ny, A, b):
+    g = L.FdfdGrid(nx, ny, 10, 10, 0, 0, OMEGA, 0.02, 1e-6)
+    levels = _front(g, -1, 0)[0][0]
+    A = A.tocsr()
+    updates, done = [], []
+    eliminated = np.zeros(nx * ny, int)
+    for level in range(-1, levels + 1):
+        new, fronts = [], []
+        for k in range(_front(g, level, 0)[0][1]):
+            info, cells, maps = _front(g, level, k)
+            s, n = info[3], len(cells)
+            assert cells.min() >= 0 and cells.max() < nx * ny
+            eliminated[cells[:s]] += 1
+            # the front's own entries: rows and columns of its separator
+            F = np.zeros((n, n), complex)
+            F[:s, :] = A[cells[:s]][:, cells].toarray()
+            F[s:, :s] = A[cells[s:]][:, cells[:s]].toarray()
+            if len(set(cells)) != n:          # no cell twice in a front
+                raise AssertionError(f"level {level} box {k}: a cell appears twice")
+            f = np.concatenate([b[cells[:s]], np.zeros(n - s)]).astype(complex)
+            if level >= 0:
+                for t in range(2):
+                    v = np.nonzero(maps[:, t] >= 0)[0]
+                    if len(v):
+                        Cc, uc, border = updates[info[5 + t]]
+                        at = maps[v, t]
+                        assert np.array_equal(border[at], cells[v])   # the same cells on both sides
+                        F[np.ix_(v, v)] += Cc[np.ix_(at, at)]
+                        f[v] += uc[at]
+            X = np.linalg.inv(F[:s, :s])
+            W = X @ F[:s, s:]
+            z = X @ f[:s]
+            new.append((F[s:, s:] - F[s:, :s] @ W, f[s:] - F[s:, :s] @ z, cells[s:]))
+            fronts.append((cells, s, z, W))
+        updates = new
+        done.append(fronts)
+    assert (eliminated == 1).all()
+    x = np.zeros(nx * ny, complex)
+    for fronts in reversed(done):
+        for cells, s, z, W in fronts:
+            x[cells[:s]] = z - W @ x[cells[s:]]
+    return x
+
+
+@pytest.mark.parametrize("N,npml,pol", [((64, 64), [8, 8], "Ez"), ((65, 97), [9, 0], "Hz"), ((200, 64), [10, 10], "Ez"),
+                                        ((71, 130), [0, 0], "Ez"), ((64, 230), [8, 12], "Hz")])
+def test_tree_and_maps_solve_the_periodic_operator(N, npml, pol):
+    rng = np.random.default_rng(N[0] + N[1])
+    A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], _eps(rng, N), npml, pol, 1e-6)
+    b = rng.standard_normal(N[0] * N[1]) + 1j * rng.standard_normal(N[0] * N[1])
+    assert relerr(_multifrontal(N[0], N[1], A, b), solver_direct(A, b)) < 1e-9
+
+
+def test_range_and_sizes():
+    """Every grid whose shorter side has 64 cells or more is in the range,
+    smaller ones are not; flags that exclude each other are refused; the two
+    kinds of factor never have one size."""
+    lib = L.lib()
+
+    def grid(nx, ny):
+        return ctypes.byref(L.FdfdGrid(nx, ny, 10, 10, 0, 0, OMEGA, 0.02, 1e-6))
+    for n in list(range(64, 460)) + [511, 512, 513, 768, 1023, 1500, 2047, 2048]:
+        for m in (64, n, n + 1, 2 * n + 1):
+            if min(n, m) > 2048 or m < 2:
+                continue
+            ny, nx = min(n, m), max(n, m)
+            assert lib.fdfd_nd_supported(grid(nx, ny)) == 1, (nx, ny)
+            for prec in (0, 1):
+                nd = lib.fdfd_factor_bytes(grid(nx, ny), prec | L.FACTOR_ND)
+                assert nd > 0 and nd != lib.fdfd_factor_bytes(grid(nx, ny), prec)
+    for shape in ((63, 64), (64, 63), (500, 40), (2, 2)):
+        assert lib.fdfd_nd_supported(grid(*shape)) == 0
+        assert lib.fdfd_factor_bytes(grid(*shape), L.FACTOR_ND) == 0
+    for bad in (L.FACTOR_ND | L.FACTOR_PIVOT, L.FACTOR_ND | L.FACTOR_STEPWISE):
+        assert lib.fdfd_factor_bytes(grid(128, 128), bad) == 0
+    prev = lib.fdfd_set_twist(0)
+    try:   # the one-chain order is a block factorization
+        assert lib.fdfd_nd_supported(grid(128, 128)) == 0
+    finally:
+        lib.fdfd_set_twist(prev)
+
+
+def _device(N, npml, pol, eps):
+    from fdfdpy_amd.device import DeviceOperator
+    op = DeviceOperator(N, OMEGA, 0.02, npml, pol, 1e-6, DEV)
+    op.set_eps(eps)
+    assert op.nested
+    return op
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,npml,pol,nrhs", [
+    ((64, 64), [8, 8], "Ez", 1), ((65, 97), [9, 12], "Hz", 2), ((128, 66), [10, 0], "Ez", 3),
+    ((129, 70), [0, 0], "Hz", 5), ((64, 300), [8, 15], "Ez", 8), ((257, 96), [20, 10], "Hz", 9)])
+@pytest.mark.parametrize("precision", ["fp64", "c64"])
+def test_solves_match_the_oracle(N, npml, pol, nrhs, precision):
+    """Edges of the tree (power-of-two sides and their neighbours, long
+    grids), both polarizations, periodic axes, a lossy cell, every count of
+    right-hand sides per pass; forward and transposed."""
+    rng = np.random.default_rng(sum(N) + nrhs)
+    eps = _eps(rng, N).astype(complex)
+    eps[N[0] // 2:, N[1] // 2:] += 0.3j
+    op = _device(N, npml, pol, eps)
+    A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], eps, npml, pol, 1e-6)
+    b = rng.standard_normal((nrhs,) + N) + 1j * rng.standard_normal((nrhs,) + N)
+    for transpose, M in ((False, A), (True, A.T.tocsr())):
+        x, rep = op.solve(torch.tensor(b, device=DEV), precision=precision, tol=1e-12, transpose=transpose)
+        assert rep.converged and not rep.fell_back
+        assert op.factors[precision][0].numel() == op.nd_bytes[precision]
+        for q in {0, nrhs - 1}:
+            assert relerr(x[q].cpu().numpy(), solver_direct(M, b[q].reshape(-1)).reshape(N)) < 1e-10
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "c64"])
+def test_kinds_are_told_apart_and_repeat_to_the_bit(precision):
+    """fdfd_solve without a kind in its precision reads the tag; fdfd_sweep on
+    this kind adds A^-1 r; two factorizations and solves have equal bits; a
+    zero right-hand side gives zeros without a sweep."""
+    N = (90, 101)
+    rng = np.random.default_rng(7)
+    op = _device(N, [10, 10], "Ez", _eps(rng, N))
+    lib, g, pr = L.lib(), ctypes.byref(op.grid), L.PREC[precision]
+    fac = op.factor(precision)
+    first = fac.clone()
+    b = op.to_solver(torch.tensor(rng.standard_normal((2,) + N) + 1j * rng.standard_normal((2,) + N), device=DEV))
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    work = torch.empty(lib.fdfd_solve_workspace_bytes(g, pr, 2), dtype=torch.uint8, device=DEV)
+    xs = []
+    for flag in (0, L.FACTOR_ND):
+        x, st = torch.full_like(b, float("nan")), L.FdfdSolveStats()
+        L.check(lib.fdfd_solve(g, ptr(op.op), ptr(fac), pr | flag, ptr(b), ptr(x), 2, 0, 1e-10, 20, ptr(work),
+                               ctypes.byref(st), None, None))
+        torch.cuda.synchronize()
+        xs.append(x)
+    assert torch.equal(xs[0], xs[1])
+    y = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    L.check(lib.fdfd_sweep(g, ptr(op.op), ptr(fac), pr, ptr(b), ptr(y), 2, ptr(work), None))
+    assert relerr(y.cpu().numpy(), xs[0].cpu().numpy()) < (1e-10 if precision == "fp64" else 1e-2)
+    op.drop_factor()
+    assert torch.equal(op.factor(precision), first)
+    x, rep = op.solve(torch.zeros(N, dtype=torch.complex128, device=DEV), precision=precision)
+    assert not x.any() and rep.sweeps == 0 and rep.converged
+    # a block factor of the same grid goes the block path
+    op.drop_factor()
+    op.factor(precision, stepwise=True)
+    xb, rep = op.solve(torch.tensor(np.ones(N) + 0j, device=DEV), precision=precision, tol=1e-10)
+    assert rep.converged and op.factors[precision][0].numel() != op.nd_bytes[precision]
+
+
+@pytest.mark.gpu
+def test_stall_without_fallback_takes_the_block_factor(monkeypatch):
+    """fallback=False keeps the precision: when the nested-dissection factor
+    does not refine (its report forced here), the block factor does."""
+    from fdfdpy_amd.device import DeviceOperator
+    N = (80, 72)
+    rng = np.random.default_rng(3)
+    eps = _eps(rng, N)
+    op = _device(N, [9, 9], "Ez", eps)
+    real = DeviceOperator._solve_one
+
+    def stalled(self, *a, **k):
+        rep = real(self, *a, **k)
+        if self.factors["c64"][0].numel() == self.nd_bytes["c64"]:
+            rep.converged = False
+        return rep
+    monkeypatch.setattr(DeviceOperator, "_solve_one", stalled)
+    b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    x, rep = op.solve(torch.tensor(b, device=DEV), precision="c64", tol=1e-10, fallback=False)
+    assert rep.converged and rep.precision == "c64"
+    assert op.factors["c64"][0].numel() != op.nd_bytes["c64"]
+    A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], eps, [9, 9], "Ez", 1e-6)
+    assert relerr(x.cpu().numpy(), solver_direct(A, b.reshape(-1)).reshape(N)) < 1e-8
