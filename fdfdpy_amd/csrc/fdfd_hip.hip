@@ -3805,9 +3805,15 @@ int fdfd_sweep(const fdfd_grid *g, const double *op, const void *factor, int pre
   if (int rc = factor_is_nd(g, factor, precision, stream, &nd, &P)) return rc;
   if (nd) {
     const NdSolveWork w = nd_solve_layout(P, precision, nrhs);
-    int rc = base_prec(precision) == FDFD_PREC_FP64
-                 ? nd_sweep<double>(P, g, factor, r, x, nrhs, 1, (char *)work, w, stream)
-                 : nd_sweep<float>(P, g, factor, r, x, nrhs, 1, (char *)work, w, stream);
+    char *wb = (char *)work;
+    int rc;
+    if (base_prec(precision) == FDFD_PREC_FP64) {
+      nd_residual<double>(g, P, op, factor, r, nullptr, nrhs, 0, wb, w, nd_parts(P), stream);
+      rc = nd_sweep<double>(P, factor, x, nrhs, 1, wb, w, stream);
+    } else {
+      nd_residual<float>(g, P, op, factor, r, nullptr, nrhs, 0, wb, w, nd_parts(P), stream);
+      rc = nd_sweep<float>(P, factor, x, nrhs, 1, wb, w, stream);
+    }
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(stream));
     return FDFD_OK;

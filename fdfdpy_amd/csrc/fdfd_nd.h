@@ -73,7 +73,7 @@ struct NdPlan {
 bool nd_plan(const fdfd_grid *g, NdPlan *P) {
   memset(P, 0, sizeof *P);
   const int nx = g->nx, ny = g->ny;
-  if (std::min(nx, ny) < ND_MIN_SIDE) return false;
+  if (std::min(nx, ny) < ND_MIN_SIDE || (long)nx * ny > (1l << 30)) return false;
   P->nx = nx;
   P->ny = ny;
   NdLevel down[ND_MAX_LEVELS];
@@ -971,281 +971,258 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
 }
 
 // -------------------------------------------------------------- solve
-// Vectors of one pass of R right-hand sides: r and x (complex FP64, caller's
-// planes of nx ny), v (complex T, the same planes: z, then x, on the
-// separators), u (complex T, [box][R][pitch]: a level's updates).
-template <typename T> struct NdSolve {
-  NdLevel L;
-  NdTab tb;
-  double alpha;
-  const T *X, *W;       // this level's
-  const double *r;      // [q][M]
-  double *x;            // [q][M]
-  T *v;                 // [q][M]
-  const T *uin;         // the children's updates
-  T *uout;
-  int nq, add;          // right-hand sides of this pass; x += (else x =)
+// Vectors of one pass of nq right-hand sides, complex T, right-hand sides
+// innermost: f (the scaled right-hand side a E r) and v (z, then x, on the
+// separators) by cell, u (a level's updates) by border entry. x is complex
+// FP64 in the caller's planes.
+//
+// The levels whose separators fit one tile run as subtrees: one workgroup
+// takes a box of level `top` with everything below it, a wave per box, with a
+// barrier between levels instead of a launch. Its u live in two regions of
+// its own, alternating by level (subtrees run at their own pace); level top
+// writes u by box for the launches above.
+constexpr int ND_TREE_MAX = 12;      // levels of a subtree
+constexpr int ND_TREE_BOXES = 512;   // least subtrees, where the grid has them (see nd_tree)
+constexpr int ND_TREE_WAVES = 8;
+struct NdTree {
+  int nx, ny, Dx, Dy, leaf_b, top, nq, add;
+  unsigned reg0, reg1;               // entries of a subtree's two u regions
+  NdLevel lev[ND_TREE_MAX];          // 0 .. top
+};
+template <typename T> struct NdVec {
+  const double *iex, *iey;
+  const T *data;                     // the factor's data
+  const T *f;
+  T *v;
+  double *x;
+  T *u0, *u1, *u2;
 };
 
 template <typename T>
-__device__ inline void nd_rhs(const NdSolve<T> &A, size_t cell, int q, T &re, T &im) {
-  const size_t M = (size_t)A.L.nx * A.L.ny;
-  const int i = (int)(cell / A.L.ny), j = (int)(cell % A.L.ny);
-  const cd e = cscale(cmul(ld_c(A.tb.ex, i), ld_c(A.tb.ey, j)), A.alpha);
-  const cd f = cmul(e, ld_c(A.r + 2 * M * q, cell));
-  re = (T)f.r;
-  im = (T)f.i;
+__device__ inline void nd_out(const double *iex, const double *iey, double *x, size_t M, int i, int j, int ny, int q,
+                              int add, T re, T im) {
+  const cd o = cmul(cmul(ld_c(iex, i), ld_c(iey, j)), cd{(double)re, (double)im});
+  double *xq = x + 2 * M * q;
+  const size_t p = (size_t)i * ny + j;
+  st_c(xq, p, add ? cadd(ld_c(xq, p), o) : o);
 }
-template <typename T>
-__device__ inline void nd_out(const NdSolve<T> &A, size_t cell, int q, T re, T im) {
-  const size_t M = (size_t)A.L.nx * A.L.ny;
-  const int i = (int)(cell / A.L.ny), j = (int)(cell % A.L.ny);
-  const cd o = cmul(cmul(ld_c(A.tb.iex, i), ld_c(A.tb.iey, j)), cd{(double)re, (double)im});
-  double *x = A.x + 2 * M * q;
-  st_c(x, cell, A.add ? cadd(ld_c(x, cell), o) : o);
+// cells as (i, j)
+__device__ inline void nd_sep_ij(const NdLevel &L, const NdBox &B, int j, int &ci, int &cj) {
+  if (L.root) {
+    const int h = L.ny - 1, w = L.nx - 1;
+    ci = j < h || j >= h + w ? 0 : j - h + 1;
+    cj = j < h ? j + 1 : 0;
+  } else if (L.ax == 0) {
+    ci = B.x0 + B.c0;
+    cj = B.y0 + j;
+  } else {
+    ci = B.x0 + j;
+    cj = B.y0 + B.c0;
+  }
 }
-// separator entry j of the children's updates plus r, right-hand side q
+// within a wave: LDS stores before this are seen by loads after it
+__device__ inline void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// f_s of separator entry j, right-hand side q: f plus the children's updates
+// (uin with the children's numbers n0, n1 in it)
 template <typename T>
-__device__ inline void nd_fs(const NdSolve<T> &A, const NdBox &B, int j, int q, T &re, T &im) {
-  nd_rhs(A, nd_sep_cell(A.L, B, j), q, re, im);
+__device__ inline void nd_fs(const NdLevel &L, const NdBox &B, const T *f, const T *uin, int n0, int n1, int nq, int j,
+                             int q, T &re, T &im) {
+  int ci, cj, m0, m1;
+  nd_sep_ij(L, B, j, ci, cj);
+  nd_sep_map(L, B, j, m0, m1);
+  T a = 0, b = 0, c = 0, d = 0;
+  nd_ld(f, ((size_t)ci * L.ny + cj) * nq + q, re, im);
+  if (m0 >= 0) nd_ld(uin, ((size_t)n0 * L.cb + m0) * nq + q, a, b);
+  if (m1 >= 0) nd_ld(uin, ((size_t)n1 * L.cb + m1) * nq + q, c, d);
+  re += a + c;
+  im += b + d;
+}
+// the children's sum at border entry j
+template <typename T>
+__device__ inline void nd_fb(const NdLevel &L, const NdBox &B, const T *uin, int n0, int n1, int nq, int j, int q,
+                             T &re, T &im) {
   int m0, m1;
-  nd_sep_map(A.L, B, j, m0, m1);
-  T a, b;
-  if (m0 >= 0) { nd_ld(A.uin, ((size_t)B.k0 * A.nq + q) * A.L.cb + m0, a, b); re += a; im += b; }
-  if (m1 >= 0) { nd_ld(A.uin, ((size_t)B.k1 * A.nq + q) * A.L.cb + m1, a, b); re += a; im += b; }
+  nd_border_map(L, B, j, m0, m1);
+  T a = 0, b = 0, c = 0, d = 0;
+  if (m0 >= 0) nd_ld(uin, ((size_t)n0 * L.cb + m0) * nq + q, a, b);
+  if (m1 >= 0) nd_ld(uin, ((size_t)n1 * L.cb + m1) * nq + q, c, d);
+  re = a + c;
+  im = b + d;
 }
 
-// Upwards, one level (and the root, whose z is x): columns [64 c, 64 c + 64)
-// of [X | W] of one box per NW waves, which split the separator's rows.
-template <typename T, int R, int NW> struct NdUp {
-  static constexpr int TASKS = NW == 1 ? 4 : 1, THREADS = 64 * NW * TASKS;
-  static constexpr int JC = NW == 1 ? TB : 64 * NW;   // rows staged at a time
-  union Mem {
-    T f[TASKS][R][2][JC];
-    T red[NW][2 * R][64];
-  };
-};
-template <typename T, int R, int NW>
-__global__ void __launch_bounds__(64 * NW * (NW == 1 ? 4 : 1)) k_nd_up(NdSolve<T> A) {
-  typedef NdUp<T, R, NW> Cfg;
-  __shared__ typename Cfg::Mem S;
-  const NdLevel &L = A.L;
-  const int tid = threadIdx.x, lane = tid & 63, task = tid / (64 * NW), wv = (tid >> 6) % NW;
-  const int chunks = (L.sp + L.bp + 63) / 64;
-  const int id = blockIdx.x * Cfg::TASKS + task;
-  const bool live = id < L.nbox * chunks;
-  const int box = live ? id / chunks : 0, c = (live ? id % chunks : 0) * 64 + lane;
+// Upwards, one wave: columns 64 chunk .. + 64 of [X | W] of a box whose
+// separator fits a tile. F: the wave's staging area.
+template <typename T, int R>
+__device__ inline void nd_up_wave(const NdTree &t, const NdVec<T> &A, const NdLevel &L, int box, int n0, int n1,
+                                  const T *uin, T *uout, int chunk, T (*F)[R][2], int lane) {
   const NdBox B = nd_box(L, box);
-  const bool inX = c < L.sp, inW = !inX && c < L.sp + L.bp;
-  const size_t pitch = inX ? L.sp : L.bp, plane = (size_t)L.sp * pitch;
-  const T *m = inX ? A.X + (size_t)box * 2 * plane + c : A.W + (size_t)box * 2 * plane + (c - L.sp);
+  const int nq = t.nq;
+  for (int e = lane; e < TB * R; e += 64) {
+    const int j = e / R, q = e % R;
+    T re = 0, im = 0;
+    if (j < B.s && q < nq) nd_fs(L, B, A.f, uin, n0, n1, nq, j, q, re, im);
+    F[j][q][0] = re;
+    F[j][q][1] = im;
+  }
+  wave_lds_fence();
+  const int c = chunk * 64 + lane;
+  const bool inX = c < TB, inW = !inX && c < TB + L.bp;
+  if (inX || inW) {
+    const int pitch = inX ? TB : L.bp;
+    const size_t plane = (size_t)TB * pitch;
+    const T *m = A.data + (inX ? L.xoff + (size_t)box * 2 * plane + c : L.woff + (size_t)box * 2 * plane + c - TB);
+    T ar[R], ai[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
+#pragma unroll 4
+    for (int j = 0; j < B.s; ++j) {
+      const T gr = m[(size_t)j * pitch], gi = m[plane + (size_t)j * pitch];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const T fr = F[j][q][0], fi = F[j][q][1];
+        ar[q] += gr * fr - gi * fi;
+        ai[q] += gr * fi + gi * fr;
+      }
+    }
+    if (c < B.s) {
+      int ci, cj;
+      nd_sep_ij(L, B, c, ci, cj);
+      const size_t at = ((size_t)ci * L.ny + cj) * nq;
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (q < nq) nd_st<T>(A.v, at + q, ar[q], ai[q]);
+    } else if (inW && c - TB < B.b) {
+      const int j = c - TB;
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (q < nq) {
+          T ur, ui;
+          nd_fb(L, B, uin, n0, n1, nq, j, q, ur, ui);
+          nd_st<T>(uout, (size_t)j * nq + q, ur - ar[q], ui - ai[q]);
+        }
+    }
+  }
+  wave_lds_fence();
+}
+
+// Downwards, one wave: x_s = z - W x_b of a box whose separator fits a tile.
+// The lanes are RP rows x 64 / RP groups of columns; a lane reads its row of W
+// in 16-byte pieces.
+template <typename T, int R, int RP>
+__device__ inline void nd_down_wave(const NdTree &t, const NdVec<T> &A, const NdLevel &L, int box, T (*XB)[R][2],
+                                    int lane) {
+  constexpr int G = 64 / RP;
+  const NdBox B = nd_box(L, box);
+  const int nq = t.nq, row = lane & (RP - 1), g = lane / RP;
+  const size_t plane = (size_t)TB * L.bp;
+  const T *W = A.data + L.woff + (size_t)box * 2 * plane + (size_t)row * L.bp;
   T ar[R], ai[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
-  for (int j0 = 0; j0 < B.s; j0 += Cfg::JC) {
-    const int nj = min(Cfg::JC, B.s - j0);
-    if (j0) __syncthreads();
-    for (int e = wv * 64 + lane; e < Cfg::JC * R; e += 64 * NW) {
-      const int q = e / Cfg::JC, j = e % Cfg::JC;
-      T fr = 0, fi = 0;
-      if (live && j < nj && q < A.nq) nd_fs(A, B, j0 + j, q, fr, fi);
-      S.f[task][q][0][j] = fr;
-      S.f[task][q][1][j] = fi;
+  for (int b0 = 0; b0 < L.b; b0 += 64) {
+    wave_lds_fence();
+    for (int e = lane; e < 64 * R; e += 64) {
+      const int c = e / R, q = e % R;
+      T xr = 0, xi = 0;
+      if (b0 + c < B.b && q < nq)
+        nd_ld(A.v, nd_border_cell(L.nx, L.ny, L.dx, L.dy, B, b0 + c) * nq + q, xr, xi);
+      XB[c][q][0] = xr;
+      XB[c][q][1] = xi;
     }
-    __syncthreads();
-    if (inX || inW) {
-      const int per = (nj + NW - 1) / NW, ja = wv * per, jb = min(nj, ja + per);
-#pragma unroll 4
-      for (int j = ja; j < jb; ++j) {
-        const T gr = m[(size_t)(j0 + j) * pitch], gi = m[plane + (size_t)(j0 + j) * pitch];
+    wave_lds_fence();
+#pragma unroll 2
+    for (int c = 4 * g; c < 64; c += 4 * G) {
+      if (b0 + c >= L.bp) break;
+      T gr[4], gi[4];
+      ld_row4(W + b0 + c, gr);
+      ld_row4(W + plane + b0 + c, gi);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-          const T fr = S.f[task][q][0][j], fi = S.f[task][q][1][j];
-          ar[q] += gr * fr - gi * fi;
-          ai[q] += gr * fi + gi * fr;
+          const T xr = XB[c + k][q][0], xi = XB[c + k][q][1];
+          ar[q] += gr[k] * xr - gi[k] * xi;
+          ai[q] += gr[k] * xi + gi[k] * xr;
         }
-      }
     }
   }
-  if (NW > 1) {
-    __syncthreads();
+#pragma unroll
+  for (int off = RP; off < 64; off <<= 1)
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      S.red[wv][2 * q][lane] = ar[q];
-      S.red[wv][2 * q + 1][lane] = ai[q];
+      ar[q] += __shfl_xor(ar[q], off);
+      ai[q] += __shfl_xor(ai[q], off);
     }
-    __syncthreads();
-  }
-  // wave w finishes right-hand sides w, w + NW, ...
+  if (row < B.s) {
+    int ci, cj;
+    nd_sep_ij(L, B, row, ci, cj);
+    const size_t at = ((size_t)ci * L.ny + cj) * nq;
 #pragma unroll
-  for (int q = 0; q < R; ++q) {
-    if (q % NW != wv || q >= A.nq || !live) continue;
-    T sr = ar[q], si = ai[q];
-    if (NW > 1) {
-      sr = si = 0;
-      for (int t = 0; t < NW; ++t) { sr += S.red[t][2 * q][lane]; si += S.red[t][2 * q + 1][lane]; }
-    }
-    if (c < B.s) {
-      const size_t cell = nd_sep_cell(L, B, c);
-      nd_st<T>(A.v, (size_t)q * L.nx * L.ny + cell, sr, si);
-      if (L.root) nd_out(A, cell, q, sr, si);
-    } else if (inW && c - L.sp < B.b) {
-      const int j = c - L.sp;
-      int m0, m1;
-      nd_border_map(L, B, j, m0, m1);
-      T ur = 0, ui = 0, a, b;
-      if (m0 >= 0) { nd_ld(A.uin, ((size_t)B.k0 * A.nq + q) * L.cb + m0, a, b); ur += a; ui += b; }
-      if (m1 >= 0) { nd_ld(A.uin, ((size_t)B.k1 * A.nq + q) * L.cb + m1, a, b); ur += a; ui += b; }
-      nd_st<T>(A.uout, ((size_t)box * A.nq + q) * L.b + j, ur - sr, ui - si);
-    }
-  }
-}
-
-// Downwards, one level: x_s = z - W x_b. LPR lanes share a row: 64 (a box's
-// rows in groups of eight per workgroup) or 8 (separators of one tile: a box
-// per wave).
-template <typename T, int R, int LPR> struct NdDown {
-  static constexpr int RW = LPR == 64 ? 2 : 1;              // rows per LPR lanes
-  static constexpr int TASKS = LPR == 64 ? 1 : 4;           // boxes per workgroup
-  static constexpr int CC = LPR == 64 ? 256 : 96;           // border entries staged at a time
-  static constexpr int ROWS = LPR == 64 ? 8 : TB;           // rows of a task
-};
-template <typename T, int R, int LPR>
-__global__ void __launch_bounds__(NT) k_nd_down(NdSolve<T> A) {
-  typedef NdDown<T, R, LPR> Cfg;
-  __shared__ T S[Cfg::TASKS][R][2][Cfg::CC];
-  const NdLevel &L = A.L;
-  const size_t M = (size_t)L.nx * L.ny;
-  const int tid = threadIdx.x, task = LPR == 64 ? 0 : tid >> 6, tl = LPR == 64 ? tid : tid & 63;
-  constexpr int TT = NT / Cfg::TASKS;                        // threads of a task
-  const int groups = (L.s + Cfg::ROWS - 1) / Cfg::ROWS;
-  const int id = blockIdx.x * Cfg::TASKS + task;
-  const bool live = id < L.nbox * groups;
-  const int box = live ? id / groups : 0, g = live ? id % groups : 0;
-  const NdBox B = nd_box(L, box);
-  const size_t plane = (size_t)L.sp * L.bp;
-  const T *W = A.W + (size_t)box * 2 * plane;
-  constexpr int RPP = TT / LPR * Cfg::RW;                    // rows at a time
-  const int l = tl % LPR;
-  for (int q0 = 0; q0 < Cfg::ROWS && q0 < L.s; q0 += RPP) {
-    const int row = g * Cfg::ROWS + q0 + tl / LPR * Cfg::RW;
-    T ar[Cfg::RW][R], ai[Cfg::RW][R];
-#pragma unroll
-    for (int w = 0; w < Cfg::RW; ++w)
-#pragma unroll
-      for (int q = 0; q < R; ++q) { ar[w][q] = 0; ai[w][q] = 0; }
-    for (int b0 = 0; b0 < L.b; b0 += Cfg::CC) {
-      const bool restage = q0 == 0 || L.b > Cfg::CC;
-      if (restage) {
-        __syncthreads();
-        for (int e = tl; e < Cfg::CC * R; e += TT) {
-          const int q = e / Cfg::CC, c = e % Cfg::CC;
-          T xr = 0, xi = 0;
-          if (live && b0 + c < B.b && q < A.nq)
-            nd_ld(A.v, (size_t)q * M + nd_border_cell(L.nx, L.ny, L.dx, L.dy, B, b0 + c), xr, xi);
-          S[task][q][0][c] = xr;
-          S[task][q][1][c] = xi;
-        }
-        __syncthreads();
-      }
-      const int nc = min(Cfg::CC, L.bp - b0);   // W is zero beyond the border
-      const T *w0 = W + (size_t)min(row, L.sp - Cfg::RW) * L.bp + b0;
-#pragma unroll 4
-      for (int c = l; c < nc; c += LPR) {
-        T gr[Cfg::RW], gi[Cfg::RW];
-#pragma unroll
-        for (int w = 0; w < Cfg::RW; ++w) {
-          gr[w] = w0[(size_t)w * L.bp + c];
-          gi[w] = w0[plane + (size_t)w * L.bp + c];
-        }
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          const T xr = S[task][q][0][c], xi = S[task][q][1][c];
-#pragma unroll
-          for (int w = 0; w < Cfg::RW; ++w) {
-            ar[w][q] += gr[w] * xr - gi[w] * xi;
-            ai[w][q] += gr[w] * xi + gi[w] * xr;
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int w = 0; w < Cfg::RW; ++w)
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-#pragma unroll
-        for (int off = LPR / 2; off >= 1; off >>= 1) {
-          ar[w][q] += __shfl_xor(ar[w][q], off);
-          ai[w][q] += __shfl_xor(ai[w][q], off);
-        }
-        // lane (w R + q) % LPR of the row finishes this sum
-        if (l == (w * R + q) % LPR && live && row + w < B.s && q < A.nq) {
-          const size_t cell = nd_sep_cell(L, B, row + w);
-          T zr, zi;
-          nd_ld(A.v, (size_t)q * M + cell, zr, zi);
-          zr -= ar[w][q];
-          zi -= ai[w][q];
-          nd_st<T>(A.v, (size_t)q * M + cell, zr, zi);
-          nd_out(A, cell, q, zr, zi);
-        }
+    for (int q = 0; q < R; ++q)
+      if (q % G == g % R && q < nq) {   // the groups share the right-hand sides
+        if (G > R && g >= R) continue;
+        T zr, zi;
+        nd_ld(A.v, at + q, zr, zi);
+        zr -= ar[q];
+        zi -= ai[q];
+        nd_st<T>(A.v, at + q, zr, zi);
+        nd_out(A.iex, A.iey, A.x, (size_t)L.nx * L.ny, ci, cj, L.ny, q, t.add, zr, zi);
       }
   }
 }
 
-// The leaves, a box per wave: X is symmetric, so lane c of each half wave
-// sums its column over half of the rows. Upwards z = X r and the updates
-// -c_a z[p_a]; downwards x = X (r - F_sb x_b).
+// A leaf, one wave: X is symmetric, so lane c of each half wave sums its
+// column over half of the rows. Upwards z = X f and the updates -c_a z[p_a];
+// downwards x = X (f - F_sb x_b).
 template <typename T, int R, bool DOWN>
-__global__ void __launch_bounds__(NT) k_nd_leaf_solve(NdSolve<T> A, const T *__restrict__ cpl) {
-  __shared__ T S[4][R][2][TB], Z[4][R][2][TB];
-  const NdLevel &L = A.L;   // dx, dy: the leaves' depth
-  const size_t M = (size_t)L.nx * L.ny;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 31, half = lane >> 5;
-  const int k = blockIdx.x * 4 + wv;
-  const bool live = k < L.nbox;
-  const int kk = live ? k : 0, ix = kk >> L.dy, iy = kk & ((1 << L.dy) - 1);
+__device__ inline void nd_leaf_wave(const NdTree &t, const NdVec<T> &A, const T *X, const T *cpl, int k, T *uout,
+                                    T (*F)[R][2], int lane) {
+  const int nq = t.nq, nx = t.nx, ny = t.ny, c = lane & 31, half = lane >> 5;
+  const int ix = k >> t.Dy, iy = k & ((1 << t.Dy) - 1);
   int x0, w, y0, h;
-  nd_seg(L.nx, L.dx, ix, x0, w);
-  nd_seg(L.ny, L.dy, iy, y0, h);
+  nd_seg(nx, t.Dx, ix, x0, w);
+  nd_seg(ny, t.Dy, iy, y0, h);
   const int s = w * h, b = 2 * (w + h);
-  const int ci = c / h, cj = c % h;
-  const size_t cell = (size_t)(x0 + ci) * L.ny + y0 + cj;
-  const T *cp = cpl + (size_t)kk * TB * 2;
-  for (int q = half; q < R; q += 2) {
+  const T *cp = cpl + (size_t)k * TB * 2;
+  const T *Xk = X + (size_t)k * 2 * TB * TB + c;
+  const int sh = (s + 1) >> 1, ja = half * sh, jb = half ? s : sh;
+  wave_lds_fence();
+  for (int e = lane; e < TB * R; e += 64) {
+    const int j = e / R, q = e % R;
     T fr = 0, fi = 0;
-    if (live && c < s && q < A.nq) {
-      nd_rhs(A, cell, q, fr, fi);
+    if (j < s && q < nq) {
+      const int ci = j / h, cj = j - ci * h;
+      const size_t cell = (size_t)(x0 + ci) * ny + y0 + cj;
+      nd_ld(A.f, cell * nq + q, fr, fi);
       if (DOWN) {
-        // the four border neighbours of an edge cell (entry order L, R, B, T)
-        const T *v = A.v + 2 * M * q;
-        T cr, cim, xr, xi;
-        auto take = [&](int e, size_t nb) {
-          nd_ld(cp, e, cr, cim);
-          nd_ld(v, nb, xr, xi);
+        // the border neighbours of an edge cell (entry order L, R, B, T)
+        auto take = [&](int en, size_t nb) {
+          T cr, cim, xr, xi;
+          nd_ld(cp, en, cr, cim);
+          nd_ld((const T *)A.v, nb * nq + q, xr, xi);
           fr -= cr * xr - cim * xi;
           fi -= cr * xi + cim * xr;
         };
-        if (ci == 0) take(cj, cell - L.ny);
-        if (ci == w - 1) take(h + cj, x0 + w == L.nx ? (size_t)(y0 + cj) : cell + L.ny);
+        if (ci == 0) take(cj, cell - ny);
+        if (ci == w - 1) take(h + cj, x0 + w == nx ? (size_t)(y0 + cj) : cell + ny);
         if (cj == 0) take(2 * h + ci, cell - 1);
-        if (cj == h - 1) take(2 * h + w + ci, y0 + h == L.ny ? (size_t)(x0 + ci) * L.ny : cell + 1);
+        if (cj == h - 1) take(2 * h + w + ci, y0 + h == ny ? (size_t)(x0 + ci) * ny : cell + 1);
       }
     }
-    S[wv][q][0][c] = fr;
-    S[wv][q][1][c] = fi;
+    F[j][q][0] = fr;
+    F[j][q][1] = fi;
   }
-  __syncthreads();
+  wave_lds_fence();
   T ar[R], ai[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
-  const T *X = A.X + (size_t)kk * 2 * TB * TB + c;
-  const int sh = (s + 1) / 2, ja = half * sh, jb = half ? s : sh;
 #pragma unroll 4
   for (int j = ja; j < jb; ++j) {
-    const T gr = X[j * TB], gi = X[TB * TB + j * TB];
+    const T gr = Xk[j * TB], gi = Xk[TB * TB + j * TB];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      const T fr = S[wv][q][0][j], fi = S[wv][q][1][j];
+      const T fr = F[j][q][0], fi = F[j][q][1];
       ar[q] += gr * fr - gi * fi;
       ai[q] += gr * fi + gi * fr;
     }
@@ -1254,41 +1231,260 @@ __global__ void __launch_bounds__(NT) k_nd_leaf_solve(NdSolve<T> A, const T *__r
   for (int q = 0; q < R; ++q) {
     ar[q] += __shfl_xor(ar[q], 32);
     ai[q] += __shfl_xor(ai[q], 32);
-    if (DOWN) {
-      if (half == (q & 1) && live && c < s && q < A.nq) nd_out(A, cell, q, ar[q], ai[q]);
-    } else if (half == 0) {
-      Z[wv][q][0][c] = ar[q];
-      Z[wv][q][1][c] = ai[q];
-    }
   }
-  if (DOWN) return;
-  __syncthreads();
-  for (int q = half; q < A.nq; q += 2) {
-    if (!live || c >= b) continue;
-    const int p = c < h ? c : c < 2 * h ? (w - 1) * h + c - h : c < 2 * h + w ? (c - 2 * h) * h : (c - 2 * h - w) * h + h - 1;
+  if (DOWN) {
+    if (c < s) {
+      const int ci = c / h, cj = c - ci * h;
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if ((R == 1 ? half == 0 : half == (q & 1)) && q < nq)
+          nd_out(A.iex, A.iey, A.x, (size_t)nx * ny, x0 + ci, y0 + cj, ny, q, t.add, ar[q], ai[q]);
+    }
+    return;
+  }
+  wave_lds_fence();
+  if (half == 0)
+#pragma unroll
+    for (int q = 0; q < R; ++q) { F[c][q][0] = ar[q]; F[c][q][1] = ai[q]; }
+  wave_lds_fence();
+  for (int e = lane; e < b * R; e += 64) {
+    const int a = e / R, q = e % R;
+    if (q >= nq) continue;
+    const int p = a < h ? a : a < 2 * h ? (w - 1) * h + a - h : a < 2 * h + w ? (a - 2 * h) * h
+                                                                 : (a - 2 * h - w) * h + h - 1;
     T cr, cim;
-    nd_ld(cp, c, cr, cim);
-    const T zr = Z[wv][q][0][p], zi = Z[wv][q][1][p];
-    nd_st<T>(A.uout, ((size_t)k * A.nq + q) * L.b + c, -(cr * zr - cim * zi), -(cr * zi + cim * zr));
+    nd_ld(cp, a, cr, cim);
+    const T zr = F[p][q][0], zi = F[p][q][1];
+    nd_st<T>(uout, (size_t)a * nq + q, -(cr * zr - cim * zi), -(cr * zi + cim * zr));
   }
 }
 
-// r = b' - A x with b' = b, or D^-1 b in the transposed solve, and per
-// right-hand side the partial sums of |r|^2 (weighted by |D|^2 in the
-// transposed solve). A null x: r = b' and the partial sums of |b|^2. Blocks
-// take every gridDim.x-th piece of a row.
+// Box n of level L inside the subtree rooted at box (ix, iy) of level Lt
+__device__ inline int nd_sub_box(const NdLevel &Lt, int ix, int iy, int dx, int dy, int n) {
+  const int ex = dx - Lt.dx, ey = dy - Lt.dy;
+  return (((ix << ex) + (n >> ey)) << dy) + (iy << ey) + (n & ((1 << ey) - 1));
+}
+
+template <typename T, int R>
+__global__ void __launch_bounds__(64 * ND_TREE_WAVES) k_nd_up_tree(NdTree t, NdVec<T> A, const T *__restrict__ X,
+                                                                   const T *__restrict__ cpl) {
+  __shared__ __align__(16) T F[ND_TREE_WAVES][TB][R][2];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const NdLevel &Lt = t.lev[t.top];
+  const int root = blockIdx.x, ix = root >> Lt.dy, iy = root & ((1 << Lt.dy) - 1);
+  T *reg[2] = {A.u0 + (size_t)2 * t.reg0 * t.nq * root, A.u1 + (size_t)2 * t.reg1 * t.nq * root};
+  const int nleaf = 1 << (t.Dx - Lt.dx + t.Dy - Lt.dy);
+  for (int n = wv; n < nleaf; n += ND_TREE_WAVES)
+    nd_leaf_wave<T, R, false>(t, A, X, cpl, nd_sub_box(Lt, ix, iy, t.Dx, t.Dy, n),
+                              reg[0] + (size_t)2 * n * t.leaf_b * t.nq, F[wv], lane);
+  for (int l = 0; l <= t.top; ++l) {
+    __syncthreads();
+    const NdLevel &L = t.lev[l];
+    const int ey = L.dy - Lt.dy, count = 1 << (L.dx - Lt.dx + ey), chunks = (TB + L.bp + 63) / 64;
+    for (int it = wv; it < count * chunks; it += ND_TREE_WAVES) {
+      const int n = it / chunks, a = n >> ey, b = n & ((1 << ey) - 1);
+      const int n0 = L.ax == 0 ? ((2 * a) << ey) + b : (a << (ey + 1)) + 2 * b;
+      const int n1 = L.ax == 0 ? n0 + (1 << ey) : n0 + 1;
+      T *uout = l == t.top ? A.u2 + (size_t)2 * root * L.b * t.nq : reg[(l + 1) & 1] + (size_t)2 * n * L.b * t.nq;
+      nd_up_wave<T, R>(t, A, L, nd_sub_box(Lt, ix, iy, L.dx, L.dy, n), n0, n1, reg[l & 1], uout, it % chunks, F[wv],
+                       lane);
+    }
+  }
+}
+template <typename T, int R>
+__global__ void __launch_bounds__(64 * ND_TREE_WAVES) k_nd_down_tree(NdTree t, NdVec<T> A, const T *__restrict__ X,
+                                                                     const T *__restrict__ cpl) {
+  __shared__ __align__(16) T F[ND_TREE_WAVES][64][R][2];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const NdLevel &Lt = t.lev[t.top];
+  const int root = blockIdx.x, ix = root >> Lt.dy, iy = root & ((1 << Lt.dy) - 1);
+  for (int l = t.top; l >= 0; --l) {
+    const NdLevel &L = t.lev[l];
+    const int count = 1 << (L.dx - Lt.dx + L.dy - Lt.dy);
+    for (int n = wv; n < count; n += ND_TREE_WAVES) {
+      const int box = nd_sub_box(Lt, ix, iy, L.dx, L.dy, n);
+      if (L.s <= 8) nd_down_wave<T, R, 8>(t, A, L, box, F[wv], lane);
+      else if (L.s <= 16) nd_down_wave<T, R, 16>(t, A, L, box, F[wv], lane);
+      else nd_down_wave<T, R, 32>(t, A, L, box, F[wv], lane);
+    }
+    __syncthreads();
+  }
+  const int nleaf = 1 << (t.Dx - Lt.dx + t.Dy - Lt.dy);
+  for (int n = wv; n < nleaf; n += ND_TREE_WAVES)
+    nd_leaf_wave<T, R, true>(t, A, X, cpl, nd_sub_box(Lt, ix, iy, t.Dx, t.Dy, n), nullptr, F[wv], lane);
+}
+
+// Upwards, one level above the subtrees (and the root, whose z is x): 32
+// columns of [X | W] of one box per workgroup, the separator's rows spread
+// over its half waves.
+template <typename T, int R, int NW>
+__global__ void __launch_bounds__(64 * NW) k_nd_up(NdLevel L, NdVec<T> A, const T *__restrict__ uin,
+                                                   T *__restrict__ uout, int nq, int add) {
+  constexpr int RG = 2 * NW, JC = 256;
+  __shared__ __align__(16) union {
+    T f[JC][R][2];
+    T red[RG][2 * R][32];
+  } S;
+  const int tid = threadIdx.x, c32 = tid & 31, rg = tid >> 5;
+  const int chunks = (L.sp + L.bp) / 32, box = blockIdx.x / chunks, c = (blockIdx.x % chunks) * 32 + c32;
+  const NdBox B = nd_box(L, box);
+  const bool inX = c < L.sp;
+  const int pitch = inX ? L.sp : L.bp;
+  const size_t plane = (size_t)L.sp * pitch;
+  const T *m = A.data + (inX ? L.xoff + (size_t)box * 2 * plane + c : L.woff + (size_t)box * 2 * plane + c - L.sp);
+  T ar[R], ai[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
+  for (int j0 = 0; j0 < B.s; j0 += JC) {
+    const int nj = min(JC, B.s - j0);
+    if (j0) __syncthreads();
+    for (int e = tid; e < nj * R; e += 64 * NW) {
+      const int j = e / R, q = e % R;
+      T re = 0, im = 0;
+      if (q < nq) nd_fs(L, B, A.f, uin, B.k0, B.k1, nq, j0 + j, q, re, im);
+      S.f[j][q][0] = re;
+      S.f[j][q][1] = im;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int j = rg; j < nj; j += RG) {
+      const T gr = m[(size_t)(j0 + j) * pitch], gi = m[plane + (size_t)(j0 + j) * pitch];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const T fr = S.f[j][q][0], fi = S.f[j][q][1];
+        ar[q] += gr * fr - gi * fi;
+        ai[q] += gr * fi + gi * fr;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    S.red[rg][2 * q][c32] = ar[q];
+    S.red[rg][2 * q + 1][c32] = ai[q];
+  }
+  __syncthreads();
+  for (int e = tid; e < 32 * R; e += 64 * NW) {
+    const int cc = e & 31, q = e >> 5, col = (blockIdx.x % chunks) * 32 + cc;
+    if (q >= nq) continue;
+    T sr = 0, si = 0;
+#pragma unroll
+    for (int g = 0; g < RG; ++g) { sr += S.red[g][2 * q][cc]; si += S.red[g][2 * q + 1][cc]; }
+    if (col < B.s) {
+      int ci, cj;
+      nd_sep_ij(L, B, col, ci, cj);
+      nd_st<T>(A.v, ((size_t)ci * L.ny + cj) * nq + q, sr, si);
+      if (L.root) nd_out(A.iex, A.iey, A.x, (size_t)L.nx * L.ny, ci, cj, L.ny, q, add, sr, si);
+    } else if (col >= L.sp && col - L.sp < B.b) {
+      T ur, ui;
+      nd_fb(L, B, uin, B.k0, B.k1, nq, col - L.sp, q, ur, ui);
+      nd_st<T>(uout, ((size_t)box * L.b + col - L.sp) * nq + q, ur - sr, ui - si);
+    }
+  }
+}
+
+// Downwards, one level above the subtrees: 16 rows of W of one box per
+// workgroup; a lane reads its row in 16-byte pieces, the columns spread over
+// the quarter waves.
+constexpr int ND_DOWN_WAVES = 8;
+template <typename T, int R>
+__global__ void __launch_bounds__(64 * ND_DOWN_WAVES) k_nd_down(NdLevel L, NdVec<T> A, int nq, int add) {
+  constexpr int CC = 256, GROUPS = 4 * ND_DOWN_WAVES;
+  __shared__ __align__(16) union {
+    T x[CC][R][2];
+    T red[ND_DOWN_WAVES][2 * R][16];
+  } S;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r16 = lane & 15, grp = wv * 4 + (lane >> 4);
+  const int groups = (L.s + 15) / 16, box = blockIdx.x / groups, row = (blockIdx.x % groups) * 16 + r16;
+  const NdBox B = nd_box(L, box);
+  const size_t plane = (size_t)L.sp * L.bp;
+  const T *W = A.data + L.woff + (size_t)box * 2 * plane + (size_t)row * L.bp;
+  T ar[R], ai[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
+  for (int b0 = 0; b0 < B.b; b0 += CC) {
+    if (b0) __syncthreads();
+    const int nb = min(CC, L.bp - b0);
+    for (int e = tid; e < nb * R; e += 64 * ND_DOWN_WAVES) {
+      const int c = e / R, q = e % R;
+      T xr = 0, xi = 0;
+      if (b0 + c < B.b && q < nq)
+        nd_ld((const T *)A.v, nd_border_cell(L.nx, L.ny, L.dx, L.dy, B, b0 + c) * nq + q, xr, xi);
+      S.x[c][q][0] = xr;
+      S.x[c][q][1] = xi;
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int c = 4 * grp; c < nb; c += 4 * GROUPS) {
+      T gr[4], gi[4];
+      ld_row4(W + b0 + c, gr);
+      ld_row4(W + plane + b0 + c, gi);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const T xr = S.x[c + k][q][0], xi = S.x[c + k][q][1];
+          ar[q] += gr[k] * xr - gi[k] * xi;
+          ai[q] += gr[k] * xi + gi[k] * xr;
+        }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    ar[q] += __shfl_xor(ar[q], 16);
+    ai[q] += __shfl_xor(ai[q], 16);
+    ar[q] += __shfl_xor(ar[q], 32);
+    ai[q] += __shfl_xor(ai[q], 32);
+  }
+  __syncthreads();
+  if (lane < 16)
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      S.red[wv][2 * q][r16] = ar[q];
+      S.red[wv][2 * q + 1][r16] = ai[q];
+    }
+  __syncthreads();
+  for (int e = tid; e < 16 * R; e += 64 * ND_DOWN_WAVES) {
+    const int r = e & 15, q = e >> 4, j = (blockIdx.x % groups) * 16 + r;
+    if (q >= nq || j >= B.s) continue;
+    T sr = 0, si = 0;
+#pragma unroll
+    for (int w = 0; w < ND_DOWN_WAVES; ++w) { sr += S.red[w][2 * q][r]; si += S.red[w][2 * q + 1][r]; }
+    int ci, cj;
+    nd_sep_ij(L, B, j, ci, cj);
+    const size_t at = ((size_t)ci * L.ny + cj) * nq + q;
+    T zr, zi;
+    nd_ld((const T *)A.v, at, zr, zi);
+    zr -= sr;
+    zi -= si;
+    nd_st<T>(A.v, at, zr, zi);
+    nd_out(A.iex, A.iey, A.x, (size_t)L.nx * L.ny, ci, cj, L.ny, q, add, zr, zi);
+  }
+}
+
+// right-hand sides of one pass over the factor
+template <typename T> constexpr int nd_rhs_per_pass() { return sizeof(T) == 8 ? 4 : 8; }
+
+// The residual v = b' - A x with b' = b, or D^-1 b in the transposed solve,
+// scaled into f (a E v, by pass), and per right-hand side the partial sums of
+// |v|^2 (weighted by |D|^2 in the transposed solve). A null x: v = b' and the
+// partial sums of |b|^2. Blocks take every gridDim.x-th piece of a row.
 constexpr int ND_RES_RHS = 4;     // right-hand sides per thread (grid.y passes)
-__global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, const double *__restrict__ op,
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, double alpha, NdTab tb, const double *__restrict__ op,
                                                     const double *__restrict__ b, const double *__restrict__ x,
-                                                    double *__restrict__ r, int nrhs, int transpose,
+                                                    T *__restrict__ f, int nrhs, int transpose,
                                                     double *__restrict__ part) {
   __shared__ double red[ND_RES_RHS][NT];
+  constexpr int most = nd_rhs_per_pass<T>();
   const int nx = g.nx, ny = g.ny, tid = threadIdx.x, q0 = blockIdx.y * ND_RES_RHS;
   const int nq = min(ND_RES_RHS, nrhs - q0), cpr = (ny + NT - 1) / NT;
+  const int pass = q0 / most, per = min(most, nrhs - pass * most), at = q0 - pass * most;
   const size_t M = (size_t)nx * ny;
+  T *fp = f + 2 * M * (size_t)pass * most;
   double acc[ND_RES_RHS] = {0, 0, 0, 0};
   for (int piece = blockIdx.x; piece < nx * cpr; piece += gridDim.x) {
-    const int i = piece / cpr, j = (piece % cpr) * NT + tid;
+    const int i = piece / cpr, j = (piece - i * cpr) * NT + tid;
     if (j >= ny) continue;
     const size_t p = (size_t)i * ny + j;
     cd dinv = {1, 0};
@@ -1299,6 +1495,7 @@ __global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, const double *_
       dinv = cinv(d);
       w2 = d.r * d.r + d.i * d.i;
     }
+    const cd e = cscale(cmul(ld_c(tb.ex, i), ld_c(tb.ey, j)), alpha);
     if (!x) {
 #pragma unroll
       for (int q = 0; q < ND_RES_RHS; ++q)
@@ -1306,7 +1503,8 @@ __global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, const double *_
           cd v = ld_c(b + 2 * M * (q0 + q), p);
           acc[q] += v.r * v.r + v.i * v.i;
           if (transpose) v = cmul(v, dinv);
-          st_c(r + 2 * M * (q0 + q), p, v);
+          v = cmul(e, v);
+          nd_st<T>(fp, p * per + at + q, (T)v.r, (T)v.i);
         }
       continue;
     }
@@ -1327,7 +1525,8 @@ __global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, const double *_
         if (transpose) v = cmul(v, dinv);
         v = csub(v, a);
         acc[q] += w2 * (v.r * v.r + v.i * v.i);
-        st_c(r + 2 * M * (q0 + q), p, v);
+        v = cmul(e, v);
+        nd_st<T>(fp, p * per + at + q, (T)v.r, (T)v.i);
       }
   }
 #pragma unroll
@@ -1342,103 +1541,107 @@ __global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, const double *_
   if (tid < nq) part[(size_t)(q0 + tid) * gridDim.x + blockIdx.x] = red[tid][0];
 }
 
-// right-hand sides of one pass over the factor
-template <typename T> constexpr int nd_rhs_per_pass() { return sizeof(T) == 8 ? 4 : 8; }
-// u of one right-hand side: the largest level's, complex T
-inline size_t nd_u_entries(const NdPlan &P) {
-  size_t n = (size_t)P.nleaf * P.leaf_b;
-  for (int i = 0; i < P.nlev; ++i) n = std::max(n, (size_t)P.lev[i].nbox * P.lev[i].b);
-  return n;
+// The subtrees of a plan: the levels whose separators fit a tile, as far up as
+// leaves ND_TREE_BOXES of them (two workgroups of eight waves per CU). 512^2
+// complex64, a solve of 4 / 8 right-hand sides in three sweeps: 1469 / 2259 us
+// with 128 subtrees (half of the CUs idle), 1164 / 1735 with 256, 1042 / 1552
+// with 512, 1146 / 1683 with 1024 and 1311 / 1945 with 2048 (more launches
+// above); a launch per level for all of them took 1850 / 3610.
+inline NdTree nd_tree(const NdPlan &P) {
+  NdTree t;
+  memset(&t, 0, sizeof t);
+  t.nx = P.nx; t.ny = P.ny; t.Dx = P.Dx; t.Dy = P.Dy; t.leaf_b = P.leaf_b;
+  while (t.top + 1 < P.nlev && t.top + 1 < ND_TREE_MAX && P.lev[t.top + 1].sp <= TB &&
+         P.lev[t.top + 1].nbox >= ND_TREE_BOXES)
+    ++t.top;
+  const NdLevel &Lt = P.lev[t.top];
+  t.reg0 = (unsigned)((P.nleaf / Lt.nbox) * P.leaf_b);
+  for (int l = 0; l <= t.top; ++l) {
+    t.lev[l] = P.lev[l];
+    const unsigned n = (unsigned)(P.lev[l].nbox / Lt.nbox * P.lev[l].b);
+    if (l < t.top) {
+      if (l & 1) t.reg0 = std::max(t.reg0, n);
+      else t.reg1 = std::max(t.reg1, n);
+    }
+  }
+  // the levels above alternate between the same buffers, whole
+  for (int l = t.top + 1; l < P.nlev; ++l) {
+    const unsigned n = (unsigned)((P.lev[l].nbox * (size_t)P.lev[l].b + Lt.nbox - 1) / Lt.nbox);
+    if ((l - t.top) & 1) t.reg0 = std::max(t.reg0, n);
+    else t.reg1 = std::max(t.reg1, n);
+  }
+  return t;
 }
-// Solve workspace: r, v and two u buffers of one pass, norm partials, norms.
+// Solve workspace: f of every right-hand side, v and the u buffers of one
+// pass, norm partials, norms.
 struct NdSolveWork {
-  size_t r, v, u[2], part, norms, total;
+  size_t f, v, u[3], part, norms, total;
 };
 inline NdSolveWork nd_solve_layout(const NdPlan &P, int precision, int nrhs) {
   const size_t M = (size_t)P.nx * P.ny, es = elem_size(precision);
   const size_t R = std::min(nrhs, es == 8 ? nd_rhs_per_pass<double>() : nd_rhs_per_pass<float>());
+  const NdTree t = nd_tree(P);
+  const NdLevel &Lt = P.lev[t.top];
   NdSolveWork w;
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t at = off; off += align_up(bytes, 256); return at; };
-  w.r = take(16 * M * nrhs);
+  w.f = take(2 * es * M * nrhs);
   w.v = take(2 * es * M * R);
-  for (int i = 0; i < 2; ++i) w.u[i] = take(2 * es * nd_u_entries(P) * R);
+  w.u[0] = take(2 * es * R * t.reg0 * Lt.nbox);
+  w.u[1] = take(2 * es * R * t.reg1 * Lt.nbox);
+  w.u[2] = take(2 * es * R * Lt.b * Lt.nbox);
   w.part = take(8 * (size_t)2 * NORM_PARTS * nrhs);
   w.norms = take(8 * 2 * (size_t)nrhs);
   w.total = off;
   return w;
 }
 
-// x (+)= A^-1 r for nq <= R right-hand sides
+// x (+)= E^-1 M^-1 f for one pass
 template <typename T, int R>
-int nd_pass(const NdPlan &P, const NdTab &tb, double alpha, const T *data, const double *r, double *x, int nq, int add,
-            T *v, T *u0, T *u1, hipStream_t s) {
-  NdSolve<T> A;
-  memset(&A, 0, sizeof A);
-  A.tb = tb;
-  A.alpha = alpha;
-  A.r = r;
-  A.x = x;
-  A.v = v;
-  A.nq = nq;
-  A.add = add;
-  T *u[2] = {u0, u1};
-  NdLevel leaf;
-  memset(&leaf, 0, sizeof leaf);
-  leaf.nx = P.nx; leaf.ny = P.ny; leaf.dx = P.Dx; leaf.dy = P.Dy; leaf.nbox = P.nleaf; leaf.b = P.leaf_b;
-  A.L = leaf;
-  A.X = data + P.leaf_off;
-  A.uout = u[0];
-  hipLaunchKernelGGL((k_nd_leaf_solve<T, R, false>), dim3((P.nleaf + 3) / 4), dim3(NT), 0, s, A, data + P.leafc_off);
-  for (int l = 0; l <= P.nlev; ++l) {
+int nd_pass(const NdPlan &P, NdTree &t, const NdVec<T> &A, int nq, int add, hipStream_t s) {
+  t.nq = nq;
+  t.add = add;
+  const T *X = A.data + P.leaf_off, *cpl = A.data + P.leafc_off;
+  const int sub = P.lev[t.top].nbox;
+  hipLaunchKernelGGL((k_nd_up_tree<T, R>), dim3(sub), dim3(64 * ND_TREE_WAVES), 0, s, t, A, X, cpl);
+  T *uin = A.u2, *uout = A.u0;
+  for (int l = t.top + 1; l <= P.nlev; ++l) {
     const NdLevel &L = P.lev[l];
-    A.L = L;
-    A.X = data + L.xoff;
-    A.W = data + L.woff;
-    A.uin = u[l & 1];
-    A.uout = u[(l + 1) & 1];
-    const int tasks = L.nbox * ((L.sp + L.bp + 63) / 64);
-    if (L.sp <= TB)
-      hipLaunchKernelGGL((k_nd_up<T, R, 1>), dim3((tasks + 3) / 4), dim3(NdUp<T, R, 1>::THREADS), 0, s, A);
-    else if (L.sp <= 128)
-      hipLaunchKernelGGL((k_nd_up<T, R, 4>), dim3(tasks), dim3(NdUp<T, R, 4>::THREADS), 0, s, A);
+    const int grid = L.nbox * ((L.sp + L.bp) / 32);
+    if (L.s <= 128)
+      hipLaunchKernelGGL((k_nd_up<T, R, 4>), dim3(grid), dim3(256), 0, s, L, A, uin, uout, nq, add);
     else
-      hipLaunchKernelGGL((k_nd_up<T, R, 8>), dim3(tasks), dim3(NdUp<T, R, 8>::THREADS), 0, s, A);
+      hipLaunchKernelGGL((k_nd_up<T, R, 8>), dim3(grid), dim3(512), 0, s, L, A, uin, uout, nq, add);
+    uin = uout;
+    uout = uin == A.u0 ? A.u1 : A.u0;
   }
-  for (int l = P.nlev - 1; l >= 0; --l) {
+  for (int l = P.nlev - 1; l > t.top; --l) {
     const NdLevel &L = P.lev[l];
-    A.L = L;
-    A.W = data + L.woff;
-    if (L.sp <= TB)
-      hipLaunchKernelGGL((k_nd_down<T, R, 8>), dim3((L.nbox + 3) / 4), dim3(NT), 0, s, A);
-    else
-      hipLaunchKernelGGL((k_nd_down<T, R, 64>), dim3(L.nbox * ((L.s + 7) / 8)), dim3(NT), 0, s, A);
+    hipLaunchKernelGGL((k_nd_down<T, R>), dim3(L.nbox * ((L.s + 15) / 16)), dim3(64 * ND_DOWN_WAVES), 0, s, L, A, nq,
+                       add);
   }
-  A.L = leaf;
-  A.X = data + P.leaf_off;
-  hipLaunchKernelGGL((k_nd_leaf_solve<T, R, true>), dim3((P.nleaf + 3) / 4), dim3(NT), 0, s, A, data + P.leafc_off);
+  hipLaunchKernelGGL((k_nd_down_tree<T, R>), dim3(sub), dim3(64 * ND_TREE_WAVES), 0, s, t, A, X, cpl);
   HIP_TRY(hipGetLastError());
   return FDFD_OK;
 }
+// x (+)= E^-1 M^-1 f, f as k_nd_residual leaves it
 template <typename T>
-int nd_sweep(const NdPlan &P, const fdfd_grid *g, const void *factor, const double *r, double *x, int nrhs, int add,
-             char *work, const NdSolveWork &w, hipStream_t s) {
-  const double *tab = (const double *)((const char *)factor + ND_HEADER);
-  const T *data = (const T *)((const char *)factor + nd_data_off(P));
-  const NdTab tb = nd_tables(tab, P.nx, P.ny);
+int nd_sweep(const NdPlan &P, const void *factor, double *x, int nrhs, int add, char *work, const NdSolveWork &w,
+             hipStream_t s) {
+  const NdTab tb = nd_tables((const double *)((const char *)factor + ND_HEADER), P.nx, P.ny);
   const size_t M = (size_t)P.nx * P.ny;
-  T *v = (T *)(work + w.v), *u0 = (T *)(work + w.u[0]), *u1 = (T *)(work + w.u[1]);
-  const double alpha = nd_alpha(g);
+  NdTree t = nd_tree(P);
   constexpr int most = nd_rhs_per_pass<T>();
   for (int q0 = 0; q0 < nrhs; q0 += most) {
     const int nq = std::min(most, nrhs - q0);
-    const double *rq = r + 2 * M * q0;
-    double *xq = x + 2 * M * q0;
+    const NdVec<T> A{tb.iex, tb.iey, (const T *)((const char *)factor + nd_data_off(P)),
+                     (const T *)(work + w.f) + 2 * M * q0, (T *)(work + w.v), x + 2 * M * q0,
+                     (T *)(work + w.u[0]), (T *)(work + w.u[1]), (T *)(work + w.u[2])};
     int rc = FDFD_OK;
-    if (nq == 1) rc = nd_pass<T, 1>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
-    else if (nq == 2) rc = nd_pass<T, 2>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
-    else if (nq <= 4) rc = nd_pass<T, 4>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
-    else if constexpr (most >= 8) rc = nd_pass<T, 8>(P, tb, alpha, data, rq, xq, nq, add, v, u0, u1, s);
+    if (nq == 1) rc = nd_pass<T, 1>(P, t, A, nq, add, s);
+    else if (nq == 2) rc = nd_pass<T, 2>(P, t, A, nq, add, s);
+    else if (nq <= 4) rc = nd_pass<T, 4>(P, t, A, nq, add, s);
+    else if constexpr (most >= 8) rc = nd_pass<T, 8>(P, t, A, nq, add, s);
     if (rc) return rc;
   }
   return FDFD_OK;
@@ -1454,6 +1657,16 @@ inline bool nd_fits(const fdfd_grid *g, NdPlan *P) {
   return true;
 }
 
+// The launch of k_nd_residual of a solve
+template <typename T>
+void nd_residual(const fdfd_grid *g, const NdPlan &P, const double *op, const void *factor, const double *b,
+                 const double *x, int nrhs, int transpose, char *work, const NdSolveWork &w, int parts, hipStream_t s) {
+  hipLaunchKernelGGL(k_nd_residual<T>, dim3(parts, (nrhs + ND_RES_RHS - 1) / ND_RES_RHS), dim3(NT), 0, s, *g,
+                     nd_alpha(g), nd_tables((const double *)((const char *)factor + ND_HEADER), P.nx, P.ny), op, b, x,
+                     (T *)(work + w.f), nrhs, transpose, (double *)(work + w.part));
+}
+inline int nd_parts(const NdPlan &P) { return std::min(2 * NORM_PARTS, P.nx * ((P.ny + NT - 1) / NT)); }
+
 // The refinement of fdfd_solve with a nested-dissection factor: x = A^-1 b,
 // then x += A^-1 (b - A x) until every right-hand side meets the tolerance.
 // With a periodic axis a step is two sweeps, as on the block path. The first
@@ -1467,12 +1680,9 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
   if (!nd_fits(g, &P)) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
   const NdSolveWork w = nd_solve_layout(P, prec, nrhs);
   char *base = (char *)work;
-  double *r = (double *)(base + w.r), *part = (double *)(base + w.part), *norms = (double *)(base + w.norms);
-  const int cpr = (P.ny + NT - 1) / NT, parts = std::min(2 * NORM_PARTS, P.nx * cpr);
-  const dim3 rgrid(parts, (nrhs + ND_RES_RHS - 1) / ND_RES_RHS);
-  auto residual = [&](const double *xi) {
-    hipLaunchKernelGGL(k_nd_residual, rgrid, dim3(NT), 0, s, *g, op, b, xi, r, nrhs, transpose, part);
-  };
+  double *part = (double *)(base + w.part), *norms = (double *)(base + w.norms);
+  const int parts = nd_parts(P);
+  auto residual = [&](const double *xi) { nd_residual<T>(g, P, op, factor, b, xi, nrhs, transpose, base, w, parts, s); };
   fdfd_solve_stats st;
   memset(&st, 0, sizeof st);
   double *nr = host, *nb = host + nrhs, *rel = host + 2 * nrhs, *prev = host + 3 * nrhs;
@@ -1484,7 +1694,7 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
   for (int it = 1; it <= max_iter; ++it) {
     for (int k = 0; k < sweeps; ++k) {
       const bool first = it == 1 && k == 0;
-      if (int rc = nd_sweep<T>(P, g, factor, r, x, nrhs, first ? 0 : 1, base, w, s)) return rc;
+      if (int rc = nd_sweep<T>(P, factor, x, nrhs, first ? 0 : 1, base, w, s)) return rc;
       residual(x);
     }
     hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts, norms);
