@@ -90,7 +90,7 @@ SIGNATURES = {
     "fdfd_set_step_symmetry": (c_int, [c_int]),
     "fdfd_set_twist": (c_int, [c_int]),
     "fdfd_twist_block": (c_int, [_G]),
-    "fdfd_nd_supported": (c_int, [_G]),
+    "fdfd_nd_supported": (c_int, [_G, c_int]),
     "fdfd_nd_front": (c_int, [_G, c_int, c_int, POINTER(c_int32), POINTER(ctypes.c_int64), POINTER(c_int32)]),
 }
 

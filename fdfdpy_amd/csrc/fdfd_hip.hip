@@ -3614,7 +3614,7 @@ namespace {
 int factor_is_nd(const fdfd_grid *g, const void *factor, int precision, hipStream_t s, bool *nd, NdPlan *P) {
   *nd = false;
   if (precision & (FDFD_FACTOR_STEPWISE | FDFD_FACTOR_PIVOT)) return FDFD_OK;
-  if (!nd_fits(g, P)) {
+  if (!nd_fits(g, precision, P)) {
     if (precision & FDFD_FACTOR_ND) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
     return FDFD_OK;
   }
@@ -3638,7 +3638,7 @@ size_t fdfd_factor_bytes(const fdfd_grid *g, int precision) {
   if (check_grid(g) || check_prec(precision)) return 0;
   if (precision & FDFD_FACTOR_ND) {
     NdPlan P;
-    if (!nd_fits(g, &P)) { fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range"); return 0; }
+    if (!nd_fits(g, precision, &P)) { fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range"); return 0; }
     return nd_factor_bytes(g, P, precision);
   }
   return factor_total_bytes(g, precision);
@@ -3647,7 +3647,7 @@ size_t fdfd_factor_workspace_bytes(const fdfd_grid *g, int precision) {
   if (check_grid(g) || check_prec(precision)) return 0;
   if (precision & FDFD_FACTOR_ND) {
     NdPlan P;
-    if (!nd_fits(g, &P)) { fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range"); return 0; }
+    if (!nd_fits(g, precision, &P)) { fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range"); return 0; }
     return nd_work_layout(P, precision).total;
   }
   return factor_work_bytes(g, precision);
@@ -4181,16 +4181,16 @@ int fdfd_twist_block(const fdfd_grid *g) {
   return twist_block(g);
 }
 
-int fdfd_nd_supported(const fdfd_grid *g) {
+int fdfd_nd_supported(const fdfd_grid *g, int precision) {
   NdPlan P;
-  if (check_grid(g)) return -1;
-  return g_twist.load() && nd_fits(g, &P) ? 1 : 0;
+  if (check_grid(g) || check_prec(precision)) return -1;
+  return g_twist.load() && nd_fits(g, precision, &P) ? 1 : 0;
 }
 
 int fdfd_nd_front(const fdfd_grid *g, int level, int box, int32_t *info, int64_t *cells, int32_t *map) {
   if (int rc = check_grid(g)) return rc;
   NdPlan P;
-  if (!info || !nd_fits(g, &P)) return fail(FDFD_ERR_ARG, "fdfd_nd_front: bad arguments, or a grid outside its range");
+  if (!info || !nd_plan(g, &P)) return fail(FDFD_ERR_ARG, "fdfd_nd_front: bad arguments, or a grid outside its range");
   NdLevel L;
   memset(&L, 0, sizeof L);
   if (level == -1) {

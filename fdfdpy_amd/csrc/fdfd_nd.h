@@ -30,7 +30,7 @@
 // order: no atomics, the same bits on every run.
 
 constexpr int ND_LEAF = 32;        // most cells of a leaf box: one pivot tile
-constexpr int ND_MIN_SIDE = 64;    // shorter grid side the path takes
+constexpr int ND_MIN_SIDE = 16;    // shorter grid side of a tree (measured: nd_fits)
 constexpr int ND_MAX_LEVELS = 40;
 constexpr size_t ND_HEADER = 256;  // the tag, at the start of the factor
 __host__ __device__ inline unsigned long long nd_tag(int i) {
@@ -1648,12 +1648,23 @@ int nd_sweep(const NdPlan &P, const void *factor, double *x, int nrhs, int add, 
 }
 
 // The path's range: a plan exists and its solve fits the workspace that
-// fdfd_solve_workspace_bytes reports without knowing the factor's kind
-inline bool nd_fits(const fdfd_grid *g, NdPlan *P) {
+// fdfd_solve_workspace_bytes reports without knowing the factor's kind. FP64,
+// new permittivity and solve / resident solve through Simulation, block path
+// against tree: 16 x 16 1.16 / 0.63 against 0.56 / 0.26 ms, 32 x 32 1.46 /
+// 0.85 against 0.61 / 0.26, 48 x 40 2.52 / 0.98 against 0.65 / 0.23, 63 x 63
+// 3.21 / 1.13 against 0.72 / 0.25; below 16 cells a tree has hardly a level.
+// Complex64 factors of grids with a side below 64 cells stay block factors:
+// how far their refinement gets in a given number of steps, and that a
+// singular leading pivot sends them to FP64, is what the fallback order is
+// tested on (a new permittivity and solve of 48 x 40 cells takes 2.17 ms
+// there; 0.94 as a tree).
+constexpr int ND_MIN_SIDE_C64 = 64;
+inline bool nd_fits(const fdfd_grid *g, int precision, NdPlan *P) {
+  const int prec = base_prec(precision);
+  if (prec == FDFD_PREC_C64 && std::min(g->nx, g->ny) < ND_MIN_SIDE_C64) return false;
   if (!nd_plan(g, P)) return false;
-  for (int prec = 0; prec < 2; ++prec)
-    for (int k = 1; k <= 8; ++k)
-      if (nd_solve_layout(*P, prec, k).total > solve_work_bytes(g, prec, k)) return false;
+  for (int k = 1; k <= 8; ++k)
+    if (nd_solve_layout(*P, prec, k).total > solve_work_bytes(g, prec, k)) return false;
   return true;
 }
 
@@ -1677,7 +1688,7 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
              hipStream_t s, double *host) {
   const int prec = sizeof(T) == 8 ? FDFD_PREC_FP64 : FDFD_PREC_C64;
   NdPlan P;
-  if (!nd_fits(g, &P)) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
+  if (!nd_fits(g, prec, &P)) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
   const NdSolveWork w = nd_solve_layout(P, prec, nrhs);
   char *base = (char *)work;
   double *part = (double *)(base + w.part), *norms = (double *)(base + w.norms);

@@ -159,13 +159,12 @@ class DeviceOperator:
         self.engine = None       # FactorEngine shared with other operators, if any
 
     # -- sizes ----------------------------------------------------------
-    @property
-    def nested(self):
+    def nested(self, precision):
         """The next factor is a nested-dissection one (unless it pivots or an engine builds it)."""
-        return self.lib.fdfd_nd_supported(ctypes.byref(self.grid)) == 1
+        return self.lib.fdfd_nd_supported(ctypes.byref(self.grid), L.PREC[precision]) == 1
 
     def factor_bytes(self, precision):
-        if self.nested:
+        if self.nested(precision):
             return self.nd_bytes[precision]
         return int(self.lib.fdfd_factor_bytes(ctypes.byref(self.grid), L.PREC[precision]))
 
@@ -221,7 +220,7 @@ class DeviceOperator:
             if not refresh or (ver == self.version and piv == pivot and not blocks):
                 return fac
         g = ctypes.byref(self.grid)
-        if self.nested and not pivot and not stepwise and self.engine is None:
+        if self.nested(precision) and not pivot and not stepwise and self.engine is None:
             p = L.PREC[precision] | L.FACTOR_ND
         else:
             p = L.PREC[precision] | (L.FACTOR_PIVOT if pivot else 0) | (L.FACTOR_STEPWISE if stepwise else 0)
@@ -275,7 +274,7 @@ class DeviceOperator:
         if fallback:
             # last resort: partial pivoting inside the 32x32 pivot tiles
             plan.append(("fp64", True, True, False))
-        elif self.nested:
+        elif self.nested(precision):
             plan.append((precision, False, True, True))
         rep, failed, spent = None, [], [0.0, 0.0, 0]
         for prec, piv, refresh, blocks in plan:

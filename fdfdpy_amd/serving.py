@@ -170,7 +170,7 @@ class ServingEngine:
                 reused = True
             else:
                 op = DeviceOperator(p.shape, p.omega, p.dl, p.npml, p.pol, p.L0, self.device)
-                if not op.nested:   # block factorizations share step launches
+                if not op.nested(self.precision):   # block factorizations share step launches
                     op.engine = self._engine_for(stream)
                 op.set_eps(p.eps)
             b = torch.as_tensor(p.rhs(), device=self.device)

@@ -292,10 +292,10 @@ int fdfd_set_twist(int on);
 int fdfd_twist_block(const fdfd_grid *g);
 
 /* 1 when FDFD_FACTOR_ND is the factor of choice for this grid (its shorter
- * side has 64 cells or more), 0 when not (also while fdfd_set_twist(0) asks
- * for the one-chain order), -1 for an invalid grid. No reference
- * counterpart. */
-int fdfd_nd_supported(const fdfd_grid *g);
+ * side has 16 cells or more, 64 in complex64), 0 when not (also while
+ * fdfd_set_twist(0) asks for the one-chain order), -1 for invalid
+ * arguments. No reference counterpart. */
+int fdfd_nd_supported(const fdfd_grid *g, int precision);
 
 /* One front of the nested-dissection tree of g, on the host (no GPU; no
  * reference counterpart): level -1 the leaves, 0 .. nlev - 1 the merges

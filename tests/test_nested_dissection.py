@@ -85,7 +85,8 @@ def _multifrontal(nx, ny, A, b):
 
 
 @pytest.mark.parametrize("N,npml,pol", [((64, 64), [8, 8], "Ez"), ((65, 97), [9, 0], "Hz"), ((200, 64), [10, 10], "Ez"),
-                                        ((71, 130), [0, 0], "Ez"), ((64, 230), [8, 12], "Hz")])
+                                        ((71, 130), [0, 0], "Ez"), ((64, 230), [8, 12], "Hz"), ((16, 16), [4, 4], "Ez"),
+                                        ((17, 90), [0, 9], "Hz"), ((31, 23), [5, 5], "Ez")])
 def test_tree_and_maps_solve_the_periodic_operator(N, npml, pol):
     rng = np.random.default_rng(N[0] + N[1])
     A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], _eps(rng, N), npml, pol, 1e-6)
@@ -94,55 +95,58 @@ def test_tree_and_maps_solve_the_periodic_operator(N, npml, pol):
 
 
 def test_range_and_sizes():
-    """Every grid whose shorter side has 64 cells or more is in the range,
-    smaller ones are not; flags that exclude each other are refused; the two
-    kinds of factor never have one size."""
+    """Every grid whose shorter side has 16 cells or more (64 in complex64) is
+    in the range, smaller ones are not; flags that exclude each other are
+    refused; the two kinds of factor never have one size."""
     lib = L.lib()
 
     def grid(nx, ny):
         return ctypes.byref(L.FdfdGrid(nx, ny, 10, 10, 0, 0, OMEGA, 0.02, 1e-6))
-    for n in list(range(64, 460)) + [511, 512, 513, 768, 1023, 1500, 2047, 2048]:
-        for m in (64, n, n + 1, 2 * n + 1):
-            if min(n, m) > 2048 or m < 2:
-                continue
+    for n in list(range(16, 460)) + [511, 512, 513, 768, 1023, 1500, 2047, 2048]:
+        for m in (16, 64, n, n + 1, 2 * n + 1):
             ny, nx = min(n, m), max(n, m)
-            assert lib.fdfd_nd_supported(grid(nx, ny)) == 1, (nx, ny)
             for prec in (0, 1):
+                assert lib.fdfd_nd_supported(grid(nx, ny), prec) == (prec == 0 or ny >= 64), (nx, ny)
+                if prec == 1 and ny < 64:
+                    continue
                 nd = lib.fdfd_factor_bytes(grid(nx, ny), prec | L.FACTOR_ND)
                 assert nd > 0 and nd != lib.fdfd_factor_bytes(grid(nx, ny), prec)
-    for shape in ((63, 64), (64, 63), (500, 40), (2, 2)):
-        assert lib.fdfd_nd_supported(grid(*shape)) == 0
-        assert lib.fdfd_factor_bytes(grid(*shape), L.FACTOR_ND) == 0
+    for shape, prec in (((63, 64), 1), ((64, 63), 1), ((500, 15), 0), ((15, 16), 0), ((2, 2), 0)):
+        assert lib.fdfd_nd_supported(grid(*shape), prec) == 0
+        assert lib.fdfd_factor_bytes(grid(*shape), prec | L.FACTOR_ND) == 0
     for bad in (L.FACTOR_ND | L.FACTOR_PIVOT, L.FACTOR_ND | L.FACTOR_STEPWISE):
         assert lib.fdfd_factor_bytes(grid(128, 128), bad) == 0
     prev = lib.fdfd_set_twist(0)
     try:   # the one-chain order is a block factorization
-        assert lib.fdfd_nd_supported(grid(128, 128)) == 0
+        assert lib.fdfd_nd_supported(grid(128, 128), 0) == 0
     finally:
         lib.fdfd_set_twist(prev)
 
 
-def _device(N, npml, pol, eps):
+def _device(N, npml, pol, eps, precision):
     from fdfdpy_amd.device import DeviceOperator
     op = DeviceOperator(N, OMEGA, 0.02, npml, pol, 1e-6, DEV)
     op.set_eps(eps)
-    assert op.nested
+    assert op.nested(precision)
     return op
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,npml,pol,nrhs", [
     ((64, 64), [8, 8], "Ez", 1), ((65, 97), [9, 12], "Hz", 2), ((128, 66), [10, 0], "Ez", 3),
-    ((129, 70), [0, 0], "Hz", 5), ((64, 300), [8, 15], "Ez", 8), ((257, 96), [20, 10], "Hz", 9)])
+    ((129, 70), [0, 0], "Hz", 5), ((64, 300), [8, 15], "Ez", 8), ((257, 96), [20, 10], "Hz", 9),
+    ((16, 16), [4, 4], "Ez", 1), ((17, 120), [0, 10], "Hz", 4), ((33, 32), [6, 6], "Ez", 5), ((47, 63), [9, 9], "Hz", 2)])
 @pytest.mark.parametrize("precision", ["fp64", "c64"])
 def test_solves_match_the_oracle(N, npml, pol, nrhs, precision):
     """Edges of the tree (power-of-two sides and their neighbours, long
     grids), both polarizations, periodic axes, a lossy cell, every count of
     right-hand sides per pass; forward and transposed."""
+    if precision == "c64" and min(N) < 64:
+        pytest.skip("complex64 factors of grids below 64 cells are block factors")
     rng = np.random.default_rng(sum(N) + nrhs)
     eps = _eps(rng, N).astype(complex)
     eps[N[0] // 2:, N[1] // 2:] += 0.3j
-    op = _device(N, npml, pol, eps)
+    op = _device(N, npml, pol, eps, precision)
     A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], eps, npml, pol, 1e-6)
     b = rng.standard_normal((nrhs,) + N) + 1j * rng.standard_normal((nrhs,) + N)
     for transpose, M in ((False, A), (True, A.T.tocsr())):
@@ -161,7 +165,7 @@ def test_kinds_are_told_apart_and_repeat_to_the_bit(precision):
     zero right-hand side gives zeros without a sweep."""
     N = (90, 101)
     rng = np.random.default_rng(7)
-    op = _device(N, [10, 10], "Ez", _eps(rng, N))
+    op = _device(N, [10, 10], "Ez", _eps(rng, N), precision)
     lib, g, pr = L.lib(), ctypes.byref(op.grid), L.PREC[precision]
     fac = op.factor(precision)
     first = fac.clone()
@@ -199,7 +203,7 @@ def test_stall_without_fallback_takes_the_block_factor(monkeypatch):
     N = (80, 72)
     rng = np.random.default_rng(3)
     eps = _eps(rng, N)
-    op = _device(N, [9, 9], "Ez", eps)
+    op = _device(N, [9, 9], "Ez", eps, "c64")
     real = DeviceOperator._solve_one
 
     def stalled(self, *a, **k):
