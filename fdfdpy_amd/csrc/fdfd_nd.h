@@ -363,10 +363,16 @@ __device__ inline unsigned row16_max(unsigned v) {
   v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
   return v;
 }
+// rows: the tile's rows that are not identity padding; the pairs beyond are
+// left alone (the step count is (rows + 1) / 2).
+// Tried: a fifth wave that keeps the diagonal blocks and picks and inverts the
+// next pair while the others update, which halves their instructions; its own
+// chain per step is then the longer one (a 512 x 512 complex64 step 17 -> 20
+// us, the leaves 110 -> 296 us).
 template <typename T, typename LT>
-__device__ void tile_inverse_pairs(LT &L, int *status) {
+__device__ void tile_inverse_pairs(LT &L, int rows, int *status) {
   static_assert(TB * TB == 4 * NT, "4 elements per thread");
-  static_assert(2 * sizeof(InvX<T>) <= offsetof(LT, mag), "exchange buffers overlay the tiles only");
+  static_assert(2 * sizeof(InvX<T>) <= offsetof(LT, end), "exchange buffers overlay the tiles only");
   const int tid = threadIdx.x, lane = tid & 63;
   const int i = tid >> 3, c0 = (tid & 7) * 4;
   T ar[4], ai[4];
@@ -378,10 +384,10 @@ __device__ void tile_inverse_pairs(LT &L, int *status) {
   }
   __syncthreads();   // every row is in registers before the exchange buffers cover Ar, Ai
   InvX<T> *X = reinterpret_cast<InvX<T> *>(&L);
-  const int mine = lane & 15, d = 2 * mine;
-  bool bad = false, taken = false;
+  const int mine = lane & 15, d = 2 * mine, pairs = min(TB, rows + 1) >> 1;
+  bool bad = false, taken = mine >= pairs;
 #pragma unroll 2
-  for (int st = 0; st < TB / 2; ++st) {
+  for (int st = 0; st < pairs; ++st) {
     InvX<T> &B = X[st & 1];
     lds_st4(&B.r[i][c0], ar);
     lds_st4(&B.i[i][c0], ai);
@@ -453,13 +459,28 @@ __device__ void tile_inverse_pairs(LT &L, int *status) {
   __syncthreads();
 }
 
+// LDS of the kernels that invert a tile: A (the tile, then its inverse), B
+// (with A: the exchange buffers of the inverse) and, where used, a third tile.
+template <typename T> struct NdLds2 {
+  T Ar[TB][TBP], Ai[TB][TBP];
+  T Br[TB][TBP], Bi[TB][TBP];
+  unsigned char pad[step_lds_pad<T>()];
+  int end[4];
+};
+template <typename T> struct NdLds3 {
+  T Ar[TB][TBP], Ai[TB][TBP];
+  T Br[TB][TBP], Bi[TB][TBP];
+  T Pr[TB][TBP], Pi[TB][TBP];
+  int end[4];
+};
+
 // A leaf box per workgroup: its five-point matrix (cells in (x, y) order,
 // identity beyond) inverted as one pivot tile; X, the border couplings c and
 // the update C[a][b] = -c_a X[p_a][p_b] c_b, p_a the cell inside border cell a.
 template <typename T>
 __global__ void __launch_bounds__(NT) k_nd_leaf(int nx, int ny, int Dx, int Dy, NdBands<T> bd, T *__restrict__ X,
                                                 T *__restrict__ cpl, T *__restrict__ C, int *status) {
-  __shared__ Lds<T> L;
+  __shared__ NdLds2<T> L;
   __shared__ T cr[TB], ci[TB];
   __shared__ int cp[TB];
   const int tid = threadIdx.x, k = blockIdx.x;
@@ -507,10 +528,13 @@ __global__ void __launch_bounds__(NT) k_nd_leaf(int nx, int ny, int Dx, int Dy, 
     nd_st<T>(cpl, (size_t)k * TB + tid, re, im);
   }
   __syncthreads();
-  tile_inverse_pairs<T>(L, status);
+  tile_inverse_pairs<T>(L, s, status);
   T *Xk = X + (size_t)k * 2 * TB * TB, *Ck = C + (size_t)k * 2 * TB * TB;
-  store4(Xk + a * TB + b0, &L.Ar[a][b0]);
-  store4(Xk + TB * TB + a * TB + b0, &L.Ai[a][b0]);
+  if (a < s) {
+    store4(Xk + a * TB + b0, &L.Ar[a][b0]);
+    store4(Xk + TB * TB + a * TB + b0, &L.Ai[a][b0]);
+  }
+  if (a >= b) return;
   T vr[4], vi[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
@@ -607,7 +631,7 @@ template <typename T> struct NdStep {
 // children, and the inverse of the first pivot tile.
 template <typename T>
 __global__ void __launch_bounds__(NT) k_nd_front(NdStep<T> A) {
-  __shared__ Lds<T> S;
+  __shared__ NdLds2<T> S;
   const NdLevel &L = A.L;
   const int ns = L.sp / TB, nb = L.bp / TB, tri = ns * (ns + 1) / 2, per = tri + ns * nb;
   int box, t;
@@ -651,7 +675,7 @@ __global__ void __launch_bounds__(NT) k_nd_front(NdStep<T> A) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) { S.Ar[a][b0 + u] = re[u]; S.Ai[a][b0 + u] = im[u]; }
       __syncthreads();
-      tile_inverse_pairs<T>(S, A.status);
+      tile_inverse_pairs<T>(S, B.s, A.status);
       store_pinv(S, A.P0 + (size_t)box * 2 * TB * TB);
       return;
     }
@@ -689,7 +713,7 @@ __global__ void __launch_bounds__(NT) k_nd_front(NdStep<T> A) {
 // contracts by 0.03-0.2 per sweep instead of 2e-4.)
 template <typename T>
 __global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
-  __shared__ Lds<T> S;
+  __shared__ NdLds3<T> S;
   const NdLevel &L = A.L;
   const int ns = L.sp / TB, nb = L.bp / TB, tri = ns * (ns + 1) / 2, per = tri + ns * nb, p = A.p;
   const bool last = p == ns - 1;
@@ -787,7 +811,7 @@ __global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
   acc_to_lds<T>(cr, ci, S.Ar, S.Ai, qi, qj, lane);
   __syncthreads();
   if (crit) {   // replaced by its inverse at the next step and read by nobody before
-    tile_inverse_pairs<T>(S, A.status);
+    tile_inverse_pairs<T>(S, nd_box(L, box).s - (p + 1) * TB, A.status);
     store_pinv(S, A.P1 + (size_t)box * 2 * TB * TB);
     return;
   }
@@ -912,6 +936,145 @@ __global__ void __launch_bounds__(NT) k_nd_update(NdLevel L, const T *__restrict
   store4(D + bp * bp + ((size_t)J * TB + a) * bp + I * TB + b0, im);
 }
 
+// A whole merge of boxes whose separator fits one tile, in one launch: X, W
+// and the update C, a workgroup per box. The border rows U = F_sb of all column
+// tiles wait in LDS (dynamic, nb tiles after the fixed part), so the children
+// are read once; C's own children entries are fetched while the matrix cores
+// form U^T W. Rows beyond the separator and the border are not written.
+// Bound by the instructions around its short products (indices, the inverse):
+// 512^2 complex64, boxes of 7 x 7, 15 x 7, 15 x 15 and 31 x 15: 148, 109, 67 and
+// 53 us as a launch each for the front, the step and the update, 67, 65, 45 and
+// 42 us here; 768^2 FP64, 11 x 5 and 11 x 11: 239 and 270 us.
+// A: F_ss, then P, then C_IJ on its way out; B: W_J.
+template <typename T>
+__global__ void __launch_bounds__(NT) k_nd_merge(NdLevel L, NdBands<T> bd, const T *__restrict__ Cin, T *__restrict__ X,
+                                                 T *__restrict__ W, T *__restrict__ Cout, int *status) {
+  extern __shared__ __align__(16) unsigned char nd_smem[];
+  NdLds2<T> &M = *reinterpret_cast<NdLds2<T> *>(nd_smem);
+  typedef T Tile[2][TB][TBP];
+  Tile *U = reinterpret_cast<Tile *>(nd_smem + sizeof(NdLds2<T>));
+  const int box = nd_item(blockIdx.x, L.nbox);
+  if (box < 0) return;
+  const int nb = L.bp / TB;
+  const NdBox B = nd_box(L, box);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, qi = wv >> 1, qj = wv & 1;
+  const int a = tid >> 3, b0 = (tid & 7) * 4;
+  int r0 = -1, r1 = -1, c0[4], c1[4];
+  T re[4], im[4];
+  if (a < B.s) nd_sep_map(L, B, a, r0, r1);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    c0[u] = c1[u] = -1;
+    if (b0 + u < B.s) nd_sep_map(L, B, b0 + u, c0[u], c1[u]);
+  }
+  nd_children(L, B, Cin, r0, r1, c0, c1, re, im);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    T mr = a == b0 + u ? T(1) : T(0), mi = 0;
+    if (a < B.s && b0 + u < B.s) nd_own_ss(L, B, bd, a, b0 + u, mr, mi);
+    M.Ar[a][b0 + u] = re[u] + mr;
+    M.Ai[a][b0 + u] = im[u] + mi;
+  }
+  for (int J = 0; J < nb; ++J) {
+    const int j0 = J * TB + b0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      c0[u] = c1[u] = -1;
+      if (j0 + u < B.b) nd_border_map(L, B, j0 + u, c0[u], c1[u]);
+    }
+    nd_children(L, B, Cin, r0, r1, c0, c1, re, im);
+    if (a == 0 || a == B.s - 1)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) nd_own_sb(L, B, bd, a, j0 + u, re[u], im[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { U[J][0][a][b0 + u] = re[u]; U[J][1][a][b0 + u] = im[u]; }
+  }
+  __syncthreads();
+  tile_inverse_pairs<T>(M, B.s, status);
+  if (a < B.s) {
+    T *D = X + (size_t)box * 2 * TB * TB + a * TB + b0;
+    store4(D, &M.Ar[a][b0]);
+    store4(D + TB * TB, &M.Ai[a][b0]);
+  }
+  // P as the left operand of W_J = P U_J, kept in registers: its tile becomes
+  // the staging tile of C (cgemm_quad's order of the inner index)
+  const int lr = lane & 15, k0 = (lane >> 5) + 16 * ((lane >> 4) & 1);
+  T pr[8], pi[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) { pr[t] = M.Ar[qi * 16 + lr][2 * t + k0]; pi[t] = M.Ai[qi * 16 + lr][2 * t + k0]; }
+  const size_t bp = L.bp, pb = TB * bp;
+  T *C = Cout + (size_t)box * 2 * bp * bp;
+  for (int J = 0; J < nb; ++J) {
+    typename Mfma<T>::v4 wr = {0, 0, 0, 0}, wi = {0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const T br = U[J][0][2 * t + k0][qj * 16 + lr], bi = U[J][1][2 * t + k0][qj * 16 + lr];
+      wr = Mfma<T>::mac(pr[t], br, wr);
+      wr = Mfma<T>::mac(-pi[t], bi, wr);
+      wi = Mfma<T>::mac(pr[t], bi, wi);
+      wi = Mfma<T>::mac(pi[t], br, wi);
+    }
+    acc_to_lds<T>(wr, wi, M.Br, M.Bi, qi, qj, lane);
+    int d0[4], d1[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      d0[u] = d1[u] = -1;
+      if (J * TB + b0 + u < B.b) nd_border_map(L, B, J * TB + b0 + u, d0[u], d1[u]);
+    }
+    __syncthreads();   // W_J is in place (and, at J = 0, every wave has its P)
+    if (a < B.s) {
+      T *D = W + (size_t)box * 2 * pb + (size_t)a * bp + J * TB + b0;
+      store4(D, &M.Br[a][b0]);
+      store4(D + pb, &M.Bi[a][b0]);
+    }
+    for (int I = 0; I <= J; ++I) {
+      int e0 = -1, e1 = -1;
+      if (I * TB + a < B.b) nd_border_map(L, B, I * TB + a, e0, e1);
+      nd_children(L, B, Cin, e0, e1, d0, d1, re, im);
+      typename Mfma<T>::v4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+      cgemm_quad_tn<T>(cr, ci, U[I][0], U[I][1], M.Br, M.Bi, qi, qj, lane, T(-1));
+      acc_to_lds<T>(cr, ci, M.Ar, M.Ai, qi, qj, lane);
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        M.Ar[a][b0 + u] = re[u] += M.Ar[a][b0 + u];
+        M.Ai[a][b0 + u] = im[u] += M.Ai[a][b0 + u];
+      }
+      __syncthreads();
+      if (I == J) {   // a diagonal tile's lower triangle mirrors its upper one
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (b0 + u < a) { re[u] = M.Ar[b0 + u][a]; im[u] = M.Ai[b0 + u][a]; }
+      }
+      if (I * TB + a < B.b) {
+        T *E = C + ((size_t)I * TB + a) * bp + J * TB + b0;
+        store4(E, re);
+        store4(E + bp * bp, im);
+      }
+      if (I != J && J * TB + a < B.b) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { re[u] = M.Ar[b0 + u][a]; im[u] = M.Ai[b0 + u][a]; }
+        T *E = C + ((size_t)J * TB + a) * bp + I * TB + b0;
+        store4(E, re);
+        store4(E + bp * bp, im);
+      }
+      __syncthreads();   // the tile is read before the next one replaces it
+    }
+  }
+}
+// Which levels k_nd_merge takes: one tile of separator, a border of at most
+// nd_merge_tiles tiles (wider ones are few boxes with more tiles than one
+// workgroup should form: with 4 and 6 tiles, 256 and 128 boxes, 75 and 72 us
+// here, 46 and 45 as a launch each for front, step and update; FP64 with 3
+// tiles and 85 KB of LDS 311 against 293)
+template <typename T> constexpr int nd_merge_tiles() { return sizeof(T) == 8 ? 2 : 3; }
+template <typename T>
+inline bool nd_merges(const NdLevel &L) { return !L.root && L.sp == TB && L.bp <= nd_merge_tiles<T>() * TB; }
+template <typename T>
+inline size_t nd_merge_lds(const NdLevel &L) {
+  return sizeof(NdLds2<T>) + (size_t)(L.bp / TB) * 2 * TB * TBP * sizeof(T);
+}
+
 template <typename T>
 int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hipStream_t s) {
   const int prec = sizeof(T) == 8 ? FDFD_PREC_FP64 : FDFD_PREC_C64;
@@ -933,6 +1096,11 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
   T *C[2] = {(T *)(base + w.C[0]), (T *)(base + w.C[1])};
   T *S[2] = {(T *)(base + w.S[0]), (T *)(base + w.S[1])}, *Bf[2] = {(T *)(base + w.B[0]), (T *)(base + w.B[1])};
   T *pv[2] = {(T *)(base + w.pinv[0]), (T *)(base + w.pinv[1])};
+  static std::once_flag lds_attr;
+  std::call_once(lds_attr, [] {
+    (void)hipFuncSetAttribute((const void *)k_nd_merge<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)(sizeof(NdLds2<T>) + nd_merge_tiles<T>() * 2 * TB * TBP * sizeof(T)));
+  });
   hipLaunchKernelGGL(k_nd_tables, dim3((std::max(P.nx + P.ny, 512) + NT - 1) / NT), dim3(NT), 0, s, *g,
                      (unsigned long long *)factor, tab, status, ND_HEADER + 32 * (size_t)(P.nx + P.ny),
                      nd_data_off(P), nd_data_off(P) + P.elems * sizeof(T), nd_factor_bytes(g, P, prec));
@@ -945,6 +1113,12 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
     const NdLevel &L = P.lev[l];
     const int ns = L.sp / TB, nb = L.bp / TB, per = ns * (ns + 1) / 2 + ns * nb;
     const int first = (L.nbox + XCDS - 1) / XCDS * XCDS;
+    if (nd_merges<T>(L)) {
+      hipLaunchKernelGGL(k_nd_merge<T>, dim3(nd_grid(L.nbox)), dim3(NT), nd_merge_lds<T>(L), s, L, A.bd,
+                         (const T *)C[cin], data + L.xoff, data + L.woff, C[cin ^ 1], status);
+      cin ^= 1;
+      continue;
+    }
     A.L = L;
     A.C = C[cin];
     A.Ds = S[1];

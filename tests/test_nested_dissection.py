@@ -168,7 +168,6 @@ def test_kinds_are_told_apart_and_repeat_to_the_bit(precision):
     op = _device(N, [10, 10], "Ez", _eps(rng, N), precision)
     lib, g, pr = L.lib(), ctypes.byref(op.grid), L.PREC[precision]
     fac = op.factor(precision)
-    first = fac.clone()
     b = op.to_solver(torch.tensor(rng.standard_normal((2,) + N) + 1j * rng.standard_normal((2,) + N), device=DEV))
     ptr = lambda t: ctypes.c_void_p(t.data_ptr())
     work = torch.empty(lib.fdfd_solve_workspace_bytes(g, pr, 2), dtype=torch.uint8, device=DEV)
@@ -185,7 +184,9 @@ def test_kinds_are_told_apart_and_repeat_to_the_bit(precision):
     L.check(lib.fdfd_sweep(g, ptr(op.op), ptr(fac), pr, ptr(b), ptr(y), 2, ptr(work), None))
     assert relerr(y.cpu().numpy(), xs[0].cpu().numpy()) < (1e-10 if precision == "fp64" else 1e-2)
     op.drop_factor()
-    assert torch.equal(op.factor(precision), first)
+    del fac
+    x, rep = op.solve(op.to_user(b), precision=precision, tol=1e-10)     # a new factor, the same bits
+    assert torch.equal(op.to_solver(x), xs[0])
     x, rep = op.solve(torch.zeros(N, dtype=torch.complex128, device=DEV), precision=precision)
     assert not x.any() and rep.sweeps == 0 and rep.converged
     # a block factor of the same grid goes the block path
