@@ -162,7 +162,7 @@ class ServingEngine:
     # ------------------------------------------------------------ one request
     def _serve(self, req, stream):
         p = req.problem
-        key = operator_key(p)
+        key = operator_key(p) if self.cache.capacity else None   # a hash of eps
         reused = False
         with torch.cuda.stream(stream):
             op = self.cache.get(key) if self.cache.capacity else None
@@ -173,7 +173,8 @@ class ServingEngine:
                 if not op.nested(self.precision):   # block factorizations share step launches
                     op.engine = self._engine_for(stream)
                 op.set_eps(p.eps)
-            b = torch.as_tensor(p.rhs(), device=self.device)
+            # Problem.rhs() on the device: the sources travel as reals
+            b = torch.as_tensor(p.srcs, device=self.device).to(torch.complex128) * (1j * p.omega)
             x, rep = op.solve(b, precision=self.precision, tol=self.tol, max_iter=self.max_iter)
             stream.synchronize()
         if self.cache.capacity and not reused:
@@ -218,6 +219,7 @@ class ServingEngine:
                     progress(len(results), len(reqs))
 
         threads = []
+        need = None   # bytes of the request to be admitted next
         with cond:
             while state["next"] < len(reqs):
                 req = reqs[state["next"]]
@@ -225,12 +227,14 @@ class ServingEngine:
                 if wait > 0:
                     cond.wait(timeout=wait)
                     continue
-                need = request_bytes(req.problem, self.precision)
+                if need is None:
+                    need = request_bytes(req.problem, self.precision)
                 if need > self.memory_budget:
                     results[req.rid] = Result(req.rid, req.problem.shape, req.problem.srcs.shape[0], None,
                                               req.arrival, now(), now(), self.precision, 0, float("nan"),
                                               False, False, "request larger than the memory budget")
                     state["next"] += 1
+                    need = None
                     continue
                 if not state["free_slots"] or state["used"] + need > self.memory_budget:
                     cond.wait(timeout=0.05)
@@ -243,6 +247,7 @@ class ServingEngine:
                 t = threading.Thread(target=worker, args=(req, slot, need, now()), daemon=True)
                 threads.append(t)
                 t.start()
+                need = None
         for t in threads:
             t.join()
         return [results[r.rid] for r in requests]
