@@ -459,6 +459,258 @@ __device__ void tile_inverse_pairs(LT &L, int rows, int *status) {
   __syncthreads();
 }
 
+// The same inverse by one wave, in its registers, for the leaves, of which
+// there are thousands. The steps are sweeps, which keep the tile symmetric:
+// with f = the pivot rows and Q = P^-1 the tile becomes M - f^T Q f off the
+// pivots, Q f on the pivot rows and columns, -Q on the block, and -M^-1 in the
+// end. The tile lies in the accumulators of 16x16x4 products, whose four inner
+// indices are the two pivots' real and imaginary parts: a step is one product
+// per quadrant and part, on the rows f that the lanes holding them publish in
+// LDS (both operands, by symmetry). Pivot rows and columns are cleared and f
+// is minus a unit vector at the pivots, so the same product leaves Q f and -Q
+// there without cancellation. The pivot blocks are kept aside, that of pair m
+// in lanes m + 16 i, updated from f as well: the next choice does not wait for
+// the products.
+// Four waves issue four times tile_inverse_pairs's choice; here it is issued
+// once. Bound by those instructions: the 8192 leaves of 512^2 complex64 110 ->
+// 53 us, the 16384 of 768^2 FP64 469 -> 206 us. As the chain of one tile it is
+// no shorter (0.53 us a pair, as four waves), and it takes 180 registers in
+// FP64, so the fronts, steps and merges keep tile_inverse_pairs (768^2 FP64
+// merges 511 -> 597 us, steps 24 -> 31 us with this one).
+template <typename T> struct WaveTile {
+  typename Mfma<T>::v4 r[2][2], i[2][2];
+};
+// LDS of one wave's inverse: the pivot rows by column, and a second set for
+// the lanes that have none to write (a branch on lanes inside the choice of
+// the accumulators makes the compiler copy the tile at every join)
+template <typename T> struct alignas(16) WaveRows {
+  T r[TB][2], i[TB][2];
+  T none[2][TB][2];
+};
+// The pivot rows j, j + 1 (j = 16 QR + jr, in accumulator TT: of one lane
+// group for f32, one each of two for f64) go to f; the pivot rows and columns
+// are cleared in the tile.
+template <int QR, int TT>
+__device__ inline void wave_rows(WaveTile<float> &M, WaveRows<float> &f, int lane, int jr) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  const int c = lane & 15;
+  const bool own = (lane >> 4) == (jr >> 2), pc = (c & ~1) == jr;
+  f2 *to = reinterpret_cast<f2 *>(own ? f.r[c] : f.none[0][c]);
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    to[16 * q] = f2{M.r[QR][q][TT], M.r[QR][q][TT + 1]};
+    to[16 * q + TB] = f2{M.i[QR][q][TT], M.i[QR][q][TT + 1]};
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bool row = t == TT || t == TT + 1, both = q == QR && row;
+      if (row) {
+        M.r[QR][q][t] = own || (both && pc) ? 0.0f : M.r[QR][q][t];
+        M.i[QR][q][t] = own || (both && pc) ? 0.0f : M.i[QR][q][t];
+      }
+      if (!both) {
+        M.r[q][QR][t] = pc ? 0.0f : M.r[q][QR][t];
+        M.i[q][QR][t] = pc ? 0.0f : M.i[q][QR][t];
+      }
+    }
+}
+template <int QR, int TT>
+__device__ inline void wave_rows(WaveTile<double> &M, WaveRows<double> &f, int lane, int jr) {
+  const int c = lane & 15, k = (lane >> 4) - (jr & 3);
+  const bool own = k == 0 || k == 1, pc = (c & ~1) == jr;
+  double *to = own ? &f.r[c][k] : f.none[0][c];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    to[32 * q] = M.r[QR][q][TT];
+    to[32 * q + 2 * TB] = M.i[QR][q][TT];
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bool row = t == TT, both = q == QR && row;
+      if (row) {
+        M.r[QR][q][t] = own || (both && pc) ? 0.0 : M.r[QR][q][t];
+        M.i[QR][q][t] = own || (both && pc) ? 0.0 : M.i[QR][q][t];
+      }
+      if (!both) {
+        M.r[q][QR][t] = pc ? 0.0 : M.r[q][QR][t];
+        M.i[q][QR][t] = pc ? 0.0 : M.i[q][QR][t];
+      }
+    }
+}
+// What one lane writes to LDS the others of its wave read next
+__device__ inline void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <typename T> struct WaveQ {   // Q = P^-1 (uniform), block of this lane's pair
+  T q00r, q00i, q01r, q01i, q11r, q11i;
+};
+// One sweep's products on the rows in accumulator TT of quadrant row QR
+template <int QR, int TT, typename T>
+__device__ inline void wave_sweep(WaveTile<T> &M, WaveRows<T> &f, int lane, int j, const WaveQ<T> &Q) {
+  const int c = lane & 15, kk = lane >> 4, k = kk & 1, part = kk >> 1;
+  wave_rows<QR, TT>(M, f, lane, j & 15);
+  wave_lds_order();
+  T *unit = lane < 2 ? f.r[j + lane] : f.none[0][0];   // minus a unit vector at the pivots
+  unit[0] = lane ? T(0) : T(-1);
+  unit[1] = lane ? T(-1) : T(0);
+  unit[2 * TB] = unit[2 * TB + 1] = 0;
+  wave_lds_order();
+  // inner index kk: -(Q f)_k, real (kk < 2) and imaginary part, against f_k
+  const T s0r = k ? Q.q01r : Q.q00r, s0i = k ? Q.q01i : Q.q00i, s1r = k ? Q.q11r : Q.q01r, s1i = k ? Q.q11i : Q.q01i;
+  const T w0 = part ? s0i : -s0r, w1 = part ? s0r : s0i, w2 = part ? s1i : -s1r, w3 = part ? s1r : s1i;
+  const T *fre = part ? &f.i[c][k] : &f.r[c][k], *fim = part ? &f.r[c][k] : &f.i[c][k];
+  T are[2], aim[2], bre[2], bim[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    bre[q] = fre[32 * q];
+    bim[q] = fim[32 * q];
+    T v0, v1, v2, v3;
+    lds_ld2(f.r[16 * q + c], v0, v2);
+    lds_ld2(f.i[16 * q + c], v1, v3);
+    are[q] = fma(v3, w3, fma(v2, w2, fma(v1, w1, v0 * w0)));
+    aim[q] = part ? -are[q] : are[q];
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      M.r[a][b] = Mfma<T>::mac(are[a], bre[b], M.r[a][b]);
+      M.i[a][b] = Mfma<T>::mac(aim[a], bim[b], M.i[a][b]);
+    }
+}
+__device__ inline void wave_sweep_at(WaveTile<float> &M, WaveRows<float> &f, int lane, int j, const WaveQ<float> &Q) {
+  if (j < 16) {
+    if (j & 2) wave_sweep<0, 2>(M, f, lane, j, Q); else wave_sweep<0, 0>(M, f, lane, j, Q);
+  } else {
+    if (j & 2) wave_sweep<1, 2>(M, f, lane, j, Q); else wave_sweep<1, 0>(M, f, lane, j, Q);
+  }
+}
+__device__ inline void wave_sweep_at(WaveTile<double> &M, WaveRows<double> &f, int lane, int j,
+                                     const WaveQ<double> &Q) {
+  if (j < 16) {
+    if (j < 8) { if (j < 4) wave_sweep<0, 0>(M, f, lane, j, Q); else wave_sweep<0, 1>(M, f, lane, j, Q); }
+    else { if (j < 12) wave_sweep<0, 2>(M, f, lane, j, Q); else wave_sweep<0, 3>(M, f, lane, j, Q); }
+  } else {
+    if (j < 24) { if (j < 20) wave_sweep<1, 0>(M, f, lane, j, Q); else wave_sweep<1, 1>(M, f, lane, j, Q); }
+    else { if (j < 28) wave_sweep<1, 2>(M, f, lane, j, Q); else wave_sweep<1, 3>(M, f, lane, j, Q); }
+  }
+}
+// p -= a b (complex)
+template <typename T> __device__ inline void wave_sub(T &pr, T &pi, T ar, T ai, T br, T bi) {
+  pr = fma(ai, bi, fma(-ar, br, pr));
+  pi = fma(-ai, br, fma(-ar, bi, pi));
+}
+__device__ inline int frexp_of(float x) { return __builtin_amdgcn_frexp_expf(x); }
+__device__ inline int frexp_of(double x) { return __builtin_amdgcn_frexp_exp(x); }
+// (Ar, Ai) in LDS -> its inverse in M, entry (16 a + crow(lane, t), 16 b + lane % 16)
+// in element t of quadrant (a, b); f: LDS that no other wave uses.
+// rows: the tile's rows that are not identity padding; the pairs beyond are
+// left alone (the step count is (rows + 1) / 2). False: singular.
+template <typename T>
+__device__ inline bool wave_inverse(WaveTile<T> &M, const T (*Ar)[TBP], const T (*Ai)[TBP], WaveRows<T> &f, int rows) {
+  const int lane = threadIdx.x & 63, mine = lane & 15;
+  const int pairs = min(TB, rows + 1) >> 1, d = 2 * mine;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * a + Mfma<T>::crow(lane, t), c = 16 * b + mine;
+        const int x = min(r, c), y = max(r, c);
+        M.r[a][b][t] = Ar[x][y];
+        M.i[a][b][t] = Ai[x][y];
+      }
+  T p00r = Ar[d][d], p00i = Ai[d][d], p01r = Ar[d][d + 1], p01i = Ai[d][d + 1];
+  T p11r = Ar[d + 1][d + 1], p11i = Ai[d + 1][d + 1];
+  bool bad = false, taken = mine >= pairs;
+#pragma unroll 1
+  for (int st = 0; st < pairs; ++st) {
+    // this lane's block, scaled by an exact power of two near 1 / max |P_ij|
+    const T mx = fmax(fmax(fabs(p00r) + fabs(p00i), fabs(p01r) + fabs(p01i)), fabs(p11r) + fabs(p11i));
+    const int e = frexp_of(mx);
+    const T a00r = ldexp(p00r, -e), a00i = ldexp(p00i, -e), a01r = ldexp(p01r, -e), a01i = ldexp(p01i, -e);
+    const T a11r = ldexp(p11r, -e), a11i = ldexp(p11i, -e);
+    const T dr = fma(a01i, a01i, fma(-a01r, a01r, fma(-a00i, a11i, a00r * a11r)));
+    const T di = fma(T(-2) * a01r, a01i, fma(a00i, a11r, a00r * a11i));
+    const T da = fabs(dr) + fabs(di);
+    const unsigned size = __float_as_uint(fabsf((float)ldexp(da, e))) & ~15u;
+    const unsigned key = row16_max(taken ? 0u : size + 16u + (unsigned)mine);
+    const int pick = __builtin_amdgcn_readfirstlane((int)(key & 15u));
+    // 1 / det: (dr - i di) / |det|^2 with det brought near 1 by an exact scale
+    const int g = frexp_of(da);
+    const T br = ldexp(dr, -g), bi = ldexp(di, -g);
+    const T rm = ldexp(rcp_nr(fma(bi, bi, br * br)), -e - g);
+    const T er = br * rm, ei = -bi * rm;
+    WaveQ<T> Q;
+    Q.q00r = lane_value(fma(-a11i, ei, a11r * er), pick);
+    Q.q00i = lane_value(fma(a11i, er, a11r * ei), pick);
+    Q.q01r = lane_value(fma(a01i, ei, -a01r * er), pick);
+    Q.q01i = lane_value(fma(-a01i, er, -a01r * ei), pick);
+    Q.q11r = lane_value(fma(-a00i, ei, a00r * er), pick);
+    Q.q11i = lane_value(fma(a00i, er, a00r * ei), pick);
+    const bool now = mine == pick;
+    bad |= now & !((da > T(0)) & (da < T(INFINITY)));
+    taken |= now;
+    wave_lds_order();
+    wave_sweep_at(M, f, lane, 2 * pick, Q);
+    // the pivot blocks: P_ab -= f(a)^T Q f(b)
+    T xr[2], xi[2], yr[2], yi[2];
+    lds_ld2(f.r[d], xr[0], xr[1]);
+    lds_ld2(f.i[d], xi[0], xi[1]);
+    lds_ld2(f.r[d + 1], yr[0], yr[1]);
+    lds_ld2(f.i[d + 1], yi[0], yi[1]);
+    T v0r = 0, v0i = 0, v1r = 0, v1i = 0, u0r = 0, u0i = 0, u1r = 0, u1i = 0;   // -Q f
+    wave_sub(v0r, v0i, Q.q00r, Q.q00i, xr[0], xi[0]);
+    wave_sub(v0r, v0i, Q.q01r, Q.q01i, xr[1], xi[1]);
+    wave_sub(v1r, v1i, Q.q01r, Q.q01i, xr[0], xi[0]);
+    wave_sub(v1r, v1i, Q.q11r, Q.q11i, xr[1], xi[1]);
+    wave_sub(u0r, u0i, Q.q00r, Q.q00i, yr[0], yi[0]);
+    wave_sub(u0r, u0i, Q.q01r, Q.q01i, yr[1], yi[1]);
+    wave_sub(u1r, u1i, Q.q01r, Q.q01i, yr[0], yi[0]);
+    wave_sub(u1r, u1i, Q.q11r, Q.q11i, yr[1], yi[1]);
+    wave_sub(p00r, p00i, -v0r, -v0i, xr[0], xi[0]);
+    wave_sub(p00r, p00i, -v1r, -v1i, xr[1], xi[1]);
+    wave_sub(p01r, p01i, -v0r, -v0i, yr[0], yi[0]);
+    wave_sub(p01r, p01i, -v1r, -v1i, yr[1], yi[1]);
+    wave_sub(p11r, p11i, -u0r, -u0i, yr[0], yi[0]);
+    wave_sub(p11r, p11i, -u1r, -u1i, yr[1], yi[1]);
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bool neg = 16 * a + Mfma<T>::crow(lane, t) < 2 * pairs;   // the padding stays
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        M.r[a][b][t] = neg ? -M.r[a][b][t] : M.r[a][b][t];
+        M.i[a][b][t] = neg ? -M.i[a][b][t] : M.i[a][b][t];
+      }
+    }
+  return !bad;
+}
+// M into a tile of pitch `pitch`
+template <typename T>
+__device__ inline void wave_store(const WaveTile<T> &M, T *re, T *im, int pitch) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int e = (16 * a + Mfma<T>::crow(lane, t)) * pitch + 16 * b + (lane & 15);
+        re[e] = M.r[a][b][t];
+        im[e] = M.i[a][b][t];
+      }
+}
+
 // LDS of the kernels that invert a tile: A (the tile, then its inverse), B
 // (with A: the exchange buffers of the inverse) and, where used, a third tile.
 template <typename T> struct NdLds2 {
@@ -474,78 +726,86 @@ template <typename T> struct NdLds3 {
   int end[4];
 };
 
-// A leaf box per workgroup: its five-point matrix (cells in (x, y) order,
+// A leaf box per wave: its five-point matrix (cells in (x, y) order,
 // identity beyond) inverted as one pivot tile; X, the border couplings c and
 // the update C[a][b] = -c_a X[p_a][p_b] c_b, p_a the cell inside border cell a.
 template <typename T>
-__global__ void __launch_bounds__(NT) k_nd_leaf(int nx, int ny, int Dx, int Dy, NdBands<T> bd, T *__restrict__ X,
+__global__ void __launch_bounds__(64, 2) k_nd_leaf(int nx, int ny, int Dx, int Dy, NdBands<T> bd, T *__restrict__ X,
                                                 T *__restrict__ cpl, T *__restrict__ C, int *status) {
-  __shared__ NdLds2<T> L;
-  __shared__ T cr[TB], ci[TB];
+  __shared__ T Ar[TB][TBP], Ai[TB][TBP], cr[TB], ci[TB];
+  __shared__ WaveRows<T> f;
   __shared__ int cp[TB];
-  const int tid = threadIdx.x, k = blockIdx.x;
+  const int lane = threadIdx.x, k = blockIdx.x;
   const int ix = k >> Dy, iy = k & ((1 << Dy) - 1);
   int x0, w, y0, h;
   nd_seg(nx, Dx, ix, x0, w);
   nd_seg(ny, Dy, iy, y0, h);
   const int s = w * h, b = 2 * (w + h);
-  const int a = tid >> 3, b0 = (tid & 7) * 4;
-  const int ai = a / h, aj = a % h;
+  const int b0 = (lane & 7) * 4, a0 = lane >> 3;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int c = b0 + u;
-    T re = a == c ? T(1) : T(0), im = 0;
-    if (a < s && c < s) {
-      const int qi = c / h, qj = c % h;
-      const size_t pa = (size_t)(x0 + ai) * ny + y0 + aj, pc = (size_t)(x0 + qi) * ny + y0 + qj;
-      re = 0;
-      if (a == c) nd_ld(bd.c, pa, re, im);
-      else if (aj == qj && (ai + 1 == qi || qi + 1 == ai)) nd_ld(bd.x, ai < qi ? pa : pc, re, im);
-      else if (ai == qi && (aj + 1 == qj || qj + 1 == aj)) nd_ld(bd.y, aj < qj ? pa : pc, re, im);
-    }
-    L.Ar[a][c] = re;
-    L.Ai[a][c] = im;
+  for (int e = lane; e < TB * TBP; e += 64) {
+    (&Ar[0][0])[e] = 0;
+    (&Ai[0][0])[e] = 0;
   }
-  if (tid < TB) {
-    T re = 0, im = 0;
+  wave_lds_order();
+  if (lane < TB) {   // the upper triangle: itself, the next cell in y and in x
+    T re = 1, im = 0;
+    if (lane < s) {
+      const int i = lane / h, j = lane - i * h;
+      const size_t p = (size_t)(x0 + i) * ny + y0 + j;
+      nd_ld(bd.c, p, re, im);
+      T yr = 0, yi = 0, xr = 0, xi = 0;
+      if (j + 1 < h) nd_ld(bd.y, p, yr, yi);
+      if (i + 1 < w) nd_ld(bd.x, p, xr, xi);
+      if (j + 1 < h) { Ar[lane][lane + 1] = yr; Ai[lane][lane + 1] = yi; }
+      if (i + 1 < w) { Ar[lane][lane + h] = xr; Ai[lane][lane + h] = xi; }
+    }
+    Ar[lane][lane] = re;
+    Ai[lane][lane] = im;
+    re = im = 0;
     int p = 0;
-    if (tid < h) {
-      p = tid;
-      nd_ld(bd.x, (size_t)(x0 - 1) * ny + y0 + tid, re, im);
-    } else if (tid < 2 * h) {
-      p = (w - 1) * h + tid - h;
-      nd_ld(bd.x, (size_t)(x0 + w - 1) * ny + y0 + tid - h, re, im);
-    } else if (tid < 2 * h + w) {
-      p = (tid - 2 * h) * h;
-      nd_ld(bd.y, (size_t)(x0 + tid - 2 * h) * ny + y0 - 1, re, im);
-    } else if (tid < b) {
-      p = (tid - 2 * h - w) * h + h - 1;
-      nd_ld(bd.y, (size_t)(x0 + tid - 2 * h - w) * ny + y0 + h - 1, re, im);
+    if (lane < h) {
+      p = lane;
+      nd_ld(bd.x, (size_t)(x0 - 1) * ny + y0 + lane, re, im);
+    } else if (lane < 2 * h) {
+      p = (w - 1) * h + lane - h;
+      nd_ld(bd.x, (size_t)(x0 + w - 1) * ny + y0 + lane - h, re, im);
+    } else if (lane < 2 * h + w) {
+      p = (lane - 2 * h) * h;
+      nd_ld(bd.y, (size_t)(x0 + lane - 2 * h) * ny + y0 - 1, re, im);
+    } else if (lane < b) {
+      p = (lane - 2 * h - w) * h + h - 1;
+      nd_ld(bd.y, (size_t)(x0 + lane - 2 * h - w) * ny + y0 + h - 1, re, im);
     }
-    cr[tid] = re;
-    ci[tid] = im;
-    cp[tid] = p;
-    nd_st<T>(cpl, (size_t)k * TB + tid, re, im);
+    cr[lane] = re;
+    ci[lane] = im;
+    cp[lane] = p;
+    nd_st<T>(cpl, (size_t)k * TB + lane, re, im);
   }
-  __syncthreads();
-  tile_inverse_pairs<T>(L, s, status);
+  wave_lds_order();
+  WaveTile<T> M;
+  if (!wave_inverse<T>(M, Ar, Ai, f, s)) *status = 1;
+  wave_lds_order();
+  wave_store<T>(M, &Ar[0][0], &Ai[0][0], TBP);
+  wave_lds_order();
   T *Xk = X + (size_t)k * 2 * TB * TB, *Ck = C + (size_t)k * 2 * TB * TB;
-  if (a < s) {
-    store4(Xk + a * TB + b0, &L.Ar[a][b0]);
-    store4(Xk + TB * TB + a * TB + b0, &L.Ai[a][b0]);
+  for (int a = a0; a < s; a += 8) {
+    store4(Xk + a * TB + b0, &Ar[a][b0]);
+    store4(Xk + TB * TB + a * TB + b0, &Ai[a][b0]);
   }
-  if (a >= b) return;
-  T vr[4], vi[4];
+  for (int a = a0; a < b; a += 8) {
+    T vr[4], vi[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int x = min(a, b0 + u), y = max(a, b0 + u);   // symmetric to the last bit
-    const T xr = L.Ar[cp[x]][cp[y]], xi = L.Ai[cp[x]][cp[y]];
-    const T tr = cr[x] * xr - ci[x] * xi, ti = cr[x] * xi + ci[x] * xr;
-    vr[u] = -(tr * cr[y] - ti * ci[y]);
-    vi[u] = -(tr * ci[y] + ti * cr[y]);
+    for (int u = 0; u < 4; ++u) {
+      const int x = min(a, b0 + u), y = max(a, b0 + u);   // symmetric to the last bit
+      const T xr = Ar[cp[x]][cp[y]], xi = Ai[cp[x]][cp[y]];
+      const T tr = cr[x] * xr - ci[x] * xi, ti = cr[x] * xi + ci[x] * xr;
+      vr[u] = -(tr * cr[y] - ti * ci[y]);
+      vi[u] = -(tr * ci[y] + ti * cr[y]);
+    }
+    store4(Ck + a * TB + b0, vr);
+    store4(Ck + TB * TB + a * TB + b0, vi);
   }
-  store4(Ck + a * TB + b0, vr);
-  store4(Ck + TB * TB + a * TB + b0, vi);
 }
 
 // Four consecutive entries (row i of the front, columns given by their
@@ -1106,7 +1366,7 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
                      nd_data_off(P), nd_data_off(P) + P.elems * sizeof(T), nd_factor_bytes(g, P, prec));
   hipLaunchKernelGGL(k_nd_bands<T>, dim3((P.ny + NT - 1) / NT, P.nx), dim3(NT), 0, s, P.nx, P.ny, nd_alpha(g), op,
                      nd_tables(tab, P.nx, P.ny), bands);
-  hipLaunchKernelGGL(k_nd_leaf<T>, dim3(P.nleaf), dim3(NT), 0, s, P.nx, P.ny, P.Dx, P.Dy, A.bd, data + P.leaf_off,
+  hipLaunchKernelGGL(k_nd_leaf<T>, dim3(P.nleaf), dim3(64), 0, s, P.nx, P.ny, P.Dx, P.Dy, A.bd, data + P.leaf_off,
                      data + P.leafc_off, C[0], status);
   int cin = 0;
   for (int l = 0; l <= P.nlev; ++l) {

@@ -158,6 +158,25 @@ def test_solves_match_the_oracle(N, npml, pol, nrhs, precision):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,cells", [((29, 21), {8, 10, 12, 15}), ((19, 19), {9, 12, 16}), ((16, 16), {21}),
+                                     ((21, 21), {16, 20, 25}), ((17, 17), {21, 24, 28, 32})])
+def test_leaves_of_every_size(N, cells):
+    """The leaf inverse from 8 cells to a full tile, odd counts (a pivot pair
+    half padding) among them. An exact factor leaves the first residual at
+    eps ||A|| ||x|| ~ 1e-16 * 1e3: one sweep meets 1e-12."""
+    g = L.FdfdGrid(*N, 4, 4, 0, 0, OMEGA, 0.02, 1e-6)
+    assert {_front(g, -1, k)[0][3] for k in range(_front(g, -1, 0)[0][1])} == cells
+    rng = np.random.default_rng(N[0])
+    eps = _eps(rng, N)
+    op = _device(N, [4, 4], "Ez", eps, "fp64")
+    b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    x, rep = op.solve(torch.tensor(b, device=DEV), precision="fp64", tol=1e-12)
+    assert rep.converged and rep.sweeps == 1
+    A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], eps, [4, 4], "Ez", 1e-6)
+    assert relerr(x.cpu().numpy(), solver_direct(A, b.reshape(-1)).reshape(N)) < 1e-10
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["fp64", "c64"])
 def test_kinds_are_told_apart_and_repeat_to_the_bit(precision):
     """fdfd_solve without a kind in its precision reads the tag; fdfd_sweep on
