@@ -971,18 +971,27 @@ __global__ void __launch_bounds__(NT) k_nd_front(NdStep<T> A) {
 // finished W loses the digits that a nearly resonant box costs twice: the
 // complex64 factor of a 512 x 512 stream grid with |X| = 550 in one box then
 // contracts by 0.03-0.2 per sweep instead of 2e-4.)
+// A workgroup takes two tiles of a column, rows I = 2 i and 2 i + 1, which
+// share P X[p,J]: three products for two tiles instead of four, P and X[p,J]
+// read once. Bound by the inverse's chain where the tiles are few and by the
+// matrix cores and the pass over the front where they are many: a step of 1200
+// tiles, complex64 20.2 -> 18.9 us, of 2600 tiles, FP64 37 -> 33 us.
+__host__ __device__ inline int nd_step_items(int ns, int nb) {
+  const int np = (ns + 1) / 2;
+  return np * (np + 1) + np * nb;
+}
 template <typename T>
 __global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
   __shared__ NdLds3<T> S;
   const NdLevel &L = A.L;
-  const int ns = L.sp / TB, nb = L.bp / TB, tri = ns * (ns + 1) / 2, per = tri + ns * nb, p = A.p;
+  const int ns = L.sp / TB, nb = L.bp / TB, np = (ns + 1) / 2, per = nd_step_items(ns, nb), p = A.p;
   const bool last = p == ns - 1;
   const int ncrit = last ? 0 : L.nbox, first = (ncrit + XCDS - 1) / XCDS * XCDS;
-  int box, I, J;
+  int box, I0, J;
   bool crit = false;
   if ((int)blockIdx.x < ncrit) {
     box = blockIdx.x;
-    I = J = p + 1;
+    I0 = J = p + 1;
     crit = true;
     __builtin_amdgcn_s_setprio(3);
   } else {
@@ -990,20 +999,24 @@ __global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
     const int it = nd_item(blockIdx.x - first, L.nbox * per);
     if (it < 0) return;
     box = it / per;
-    const int t = it % per;
-    if (t < tri) { const int e = upper_tile(ns, t); I = e / ns; J = e % ns; }
-    else { I = (t - tri) / nb; J = ns + (t - tri) % nb; }
-    if (!last && I == p + 1 && J == p + 1) return;
+    const int t = it % per, tri = np * (np + 1);
+    if (t < tri) { const int e = upper_tile(np, t >> 1); I0 = e / np * 2; J = e % np * 2 + (t & 1); }
+    else { I0 = (t - tri) / nb * 2; J = ns + (t - tri) % nb; }
+    if (J < I0 || (J >= ns && t < tri)) return;   // ns is odd
   }
+  // which of the two there are
+  const auto skips = [&](int I) { return I >= ns || I > J || (!crit && !last && I == p + 1 && J == p + 1); };
+  const bool has[2] = {!skips(I0), !crit && !skips(I0 + 1)};
+  if (!has[0] && !has[1]) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, qi = wv >> 1, qj = wv & 1;
   const int a = tid >> 3, b0 = (tid & 7) * 4;
   const size_t sp = L.sp, bp = L.bp, ps = sp * sp, pb = sp * bp;
   const T *Ss = A.Ss + (size_t)box * 2 * ps, *Sb = A.Sb + (size_t)box * 2 * pb;
   const T *P = A.P0 + (size_t)box * 2 * TB * TB;
-  const bool row = I == p, col = J == p, mirA = J < p, mirB = I > p;
-  // every global read first: P, X[p,J], X[I,p] and the tile itself
-  T pr[4], pi[4], ar[4], ai[4], br[4], bi[4];
-  typename Mfma<T>::v4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+  const bool col = J == p, mirA = J < p;
+  // every global read first: P, X[p,J], X[I,p] and the tiles themselves
+  T pr[4], pi[4], ar[4], ai[4], br[2][4], bi[2][4];
+  typename Mfma<T>::v4 cr[2], ci[2];
   ld_row4(P + a * TB + b0, pr);
   ld_row4(P + TB * TB + a * TB + b0, pi);
   if (!col) {
@@ -1014,21 +1027,34 @@ __global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
     ld_row4(q, ar);
     ld_row4(q + pl, ai);
   }
-  if (!row) {
-    const T *q = mirB ? Ss + ((size_t)p * TB + a) * sp + I * TB + b0 : Ss + ((size_t)I * TB + a) * sp + p * TB + b0;
-    ld_row4(q, br);
-    ld_row4(q + ps, bi);
-  }
-  if (!row && !col) {
-    const T *q = J >= ns ? Sb + (size_t)(J - ns) * TB : Ss + (size_t)J * TB;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int I = I0 + h;
+    cr[h] = ci[h] = typename Mfma<T>::v4{0, 0, 0, 0};
+    if (!has[h] || I == p) continue;
+    const T *q = I > p ? Ss + ((size_t)p * TB + a) * sp + I * TB + b0 : Ss + ((size_t)I * TB + a) * sp + p * TB + b0;
+    ld_row4(q, br[h]);
+    ld_row4(q + ps, bi[h]);
+    if (col) continue;
+    q = J >= ns ? Sb + (size_t)(J - ns) * TB : Ss + (size_t)J * TB;
     const size_t pitch = J >= ns ? bp : sp, pl = J >= ns ? pb : ps;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const size_t e = (size_t)(I * TB + qi * 16 + Mfma<T>::crow(lane, t)) * pitch + qj * 16 + (lane & 15);
-      cr[t] = q[e];
-      ci[t] = q[pl + e];
+      cr[h][t] = q[e];
+      ci[h][t] = q[pl + e];
     }
   }
+  // X[I,p] of the first row to B, of the second to A (J == p) or, once P X[p,J] is formed, to P
+  const auto put = [&](int h, T (*dr)[TBP], T (*di)[TBP]) {
+    if (!has[h] || I0 + h == p) return;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = b0 + u;
+      if (I0 + h > p) { dr[c][a] = br[h][u]; di[c][a] = bi[h][u]; }
+      else { dr[a][c] = br[h][u]; di[a][c] = bi[h][u]; }
+    }
+  };
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int c = b0 + u;
@@ -1038,66 +1064,80 @@ __global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
       if (mirA) { S.Ar[c][a] = -ar[u]; S.Ai[c][a] = -ai[u]; }
       else { S.Ar[a][c] = ar[u]; S.Ai[a][c] = ai[u]; }
     }
-    if (!row) {
-      if (mirB) { S.Br[c][a] = br[u]; S.Bi[c][a] = bi[u]; }
-      else { S.Br[a][c] = br[u]; S.Bi[a][c] = bi[u]; }
-    }
   }
+  put(0, S.Br, S.Bi);
+  if (col) put(1, S.Ar, S.Ai);
   __syncthreads();
-  if (row && col) {
+  if (col) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int x = qi * 16 + Mfma<T>::crow(lane, t), y = qj * 16 + (lane & 15);
-      cr[t] = S.Pr[x][y];
-      ci[t] = S.Pi[x][y];
+    for (int h = 0; h < 2; ++h) {
+      if (!has[h]) continue;
+      if (I0 + h == p) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int x = qi * 16 + Mfma<T>::crow(lane, t), y = qj * 16 + (lane & 15);
+          cr[h][t] = S.Pr[x][y];
+          ci[h][t] = S.Pi[x][y];
+        }
+      } else {
+        cgemm_quad<T>(cr[h], ci[h], h ? S.Ar : S.Br, h ? S.Ai : S.Bi, S.Pr, S.Pi, qi, qj, lane, T(-1));
+      }
     }
-  } else if (col) {
-    cgemm_quad<T>(cr, ci, S.Br, S.Bi, S.Pr, S.Pi, qi, qj, lane, T(-1));
   } else {
     typename Mfma<T>::v4 rr = {0, 0, 0, 0}, ri = {0, 0, 0, 0};
     cgemm_quad<T>(rr, ri, S.Pr, S.Pi, S.Ar, S.Ai, qi, qj, lane, T(1));
-    if (row) {
-      cr = rr;
-      ci = ri;
-    } else {
-      __syncthreads();   // every wave has read X[p,J]
-      acc_to_lds<T>(rr, ri, S.Ar, S.Ai, qi, qj, lane);
-      __syncthreads();
-      cgemm_quad<T>(cr, ci, S.Br, S.Bi, S.Ar, S.Ai, qi, qj, lane, T(-1));
+    __syncthreads();   // every wave has read P and X[p,J]
+    acc_to_lds<T>(rr, ri, S.Ar, S.Ai, qi, qj, lane);
+    put(1, S.Pr, S.Pi);
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!has[h]) continue;
+      if (I0 + h == p) { cr[h] = rr; ci[h] = ri; }
+      else cgemm_quad<T>(cr[h], ci[h], h ? S.Pr : S.Br, h ? S.Pi : S.Bi, S.Ar, S.Ai, qi, qj, lane, T(-1));
     }
   }
   // out through LDS as whole rows
   __syncthreads();
-  acc_to_lds<T>(cr, ci, S.Ar, S.Ai, qi, qj, lane);
-  __syncthreads();
   if (crit) {   // replaced by its inverse at the next step and read by nobody before
+    acc_to_lds<T>(cr[0], ci[0], S.Ar, S.Ai, qi, qj, lane);
+    __syncthreads();
     tile_inverse_pairs<T>(S, nd_box(L, box).s - (p + 1) * TB, A.status);
     store_pinv(S, A.P1 + (size_t)box * 2 * TB * TB);
     return;
   }
-  if (J >= ns) {
-    const size_t o = (size_t)box * 2 * pb + ((size_t)I * TB + a) * bp + (size_t)(J - ns) * TB + b0;
-    store4(A.Db + o, &S.Ar[a][b0]);
-    store4(A.Db + o + pb, &S.Ai[a][b0]);
-    if (row && ns > 1) {
-      store4(A.R + o, &S.Ar[a][b0]);
-      store4(A.R + o + pb, &S.Ai[a][b0]);
-      if (p > 0) {   // at p = 0 U holds F_sb itself
-        store4(A.U + o, ar);
-        store4(A.U + o + pb, ai);
-      }
-    }
-    return;
-  }
-  T *D = A.Ds + (size_t)box * 2 * ps;
-  store4(D + ((size_t)I * TB + a) * sp + J * TB + b0, &S.Ar[a][b0]);
-  store4(D + ps + ((size_t)I * TB + a) * sp + J * TB + b0, &S.Ai[a][b0]);
-  if (last && I != J) {
-    T mr[4], mi[4];
+  if (has[0]) acc_to_lds<T>(cr[0], ci[0], S.Br, S.Bi, qi, qj, lane);
+  if (has[1]) acc_to_lds<T>(cr[1], ci[1], S.Pr, S.Pi, qi, qj, lane);
+  __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 4; ++u) { mr[u] = S.Ar[b0 + u][a]; mi[u] = S.Ai[b0 + u][a]; }
-    store4(D + ((size_t)J * TB + a) * sp + I * TB + b0, mr);
-    store4(D + ps + ((size_t)J * TB + a) * sp + I * TB + b0, mi);
+  for (int h = 0; h < 2; ++h) {
+    if (!has[h]) continue;
+    const int I = I0 + h;
+    const T (*Or)[TBP] = h ? S.Pr : S.Br, (*Oi)[TBP] = h ? S.Pi : S.Bi;
+    if (J >= ns) {
+      const size_t o = (size_t)box * 2 * pb + ((size_t)I * TB + a) * bp + (size_t)(J - ns) * TB + b0;
+      store4(A.Db + o, &Or[a][b0]);
+      store4(A.Db + o + pb, &Oi[a][b0]);
+      if (I == p && ns > 1) {
+        store4(A.R + o, &Or[a][b0]);
+        store4(A.R + o + pb, &Oi[a][b0]);
+        if (p > 0) {   // at p = 0 U holds F_sb itself
+          store4(A.U + o, ar);
+          store4(A.U + o + pb, ai);
+        }
+      }
+      continue;
+    }
+    T *D = A.Ds + (size_t)box * 2 * ps;
+    store4(D + ((size_t)I * TB + a) * sp + J * TB + b0, &Or[a][b0]);
+    store4(D + ps + ((size_t)I * TB + a) * sp + J * TB + b0, &Oi[a][b0]);
+    if (last && I != J) {
+      T mr[4], mi[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { mr[u] = Or[b0 + u][a]; mi[u] = Oi[b0 + u][a]; }
+      store4(D + ((size_t)J * TB + a) * sp + I * TB + b0, mr);
+      store4(D + ps + ((size_t)J * TB + a) * sp + I * TB + b0, mi);
+    }
   }
 }
 
@@ -1393,7 +1433,8 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
       A.Db = last ? data + L.woff : Bf[p & 1];
       A.P0 = pv[p & 1];
       A.P1 = pv[(p + 1) & 1];
-      hipLaunchKernelGGL(k_nd_step<T>, dim3((last ? 0 : first) + nd_grid(L.nbox * per)), dim3(NT), 0, s, A);
+      hipLaunchKernelGGL(k_nd_step<T>, dim3((last ? 0 : first) + nd_grid(L.nbox * nd_step_items(ns, nb))),
+                         dim3(NT), 0, s, A);
     }
     if (L.root) break;
     hipLaunchKernelGGL(k_nd_update<T>, dim3(nd_grid(L.nbox * (nb * (nb + 1) / 2))), dim3(NT), 0, s, L,
