@@ -332,21 +332,27 @@ __global__ void __launch_bounds__(NT) k_nd_bands(int nx, int ny, double alpha, c
   nd_st<T>(bands + 4 * M, p, (T)y.r, (T)y.i);
 }
 
-// Inverse of the TB x TB tile in (Ar, Ai), in place, by Gauss-Jordan with
-// 2 x 2 diagonal block pivots taken in the order of their size: each step
-// picks, of the adjacent pairs not yet taken, the block P with the largest
-// |det P| / max |P_ij| (about 1 / ||P^-1||). The fronts of interior boxes are
-// real and indefinite, and a fixed order meets small leading minors: on the
-// request stream's 512 x 512 grid the complex64 factor of seed 7 then does not
-// refine at all, against a contraction of 2e-4 per sweep with the picked
-// order (2e-4 too for row pivoting inside the tile). Diagonal pivots move no
-// rows, so the order costs only the choice: lane l of every wave forms det and
-// inverse of pair l % 16 while the others do, a maximum over 16 lanes (row
-// rotations) names the pair, and its inverse comes by readlane. Only the
-// upper triangle is read: the fronts stay symmetric to the last bit, without
-// which the rounding of a nearly resonant box (|X| ~ 10^3) grows by another
-// two digits on the way up.
-// Layout and exchange as in tile_inverse_diag.
+// Inverse of a symmetric TB x TB tile with 2 x 2 diagonal pivots taken in the
+// order of their size: each step picks, of the adjacent pairs not yet taken,
+// the block P with the largest |det P| / max |P_ij| (about 1 / ||P^-1||). The
+// fronts of interior boxes are real and indefinite, and a fixed order meets
+// small leading minors: on the request stream's 512 x 512 grid the complex64
+// factor of seed 7 then does not refine at all, against a contraction of 2e-4
+// per sweep with the picked order (2e-4 too for row pivoting inside the tile).
+// Diagonal pivots move no rows. Only the upper triangle is read: the fronts
+// stay symmetric to the last bit, without which the rounding of a nearly
+// resonant box (|X| ~ 10^3) grows by another two digits on the way up.
+//
+// The steps are sweeps, which keep the tile symmetric: with f = the pivot rows
+// and Q = P^-1 the tile becomes M - f^T Q f off the pivots, Q f on the pivot
+// rows and columns, -Q on the block, and -M^-1 in the end. The tile lies in
+// accumulators of 16x16x4 products, whose four inner indices are the two
+// pivots' real and imaginary parts: a step is one product per quadrant and
+// part, on the rows f that the lanes holding them publish in LDS (both
+// operands, by symmetry). Pivot rows and columns are cleared and f is minus a
+// unit vector at the pivots, so the same product leaves Q f and -Q there
+// without cancellation. The diagonal blocks are kept aside and updated from f
+// too: the next choice does not wait for the products.
 __device__ inline float lane_value(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
@@ -356,135 +362,242 @@ __device__ inline double lane_value(double v, int l) {
   const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
   return __longlong_as_double(((long long)hi << 32) | lo);
 }
-__device__ inline unsigned row16_max(unsigned v) {
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));   // row_ror:8
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
-  return v;
+// maximum over the quads of a wave (uniform)
+__device__ inline int wave16_max(unsigned v) {
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));   // row_ror:4
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));   // row_bcast:15
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));   // row_bcast:31
+  return __builtin_amdgcn_readlane((int)v, 63);
 }
-// rows: the tile's rows that are not identity padding; the pairs beyond are
-// left alone (the step count is (rows + 1) / 2).
-// Tried: a fifth wave that keeps the diagonal blocks and picks and inverts the
-// next pair while the others update, which halves their instructions; its own
-// chain per step is then the longer one (a 512 x 512 complex64 step 17 -> 20
-// us, the leaves 110 -> 296 us).
+template <typename T> struct WaveQ {   // Q = P^-1, uniform
+  T q00r, q00i, q01r, q01i, q11r, q11i;
+};
+// p -= a b (complex)
+template <typename T> __device__ inline void wave_sub(T &pr, T &pi, T ar, T ai, T br, T bi) {
+  pr = fma(ai, bi, fma(-ar, br, pr));
+  pi = fma(-ai, br, fma(-ar, bi, pi));
+}
+__device__ inline int frexp_of(float x) { return __builtin_amdgcn_frexp_expf(x); }
+__device__ inline int frexp_of(double x) { return __builtin_amdgcn_frexp_exp(x); }
+// LDS of an inverse: the pivot rows by column
+template <typename T> struct alignas(16) PivotRows {
+  T r[TB][2], i[TB][2];
+};
+// The diagonal blocks: lane 4 m + e of every wave keeps P00, P01, P11, P01 of
+// pair m (e = 0 .. 3); quads exchange them by DPP
+template <int E0, int E1, int E2, int E3> __device__ inline int quad(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, E0 | E1 << 2 | E2 << 4 | E3 << 6, 0xf, 0xf, true);
+}
+template <int E0, int E1, int E2, int E3> __device__ inline float quad(float v) {
+  return __int_as_float(quad<E0, E1, E2, E3>(__float_as_int(v)));
+}
+template <int E0, int E1, int E2, int E3> __device__ inline double quad(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = quad<E0, E1, E2, E3>((int)(b & 0xffffffffll)), hi = quad<E0, E1, E2, E3>((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+template <typename T> struct PivotBlocks {
+  T pr, pi, ar, ai, dr, di, da;
+  int e;
+  bool taken, bad;
+  __device__ inline PivotBlocks(const T (*Ar)[TBP], const T (*Ai)[TBP], int pairs) {
+    const int m = (threadIdx.x & 63) >> 2, q = threadIdx.x & 3, x = 2 * m + (q == 2), y = 2 * m + (q != 0);
+    pr = Ar[x][y];
+    pi = Ai[x][y];
+    taken = m >= pairs;
+    bad = false;
+  }
+  // the pair to eliminate next
+  __device__ inline int pick() {
+    const int m = (threadIdx.x & 63) >> 2;
+    // scaled by an exact power of two near 1 / max |P_ij|
+    T mx = fabs(pr) + fabs(pi);
+    mx = fmax(mx, quad<1, 0, 3, 2>(mx));
+    mx = fmax(mx, quad<2, 3, 0, 1>(mx));
+    e = frexp_of(mx);
+    ar = ldexp(pr, -e);
+    ai = ldexp(pi, -e);
+    const T a00r = quad<0, 0, 0, 0>(ar), a00i = quad<0, 0, 0, 0>(ai), a01r = quad<1, 1, 1, 1>(ar);
+    const T a01i = quad<1, 1, 1, 1>(ai), a11r = quad<2, 2, 2, 2>(ar), a11i = quad<2, 2, 2, 2>(ai);
+    dr = fma(a01i, a01i, fma(-a01r, a01r, fma(-a00i, a11i, a00r * a11r)));
+    di = fma(T(-2) * a01r, a01i, fma(a00i, a11r, a00r * a11i));
+    da = fabs(dr) + fabs(di);
+    const unsigned size = __float_as_uint(fabsf((float)ldexp(da, e))) & ~15u;
+    const int at = wave16_max(taken ? 0u : size + 16u + (unsigned)m) & 15;
+    const bool now = m == at;
+    bad |= now & !((da > T(0)) & (da < T(INFINITY)));
+    taken |= now;
+    return at;
+  }
+  // its inverse: 1 / det = (dr - i di) / |det|^2, det brought near 1 by an exact scale
+  __device__ inline void inverse(int at, WaveQ<T> &Q) const {
+    const int g = frexp_of(da);
+    const T br = ldexp(dr, -g), bi = ldexp(di, -g);
+    T rm = ldexp(rcp_nr(fma(bi, bi, br * br)), -e - g);
+    rm = threadIdx.x & 1 ? -rm : rm;
+    const T er = br * rm, ei = -bi * rm, nr = quad<2, 1, 0, 1>(ar), ni = quad<2, 1, 0, 1>(ai);
+    const T qr = fma(-ni, ei, nr * er), qi = fma(ni, er, nr * ei);
+    Q.q00r = lane_value(qr, 4 * at);
+    Q.q00i = lane_value(qi, 4 * at);
+    Q.q01r = lane_value(qr, 4 * at + 1);
+    Q.q01i = lane_value(qi, 4 * at + 1);
+    Q.q11r = lane_value(qr, 4 * at + 2);
+    Q.q11i = lane_value(qi, 4 * at + 2);
+  }
+  // P_ab -= f(a)^T Q f(b)
+  T xr[2], xi[2], yr[2], yi[2];
+  __device__ inline void read(const PivotRows<T> &f) {
+    const int m = (threadIdx.x & 63) >> 2, q = threadIdx.x & 3, x = 2 * m + (q == 2), y = 2 * m + (q != 0);
+    lds_ld2(f.r[x], xr[0], xr[1]);
+    lds_ld2(f.i[x], xi[0], xi[1]);
+    lds_ld2(f.r[y], yr[0], yr[1]);
+    lds_ld2(f.i[y], yi[0], yi[1]);
+  }
+  __device__ inline void update(const WaveQ<T> &Q) {
+    T v0r = 0, v0i = 0, v1r = 0, v1i = 0;   // -Q f
+    wave_sub(v0r, v0i, Q.q00r, Q.q00i, xr[0], xi[0]);
+    wave_sub(v0r, v0i, Q.q01r, Q.q01i, xr[1], xi[1]);
+    wave_sub(v1r, v1i, Q.q01r, Q.q01i, xr[0], xi[0]);
+    wave_sub(v1r, v1i, Q.q11r, Q.q11i, xr[1], xi[1]);
+    wave_sub(pr, pi, -v0r, -v0i, yr[0], yi[0]);
+    wave_sub(pr, pi, -v1r, -v1i, yr[1], yi[1]);
+  }
+};
+// The inner index kk = lane / 16 of a sweep's products (k = kk & 1, imaginary
+// part for kk >= 2): w of -(Q f)_k as a combination of f's four values
+template <typename T> struct SweepCoef {
+  T w0, w1, w2, w3;
+  bool part;
+  __device__ inline SweepCoef(const WaveQ<T> &Q) {
+    const int kk = (threadIdx.x >> 4) & 3, k = kk & 1;
+    part = kk >> 1;
+    const T s0r = k ? Q.q01r : Q.q00r, s0i = k ? Q.q01i : Q.q00i, s1r = k ? Q.q11r : Q.q01r, s1i = k ? Q.q11i : Q.q01i;
+    w0 = part ? s0i : -s0r;
+    w1 = part ? s0r : s0i;
+    w2 = part ? s1i : -s1r;
+    w3 = part ? s1r : s1i;
+  }
+  // left operands of the real and the imaginary products, for row values f[2]
+  __device__ inline void left(T v0, T v1, T v2, T v3, T &re, T &im) const {
+    re = fma(v3, w3, fma(v2, w2, fma(v1, w1, v0 * w0)));
+    im = part ? -re : re;
+  }
+};
+// Pivot rows jr, jr + 1 of a 16-row quadrant: in accumulators tt, tt + 1 of one
+// lane group (f32), in accumulator tt of two groups (f64). Writes this lane's
+// column of them, minus a unit vector at the pivots if the quadrant is
+// diagonal; whether this lane holds them.
+template <typename T> __device__ inline int pivot_acc(int jr) { return sizeof(T) == 8 ? jr >> 2 : jr & 2; }
+template <typename T> __device__ inline constexpr int pivot_tt(int t) { return sizeof(T) == 8 ? t : t & 2; }
+__device__ inline bool pivot_rows(PivotRows<float> &f, const Mfma<float>::v4 &mr, const Mfma<float>::v4 &mi, int col,
+                                  int group, int jr, bool diagonal) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  const bool own = group == jr >> 2;
+  if (own) {
+    const int c = col & 15;
+    f2 r = f2{mr[0], mr[1]}, i = f2{mi[0], mi[1]};
+    if (jr & 2) { r = f2{mr[2], mr[3]}; i = f2{mi[2], mi[3]}; }
+    if (diagonal && (c & ~1) == jr) { r = f2{c == jr ? -1.0f : 0.0f, c == jr ? 0.0f : -1.0f}; i = f2{0, 0}; }
+    *reinterpret_cast<f2 *>(f.r[col]) = r;
+    *reinterpret_cast<f2 *>(f.i[col]) = i;
+  }
+  return own;
+}
+__device__ inline bool pivot_rows(PivotRows<double> &f, const Mfma<double>::v4 &mr, const Mfma<double>::v4 &mi, int col,
+                                  int group, int jr, bool diagonal) {
+  const int k = group - (jr & 3);
+  const bool own = (k & ~1) == 0;
+  if (own) {
+    const int c = col & 15;
+    double r, i;
+    if (jr < 8) {
+      if (jr < 4) { r = mr[0]; i = mi[0]; } else { r = mr[1]; i = mi[1]; }
+    } else {
+      if (jr < 12) { r = mr[2]; i = mi[2]; } else { r = mr[3]; i = mi[3]; }
+    }
+    if (diagonal && (c & ~1) == jr) { r = c == jr + k ? -1.0 : 0.0; i = 0; }
+    f.r[col][k] = r;
+    f.i[col][k] = i;
+  }
+  return own;
+}
+// The inverse of the tile in (Ar, Ai), in place, by four waves, a quadrant
+// each; every wave keeps all diagonal blocks and makes the same choice, so a
+// step has one barrier, between the rows' way into LDS (one of two buffers in
+// turn) and out of it. rows: the tile's rows that are not identity padding; the
+// pairs beyond are left alone (the step count is (rows + 1) / 2).
+// Bound by one step's chain: choice, rows, barrier, blocks; about 150
+// instructions, 0.34 us a pair. With the tile in registers row by row, the
+// blocks read back from LDS and the update on vector units, 0.53 us: the factor
+// of 512^2 complex64 2.04 -> 1.87 ms, of 120^2 FP64 0.61 -> 0.56 ms, of 768^2
+// FP64 6.30 -> 6.03 ms. Tried with that layout: a fifth wave that picks and
+// inverts the next pair while the others update (a step of 512^2 17 -> 20 us),
+// and eight waves (18.6 us).
 template <typename T, typename LT>
 __device__ void tile_inverse_pairs(LT &L, int rows, int *status) {
-  static_assert(TB * TB == 4 * NT, "4 elements per thread");
-  static_assert(2 * sizeof(InvX<T>) <= offsetof(LT, end), "exchange buffers overlay the tiles only");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int i = tid >> 3, c0 = (tid & 7) * 4;
-  T ar[4], ai[4];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, qi = wv >> 1, qj = wv & 1, c = lane & 15;
+  const int kk = lane >> 4, k = kk & 1, part = kk >> 1, pairs = min(TB, rows + 1) >> 1;
+  typename Mfma<T>::v4 mr, mi;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {   // the upper triangle
-    const int x = min(i, c0 + q), y = max(i, c0 + q);
-    ar[q] = L.Ar[x][y];
-    ai[q] = L.Ai[x][y];
+  for (int t = 0; t < 4; ++t) {   // the upper triangle
+    const int r = 16 * qi + Mfma<T>::crow(lane, t), x = min(r, 16 * qj + c), y = max(r, 16 * qj + c);
+    mr[t] = L.Ar[x][y];
+    mi[t] = L.Ai[x][y];
   }
-  __syncthreads();   // every row is in registers before the exchange buffers cover Ar, Ai
-  InvX<T> *X = reinterpret_cast<InvX<T> *>(&L);
-  const int mine = lane & 15, d = 2 * mine, pairs = min(TB, rows + 1) >> 1;
-  bool bad = false, taken = mine >= pairs;
+  PivotBlocks<T> B(L.Ar, L.Ai, pairs);
 #pragma unroll 2
   for (int st = 0; st < pairs; ++st) {
-    InvX<T> &B = X[st & 1];
-    lds_st4(&B.r[i][c0], ar);
-    lds_st4(&B.i[i][c0], ai);
-    __syncthreads();
-    // this lane's pair: P, scaled by an exact power of two near 1 / max |P_ij|,
-    // and Q = P^-1 = adj(P') sc / det(P')
-    T p00r, p01r, p00i, p01i, p10r, p11r, p10i, p11i;
-    lds_ld2(&B.r[d][d], p00r, p01r);
-    lds_ld2(&B.i[d][d], p00i, p01i);
-    lds_ld2(&B.r[d + 1][d], p10r, p11r);
-    lds_ld2(&B.i[d + 1][d], p10i, p11i);
-    const T mx = fmax(fmax(fmax(fabs(p00r), fabs(p00i)), fmax(fabs(p01r), fabs(p01i))),
-                      fmax(fmax(fabs(p10r), fabs(p10i)), fmax(fabs(p11r), fabs(p11i))));
-    const T sc = exp_scale(mx);
-    const T a00r = p00r * sc, a00i = p00i * sc, a01r = p01r * sc, a01i = p01i * sc;
-    const T a10r = p10r * sc, a10i = p10i * sc, a11r = p11r * sc, a11i = p11i * sc;
-    const T dr = (a00r * a11r - a00i * a11i) - (a01r * a10r - a01i * a10i);
-    const T di = (a00r * a11i + a00i * a11r) - (a01r * a10i + a01i * a10r);
-    const T da = fabs(dr) + fabs(di);
-    const bool ok = da > T(0) && isfinite(da) && mx > T(0) && isfinite(mx);
-    const unsigned size = __float_as_uint(fabsf((float)(da * exp_scale(sc)))) & ~15u;
-    const unsigned key = row16_max(taken ? 0u : size + 16u + (unsigned)mine);
-    const int pick = __builtin_amdgcn_readfirstlane((int)(key & 15u)), j = 2 * pick;
-    T f0r, f1r, f0i, f1i, h0r[4], h0i[4], h1r[4], h1i[4];
-    lds_ld2(&B.r[i][j], f0r, f1r);
-    lds_ld2(&B.i[i][j], f0i, f1i);
-    lds_ld4(&B.r[j][c0], h0r);
-    lds_ld4(&B.i[j][c0], h0i);
-    lds_ld4(&B.r[j + 1][c0], h1r);
-    lds_ld4(&B.i[j + 1][c0], h1i);
-    // 1 / det: (dr - i di) / |det|^2 with det brought to [0.5, 1) by an exact scale
-    const T ds = exp_scale(fmax(fabs(dr), fabs(di)));
-    const T br = dr * ds, bi = di * ds;
-    const T rm = rcp_nr(br * br + bi * bi) * ds * sc;
-    const T er = br * rm, ei = -bi * rm;
-    const T q00r = lane_value(a11r * er - a11i * ei, pick), q00i = lane_value(a11r * ei + a11i * er, pick);
-    const T q01r = lane_value(-(a01r * er - a01i * ei), pick), q01i = lane_value(-(a01r * ei + a01i * er), pick);
-    const T q10r = lane_value(-(a10r * er - a10i * ei), pick), q10i = lane_value(-(a10r * ei + a10i * er), pick);
-    const T q11r = lane_value(a00r * er - a00i * ei, pick), q11i = lane_value(a00r * ei + a00i * er, pick);
-    if (!__builtin_amdgcn_readlane((int)ok, pick)) bad = true;
-    taken = taken || mine == pick;
-    // new row = base - g0 h0 - g1 h1: off the pivot rows base = row and
-    // g = [f0 f1] Q; on them base = 0 and g = -(row of Q)
-    T g0r = f0r * q00r - f0i * q00i + f1r * q10r - f1i * q10i;
-    T g0i = f0r * q00i + f0i * q00r + f1r * q10i + f1i * q10r;
-    T g1r = f0r * q01r - f0i * q01i + f1r * q11r - f1i * q11i;
-    T g1i = f0r * q01i + f0i * q01r + f1r * q11i + f1i * q11r;
-    const bool r0 = i == j, r1 = i == j + 1, prow = r0 || r1;
-    g0r = r0 ? -q00r : (r1 ? -q10r : g0r);
-    g0i = r0 ? -q00i : (r1 ? -q10i : g0i);
-    g1r = r0 ? -q01r : (r1 ? -q11r : g1r);
-    g1i = r0 ? -q01i : (r1 ? -q11i : g1i);
-    // the pivot columns: Q on the pivot rows, -g elsewhere
-    const T cjr = -g0r, cji = -g0i, ckr = -g1r, cki = -g1i;
+    PivotRows<T> &f = L.f[st & 1];
+    const int at = B.pick(), j = 2 * at, jr = j & 15;
+    const bool inr = j >> 4 == qi, inc = j >> 4 == qj, pc = inc && (c & ~1) == jr;
+    bool own = inr;
+    if (inr) own = pivot_rows(f, mr, mi, 16 * qj + c, kk, jr, inc);
+    const int tt = pivot_acc<T>(jr);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const T xr0 = prow ? T(0) : ar[q], xi0 = prow ? T(0) : ai[q];
-      const T xr = xr0 - (g0r * h0r[q] - g0i * h0i[q]) - (g1r * h1r[q] - g1i * h1i[q]);
-      const T xi = xi0 - (g0r * h0i[q] + g0i * h0r[q]) - (g1r * h1i[q] + g1i * h1r[q]);
-      const int c = c0 + q;
-      ar[q] = c == j ? cjr : (c == j + 1 ? ckr : xr);
-      ai[q] = c == j ? cji : (c == j + 1 ? cki : xi);
+    for (int t = 0; t < 4; ++t) {
+      const bool zero = pc || (own && pivot_tt<T>(t) == tt);
+      mr[t] = zero ? T(0) : mr[t];
+      mi[t] = zero ? T(0) : mi[t];
     }
+    WaveQ<T> Q;
+    B.inverse(at, Q);
+    const SweepCoef<T> W(Q);
+    __syncthreads();
+    T v0, v1, v2, v3, are, aim;
+    lds_ld2(f.r[16 * qi + c], v0, v2);
+    lds_ld2(f.i[16 * qi + c], v1, v3);
+    const T bre = (&f.r[16 * qj + c][k])[part * 2 * TB], bim = (&f.i[16 * qj + c][k])[-part * 2 * TB];
+    B.read(f);
+    __builtin_amdgcn_sched_barrier(0);   // all reads first: they wait for LDS once
+    W.left(v0, v1, v2, v3, are, aim);
+    mr = Mfma<T>::mac(are, bre, mr);
+    mi = Mfma<T>::mac(aim, bim, mi);
+    B.update(Q);
   }
-  __syncthreads();   // the last step's reads are done before Ar, Ai are written
+  // the padding stays
 #pragma unroll
-  for (int q = 0; q < 4; ++q) { L.Ar[i][c0 + q] = ar[q]; L.Ai[i][c0 + q] = ai[q]; }
-  if (bad) *status = 1;
+  for (int t = 0; t < 4; ++t) {
+    const int r = 16 * qi + Mfma<T>::crow(lane, t);
+    L.Ar[r][16 * qj + c] = r < 2 * pairs ? -mr[t] : mr[t];
+    L.Ai[r][16 * qj + c] = r < 2 * pairs ? -mi[t] : mi[t];
+  }
+  if (B.bad) *status = 1;
   __syncthreads();
 }
 
-// The same inverse by one wave, in its registers, for the leaves, of which
-// there are thousands. The steps are sweeps, which keep the tile symmetric:
-// with f = the pivot rows and Q = P^-1 the tile becomes M - f^T Q f off the
-// pivots, Q f on the pivot rows and columns, -Q on the block, and -M^-1 in the
-// end. The tile lies in the accumulators of 16x16x4 products, whose four inner
-// indices are the two pivots' real and imaginary parts: a step is one product
-// per quadrant and part, on the rows f that the lanes holding them publish in
-// LDS (both operands, by symmetry). Pivot rows and columns are cleared and f
-// is minus a unit vector at the pivots, so the same product leaves Q f and -Q
-// there without cancellation. The pivot blocks are kept aside, that of pair m
-// in lanes m + 16 i, updated from f as well: the next choice does not wait for
-// the products.
-// Four waves issue four times tile_inverse_pairs's choice; here it is issued
-// once. Bound by those instructions: the 8192 leaves of 512^2 complex64 110 ->
-// 53 us, the 16384 of 768^2 FP64 469 -> 206 us. As the chain of one tile it is
-// no shorter (0.53 us a pair, as four waves), and it takes 180 registers in
-// FP64, so the fronts, steps and merges keep tile_inverse_pairs (768^2 FP64
-// merges 511 -> 597 us, steps 24 -> 31 us with this one).
+// The same inverse by one wave, for the leaves, of which there are thousands:
+// the choice's instructions are issued once a leaf and not by four waves. Bound
+// by them: the 8192 leaves of 512^2 complex64 110 -> 51 us, the 16384 of 768^2
+// FP64 469 -> 200 us. As the chain of one tile it is slower than four waves
+// and takes 180 registers in FP64.
 template <typename T> struct WaveTile {
   typename Mfma<T>::v4 r[2][2], i[2][2];
 };
 // LDS of one wave's inverse: the pivot rows by column, and a second set for
 // the lanes that have none to write (a branch on lanes inside the choice of
 // the accumulators makes the compiler copy the tile at every join)
-template <typename T> struct alignas(16) WaveRows {
-  T r[TB][2], i[TB][2];
+template <typename T> struct WaveRows : PivotRows<T> {
   T none[2][TB][2];
 };
 // The pivot rows j, j + 1 (j = 16 QR + jr, in accumulator TT: of one lane
@@ -547,9 +660,6 @@ __device__ inline void wave_lds_order() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-template <typename T> struct WaveQ {   // Q = P^-1 (uniform), block of this lane's pair
-  T q00r, q00i, q01r, q01i, q11r, q11i;
-};
 // One sweep's products on the rows in accumulator TT of quadrant row QR
 template <int QR, int TT, typename T>
 __device__ inline void wave_sweep(WaveTile<T> &M, WaveRows<T> &f, int lane, int j, const WaveQ<T> &Q) {
@@ -561,9 +671,7 @@ __device__ inline void wave_sweep(WaveTile<T> &M, WaveRows<T> &f, int lane, int 
   unit[1] = lane ? T(-1) : T(0);
   unit[2 * TB] = unit[2 * TB + 1] = 0;
   wave_lds_order();
-  // inner index kk: -(Q f)_k, real (kk < 2) and imaginary part, against f_k
-  const T s0r = k ? Q.q01r : Q.q00r, s0i = k ? Q.q01i : Q.q00i, s1r = k ? Q.q11r : Q.q01r, s1i = k ? Q.q11i : Q.q01i;
-  const T w0 = part ? s0i : -s0r, w1 = part ? s0r : s0i, w2 = part ? s1i : -s1r, w3 = part ? s1r : s1i;
+  const SweepCoef<T> W(Q);
   const T *fre = part ? &f.i[c][k] : &f.r[c][k], *fim = part ? &f.r[c][k] : &f.i[c][k];
   T are[2], aim[2], bre[2], bim[2];
 #pragma unroll
@@ -573,8 +681,7 @@ __device__ inline void wave_sweep(WaveTile<T> &M, WaveRows<T> &f, int lane, int 
     T v0, v1, v2, v3;
     lds_ld2(f.r[16 * q + c], v0, v2);
     lds_ld2(f.i[16 * q + c], v1, v3);
-    are[q] = fma(v3, w3, fma(v2, w2, fma(v1, w1, v0 * w0)));
-    aim[q] = part ? -are[q] : are[q];
+    W.left(v0, v1, v2, v3, are[q], aim[q]);
   }
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -601,13 +708,6 @@ __device__ inline void wave_sweep_at(WaveTile<double> &M, WaveRows<double> &f, i
     else { if (j < 28) wave_sweep<1, 2>(M, f, lane, j, Q); else wave_sweep<1, 3>(M, f, lane, j, Q); }
   }
 }
-// p -= a b (complex)
-template <typename T> __device__ inline void wave_sub(T &pr, T &pi, T ar, T ai, T br, T bi) {
-  pr = fma(ai, bi, fma(-ar, br, pr));
-  pi = fma(-ai, br, fma(-ar, bi, pi));
-}
-__device__ inline int frexp_of(float x) { return __builtin_amdgcn_frexp_expf(x); }
-__device__ inline int frexp_of(double x) { return __builtin_amdgcn_frexp_exp(x); }
 // (Ar, Ai) in LDS -> its inverse in M, entry (16 a + crow(lane, t), 16 b + lane % 16)
 // in element t of quadrant (a, b); f: LDS that no other wave uses.
 // rows: the tile's rows that are not identity padding; the pairs beyond are
@@ -615,7 +715,7 @@ __device__ inline int frexp_of(double x) { return __builtin_amdgcn_frexp_exp(x);
 template <typename T>
 __device__ inline bool wave_inverse(WaveTile<T> &M, const T (*Ar)[TBP], const T (*Ai)[TBP], WaveRows<T> &f, int rows) {
   const int lane = threadIdx.x & 63, mine = lane & 15;
-  const int pairs = min(TB, rows + 1) >> 1, d = 2 * mine;
+  const int pairs = min(TB, rows + 1) >> 1;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -627,60 +727,16 @@ __device__ inline bool wave_inverse(WaveTile<T> &M, const T (*Ar)[TBP], const T 
         M.r[a][b][t] = Ar[x][y];
         M.i[a][b][t] = Ai[x][y];
       }
-  T p00r = Ar[d][d], p00i = Ai[d][d], p01r = Ar[d][d + 1], p01i = Ai[d][d + 1];
-  T p11r = Ar[d + 1][d + 1], p11i = Ai[d + 1][d + 1];
-  bool bad = false, taken = mine >= pairs;
+  PivotBlocks<T> B(Ar, Ai, pairs);
 #pragma unroll 1
   for (int st = 0; st < pairs; ++st) {
-    // this lane's block, scaled by an exact power of two near 1 / max |P_ij|
-    const T mx = fmax(fmax(fabs(p00r) + fabs(p00i), fabs(p01r) + fabs(p01i)), fabs(p11r) + fabs(p11i));
-    const int e = frexp_of(mx);
-    const T a00r = ldexp(p00r, -e), a00i = ldexp(p00i, -e), a01r = ldexp(p01r, -e), a01i = ldexp(p01i, -e);
-    const T a11r = ldexp(p11r, -e), a11i = ldexp(p11i, -e);
-    const T dr = fma(a01i, a01i, fma(-a01r, a01r, fma(-a00i, a11i, a00r * a11r)));
-    const T di = fma(T(-2) * a01r, a01i, fma(a00i, a11r, a00r * a11i));
-    const T da = fabs(dr) + fabs(di);
-    const unsigned size = __float_as_uint(fabsf((float)ldexp(da, e))) & ~15u;
-    const unsigned key = row16_max(taken ? 0u : size + 16u + (unsigned)mine);
-    const int pick = __builtin_amdgcn_readfirstlane((int)(key & 15u));
-    // 1 / det: (dr - i di) / |det|^2 with det brought near 1 by an exact scale
-    const int g = frexp_of(da);
-    const T br = ldexp(dr, -g), bi = ldexp(di, -g);
-    const T rm = ldexp(rcp_nr(fma(bi, bi, br * br)), -e - g);
-    const T er = br * rm, ei = -bi * rm;
+    const int pick = B.pick();
     WaveQ<T> Q;
-    Q.q00r = lane_value(fma(-a11i, ei, a11r * er), pick);
-    Q.q00i = lane_value(fma(a11i, er, a11r * ei), pick);
-    Q.q01r = lane_value(fma(a01i, ei, -a01r * er), pick);
-    Q.q01i = lane_value(fma(-a01i, er, -a01r * ei), pick);
-    Q.q11r = lane_value(fma(-a00i, ei, a00r * er), pick);
-    Q.q11i = lane_value(fma(a00i, er, a00r * ei), pick);
-    const bool now = mine == pick;
-    bad |= now & !((da > T(0)) & (da < T(INFINITY)));
-    taken |= now;
+    B.inverse(pick, Q);
     wave_lds_order();
     wave_sweep_at(M, f, lane, 2 * pick, Q);
-    // the pivot blocks: P_ab -= f(a)^T Q f(b)
-    T xr[2], xi[2], yr[2], yi[2];
-    lds_ld2(f.r[d], xr[0], xr[1]);
-    lds_ld2(f.i[d], xi[0], xi[1]);
-    lds_ld2(f.r[d + 1], yr[0], yr[1]);
-    lds_ld2(f.i[d + 1], yi[0], yi[1]);
-    T v0r = 0, v0i = 0, v1r = 0, v1i = 0, u0r = 0, u0i = 0, u1r = 0, u1i = 0;   // -Q f
-    wave_sub(v0r, v0i, Q.q00r, Q.q00i, xr[0], xi[0]);
-    wave_sub(v0r, v0i, Q.q01r, Q.q01i, xr[1], xi[1]);
-    wave_sub(v1r, v1i, Q.q01r, Q.q01i, xr[0], xi[0]);
-    wave_sub(v1r, v1i, Q.q11r, Q.q11i, xr[1], xi[1]);
-    wave_sub(u0r, u0i, Q.q00r, Q.q00i, yr[0], yi[0]);
-    wave_sub(u0r, u0i, Q.q01r, Q.q01i, yr[1], yi[1]);
-    wave_sub(u1r, u1i, Q.q01r, Q.q01i, yr[0], yi[0]);
-    wave_sub(u1r, u1i, Q.q11r, Q.q11i, yr[1], yi[1]);
-    wave_sub(p00r, p00i, -v0r, -v0i, xr[0], xi[0]);
-    wave_sub(p00r, p00i, -v1r, -v1i, xr[1], xi[1]);
-    wave_sub(p01r, p01i, -v0r, -v0i, yr[0], yi[0]);
-    wave_sub(p01r, p01i, -v1r, -v1i, yr[1], yi[1]);
-    wave_sub(p11r, p11i, -u0r, -u0i, yr[0], yi[0]);
-    wave_sub(p11r, p11i, -u1r, -u1i, yr[1], yi[1]);
+    B.read(f);
+    B.update(Q);
   }
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -693,7 +749,7 @@ __device__ inline bool wave_inverse(WaveTile<T> &M, const T (*Ar)[TBP], const T 
         M.i[a][b][t] = neg ? -M.i[a][b][t] : M.i[a][b][t];
       }
     }
-  return !bad;
+  return !B.bad;
 }
 // M into a tile of pitch `pitch`
 template <typename T>
@@ -715,15 +771,18 @@ __device__ inline void wave_store(const WaveTile<T> &M, T *re, T *im, int pitch)
 // (with A: the exchange buffers of the inverse) and, where used, a third tile.
 template <typename T> struct NdLds2 {
   T Ar[TB][TBP], Ai[TB][TBP];
-  T Br[TB][TBP], Bi[TB][TBP];
-  unsigned char pad[step_lds_pad<T>()];
-  int end[4];
+  union {
+    struct { T Br[TB][TBP], Bi[TB][TBP]; };
+    PivotRows<T> f[2];
+  };
 };
 template <typename T> struct NdLds3 {
   T Ar[TB][TBP], Ai[TB][TBP];
-  T Br[TB][TBP], Bi[TB][TBP];
+  union {
+    struct { T Br[TB][TBP], Bi[TB][TBP]; };
+    PivotRows<T> f[2];
+  };
   T Pr[TB][TBP], Pi[TB][TBP];
-  int end[4];
 };
 
 // A leaf box per wave: its five-point matrix (cells in (x, y) order,
@@ -890,7 +949,7 @@ template <typename T> struct NdStep {
 // The front's [F_ss | F_sb] (tiles I <= J and the border's) from the
 // children, and the inverse of the first pivot tile.
 template <typename T>
-__global__ void __launch_bounds__(NT) k_nd_front(NdStep<T> A) {
+__global__ void __launch_bounds__(NT, 2) k_nd_front(NdStep<T> A) {
   __shared__ NdLds2<T> S;
   const NdLevel &L = A.L;
   const int ns = L.sp / TB, nb = L.bp / TB, tri = ns * (ns + 1) / 2, per = tri + ns * nb;
@@ -981,7 +1040,7 @@ __host__ __device__ inline int nd_step_items(int ns, int nb) {
   return np * (np + 1) + np * nb;
 }
 template <typename T>
-__global__ void __launch_bounds__(NT) k_nd_step(NdStep<T> A) {
+__global__ void __launch_bounds__(NT, 2) k_nd_step(NdStep<T> A) {
   __shared__ NdLds3<T> S;
   const NdLevel &L = A.L;
   const int ns = L.sp / TB, nb = L.bp / TB, np = (ns + 1) / 2, per = nd_step_items(ns, nb), p = A.p;
@@ -1247,7 +1306,7 @@ __global__ void __launch_bounds__(NT) k_nd_update(NdLevel L, const T *__restrict
 // 42 us here; 768^2 FP64, 11 x 5 and 11 x 11: 239 and 270 us.
 // A: F_ss, then P, then C_IJ on its way out; B: W_J.
 template <typename T>
-__global__ void __launch_bounds__(NT) k_nd_merge(NdLevel L, NdBands<T> bd, const T *__restrict__ Cin, T *__restrict__ X,
+__global__ void __launch_bounds__(NT, 2) k_nd_merge(NdLevel L, NdBands<T> bd, const T *__restrict__ Cin, T *__restrict__ X,
                                                  T *__restrict__ W, T *__restrict__ Cout, int *status) {
   extern __shared__ __align__(16) unsigned char nd_smem[];
   NdLds2<T> &M = *reinterpret_cast<NdLds2<T> *>(nd_smem);
