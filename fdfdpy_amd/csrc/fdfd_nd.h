@@ -1850,16 +1850,23 @@ __global__ void __launch_bounds__(64 * ND_TREE_WAVES) k_nd_down_tree(NdTree t, N
 
 // Upwards, one level above the subtrees (and the root, whose z is x): 32
 // columns of [X | W] of one box per workgroup, the separator's rows spread
-// over its half waves.
-template <typename T, int R, int NW>
+// over its half waves, UN at a time. These matrix rows do not depend on f:
+// their loads go out before f is gathered, so a batch of 2 NW UN rows costs one
+// trip to memory. Bound by the latencies of one launch: 512^2 complex64 with 4
+// right-hand sides, the root's 1023 rows 20.6 -> 15 us, the levels below it
+// 12.5 .. 7 -> 10 .. 6 us against rows loaded four at a time after f; the solve
+// 1.05 -> 0.99 ms, of 512^2 FP64 with one 0.42 -> 0.35 ms. The caller's NW and
+// UN make one batch of a separator up to 512 rows; larger batches than the
+// separator needs would load rows for nothing.
+template <typename T, int R, int NW, int UN>
 __global__ void __launch_bounds__(64 * NW) k_nd_up(NdLevel L, NdVec<T> A, const T *__restrict__ uin,
                                                    T *__restrict__ uout, int nq, int add) {
-  constexpr int RG = 2 * NW, JC = 256;
+  constexpr int RG = 2 * NW, JC = RG * UN;
   __shared__ __align__(16) union {
     T f[JC][R][2];
-    T red[RG][2 * R][32];
+    T red[NW][2 * R][32];
   } S;
-  const int tid = threadIdx.x, c32 = tid & 31, rg = tid >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c32 = tid & 31, rg = tid >> 5;
   const int chunks = (L.sp + L.bp) / 32, box = blockIdx.x / chunks, c = (blockIdx.x % chunks) * 32 + c32;
   const NdBox B = nd_box(L, box);
   const bool inX = c < L.sp;
@@ -1870,40 +1877,50 @@ __global__ void __launch_bounds__(64 * NW) k_nd_up(NdLevel L, NdVec<T> A, const 
 #pragma unroll
   for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
   for (int j0 = 0; j0 < B.s; j0 += JC) {
-    const int nj = min(JC, B.s - j0);
+    T gr[UN], gi[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {   // past the separator: its last row, against f = 0
+      const T *row = m + (size_t)min(j0 + rg + u * RG, B.s - 1) * pitch;
+      gr[u] = row[0];
+      gi[u] = row[plane];
+    }
     if (j0) __syncthreads();
-    for (int e = tid; e < nj * R; e += 64 * NW) {
+    for (int e = tid; e < JC * R; e += 64 * NW) {
       const int j = e / R, q = e % R;
       T re = 0, im = 0;
-      if (q < nq) nd_fs(L, B, A.f, uin, B.k0, B.k1, nq, j0 + j, q, re, im);
+      if (j0 + j < B.s && q < nq) nd_fs(L, B, A.f, uin, B.k0, B.k1, nq, j0 + j, q, re, im);
       S.f[j][q][0] = re;
       S.f[j][q][1] = im;
     }
     __syncthreads();
-#pragma unroll 4
-    for (int j = rg; j < nj; j += RG) {
-      const T gr = m[(size_t)(j0 + j) * pitch], gi = m[plane + (size_t)(j0 + j) * pitch];
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
 #pragma unroll
       for (int q = 0; q < R; ++q) {
-        const T fr = S.f[j][q][0], fi = S.f[j][q][1];
-        ar[q] += gr * fr - gi * fi;
-        ai[q] += gr * fi + gi * fr;
+        const T fr = S.f[rg + u * RG][q][0], fi = S.f[rg + u * RG][q][1];
+        ar[q] += gr[u] * fr - gi[u] * fi;
+        ai[q] += gr[u] * fi + gi[u] * fr;
       }
-    }
   }
-  __syncthreads();
 #pragma unroll
   for (int q = 0; q < R; ++q) {
-    S.red[rg][2 * q][c32] = ar[q];
-    S.red[rg][2 * q + 1][c32] = ai[q];
+    ar[q] += __shfl_xor(ar[q], 32);
+    ai[q] += __shfl_xor(ai[q], 32);
   }
+  __syncthreads();
+  if (lane < 32)
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      S.red[wv][2 * q][c32] = ar[q];
+      S.red[wv][2 * q + 1][c32] = ai[q];
+    }
   __syncthreads();
   for (int e = tid; e < 32 * R; e += 64 * NW) {
     const int cc = e & 31, q = e >> 5, col = (blockIdx.x % chunks) * 32 + cc;
     if (q >= nq) continue;
     T sr = 0, si = 0;
 #pragma unroll
-    for (int g = 0; g < RG; ++g) { sr += S.red[g][2 * q][cc]; si += S.red[g][2 * q + 1][cc]; }
+    for (int g = 0; g < NW; ++g) { sr += S.red[g][2 * q][cc]; si += S.red[g][2 * q + 1][cc]; }
     if (col < B.s) {
       int ci, cj;
       nd_sep_ij(L, B, col, ci, cj);
@@ -1919,11 +1936,11 @@ __global__ void __launch_bounds__(64 * NW) k_nd_up(NdLevel L, NdVec<T> A, const 
 
 // Downwards, one level above the subtrees: 16 rows of W of one box per
 // workgroup; a lane reads its row in 16-byte pieces, the columns spread over
-// the quarter waves.
+// the quarter waves, UN pieces at a time and before x is gathered, as in k_nd_up.
 constexpr int ND_DOWN_WAVES = 8;
-template <typename T, int R>
+template <typename T, int R, int UN>
 __global__ void __launch_bounds__(64 * ND_DOWN_WAVES) k_nd_down(NdLevel L, NdVec<T> A, int nq, int add) {
-  constexpr int CC = 256, GROUPS = 4 * ND_DOWN_WAVES;
+  constexpr int GROUPS = 4 * ND_DOWN_WAVES, CC = 4 * GROUPS * UN;
   __shared__ __align__(16) union {
     T x[CC][R][2];
     T red[ND_DOWN_WAVES][2 * R][16];
@@ -1937,31 +1954,41 @@ __global__ void __launch_bounds__(64 * ND_DOWN_WAVES) k_nd_down(NdLevel L, NdVec
 #pragma unroll
   for (int q = 0; q < R; ++q) { ar[q] = 0; ai[q] = 0; }
   for (int b0 = 0; b0 < B.b; b0 += CC) {
+    T gr[UN][4], gi[UN][4];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {   // past the border: its last piece, against x = 0
+      const int c = min(b0 + 4 * (grp + u * GROUPS), L.bp - 4);
+      ld_row4(W + c, gr[u]);
+      ld_row4(W + plane + c, gi[u]);
+    }
     if (b0) __syncthreads();
-    const int nb = min(CC, L.bp - b0);
-    for (int e = tid; e < nb * R; e += 64 * ND_DOWN_WAVES) {
-      const int c = e / R, q = e % R;
-      T xr = 0, xi = 0;
-      if (b0 + c < B.b && q < nq)
-        nd_ld((const T *)A.v, nd_border_cell(L.nx, L.ny, L.dx, L.dy, B, b0 + c) * nq + q, xr, xi);
-      S.x[c][q][0] = xr;
-      S.x[c][q][1] = xi;
+    constexpr int TS = 64 * ND_DOWN_WAVES, G = (CC * R + TS - 1) / TS;
+    T xr[G], xi[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const int e = tid + u * TS, q = min(e % R, nq - 1);
+      nd_ld((const T *)A.v, nd_border_cell(L.nx, L.ny, L.dx, L.dy, B, min(b0 + e / R, B.b - 1)) * nq + q, xr[u], xi[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const int e = tid + u * TS, c = e / R, q = e % R;
+      if (CC * R < TS && e >= CC * R) break;
+      const bool has = b0 + c < B.b && q < nq;
+      S.x[c][q][0] = has ? xr[u] : T(0);
+      S.x[c][q][1] = has ? xi[u] : T(0);
     }
     __syncthreads();
-#pragma unroll 2
-    for (int c = 4 * grp; c < nb; c += 4 * GROUPS) {
-      T gr[4], gi[4];
-      ld_row4(W + b0 + c, gr);
-      ld_row4(W + plane + b0 + c, gi);
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-          const T xr = S.x[c + k][q][0], xi = S.x[c + k][q][1];
-          ar[q] += gr[k] * xr - gi[k] * xi;
-          ai[q] += gr[k] * xi + gi[k] * xr;
+          const int c = 4 * (grp + u * GROUPS) + k;
+          const T xr = S.x[c][q][0], xi = S.x[c][q][1];
+          ar[q] += gr[u][k] * xr - gi[u][k] * xi;
+          ai[q] += gr[u][k] * xi + gi[u][k] * xr;
         }
-    }
   }
 #pragma unroll
   for (int q = 0; q < R; ++q) {
@@ -2142,17 +2169,17 @@ int nd_pass(const NdPlan &P, NdTree &t, const NdVec<T> &A, int nq, int add, hipS
   for (int l = t.top + 1; l <= P.nlev; ++l) {
     const NdLevel &L = P.lev[l];
     const int grid = L.nbox * ((L.sp + L.bp) / 32);
-    if (L.s <= 128)
-      hipLaunchKernelGGL((k_nd_up<T, R, 4>), dim3(grid), dim3(256), 0, s, L, A, uin, uout, nq, add);
-    else
-      hipLaunchKernelGGL((k_nd_up<T, R, 8>), dim3(grid), dim3(512), 0, s, L, A, uin, uout, nq, add);
+    const auto up = L.s <= 64 ? k_nd_up<T, R, 4, 8> : L.s <= 128 ? k_nd_up<T, R, 4, 16>
+                  : L.s <= 256 ? k_nd_up<T, R, 8, 16> : k_nd_up<T, R, 16, 16>;
+    hipLaunchKernelGGL(up, dim3(grid), dim3(L.s <= 128 ? 256 : L.s <= 256 ? 512 : 1024), 0, s, L, A, uin, uout, nq, add);
     uin = uout;
     uout = uin == A.u0 ? A.u1 : A.u0;
   }
   for (int l = P.nlev - 1; l > t.top; --l) {
     const NdLevel &L = P.lev[l];
-    hipLaunchKernelGGL((k_nd_down<T, R>), dim3(L.nbox * ((L.s + 15) / 16)), dim3(64 * ND_DOWN_WAVES), 0, s, L, A, nq,
-                       add);
+    const auto down = L.b <= 256 ? k_nd_down<T, R, 2> : L.b <= 512 || sizeof(T) == 8 ? k_nd_down<T, R, 4>
+                                                      : k_nd_down<T, R, 8>;
+    hipLaunchKernelGGL(down, dim3(L.nbox * ((L.s + 15) / 16)), dim3(64 * ND_DOWN_WAVES), 0, s, L, A, nq, add);
   }
   hipLaunchKernelGGL((k_nd_down_tree<T, R>), dim3(sub), dim3(64 * ND_TREE_WAVES), 0, s, t, A, X, cpl);
   HIP_TRY(hipGetLastError());

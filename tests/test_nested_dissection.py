@@ -135,12 +135,14 @@ def _device(N, npml, pol, eps, precision):
 @pytest.mark.parametrize("N,npml,pol,nrhs", [
     ((64, 64), [8, 8], "Ez", 1), ((65, 97), [9, 12], "Hz", 2), ((128, 66), [10, 0], "Ez", 3),
     ((129, 70), [0, 0], "Hz", 5), ((64, 300), [8, 15], "Ez", 8), ((257, 96), [20, 10], "Hz", 9),
-    ((16, 16), [4, 4], "Ez", 1), ((17, 120), [0, 10], "Hz", 4), ((33, 32), [6, 6], "Ez", 5), ((47, 63), [9, 9], "Hz", 2)])
+    ((16, 16), [4, 4], "Ez", 1), ((17, 120), [0, 10], "Hz", 4), ((33, 32), [6, 6], "Ez", 5), ((47, 63), [9, 9], "Hz", 2),
+    ((301, 290), [12, 12], "Ez", 4)])
 @pytest.mark.parametrize("precision", ["fp64", "c64"])
 def test_solves_match_the_oracle(N, npml, pol, nrhs, precision):
     """Edges of the tree (power-of-two sides and their neighbours, long
     grids), both polarizations, periodic axes, a lossy cell, every count of
-    right-hand sides per pass; forward and transposed."""
+    right-hand sides per pass, separators and borders over 512 cells (more than
+    one batch of a sweep's rows); forward and transposed."""
     if precision == "c64" and min(N) < 64:
         pytest.skip("complex64 factors of grids below 64 cells are block factors")
     rng = np.random.default_rng(sum(N) + nrhs)
