@@ -2262,6 +2262,12 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
   residual(nullptr);
   hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts, norms + nrhs);
   const int sweeps = wrap_exact(g) ? 2 : 1;
+  // A complex64 sweep leaves 1e-5 .. 1e-2 of the residual; one that ends within
+  // tol but above a quarter of it is followed by one more (a solve in six), so
+  // that fields that stop just below tol are no further off than the block
+  // factor's.
+  const double want = sizeof(T) == 4 ? 0.25 * tol : tol;
+  bool near = false;
   int stall_count = 0;
   for (int it = 1; it <= max_iter; ++it) {
     for (int k = 0; k < sweeps; ++k) {
@@ -2297,9 +2303,10 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
       if (rel[q] > tol && rel[q] < 0.7 * prev[q]) contracting = true;
     }
     st.max_rel_residual = worst;
-    if (worst <= tol) { st.converged = 1; break; }
+    if (worst <= want || (worst <= tol && (near || it == max_iter))) { st.converged = 1; break; }
     if (!std::isfinite(worst)) { st.stalled = 1; break; }
-    stall_count = contracting ? 0 : stall_count + 1;
+    near = worst <= tol;
+    stall_count = contracting || near ? 0 : stall_count + 1;
     if (stall_count >= 2) { st.stalled = 1; break; }
     for (int q = 0; q < nrhs; ++q) prev[q] = rel[q];
   }
