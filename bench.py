@@ -13,19 +13,19 @@ each the equivalent of one reference solve_fields call) with p50/p99
 latency, for the complex64-factor + FP64-refinement path (the headline
 value) and for the FP64-factor path on the same trace.
 
-Two loads: the throughput leg offers the stream faster than it is served
-(Poisson arrivals at --rate), so solves/s is the saturated rate and its
-latencies include queueing; the latency leg replays the first
+Three loads: the throughput leg offers the stream at --rate (Poisson
+arrivals) and gives the headline solves/s, which that rate bounds once the
+service is faster; the capacity leg has the whole stream queued at the start
+("saturated": the service's own rate); the latency leg replays the first
 --latency-requests requests at --latency-load (0.25) x the FP64 path's saturated request rate,
 below both paths' capacity at that load (the factorizations batch less when
 fewer requests are in flight, so capacity falls with the load), and its
 p50/p99 are the headline latencies.
 
-Also reported: the roofline of the dominant kernel (the Gauss-Jordan step
-of the complex64 factor, 8 factorizations per launch as in the stream,
-timed with HIP events on its stream; HBM bytes per launch from two
-rocprofv3 --pmc passes over the same launches, scaled by a copy of known
-size) and a CPU baseline: the oracle's SuperLU restatement of the
+Also reported: the roofline of the dominant work (the complex64
+nested-dissection factor, timed with HIP events on its stream; HBM bytes per
+launch of its step kernel from two rocprofv3 --pmc passes, scaled by a copy of
+known size) and a CPU baseline: the oracle's SuperLU restatement of the
 reference's 'scipy' branch in a pool of one worker per host core, replaying
 a bounded prefix of the same stream.
 """
@@ -47,7 +47,6 @@ sys.path.insert(0, ROOT)
 FP32_MFMA_PEAK_TFLOPS = 157.3
 FP64_MFMA_PEAK_TFLOPS = 78.6
 ROOF_N = 512          # grid of the roofline leg's factorizations
-ROOF_JOBS = 10        # factorizations per step launch: 20 chains (the stream's launches carry 18-22)
 COPY_BYTES = 256 << 20
 
 
@@ -104,27 +103,6 @@ def _timed_factor(op, precision, stepwise):
     return e0.elapsed_time(e1)
 
 
-def _timed_wrap(op, precision):
-    """The x-wrap correction step alone (fdfd_factor_wrap) on op's resident
-    factor, timed with HIP events on its stream."""
-    import ctypes
-    import torch
-    from fdfdpy_amd import _lib as L
-    from fdfdpy_amd.device import _stream, _vp
-    lib = L.lib()
-    g = ctypes.byref(op.grid)
-    fac = op.factors[precision][0]
-    work = torch.empty(lib.fdfd_factor_workspace_bytes(g, L.PREC[precision]), dtype=torch.uint8, device="cuda:0")
-    s = torch.cuda.current_stream()
-    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    torch.cuda.synchronize()
-    e0.record(s)
-    L.check(lib.fdfd_factor_wrap(g, _vp(op.op), _vp(fac), L.PREC[precision], _vp(work), _stream("cuda:0")))
-    e1.record(s)
-    torch.cuda.synchronize()
-    return e0.elapsed_time(e1)
-
-
 def _roof_ops(n, njobs):
     """njobs operators of the stream's n x n grid (request seeds 7, 8, ...)."""
     from fdfdpy_amd import configs as C
@@ -138,108 +116,62 @@ def _roof_ops(n, njobs):
     return ops
 
 
-def _batched_factor(ops, precision, stream_timed=True):
-    """fdfd_factor_batch over ops (one grid) on the current stream, twice:
-    warm, then timed with HIP events on that stream. Returns ms."""
-    import ctypes
-    import torch
-    from fdfdpy_amd import _lib as L
-    from fdfdpy_amd.device import _stream
-    lib = L.lib()
-    g = ctypes.byref(ops[0].grid)
-    pr = L.PREC[precision]
-    nj = len(ops)
-    facs = [torch.empty(lib.fdfd_factor_bytes(g, pr), dtype=torch.uint8, device="cuda:0") for _ in ops]
-    works = [torch.empty(lib.fdfd_factor_workspace_bytes(g, pr), dtype=torch.uint8, device="cuda:0") for _ in ops]
-    arr = lambda ts: (ctypes.c_void_p * nj)(*[t.data_ptr() for t in ts])
-    a_ops, a_fac, a_work = arr([o.op for o in ops]), arr(facs), arr(works)
-    ms = None
-    for rep in range(2 if stream_timed else 1):
-        s = torch.cuda.current_stream()
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        torch.cuda.synchronize()
-        e0.record(s)
-        L.check(lib.fdfd_factor_batch(g, a_ops, a_fac, nj, pr, a_work, _stream("cuda:0")))
-        e1.record(s)
-        torch.cuda.synchronize()
-        ms = e0.elapsed_time(e1)
-    for w in works:
-        L.check(lib.fdfd_factor_status(g, pr, ctypes.c_void_p(w.data_ptr()), _stream("cuda:0")))
-    for op, f in zip(ops, facs):
-        op.factors[precision] = (f, op.version, False)
-    return ms
-
-
-def roofline_leg(n=ROOF_N, precision="c64", njobs=ROOF_JOBS, traffic=None):
-    """The dominant kernel of the stream, k_gj_step, at the stream's batching.
-
-    njobs twisted factorizations of n x n operators share each step launch
-    (fdfd_factor_batch: every launch carries a step of each operator's top
-    chain and, until it ends, of its bottom chain; (c + 1) n/32 + 1 launches
-    for twist block c), timed with HIP events on their stream; the x-wrap
-    corrections that follow them are timed alone and taken out. Algorithmic
-    flops: 8 m n^3 per factorization (m = n blocks), spread over the
-    launches. One factorization alone (its two chains per launch) is timed
-    too, and, for comparison, the one-chain factorization (stepwise and the
-    persistent single-launch kernel), both with their wrap corrections.
-    """
+def _nd_counts(op):
+    """Real flops of op's nested-dissection factor (per front of separator s
+    and border b, complex symmetric: 4 s^3 for the inverse, 8 s^2 b for W,
+    4 s b^2 for the update), its pivot-step launches, and the bytes those read
+    and write (the upper tiles of F_ss and the tiles of F_sb, once each way)."""
     import ctypes
     from fdfdpy_amd import _lib as L
-    lib = L.lib()
-    ops = _roof_ops(n, njobs)
-    c = lib.fdfd_twist_block(ctypes.byref(ops[0].grid))
-    ms_all = _batched_factor(ops, precision)
-    ms_wrap = sum(_timed_wrap(op, precision) for op in ops)
-    ms = ms_all - ms_wrap
-    one = ops[0]
-    ms1 = _timed_factor(one, precision, stepwise=True) - ms_wrap / njobs
-    ms_single = _timed_factor(one, precision, stepwise=False)          # with its wrap correction
-    prev = lib.fdfd_set_twist(0)
-    try:
-        ms_chain = _timed_factor(one, precision, stepwise=True)        # one chain, with its wrap correction
-        ms_persist = _timed_factor(one, precision, stepwise=False)
-        one.drop_factor()
-    finally:
-        lib.fdfd_set_twist(prev)
-    nt = (n + 31) // 32
-    launches = (c + 1) * nt + 1
-    flops = 8.0 * n ** 4                       # 8 m n^3 real flops per factorization, m = n blocks
-    avg_us = ms * 1e3 / launches
-    achieved = njobs * flops / (ms * 1e-3) / 1e12
+    lib, g = L.lib(), ctypes.byref(op.grid)
+    info = (ctypes.c_int32 * 8)()
+    flops = steps = nbytes = 0
+    L.check(lib.fdfd_nd_front(g, -1, 0, info, None, None))
+    for level in range(-1, info[0] + 1):
+        L.check(lib.fdfd_nd_front(g, level, 0, info, None, None))
+        boxes, ns, nb = info[1], -(-info[3] // 32), -(-info[4] // 32)
+        for k in range(boxes):
+            L.check(lib.fdfd_nd_front(g, level, k, info, None, None))
+            sep, border = info[3], info[4]
+            flops += 4 * sep ** 3 + 8 * sep ** 2 * border + 4 * sep * border ** 2
+        if level >= 0 and (ns > 1 or nb > 3):     # narrower merges are one launch
+            steps += ns
+            nbytes += boxes * ns * 2 * (ns * (ns + 1) // 2 + ns * nb) * 32 * 32 * 8
+    return flops, steps, nbytes
+
+
+def roofline_leg(n=ROOF_N, precision="c64", traffic=None):
+    """The dominant work of the stream: the nested-dissection factor of an
+    n x n operator, timed with HIP events on its stream; its pivot steps
+    (k_nd_step) are a chain of dependent launches, so the rate of the matrix
+    cores is reported for the whole factor. For comparison, the block
+    factorization of the same operator (stepwise, twisted)."""
+    one = _roof_ops(n, 1)[0]
+    ms = min(_timed_factor(one, precision, stepwise=False) for _ in range(3))
+    flops, steps, nbytes = _nd_counts(one)
+    one.drop_factor()
+    ms_block = _timed_factor(one, precision, stepwise=True)
+    one.drop_factor()
+    achieved = flops / (ms * 1e-3) / 1e12
     peak = FP32_MFMA_PEAK_TFLOPS if precision == "c64" else FP64_MFMA_PEAK_TFLOPS
-    tname = "float" if precision == "c64" else "double"
     out = {
-        "kernel": f"k_gj_step<{tname}, false>",
+        "kernel": f"k_nd_step<{'float' if precision == 'c64' else 'double'}>",
         "bound": "mfma", "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
         "frac": round(achieved / peak, 5), "traffic": None,
-        "workload": f"{njobs} twisted complex factors of {n}x{n} Ez operators (twist block {c}) sharing "
-                    f"{launches} step launches: {njobs * flops:.3e} flops, {njobs * flops / launches:.3e} per launch",
-        "avg_launch_us": round(avg_us, 3), "batched_factor_ms": round(ms, 3), "wrap_ms": round(ms_wrap, 3),
-        "hbm_gbs_algorithmic": None,
-        "one_request": {"avg_launch_us": round(ms1 * 1e3 / launches, 3), "factor_ms": round(ms1, 3),
-                        "achieved_tflops": round(flops / (ms1 * 1e-3) / 1e12, 3),
-                        "factor_with_wrap_ms": round(ms_single, 3)},
-        "one_chain": {"stepwise_with_wrap_ms": round(ms_chain, 3), "persistent_with_wrap_ms": round(ms_persist, 3)},
+        "workload": f"one nested-dissection factor of a {n}x{n} Ez operator: {flops:.3e} flops, "
+                    f"{steps} dependent pivot-step launches among its launches",
+        "factor_ms": round(ms, 3), "block_factor_ms": round(ms_block, 3),
+        "step_algorithmic_bytes_per_launch": round(nbytes / steps),
     }
-    # algorithmic bytes: per block step, the upper tiles of the working matrix
-    # read and written once (symmetric steps), plus the tiles below the
-    # diagonal written at each block's last step; n blocks of nt steps per
-    # factorization, over the launches
-    es = 8 if precision == "c64" else 16
-    upper = nt * (nt + 1) // 2 * 32 * 32 * es * 2
-    lower = nt * (nt - 1) // 2 * 32 * 32 * es / nt
-    alg = njobs * n * nt * (upper + lower) / launches
-    out["algorithmic_bytes_per_launch"] = round(alg)
-    out["hbm_gbs_algorithmic"] = round(alg / (avg_us * 1e-6) / 1e9, 1)
     if traffic:
         out["traffic"] = traffic.get("bytes_per_launch")
         out["traffic_detail"] = traffic
     return out
 
 
-def traffic_child(n=ROOF_N, precision="c64", njobs=ROOF_JOBS):
+def traffic_child(n=ROOF_N, precision="c64"):
     """Run under rocprofv3 --pmc: a plain copy of known size (three times),
-    then the roofline leg's batched factorization once."""
+    then the roofline leg's factor once."""
     import torch
     a = torch.empty(COPY_BYTES // 4, dtype=torch.float32, device="cuda:0").fill_(1.0)
     b = torch.empty_like(a)
@@ -247,27 +179,26 @@ def traffic_child(n=ROOF_N, precision="c64", njobs=ROOF_JOBS):
         b.copy_(a)
     torch.cuda.synchronize()
     del a, b
-    _batched_factor(_roof_ops(n, njobs), precision, stream_timed=False)
+    _roof_ops(n, 1)[0].factor(precision)
+    torch.cuda.synchronize()
     print("traffic child done", flush=True)
 
 
-def kernels_only(n=ROOF_N, njobs=ROOF_JOBS, nrhs=4):
-    """The copy calibration, the roofline leg's batched factorization in both
-    precisions, and one n x n solve with nrhs right-hand sides to 1e-10 in
-    both precisions (persistent sweeps, wrap correction, FP64 stencil
-    residuals): the kernels whose counters the profiles report."""
+def kernels_only(n=ROOF_N, nrhs=4):
+    """The copy calibration, the roofline leg's factor in both precisions, and
+    one n x n solve with nrhs right-hand sides to 1e-10 in both precisions:
+    the kernels whose counters the profiles report."""
     import torch
     copy_calibration()
-    ops = _roof_ops(n, njobs)
+    op = _roof_ops(n, 1)[0]
     rng = torch.Generator(device="cpu").manual_seed(1)
     out = {}
     for prec in ("c64", "fp64"):
-        out[prec + "_batched_factor_ms"] = round(_batched_factor(ops, prec, stream_timed=False), 3)
-        b = torch.randn((nrhs,) + ops[0].shape, dtype=torch.complex128, generator=rng).to("cuda:0")
-        x, rep = ops[0].solve(b, precision=prec, tol=1e-10)
+        out[prec + "_factor_ms"] = round(_timed_factor(op, prec, stepwise=False), 3)
+        b = torch.randn((nrhs,) + op.shape, dtype=torch.complex128, generator=rng).to("cuda:0")
+        x, rep = op.solve(b, precision=prec, tol=1e-10)
         out[prec + "_solve"] = {"steps": rep.iterations, "sweeps": rep.sweeps, "residual": rep.max_rel_residual}
-        for op in ops:
-            op.drop_factor()
+        op.drop_factor()
     torch.cuda.synchronize()
     return out
 
@@ -296,8 +227,8 @@ def _pmc_means(counter, timeout_s=240):
                         continue
                     key = (row["Kernel_Name"], row.get("Dispatch_Id", ""))
                     per[key] = per.get(key, 0.0) + float(row["Counter_Value"])
-        # demangled ("k_gj_step<float, false>") or mangled ("k_gj_stepIfLb0E") names
-        step = [v for (k, _), v in per.items() if "k_gj_step<float, false>" in k or "k_gj_stepIfLb0E" in k]
+        # demangled ("k_nd_step<float>") or mangled ("k_nd_stepIf") names
+        step = [v for (k, _), v in per.items() if "k_nd_step<float>" in k or "k_nd_stepIf" in k]
         copy = [v for (k, _), v in per.items() if "copyBuffer" in k]
         if not step or not copy:
             names = sorted({k for k, _ in per})[:6]
@@ -308,7 +239,7 @@ def _pmc_means(counter, timeout_s=240):
 
 
 def traffic_leg():
-    """HBM bytes per batched step launch: FETCH_SIZE and WRITE_SIZE (KiB per
+    """HBM bytes per step launch: FETCH_SIZE and WRITE_SIZE (KiB per
     dispatch) in two rocprofv3 --pmc passes, each scaled by what the counter
     reads for the 256 MiB copy. Runs before this process touches the GPU
     (the passes are child processes)."""
@@ -548,12 +479,6 @@ def run_stream(reqs, precision, slots, tol, engines=2, keep=False, fresh_cache=F
     errs = sorted({r.error for r in res if r.error})
     if errs:
         log(f"  {precision}: {summ['failed']} failed requests; errors: {errs[:4]}")
-    if eng.factor_engines:
-        # batching of the factorizations: job-steps per shared step launch
-        steps = sum(r.problem.shape[0] * (-(-r.problem.shape[1] // 32)) + 1 for r in reqs)
-        launches = sum(e.launches for e in eng.factor_engines)
-        summ["engine_launches"] = launches
-        summ["jobs_per_launch"] = round(steps / launches, 3) if launches else None
     return summ, res
 
 
@@ -625,8 +550,8 @@ def main():
             s, _ = run_stream(wreqs, prec, args.slots, args.tol, args.engines)
             log(f"warmup {w} {prec}: {s['solves']} solves in {s['wall_s']:.2f}s")
 
-    # throughput leg: the whole stream, offered faster than it is served; the
-    # results are kept (outside the timing) for the per-result errors
+    # throughput leg: the whole stream at its arrivals; the results are kept
+    # (outside the timing) for the per-result errors
     mixed, res_m = run_stream(reqs, "c64", args.slots, args.tol, args.engines, keep=True)
     log(f"mixed: {json.dumps(mixed)}")
     fp64 = None
@@ -645,10 +570,13 @@ def main():
                                                 "the FP64-factor path's result of the same request and RHS")
         del res_f, ref
     del res_m
+    capacity, _ = run_stream([Request(i, p, 0.0) for i, p in enumerate(problems[:n_req])], "c64", args.slots, args.tol,
+                             args.engines)
+    log(f"capacity: {json.dumps(capacity)}")
     if errors:
         log(f"errors: {json.dumps({k_: {a: b for a, b in v.items() if a != 'per_result'} for k_, v in errors.items() if v})}")
     if args.stream_only:
-        print(json.dumps({"stream_c64": mixed, "stream_fp64": fp64}), flush=True)
+        print(json.dumps({"stream_c64": mixed, "stream_fp64": fp64, "capacity_c64": capacity}), flush=True)
         return
     # latency leg: a prefix of the stream at latency_load x the FP64 path's saturated request rate
     cap = (fp64 or mixed)["requests_per_s"]
@@ -692,8 +620,7 @@ def main():
         "fallbacks": mixed["fallbacks"], "failed": mixed["failed"] + lat_m["failed"],
         "mean_steps": mixed["mean_steps"], "mean_sweeps": mixed["mean_sweeps"],
         "error_per_result": errors or None,
-        "saturated": _path_summary(mixed) | {"engine_launches": mixed.get("engine_launches"),
-                                             "jobs_per_launch": mixed.get("jobs_per_launch")},
+        "saturated": _path_summary(capacity),
         "roofline": {k_: roof[k_] for k_ in ("bound", "achieved", "peak", "unit", "frac", "traffic")},
         "roofline_detail": {k_: v for k_, v in roof.items()
                             if k_ not in ("bound", "achieved", "peak", "unit", "frac", "traffic")},

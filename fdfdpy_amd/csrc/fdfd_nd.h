@@ -4,8 +4,12 @@
 // The block sweep of fdfd_hip.hip is serial in the long axis: m n/32 dependent
 // pivot steps to factor, m dependent blocks per sweep, 8 m n^3 flops. Here the
 // cells are ordered by nested dissection on a regular tree: about 5n/32
-// dependent pivot steps on an n x n grid, two launches per tree level per
-// sweep, and O(n^3) flops.
+// dependent pivot steps on an n x n grid, one launch per direction of a sweep
+// for the lower levels and one per level above, and O(n^3) flops. 512^2
+// complex64: factor 65.7 -> 1.87 ms, a sweep 2.1 -> 0.33 ms; 768^2 FP64: 222 ->
+// 6.0 ms. The block path keeps what asks for it by kind (pivoted, stepwise and
+// batched factors) and the grids with a side under ND_MIN_SIDE cells, complex64
+// under ND_MIN_SIDE_C64.
 //
 // Tree. Cell column 0 and cell row 0 (the cross) are the root separator, so
 // what is left, cells 1..nx-1 x 1..ny-1, is not periodic. A box is split by
@@ -22,8 +26,8 @@
 // For a box with front [[F_ss, F_sb], [F_sb^T, F_bb]] summed from its two
 // children's updates and its separator's own entries:
 //   X = F_ss^-1,  W = X F_sb,  C = F_bb - F_sb^T X F_sb  (to the parent).
-// X comes from the tiled Gauss-Jordan steps of the block factorization on
-// the upper tiles of [F_ss | F_sb]; C is one MFMA product per level.
+// X comes from tiled Gauss-Jordan steps on the upper tiles of [F_ss | F_sb]
+// (k_nd_step); C from the panels that these leave, one MFMA product per level.
 //
 // Solve. Upwards f_s = r_s + (children), z = X f_s, u = (children) - W^T f_s;
 // downwards x_s = z - W x_b. Everything is gathered by the reader in a fixed
