@@ -17,9 +17,8 @@ Three loads: the throughput leg offers the stream at --rate (Poisson
 arrivals) and gives the headline solves/s, which that rate bounds once the
 service is faster; the capacity leg has the whole stream queued at the start
 ("saturated": the service's own rate); the latency leg replays the first
---latency-requests requests at --latency-load (0.25) x the FP64 path's saturated request rate,
-below both paths' capacity at that load (the factorizations batch less when
-fewer requests are in flight, so capacity falls with the load), and its
+--latency-requests requests at --latency-load (0.25) x the request rate of the
+FP64 path's throughput leg, below both paths' capacity at that load, and its
 p50/p99 are the headline latencies.
 
 Also reported: the roofline of the dominant work (the complex64
@@ -578,7 +577,7 @@ def main():
     if args.stream_only:
         print(json.dumps({"stream_c64": mixed, "stream_fp64": fp64, "capacity_c64": capacity}), flush=True)
         return
-    # latency leg: a prefix of the stream at latency_load x the FP64 path's saturated request rate
+    # latency leg: a prefix of the stream at latency_load x the FP64 path's request rate
     cap = (fp64 or mixed)["requests_per_s"]
     lat_rate = args.latency_load * cap
     k = min(args.latency_requests, n_req)

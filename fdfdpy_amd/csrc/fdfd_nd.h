@@ -384,9 +384,9 @@ template <typename T> __device__ inline void wave_sub(T &pr, T &pi, T ar, T ai, 
 }
 __device__ inline int frexp_of(float x) { return __builtin_amdgcn_frexp_expf(x); }
 __device__ inline int frexp_of(double x) { return __builtin_amdgcn_frexp_exp(x); }
-// LDS of an inverse: the pivot rows by column
+// LDS of an inverse: the pivot rows by column, real and imaginary parts
 template <typename T> struct alignas(16) PivotRows {
-  T r[TB][2], i[TB][2];
+  T v[2][TB][2];
 };
 // The diagonal blocks: lane 4 m + e of every wave keeps P00, P01, P11, P01 of
 // pair m (e = 0 .. 3); quads exchange them by DPP
@@ -453,10 +453,10 @@ template <typename T> struct PivotBlocks {
   T xr[2], xi[2], yr[2], yi[2];
   __device__ inline void read(const PivotRows<T> &f) {
     const int m = (threadIdx.x & 63) >> 2, q = threadIdx.x & 3, x = 2 * m + (q == 2), y = 2 * m + (q != 0);
-    lds_ld2(f.r[x], xr[0], xr[1]);
-    lds_ld2(f.i[x], xi[0], xi[1]);
-    lds_ld2(f.r[y], yr[0], yr[1]);
-    lds_ld2(f.i[y], yi[0], yi[1]);
+    lds_ld2(f.v[0][x], xr[0], xr[1]);
+    lds_ld2(f.v[1][x], xi[0], xi[1]);
+    lds_ld2(f.v[0][y], yr[0], yr[1]);
+    lds_ld2(f.v[1][y], yi[0], yi[1]);
   }
   __device__ inline void update(const WaveQ<T> &Q) {
     T v0r = 0, v0i = 0, v1r = 0, v1i = 0;   // -Q f
@@ -503,8 +503,8 @@ __device__ inline bool pivot_rows(PivotRows<float> &f, const Mfma<float>::v4 &mr
     f2 r = f2{mr[0], mr[1]}, i = f2{mi[0], mi[1]};
     if (jr & 2) { r = f2{mr[2], mr[3]}; i = f2{mi[2], mi[3]}; }
     if (diagonal && (c & ~1) == jr) { r = f2{c == jr ? -1.0f : 0.0f, c == jr ? 0.0f : -1.0f}; i = f2{0, 0}; }
-    *reinterpret_cast<f2 *>(f.r[col]) = r;
-    *reinterpret_cast<f2 *>(f.i[col]) = i;
+    *reinterpret_cast<f2 *>(f.v[0][col]) = r;
+    *reinterpret_cast<f2 *>(f.v[1][col]) = i;
   }
   return own;
 }
@@ -521,8 +521,8 @@ __device__ inline bool pivot_rows(PivotRows<double> &f, const Mfma<double>::v4 &
       if (jr < 12) { r = mr[2]; i = mi[2]; } else { r = mr[3]; i = mi[3]; }
     }
     if (diagonal && (c & ~1) == jr) { r = c == jr + k ? -1.0 : 0.0; i = 0; }
-    f.r[col][k] = r;
-    f.i[col][k] = i;
+    f.v[0][col][k] = r;
+    f.v[1][col][k] = i;
   }
   return own;
 }
@@ -569,9 +569,9 @@ __device__ void tile_inverse_pairs(LT &L, int rows, int *status) {
     const SweepCoef<T> W(Q);
     __syncthreads();
     T v0, v1, v2, v3, are, aim;
-    lds_ld2(f.r[16 * qi + c], v0, v2);
-    lds_ld2(f.i[16 * qi + c], v1, v3);
-    const T bre = (&f.r[16 * qj + c][k])[part * 2 * TB], bim = (&f.i[16 * qj + c][k])[-part * 2 * TB];
+    lds_ld2(f.v[0][16 * qi + c], v0, v2);
+    lds_ld2(f.v[1][16 * qi + c], v1, v3);
+    const T bre = f.v[part][16 * qj + c][k], bim = f.v[1 - part][16 * qj + c][k];
     B.read(f);
     __builtin_amdgcn_sched_barrier(0);   // all reads first: they wait for LDS once
     W.left(v0, v1, v2, v3, are, aim);
@@ -594,15 +594,17 @@ __device__ void tile_inverse_pairs(LT &L, int rows, int *status) {
 // the choice's instructions are issued once a leaf and not by four waves. Bound
 // by them: the 8192 leaves of 512^2 complex64 110 -> 51 us, the 16384 of 768^2
 // FP64 469 -> 200 us. As the chain of one tile it is slower than four waves
-// and takes 180 registers in FP64.
+// and takes over 200 registers in FP64.
+// within a wave: LDS stores before this are seen by loads after it
+__device__ inline void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 template <typename T> struct WaveTile {
   typename Mfma<T>::v4 r[2][2], i[2][2];
 };
 // LDS of one wave's inverse: the pivot rows by column, and a second set for
 // the lanes that have none to write (a branch on lanes inside the choice of
 // the accumulators makes the compiler copy the tile at every join)
-template <typename T> struct WaveRows : PivotRows<T> {
-  T none[2][TB][2];
+template <typename T> struct WaveRows {
+  PivotRows<T> rows, none;
 };
 // The pivot rows j, j + 1 (j = 16 QR + jr, in accumulator TT: of one lane
 // group for f32, one each of two for f64) go to f; the pivot rows and columns
@@ -612,11 +614,11 @@ __device__ inline void wave_rows(WaveTile<float> &M, WaveRows<float> &f, int lan
   typedef float f2 __attribute__((ext_vector_type(2)));
   const int c = lane & 15;
   const bool own = (lane >> 4) == (jr >> 2), pc = (c & ~1) == jr;
-  f2 *to = reinterpret_cast<f2 *>(own ? f.r[c] : f.none[0][c]);
+  PivotRows<float> &to = own ? f.rows : f.none;
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-    to[16 * q] = f2{M.r[QR][q][TT], M.r[QR][q][TT + 1]};
-    to[16 * q + TB] = f2{M.i[QR][q][TT], M.i[QR][q][TT + 1]};
+    *reinterpret_cast<f2 *>(to.v[0][16 * q + c]) = f2{M.r[QR][q][TT], M.r[QR][q][TT + 1]};
+    *reinterpret_cast<f2 *>(to.v[1][16 * q + c]) = f2{M.i[QR][q][TT], M.i[QR][q][TT + 1]};
   }
 #pragma unroll
   for (int q = 0; q < 2; ++q)
@@ -637,11 +639,11 @@ template <int QR, int TT>
 __device__ inline void wave_rows(WaveTile<double> &M, WaveRows<double> &f, int lane, int jr) {
   const int c = lane & 15, k = (lane >> 4) - (jr & 3);
   const bool own = k == 0 || k == 1, pc = (c & ~1) == jr;
-  double *to = own ? &f.r[c][k] : f.none[0][c];
+  PivotRows<double> &to = own ? f.rows : f.none;
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-    to[32 * q] = M.r[QR][q][TT];
-    to[32 * q + 2 * TB] = M.i[QR][q][TT];
+    to.v[0][16 * q + c][k & 1] = M.r[QR][q][TT];
+    to.v[1][16 * q + c][k & 1] = M.i[QR][q][TT];
   }
 #pragma unroll
   for (int q = 0; q < 2; ++q)
@@ -658,33 +660,27 @@ __device__ inline void wave_rows(WaveTile<double> &M, WaveRows<double> &f, int l
       }
     }
 }
-// What one lane writes to LDS the others of its wave read next
-__device__ inline void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 // One sweep's products on the rows in accumulator TT of quadrant row QR
 template <int QR, int TT, typename T>
 __device__ inline void wave_sweep(WaveTile<T> &M, WaveRows<T> &f, int lane, int j, const WaveQ<T> &Q) {
   const int c = lane & 15, kk = lane >> 4, k = kk & 1, part = kk >> 1;
   wave_rows<QR, TT>(M, f, lane, j & 15);
-  wave_lds_order();
-  T *unit = lane < 2 ? f.r[j + lane] : f.none[0][0];   // minus a unit vector at the pivots
-  unit[0] = lane ? T(0) : T(-1);
-  unit[1] = lane ? T(-1) : T(0);
-  unit[2 * TB] = unit[2 * TB + 1] = 0;
-  wave_lds_order();
+  wave_lds_fence();
+  PivotRows<T> &unit = lane < 2 ? f.rows : f.none;   // minus a unit vector at the pivots
+  const int l = lane & 1;
+  unit.v[0][j + l][0] = l ? T(0) : T(-1);
+  unit.v[0][j + l][1] = l ? T(-1) : T(0);
+  unit.v[1][j + l][0] = unit.v[1][j + l][1] = 0;
+  wave_lds_fence();
   const SweepCoef<T> W(Q);
-  const T *fre = part ? &f.i[c][k] : &f.r[c][k], *fim = part ? &f.r[c][k] : &f.i[c][k];
   T are[2], aim[2], bre[2], bim[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-    bre[q] = fre[32 * q];
-    bim[q] = fim[32 * q];
+    bre[q] = f.rows.v[part][16 * q + c][k];
+    bim[q] = f.rows.v[1 - part][16 * q + c][k];
     T v0, v1, v2, v3;
-    lds_ld2(f.r[16 * q + c], v0, v2);
-    lds_ld2(f.i[16 * q + c], v1, v3);
+    lds_ld2(f.rows.v[0][16 * q + c], v0, v2);
+    lds_ld2(f.rows.v[1][16 * q + c], v1, v3);
     W.left(v0, v1, v2, v3, are[q], aim[q]);
   }
 #pragma unroll
@@ -737,9 +733,9 @@ __device__ inline bool wave_inverse(WaveTile<T> &M, const T (*Ar)[TBP], const T 
     const int pick = B.pick();
     WaveQ<T> Q;
     B.inverse(pick, Q);
-    wave_lds_order();
+    wave_lds_fence();
     wave_sweep_at(M, f, lane, 2 * pick, Q);
-    B.read(f);
+    B.read(f.rows);
     B.update(Q);
   }
 #pragma unroll
@@ -810,7 +806,7 @@ __global__ void __launch_bounds__(64, 2) k_nd_leaf(int nx, int ny, int Dx, int D
     (&Ar[0][0])[e] = 0;
     (&Ai[0][0])[e] = 0;
   }
-  wave_lds_order();
+  wave_lds_fence();
   if (lane < TB) {   // the upper triangle: itself, the next cell in y and in x
     T re = 1, im = 0;
     if (lane < s) {
@@ -845,12 +841,12 @@ __global__ void __launch_bounds__(64, 2) k_nd_leaf(int nx, int ny, int Dx, int D
     cp[lane] = p;
     nd_st<T>(cpl, (size_t)k * TB + lane, re, im);
   }
-  wave_lds_order();
+  wave_lds_fence();
   WaveTile<T> M;
   if (!wave_inverse<T>(M, Ar, Ai, f, s)) *status = 1;
-  wave_lds_order();
+  wave_lds_fence();
   wave_store<T>(M, &Ar[0][0], &Ai[0][0], TBP);
-  wave_lds_order();
+  wave_lds_fence();
   T *Xk = X + (size_t)k * 2 * TB * TB, *Ck = C + (size_t)k * 2 * TB * TB;
   for (int a = a0; a < s; a += 8) {
     store4(Xk + a * TB + b0, &Ar[a][b0]);
@@ -1558,8 +1554,6 @@ __device__ inline void nd_sep_ij(const NdLevel &L, const NdBox &B, int j, int &c
     cj = B.y0 + B.c0;
   }
 }
-// within a wave: LDS stores before this are seen by loads after it
-__device__ inline void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 // f_s of separator entry j, right-hand side q: f plus the children's updates
 // (uin with the children's numbers n0, n1 in it)
