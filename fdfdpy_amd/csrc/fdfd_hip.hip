@@ -3654,7 +3654,10 @@ size_t fdfd_factor_workspace_bytes(const fdfd_grid *g, int precision) {
 }
 size_t fdfd_solve_workspace_bytes(const fdfd_grid *g, int precision, int nrhs) {
   if (check_grid(g) || check_prec(precision) || nrhs < 1) return 0;
-  return solve_work_bytes(g, precision, nrhs);
+  const size_t n = solve_work_bytes(g, precision, nrhs);
+  NdPlan P;
+  if ((precision & (FDFD_FACTOR_STEPWISE | FDFD_FACTOR_PIVOT)) || !nd_fits(g, precision, &P)) return n;
+  return std::max(n, nd_solve_layout(P, precision, nrhs).total);   // either kind of factor
 }
 
 int fdfd_sfactors(const fdfd_grid *g, double *isxf, double *isxb, double *isyf, double *isyb) {
@@ -3854,19 +3857,21 @@ int fdfd_stretch_scale(const fdfd_grid *g, double *v, int nrhs, int inverse, hip
 }  // extern "C"
 
 namespace {
-// The refinement of fdfd_solve. work: the solve workspace (device); host:
-// 4 * nrhs doubles of host scratch (norms of b, of the residual, the relative
-// residuals and the previous step's).
+// The refinement of fdfd_solve. work: the solve workspace (device) of room
+// bytes; host: 4 * nrhs doubles of host scratch (norms of b, of the residual,
+// the relative residuals and the previous step's).
 int solve_impl(const fdfd_grid *g, const double *op, const void *factor, int precision, const double *b,
                double *x, int nrhs, int transpose, double tol, int max_iter, void *work,
-               fdfd_solve_stats *stats, double *rel_res, hipStream_t stream, double *host) {
+               fdfd_solve_stats *stats, double *rel_res, hipStream_t stream, double *host, size_t room) {
   bool nd = false;
   NdPlan P;
   if (int rc = factor_is_nd(g, factor, precision, stream, &nd, &P)) return rc;
   if (nd)
     return base_prec(precision) == FDFD_PREC_FP64
-               ? nd_solve<double>(g, op, factor, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res, stream, host)
-               : nd_solve<float>(g, op, factor, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res, stream, host);
+               ? nd_solve<double>(g, op, factor, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res, stream, host,
+                                  room)
+               : nd_solve<float>(g, op, factor, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res, stream, host,
+                                 room);
   SolveWork sw = solve_work_layout(g, precision, nrhs, work);
   const size_t M = (size_t)g->nx * g->ny;
   const dim3 sgrid((g->ny + NT - 1) / NT, g->nx);
@@ -4024,7 +4029,7 @@ int fdfd_solve(const fdfd_grid *g, const double *op, const void *factor, int pre
     return fail(FDFD_ERR_ARG, "bad arguments to fdfd_solve");
   std::vector<double> host(4 * (size_t)nrhs);
   return solve_impl(g, op, factor, precision, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res,
-                    stream, host.data());
+                    stream, host.data(), SIZE_MAX);
 }
 
 int fdfd_solve_static(const fdfd_grid *g, const double *op, const void *factor, int precision,
@@ -4045,7 +4050,7 @@ int fdfd_solve_static(const fdfd_grid *g, const double *op, const void *factor, 
   if (int rc = static_scratch(&work)) return rc;
   double host[4 * STATIC_MAX_RHS];
   return solve_impl(g, op, factor, precision, b, x, nrhs, transpose, tol, max_iter, work, stats, rel_res,
-                    stream, host);
+                    stream, host, STATIC_SCRATCH_BYTES);
 }
 
 int fdfd_grad_eps(const fdfd_grid *g, const double *lam, const double *e, double *grad,

@@ -2132,9 +2132,10 @@ inline NdTree nd_tree(const NdPlan &P) {
   return t;
 }
 // Solve workspace: f of every right-hand side, v and the u buffers of one
-// pass, norm partials, norms.
+// pass, norm partials, norms (`base` bytes), and an iterate within the
+// tolerance (nd_solve).
 struct NdSolveWork {
-  size_t f, v, u[3], part, norms, total;
+  size_t f, v, u[3], part, norms, base, kept, total;
 };
 inline NdSolveWork nd_solve_layout(const NdPlan &P, int precision, int nrhs) {
   const size_t M = (size_t)P.nx * P.ny, es = elem_size(precision);
@@ -2151,6 +2152,8 @@ inline NdSolveWork nd_solve_layout(const NdPlan &P, int precision, int nrhs) {
   w.u[2] = take(2 * es * R * Lt.b * Lt.nbox);
   w.part = take(8 * (size_t)2 * NORM_PARTS * nrhs);
   w.norms = take(8 * 2 * (size_t)nrhs);
+  w.base = off;
+  w.kept = take(16 * M * nrhs);
   w.total = off;
   return w;
 }
@@ -2206,8 +2209,9 @@ int nd_sweep(const NdPlan &P, const void *factor, double *x, int nrhs, int add, 
   return FDFD_OK;
 }
 
-// The path's range: a plan exists and its solve fits the workspace that
-// fdfd_solve_workspace_bytes reports without knowing the factor's kind. FP64,
+// The path's range: a plan exists and its solve fits the block path's
+// workspace, which fdfd_solve_static is limited by (except the kept iterate,
+// which that call does without where it has no room). FP64,
 // new permittivity and solve / resident solve through Simulation, block path
 // against tree: 16 x 16 1.16 / 0.63 against 0.56 / 0.26 ms, 32 x 32 1.46 /
 // 0.85 against 0.61 / 0.26, 48 x 40 2.52 / 0.98 against 0.65 / 0.23, 63 x 63
@@ -2223,7 +2227,7 @@ inline bool nd_fits(const fdfd_grid *g, int precision, NdPlan *P) {
   if (prec == FDFD_PREC_C64 && std::min(g->nx, g->ny) < ND_MIN_SIDE_C64) return false;
   if (!nd_plan(g, P)) return false;
   for (int k = 1; k <= 8; ++k)
-    if (nd_solve_layout(*P, prec, k).total > solve_work_bytes(g, prec, k)) return false;
+    if (nd_solve_layout(*P, prec, k).base > solve_work_bytes(g, prec, k)) return false;
   return true;
 }
 
@@ -2240,11 +2244,12 @@ inline int nd_parts(const NdPlan &P) { return std::min(2 * NORM_PARTS, P.nx * ((
 // The refinement of fdfd_solve with a nested-dissection factor: x = A^-1 b,
 // then x += A^-1 (b - A x) until every right-hand side meets the tolerance.
 // With a periodic axis a step is two sweeps, as on the block path. The first
-// sweep starts before ||b|| is known on the host; a zero b gives x = 0.
+// sweep starts before ||b|| is known on the host; a zero b gives x = 0. room:
+// the workspace's bytes.
 template <typename T>
 int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const double *b, double *x, int nrhs,
              int transpose, double tol, int max_iter, void *work, fdfd_solve_stats *stats, double *rel_res,
-             hipStream_t s, double *host) {
+             hipStream_t s, double *host, size_t room) {
   const int prec = sizeof(T) == 8 ? FDFD_PREC_FP64 : FDFD_PREC_C64;
   NdPlan P;
   if (!nd_fits(g, prec, &P)) return fail(FDFD_ERR_ARG, "the grid is outside the nested-dissection factor's range");
@@ -2263,9 +2268,11 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
   // A complex64 sweep leaves 1e-5 .. 1e-2 of the residual; one that ends within
   // tol but above a quarter of it is followed by one more (a solve in six), so
   // that fields that stop just below tol are no further off than the block
-  // factor's.
+  // factor's. The iterate within tol is kept meanwhile: near the floor of the
+  // FP64 residual the next one may lie above tol, and is then taken back.
   const double want = sizeof(T) == 4 ? 0.25 * tol : tol;
-  bool near = false;
+  const size_t xbytes = 16 * (size_t)P.nx * P.ny * nrhs;
+  bool held = false;
   int stall_count = 0;
   for (int it = 1; it <= max_iter; ++it) {
     for (int k = 0; k < sweeps; ++k) {
@@ -2281,7 +2288,7 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
       bool all_zero = true;
       for (int q = 0; q < nrhs; ++q) all_zero = all_zero && nb[q] == 0.0;
       if (all_zero) {   // linalg.py:128-129
-        HIP_TRY(hipMemsetAsync(x, 0, 16 * (size_t)P.nx * P.ny * nrhs, s));
+        HIP_TRY(hipMemsetAsync(x, 0, xbytes, s));
         HIP_TRY(hipStreamSynchronize(s));
         st.zero_rhs = 1;
         st.converged = 1;
@@ -2301,11 +2308,22 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
       if (rel[q] > tol && rel[q] < 0.7 * prev[q]) contracting = true;
     }
     st.max_rel_residual = worst;
-    if (worst <= want || (worst <= tol && (near || it == max_iter))) { st.converged = 1; break; }
-    if (!std::isfinite(worst)) { st.stalled = 1; break; }
-    near = worst <= tol;
-    stall_count = contracting || near ? 0 : stall_count + 1;
-    if (stall_count >= 2) { st.stalled = 1; break; }
+    if (worst <= tol) {
+      st.converged = 1;
+      if (worst <= want || held || it == max_iter || w.total > room) break;
+      HIP_TRY(hipMemcpyAsync(base + w.kept, x, xbytes, hipMemcpyDeviceToDevice, s));
+      held = true;
+    } else if (held) {   // back to the iterate before
+      HIP_TRY(hipMemcpyAsync(x, base + w.kept, xbytes, hipMemcpyDeviceToDevice, s));
+      HIP_TRY(hipStreamSynchronize(s));
+      st.max_rel_residual = 0;
+      for (int q = 0; q < nrhs; ++q) st.max_rel_residual = std::max(st.max_rel_residual, rel[q] = prev[q]);
+      break;
+    } else {
+      if (!std::isfinite(worst)) { st.stalled = 1; break; }
+      stall_count = contracting ? 0 : stall_count + 1;
+      if (stall_count >= 2) { st.stalled = 1; break; }
+    }
     for (int q = 0; q < nrhs; ++q) prev[q] = rel[q];
   }
   if (transpose) {   // x = D x'

@@ -99,6 +99,8 @@ const char *fdfd_last_error(void);
 size_t fdfd_op_bytes(const fdfd_grid *g);
 size_t fdfd_factor_bytes(const fdfd_grid *g, int precision);
 size_t fdfd_factor_workspace_bytes(const fdfd_grid *g, int precision);
+/* enough for either kind of factor, or, with FDFD_FACTOR_STEPWISE or
+ * FDFD_FACTOR_PIVOT in precision, for a block factor */
 size_t fdfd_solve_workspace_bytes(const fdfd_grid *g, int precision, int nrhs);
 int fdfd_block_padding(void);   /* block size is padded to this multiple */
 
@@ -199,8 +201,8 @@ int fdfd_solve(const fdfd_grid *g, const double *op, const void *factor, int pre
  * loops, harnesses that forbid hipMalloc). No counterpart in the reference.
  * The workspace is a static 64 MiB array of the library on each device
  * (held until the process ends); a solve whose fdfd_solve_workspace_bytes
- * exceeds it, or with more than 16 right-hand sides, fails with FDFD_ERR_ARG
- * (use fdfd_solve). Every call on one device shares that array: calls that
+ * with FDFD_FACTOR_STEPWISE (the block factor's) exceeds it, or with more
+ * than 16 right-hand sides, fails with FDFD_ERR_ARG (use fdfd_solve). Every call on one device shares that array: calls that
  * overlap on one GPU (other streams, other host threads) race and must be
  * serialized by the caller. Nothing in the array needs to start at zero; the
  * solve clears what it reads before reading it. Other arguments, results

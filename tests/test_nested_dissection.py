@@ -218,6 +218,38 @@ def test_kinds_are_told_apart_and_repeat_to_the_bit(precision):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,npml", [((64, 80), [8, 8]), ((129, 96), [10, 10])])
+def test_a_solve_that_met_its_tolerance_stays_converged(N, npml):
+    """The tolerance is the smallest residual that the complex64 refinement
+    passes through, at its floor: the sweep that follows such an iterate lies
+    above it, and the solve ends with the iterate that met it."""
+    lib, found = L.lib(), 0
+    for seed in range(8):
+        rng = np.random.default_rng(seed)
+        op = _device(N, npml, "Ez", _eps(rng, N), "c64")
+        g, fac = ctypes.byref(op.grid), op.factor("c64")
+        b = op.to_solver(torch.tensor(rng.standard_normal(N) + 1j * rng.standard_normal(N), device=DEV))
+        work = torch.empty(lib.fdfd_solve_workspace_bytes(g, 1, 1), dtype=torch.uint8, device=DEV)
+
+        def solve(tol, steps):
+            x, st, ptr = torch.empty_like(b), L.FdfdSolveStats(), lambda t: ctypes.c_void_p(t.data_ptr())
+            torch.cuda.synchronize()
+            rc = lib.fdfd_solve(g, ptr(op.op), ptr(fac), 1 | L.FACTOR_ND, ptr(b), ptr(x), 1, 0, tol, steps, ptr(work),
+                                ctypes.byref(st), None, None)
+            return rc, x, st
+        seq = [solve(1e-30, k) for k in range(1, 13)]
+        res = [st.max_rel_residual for _, _, st in seq]
+        k = int(np.argmin(res))
+        if seq[k][2].iterations != k + 1 or k + 1 >= seq[-1][2].iterations:
+            continue                   # the smallest one is the last before the stall
+        found += 1
+        rc, x, st = solve(res[k], 20)
+        assert rc == L.FDFD_OK and st.converged and st.max_rel_residual <= res[k]
+        assert torch.equal(x, seq[k][1])
+    assert found
+
+
+@pytest.mark.gpu
 def test_stall_without_fallback_takes_the_block_factor(monkeypatch):
     """fallback=False keeps the precision: when the nested-dissection factor
     does not refine (its report forced here), the block factor does."""
