@@ -2151,7 +2151,7 @@ inline NdSolveWork nd_solve_layout(const NdPlan &P, int precision, int nrhs) {
   w.u[1] = take(2 * es * R * t.reg1 * Lt.nbox);
   w.u[2] = take(2 * es * R * Lt.b * Lt.nbox);
   w.part = take(8 * (size_t)2 * NORM_PARTS * nrhs);
-  w.norms = take(8 * 2 * (size_t)nrhs);
+  w.norms = take(8 * 3 * (size_t)nrhs);
   w.base = off;
   w.kept = take(16 * M * nrhs);
   w.total = off;
@@ -2265,14 +2265,29 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
   residual(nullptr);
   hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts, norms + nrhs);
   const int sweeps = wrap_exact(g) ? 2 : 1;
-  // A complex64 sweep leaves 1e-5 .. 1e-2 of the residual; one that ends within
-  // tol but above a quarter of it is followed by one more (a solve in six), so
-  // that fields that stop just below tol are no further off than the block
-  // factor's. The iterate within tol is kept meanwhile: near the floor of the
-  // FP64 residual the next one may lie above tol, and is then taken back.
-  const double want = sizeof(T) == 4 ? 0.25 * tol : tol;
+  // Which iterate within tol is the last. The first one can be a hundred times
+  // as far from the solution as the block factor's, whose steps leave the wrap
+  // coupling to a second one: what a sweep leaves lies in the directions that
+  // A^-1 amplifies most. Errors of 246 drawn operators (40 to 640 cells a side)
+  // against the block factor's at the same tol, as the mean of the ratio, its
+  // maximum and how many are larger:
+  //   FP64, tol 1e-12: one sweep 0.47, 184, 65; two 0.09, 1.4 (rounding), 9.
+  //   complex64, tol 1e-12: first iterate below tol 0.19, 311, 57 of 205; one
+  //   more from above tol/4 0.10, 46, 38; from above tol/100 0.02, 1.9, 4.
+  //   complex64, tol 1e-10: 0.03, 1363, 43; 0.01, 85, 26; 0.004, 85, 12 (the
+  //   85: a residual of tol/2 after eight sweeps).
+  // So FP64 takes two sweeps at least, the first two without a look between
+  // them, and complex64 one more from above tol/100 (0.1 to 0.6 sweeps a solve).
+  // The iterate within tol is kept meanwhile: near the floor of the FP64
+  // residual the next one may lie above tol, and is then taken back.
+  const bool keeps = w.total <= room, pair = sizeof(T) == 8 && sweeps == 1 && max_iter > 1 && keeps;
+  const auto enough = [&](double worst) { return sizeof(T) == 8 ? st.sweeps >= 2 : worst <= 0.01 * tol; };
+  const auto relative = [](double r2, double b2) {
+    const double v = b2 > 0 ? sqrt(r2 / b2) : 0.0;
+    return std::isfinite(v) ? v : INFINITY;
+  };
   const size_t xbytes = 16 * (size_t)P.nx * P.ny * nrhs;
-  bool held = false;
+  bool held = false, looked = false;
   int stall_count = 0;
   for (int it = 1; it <= max_iter; ++it) {
     for (int k = 0; k < sweeps; ++k) {
@@ -2280,40 +2295,56 @@ int nd_solve(const fdfd_grid *g, const double *op, const void *factor, const dou
       if (int rc = nd_sweep<T>(P, factor, x, nrhs, first ? 0 : 1, base, w, s)) return rc;
       residual(x);
     }
-    hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts, norms);
+    const bool unseen = pair && it == 1;   // its norms are read with the next ones
+    hipLaunchKernelGGL(k_norm_final, dim3(nrhs), dim3(NT), 0, s, (const double *)part, parts,
+                       norms + (unseen ? 2 * nrhs : 0));
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(nr, norms, sizeof(double) * (it == 1 ? 2 : 1) * nrhs, hipMemcpyDeviceToHost, s));
+    st.iterations = it;
+    st.sweeps += sweeps;
+    if (unseen) {
+      HIP_TRY(hipMemcpyAsync(base + w.kept, x, xbytes, hipMemcpyDeviceToDevice, s));
+      continue;
+    }
+    // nr, and at the first look nb and (in rel's place) the unseen iterate's
+    HIP_TRY(hipMemcpyAsync(nr, norms, sizeof(double) * (looked ? 1 : pair ? 3 : 2) * nrhs, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (it == 1) {
+    if (!looked) {
+      looked = true;
       bool all_zero = true;
       for (int q = 0; q < nrhs; ++q) all_zero = all_zero && nb[q] == 0.0;
       if (all_zero) {   // linalg.py:128-129
         HIP_TRY(hipMemsetAsync(x, 0, xbytes, s));
         HIP_TRY(hipStreamSynchronize(s));
+        memset(&st, 0, sizeof st);
         st.zero_rhs = 1;
         st.converged = 1;
         if (stats) *stats = st;
         if (rel_res) for (int q = 0; q < nrhs; ++q) rel_res[q] = 0;
         return FDFD_OK;
       }
+      if (pair) {
+        held = true;
+        for (int q = 0; q < nrhs; ++q) {
+          prev[q] = relative(rel[q], nb[q]);
+          held = held && prev[q] <= tol;
+        }
+      }
     }
-    st.iterations = it;
-    st.sweeps += sweeps;
     double worst = 0;
     bool contracting = false;
     for (int q = 0; q < nrhs; ++q) {
-      rel[q] = nb[q] > 0 ? sqrt(nr[q] / nb[q]) : 0.0;
-      if (!std::isfinite(rel[q])) rel[q] = INFINITY;
+      rel[q] = relative(nr[q], nb[q]);
       worst = std::max(worst, rel[q]);
       if (rel[q] > tol && rel[q] < 0.7 * prev[q]) contracting = true;
     }
     st.max_rel_residual = worst;
     if (worst <= tol) {
       st.converged = 1;
-      if (worst <= want || held || it == max_iter || w.total > room) break;
+      if (enough(worst) || held || it == max_iter || !keeps) break;
       HIP_TRY(hipMemcpyAsync(base + w.kept, x, xbytes, hipMemcpyDeviceToDevice, s));
       held = true;
     } else if (held) {   // back to the iterate before
+      st.converged = 1;
       HIP_TRY(hipMemcpyAsync(x, base + w.kept, xbytes, hipMemcpyDeviceToDevice, s));
       HIP_TRY(hipStreamSynchronize(s));
       st.max_rel_residual = 0;

@@ -188,8 +188,11 @@ int fdfd_sweep(const fdfd_grid *g, const double *op, const void *factor, int pre
  * block sweep: the correction of the coupling the previous iteration left
  * on the boundary blocks is added to its right-hand side. With the exact
  * correction an iteration is two sweeps (T^-1 r, then T^-1 of the
- * capacitance product's forcing). An all-zero b gives x = 0 without a sweep
- * (linalg.py:128-129). rel_res (optional, device-independent host array of
+ * capacitance product's forcing). With a nested-dissection factor FP64 takes
+ * two sweeps at least and complex64 one more from a residual above tol / 100
+ * (max_iter allowing), so that the field is as exact as with a block factor;
+ * of the iterates that met tol the last one is returned. An all-zero b gives
+ * x = 0 (linalg.py:128-129). rel_res (optional, device-independent host array of
  * nrhs doubles) receives the final relative residuals. */
 int fdfd_solve(const fdfd_grid *g, const double *op, const void *factor, int precision,
                const double *b, double *x, int nrhs, int transpose, double tol,

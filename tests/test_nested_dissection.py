@@ -172,7 +172,7 @@ def test_leaves_of_every_size(N, cells):
     eps = _eps(rng, N)
     op = _device(N, [4, 4], "Ez", eps, "fp64")
     b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
-    x, rep = op.solve(torch.tensor(b, device=DEV), precision="fp64", tol=1e-12)
+    x, rep = op.solve(torch.tensor(b, device=DEV), precision="fp64", tol=1e-12, max_iter=1)
     assert rep.converged and rep.sweeps == 1
     A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], eps, [4, 4], "Ez", 1e-6)
     assert relerr(x.cpu().numpy(), solver_direct(A, b.reshape(-1)).reshape(N)) < 1e-10
@@ -247,6 +247,43 @@ def test_a_solve_that_met_its_tolerance_stays_converged(N, npml):
         assert rc == L.FDFD_OK and st.converged and st.max_rel_residual <= res[k]
         assert torch.equal(x, seq[k][1])
     assert found
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,seed,precision,tol", [(128, 24, "fp64", 1e-12), (96, 10, "c64", 1e-12),
+                                                  (192, 38, "c64", 1e-12), (128, 15, "c64", 1e-10)])
+def test_solves_are_as_exact_as_the_block_factors(n, seed, precision, tol):
+    """Operators whose first iterate within the tolerance is 9 to 28 times
+    as far from the solution as the block factor's result at that tolerance.
+    The solution is FP64 refinement run to its floor, good to the rounding of
+    the residual, 1e-16 ||A|| ||x|| / ||b|| ~ 1e-14, times the amplification
+    seen above (10): the block factor's error is above 1e-13 in every case."""
+    lib = L.lib()
+    p = C.c3_request(seed, n=n)
+    op = _device(p.shape, p.npml, p.pol, p.eps, "fp64")
+    assert (p.dl, p.L0) == (0.02, 1e-6)
+    op.grid.omega = op.grid_user.omega = p.omega
+    op.set_eps(p.eps)
+    b = torch.tensor(p.rhs(), device=DEV)
+
+    def error(x):
+        return max(relerr(x[q].cpu().numpy(), ref[q].cpu().numpy()) for q in range(b.shape[0]))
+    bs, fac, g = op.to_solver(b), op.factor("fp64"), ctypes.byref(op.grid)
+    work = torch.empty(lib.fdfd_solve_workspace_bytes(g, L.FACTOR_ND, b.shape[0]), dtype=torch.uint8, device=DEV)
+    ref, ptr = torch.empty_like(bs), lambda t: ctypes.c_void_p(t.data_ptr())
+    torch.cuda.synchronize()
+    lib.fdfd_solve(g, ptr(op.op), ptr(fac), L.FACTOR_ND, ptr(bs), ptr(ref), b.shape[0], 0, 1e-30, 5, ptr(work), None, None,
+                   None)
+    ref = op.to_user(ref)
+    op.drop_factor()
+    x, rep = op.solve(b, precision=precision, tol=tol, fallback=False)
+    assert op.factors[precision][0].numel() == op.nd_bytes[precision]
+    op.drop_factor()
+    op.factor(precision, stepwise=True)
+    y, _ = op.solve(b, precision=precision, tol=tol, fallback=False)
+    assert op.factors[precision][0].numel() != op.nd_bytes[precision]
+    print(f"{n} {seed} {precision} {tol:g}: error {error(x):.1e} in {rep.sweeps} sweeps, block {error(y):.1e}")
+    assert error(y) > 1e-13 and error(x) <= error(y)
 
 
 @pytest.mark.gpu
