@@ -4189,7 +4189,7 @@ int fdfd_twist_block(const fdfd_grid *g) {
 int fdfd_nd_supported(const fdfd_grid *g, int precision) {
   NdPlan P;
   if (check_grid(g) || check_prec(precision)) return -1;
-  return g_twist.load() && nd_fits(g, precision, &P) ? 1 : 0;
+  return g_twist.load() && nd_fits(g, precision, &P) && !nd_long(g) ? 1 : 0;
 }
 
 int fdfd_nd_front(const fdfd_grid *g, int level, int box, int32_t *info, int64_t *cells, int32_t *map) {

@@ -2231,6 +2231,20 @@ inline bool nd_fits(const fdfd_grid *g, int precision, NdPlan *P) {
   return true;
 }
 
+// Grids too long for the tree to be the factor of choice. Its root front is the
+// cross, of order nx + ny - 1 and eliminated whole: the factor's time grows
+// with the cube of the long side and its memory with the square, the block
+// chain's with the side itself. FP64 factor, tree against block path: 6144 x 16
+// 36 against 58 ms, 8192 x 16 81 / 78 (5.8 GB against 0.13), 12288 x 16 266 /
+// 117, 11584 x 64 230 / 326, 16384 x 64 632 / 462, 16384 x 128 645 / 776;
+// complex64 11584 x 64 116 / 254, 16384 x 64 317 / 359. A chain's step costs
+// about its block's tiles: the lines cross near a^2 = 2^21 b for a long side a
+// and a short side padded to b.
+inline bool nd_long(const fdfd_grid *g) {
+  const size_t a = std::max(g->nx, g->ny), b = pad_n(std::min(g->nx, g->ny));
+  return a * a > b << 21;
+}
+
 // The launch of k_nd_residual of a solve
 template <typename T>
 void nd_residual(const fdfd_grid *g, const NdPlan &P, const double *op, const void *factor, const double *b,

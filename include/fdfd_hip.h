@@ -58,7 +58,8 @@ enum { FDFD_PREC_FP64 = 0, FDFD_PREC_C64 = 1 };      /* factor precision  */
 #define FDFD_FACTOR_STEPWISE 0x200
 /* OR'ed, alone, into the precision argument of fdfd_factor and of the size
  * functions: the nested-dissection factor of the whole periodic operator
- * (grids that fdfd_nd_supported accepts) instead of the block factorization.
+ * (grids of 16 cells a side or more, 64 in complex64) instead of the block
+ * factorization; fdfd_nd_supported says where it is the better one.
  * Its buffers have sizes of their own. fdfd_solve, fdfd_solve_static and
  * fdfd_sweep recognise it by a tag at its start, which costs a read of the
  * device; with FDFD_FACTOR_ND (or, for a block factor, FDFD_FACTOR_STEPWISE)
@@ -297,8 +298,9 @@ int fdfd_set_twist(int on);
 int fdfd_twist_block(const fdfd_grid *g);
 
 /* 1 when FDFD_FACTOR_ND is the factor of choice for this grid (its shorter
- * side has 16 cells or more, 64 in complex64), 0 when not (also while
- * fdfd_set_twist(0) asks for the one-chain order), -1 for invalid
+ * side has 16 cells or more, 64 in complex64, and its longer side a is not
+ * beyond a^2 = 2^21 b, b the shorter one padded to 32), 0 when not (also
+ * while fdfd_set_twist(0) asks for the one-chain order), -1 for invalid
  * arguments. No reference counterpart. */
 int fdfd_nd_supported(const fdfd_grid *g, int precision);
 

@@ -123,6 +123,20 @@ def test_range_and_sizes():
         lib.fdfd_set_twist(prev)
 
 
+@pytest.mark.parametrize("longest,short", [(8192, 16), (8192, 32), (11585, 33), (11585, 64), (16384, 128), (32768, 512)])
+def test_long_grids_are_block_factors(longest, short):
+    """The root front grows with the square of the long side, a block factor
+    with the side: beyond the line the block factor is the one of choice, and
+    the tree stays there for who asks for it."""
+    lib = L.lib()
+    for nx, want in ((longest, 1), (longest + 1, 0), (10 * longest, 0)):
+        g = ctypes.byref(L.FdfdGrid(nx, short, 8, 8, 0, 0, OMEGA, 0.02, 1e-6))
+        assert lib.fdfd_nd_supported(g, 0) == want
+        assert lib.fdfd_nd_supported(g, 1) == (want if short >= 64 else 0)
+    g = ctypes.byref(L.FdfdGrid(longest + 1, short, 8, 8, 0, 0, OMEGA, 0.02, 1e-6))
+    assert lib.fdfd_factor_bytes(g, L.FACTOR_ND) > 0
+
+
 def _device(N, npml, pol, eps, precision):
     from fdfdpy_amd.device import DeviceOperator
     op = DeviceOperator(N, OMEGA, 0.02, npml, pol, 1e-6, DEV)
