@@ -137,9 +137,20 @@ inline size_t nd_factor_bytes(const fdfd_grid *g, const NdPlan &P, int precision
   const size_t n = nd_data_off(P) + align_up(P.elems * elem_size(precision), 256);
   return n == factor_total_bytes(g, base_prec(precision)) ? n + 256 : n;
 }
+// Which levels k_nd_merge takes: one tile of separator, a border of at most
+// nd_merge_tiles tiles (wider ones are few boxes with more tiles than one
+// workgroup should form: with 4 and 6 tiles, 256 and 128 boxes, 75 and 72 us
+// there, 46 and 45 as a launch each for front, step and update; FP64 with 3
+// tiles and 85 KB of LDS 311 against 293). es: bytes of a real.
+constexpr int nd_merge_tiles(size_t es) { return es == 8 ? 2 : 3; }
+inline bool nd_merges(const NdLevel &L, size_t es) {
+  return !L.root && L.sp == TB && L.bp <= nd_merge_tiles(es) * TB;
+}
 // Factor workspace (after the status header): the scaled bands, the pivot
 // inverses of two steps, the ping-pong pairs of [F_ss] and [F_sb], the panels
-// U and R of the elimination (k_nd_step), the updates C of two levels.
+// U and R of the elimination (k_nd_step), the updates C of two levels. All but
+// the bands and C belong to the levels that k_nd_merge does not take: 512^2
+// complex64 195 MB instead of 283, 768^2 FP64 1027 instead of 1261.
 struct NdWork {
   size_t bands, pinv[2], S[2], B[2], U, R, C[2], total;
 };
@@ -148,11 +159,12 @@ NdWork nd_work_layout(const NdPlan &P, int precision) {
   size_t boxes = 0, ss = 0, sb = 0, sb1 = 0, cc = (size_t)P.nleaf * P.leaf_bp * P.leaf_bp;
   for (int i = 0; i <= P.nlev; ++i) {
     const NdLevel &L = P.lev[i];
+    cc = std::max(cc, (size_t)L.nbox * L.bp * L.bp);
+    if (nd_merges(L, es)) continue;
     boxes = std::max(boxes, (size_t)L.nbox);
     if (L.sp > TB) ss = std::max(ss, (size_t)L.nbox * L.sp * L.sp);
     sb = std::max(sb, (size_t)L.nbox * L.sp * L.bp);
     if (L.sp > TB) sb1 = std::max(sb1, (size_t)L.nbox * L.sp * L.bp);
-    cc = std::max(cc, (size_t)L.nbox * L.bp * L.bp);
   }
   NdWork w;
   size_t off = WORK_HEADER;
@@ -1421,14 +1433,6 @@ __global__ void __launch_bounds__(NT, 2) k_nd_merge(NdLevel L, NdBands<T> bd, co
     }
   }
 }
-// Which levels k_nd_merge takes: one tile of separator, a border of at most
-// nd_merge_tiles tiles (wider ones are few boxes with more tiles than one
-// workgroup should form: with 4 and 6 tiles, 256 and 128 boxes, 75 and 72 us
-// here, 46 and 45 as a launch each for front, step and update; FP64 with 3
-// tiles and 85 KB of LDS 311 against 293)
-template <typename T> constexpr int nd_merge_tiles() { return sizeof(T) == 8 ? 2 : 3; }
-template <typename T>
-inline bool nd_merges(const NdLevel &L) { return !L.root && L.sp == TB && L.bp <= nd_merge_tiles<T>() * TB; }
 template <typename T>
 inline size_t nd_merge_lds(const NdLevel &L) {
   return sizeof(NdLds2<T>) + (size_t)(L.bp / TB) * 2 * TB * TBP * sizeof(T);
@@ -1458,7 +1462,7 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
   static std::once_flag lds_attr;
   std::call_once(lds_attr, [] {
     (void)hipFuncSetAttribute((const void *)k_nd_merge<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)(sizeof(NdLds2<T>) + nd_merge_tiles<T>() * 2 * TB * TBP * sizeof(T)));
+                              (int)(sizeof(NdLds2<T>) + nd_merge_tiles(sizeof(T)) * 2 * TB * TBP * sizeof(T)));
   });
   hipLaunchKernelGGL(k_nd_tables, dim3((std::max(P.nx + P.ny, 512) + NT - 1) / NT), dim3(NT), 0, s, *g,
                      (unsigned long long *)factor, tab, status, ND_HEADER + 32 * (size_t)(P.nx + P.ny),
@@ -1472,7 +1476,7 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
     const NdLevel &L = P.lev[l];
     const int ns = L.sp / TB, nb = L.bp / TB, per = ns * (ns + 1) / 2 + ns * nb;
     const int first = (L.nbox + XCDS - 1) / XCDS * XCDS;
-    if (nd_merges<T>(L)) {
+    if (nd_merges(L, sizeof(T))) {
       hipLaunchKernelGGL(k_nd_merge<T>, dim3(nd_grid(L.nbox)), dim3(NT), nd_merge_lds<T>(L), s, L, A.bd,
                          (const T *)C[cin], data + L.xoff, data + L.woff, C[cin ^ 1], status);
       cin ^= 1;

@@ -137,6 +137,36 @@ def test_long_grids_are_block_factors(longest, short):
     assert lib.fdfd_factor_bytes(g, L.FACTOR_ND) > 0
 
 
+@pytest.mark.parametrize("nx,ny", [(16, 16), (64, 64), (200, 96), (512, 512), (1000, 64)])
+@pytest.mark.parametrize("es", [8, 4])
+def test_workspace_holds_what_the_launches_use(nx, ny, es):
+    """The bands and the updates of two levels; pivot inverses, fronts and
+    panels only of the levels that are eliminated step by step (a separator
+    over one tile, or a border over 2 tiles, 3 in complex64, and the root)."""
+    if es == 4 and ny < 64:
+        pytest.skip("complex64 factors of grids below 64 cells are block factors")
+    lib, pad = L.lib(), lambda n: -(-n // 32) * 32
+    g = L.FdfdGrid(nx, ny, 8, 8, 0, 0, OMEGA, 0.02, 1e-6)
+    levels = _front(g, -1, 0)[0][0]
+    info = (ctypes.c_int32 * 8)()
+    boxes = ss = sb = panels = updates = 0
+    for level in range(-1, levels + 1):
+        s = b = k = 0
+        while k == 0 or k < info[1]:
+            L.check(lib.fdfd_nd_front(ctypes.byref(g), level, k, info, None, None))
+            s, b, k = max(s, info[3]), max(b, info[4]), k + 1
+        sp, bp = (32, 32) if level == -1 else (pad(s), pad(b))
+        updates = max(updates, k * bp * bp)
+        if level == -1 or (level < levels and sp == 32 and bp <= (64 if es == 8 else 96)):
+            continue
+        boxes, panels = max(boxes, k), max(panels, k * sp * bp)
+        if sp > 32:
+            ss, sb = max(ss, k * sp * sp), max(sb, k * sp * bp)
+    need = 2 * es * (3 * nx * ny + 2 * boxes * 32 * 32 + 2 * ss + 2 * sb + panels + sb + 2 * updates)
+    got = lib.fdfd_factor_workspace_bytes(ctypes.byref(g), (0 if es == 8 else 1) | L.FACTOR_ND)
+    assert 0 <= got - need <= 1024 + 11 * 256      # the status header, and the parts' alignment
+
+
 def _device(N, npml, pol, eps, precision):
     from fdfdpy_amd.device import DeviceOperator
     op = DeviceOperator(N, OMEGA, 0.02, npml, pol, 1e-6, DEV)
