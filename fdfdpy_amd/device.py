@@ -157,11 +157,13 @@ class DeviceOperator:
         self.factors = {}        # precision -> (uint8 tensor, operator version, pivoted)
         self.factor_seconds = {}
         self.engine = None       # FactorEngine shared with other operators, if any
+        self.tree = True         # nested-dissection factors where the grid is in their range
 
     # -- sizes ----------------------------------------------------------
     def nested(self, precision):
-        """The next factor is a nested-dissection one (unless it pivots or an engine builds it)."""
-        return self.lib.fdfd_nd_supported(ctypes.byref(self.grid), L.PREC[precision]) == 1
+        """The next factor is a nested-dissection one (unless it pivots)."""
+        return (self.tree and self.engine is None and
+                self.lib.fdfd_nd_supported(ctypes.byref(self.grid), L.PREC[precision]) == 1)
 
     def factor_bytes(self, precision):
         if self.nested(precision):
@@ -220,7 +222,7 @@ class DeviceOperator:
             if not refresh or (ver == self.version and piv == pivot and not blocks):
                 return fac
         g = ctypes.byref(self.grid)
-        if self.nested(precision) and not pivot and not stepwise and self.engine is None:
+        if self.nested(precision) and not pivot and not stepwise:
             p = L.PREC[precision] | L.FACTOR_ND
         else:
             p = L.PREC[precision] | (L.FACTOR_PIVOT if pivot else 0) | (L.FACTOR_STEPWISE if stepwise else 0)

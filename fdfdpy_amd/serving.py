@@ -11,6 +11,7 @@ identical operators are kept in an LRU cache across requests.
 
 from __future__ import annotations
 
+import ctypes
 import hashlib
 import threading
 import time
@@ -21,7 +22,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .device import DeviceOperator, FactorEngine
+from .device import DeviceOperator, FactorEngine, choose_transpose
 
 
 @dataclass
@@ -63,20 +64,25 @@ def operator_key(p):
     return (p.shape, p.pol, float(p.omega), float(p.dl), float(p.L0), tuple(p.npml), h)
 
 
-def request_bytes(p, precision, nrhs=None):
-    """Device bytes a request may hold while it runs (operator, factor,
-    workspaces, vectors), with a block factor of its precision, the larger
-    kind, which a solve without its nested-dissection factor falls back to."""
+def request_bytes(p, precision, nrhs=None, nested=True):
+    """Device bytes a request holds while it runs (operator, factor,
+    workspaces, vectors) with a factor of its precision, of the larger kind:
+    block, or (nested) nested dissection where the grid is in its range, which
+    is the larger one on small and on long grids."""
     lib = L.lib()
     Nx, Ny = p.shape
-    g = L.FdfdGrid(Nx, Ny, p.npml[0], p.npml[1], L.POL[p.pol], 0, p.omega, p.dl, p.L0)
-    import ctypes
+    turn = choose_transpose(Nx, Ny, p.npml)
+    nx, ny, npx, npy = (Ny, Nx, p.npml[1], p.npml[0]) if turn else (Nx, Ny, p.npml[0], p.npml[1])
+    g = L.FdfdGrid(nx, ny, npx, npy, L.POL[p.pol], 0, p.omega, p.dl, p.L0)
     gp = ctypes.byref(g)
     k = p.srcs.shape[0] if nrhs is None else nrhs
     pr = L.PREC[precision]
-    return int(lib.fdfd_op_bytes(gp) * 1.2 + lib.fdfd_factor_bytes(gp, pr)
-               + lib.fdfd_factor_workspace_bytes(gp, pr) + lib.fdfd_solve_workspace_bytes(gp, pr, k)
-               + 16 * Nx * Ny * (3 * k + 2))
+    kinds = [pr | L.FACTOR_STEPWISE]
+    if nested and lib.fdfd_nd_supported(gp, pr) == 1:
+        kinds.append(pr | L.FACTOR_ND)
+    return int(lib.fdfd_op_bytes(gp) * 1.2 + 16 * Nx * Ny * (3 * k + 2)
+               + max(lib.fdfd_factor_bytes(gp, f) + lib.fdfd_factor_workspace_bytes(gp, f)
+                     + lib.fdfd_solve_workspace_bytes(gp, f, k) for f in kinds))
 
 
 class FactorCache:
@@ -170,6 +176,8 @@ class ServingEngine:
                 reused = True
             else:
                 op = DeviceOperator(p.shape, p.omega, p.dl, p.npml, p.pol, p.L0, self.device)
+                # a request that the budget only holds with a block factor takes one
+                op.tree = request_bytes(p, self.precision) <= self.memory_budget
                 if not op.nested(self.precision):   # block factorizations share step launches
                     op.engine = self._engine_for(stream)
                 op.set_eps(p.eps)
@@ -229,6 +237,8 @@ class ServingEngine:
                     continue
                 if need is None:
                     need = request_bytes(req.problem, self.precision)
+                    if need > self.memory_budget:
+                        need = request_bytes(req.problem, self.precision, nested=False)
                 if need > self.memory_budget:
                     results[req.rid] = Result(req.rid, req.problem.shape, req.problem.srcs.shape[0], None,
                                               req.arrival, now(), now(), self.precision, 0, float("nan"),

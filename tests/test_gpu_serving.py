@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from fdfdpy_amd import configs as C
-from fdfdpy_amd.serving import Request, ServingEngine, summarize
+from fdfdpy_amd.serving import Request, ServingEngine, request_bytes, summarize
 from oracle import construct_A
 
 pytestmark = pytest.mark.gpu
@@ -48,6 +48,25 @@ def test_memory_budget_and_factor_cache():
     assert np.array_equal(res2[0].fields.cpu().numpy(), res[1].fields.cpu().numpy())
     s = summarize(res, max(r.done for r in res))
     assert s["failed"] == 0 and s["max_rel_residual"] <= 1e-10
+
+
+def test_budget_for_a_block_factor_alone_gets_one():
+    """64 x 64 cells: the nested-dissection factor and its workspace are three
+    times the block factor's."""
+    rng = np.random.default_rng(0)
+    src = np.zeros((1, 64, 64))
+    src[0, 20, 30] = 1
+    p = C.Problem("small", "Ez", C.omega_of(1.55e-6), 1 + 11.25 * (rng.random((64, 64)) < 0.5), [8, 8], src)
+    block, most = request_bytes(p, "fp64", nested=False), request_bytes(p, "fp64")
+    fields, launches = [], []
+    for budget in (most, (block + most) // 2):
+        eng = ServingEngine("cuda:0", precision="fp64", slots=2, keep_fields=True, memory_budget=budget)
+        r = eng.run([Request(0, p, 0.0)])[0]
+        assert not r.error and r.max_rel_residual <= 1e-10
+        fields.append(r.fields.cpu().numpy())
+        launches.append(sum(e.launches for e in eng.factor_engines))
+    assert launches[0] == 0 and launches[1] > 0
+    assert np.linalg.norm(fields[1] - fields[0]) < 1e-8 * np.linalg.norm(fields[0])
 
 
 def test_engine_factors_match_direct_factors():

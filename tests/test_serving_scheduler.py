@@ -1,12 +1,15 @@
 """Admission and scheduling of the serving loop, with the device work replaced (CPU)."""
 
+import ctypes
 import threading
 import time
 
 import numpy as np
+import pytest
 
+from fdfdpy_amd import _lib as L
 from fdfdpy_amd import configs as C
-from fdfdpy_amd.device import SolveReport
+from fdfdpy_amd.device import SolveReport, choose_transpose
 from fdfdpy_amd.serving import FactorCache, Request, ServingEngine, request_bytes, summarize
 
 
@@ -78,6 +81,42 @@ def test_request_bytes_scale_with_precision():
     p = C.c3_request(0, n=512)
     assert request_bytes(p, "fp64") > 1.8 * request_bytes(p, "c64") * 0.9
     assert request_bytes(p, "c64") > 512 * 2 * 512 * 512 * 4
+
+
+def _sized(nx, ny, npml=(8, 8), k=2):
+    return C.Problem("sized", "Ez", C.omega_of(1.55e-6), np.ones((nx, ny)), list(npml), np.zeros((k, nx, ny)))
+
+
+@pytest.mark.parametrize("shape,npml", [((64, 64), (8, 8)), ((128, 128), (8, 8)), ((200, 200), (8, 8)),
+                                        ((256, 256), (8, 8)), ((512, 512), (8, 8)), ((768, 768), (8, 8)),
+                                        ((1000, 64), (8, 8)), ((64, 1000), (8, 8)), ((5000, 16), (8, 8)),
+                                        ((300, 120), (0, 8)), ((100000, 16), (8, 8))])
+@pytest.mark.parametrize("precision", ["fp64", "c64"])
+def test_request_bytes_cover_what_the_operator_allocates(shape, npml, precision):
+    """Factor, factor workspace and solve workspace of either kind, in the
+    orientation that the operator is solved in."""
+    lib, p, pr = L.lib(), _sized(*shape, npml), L.PREC[precision]
+    turn = choose_transpose(*shape, npml)
+    g = ctypes.byref(L.FdfdGrid(*(shape[::-1] if turn else shape), *(npml[::-1] if turn else npml), 0, 0, p.omega,
+                                p.dl, p.L0))
+
+    def held(f):
+        return (lib.fdfd_factor_bytes(g, f) + lib.fdfd_factor_workspace_bytes(g, f) +
+                lib.fdfd_solve_workspace_bytes(g, f, 2))
+    nested = lib.fdfd_nd_supported(g, pr) == 1
+    rest = lib.fdfd_op_bytes(g) * 1.2 + 16 * shape[0] * shape[1] * 8      # b twice, x twice, per source
+    need = max(held(pr), held(pr | L.FACTOR_ND)) if nested else held(pr)
+    assert need < request_bytes(p, precision) <= need + rest + 1
+    assert request_bytes(p, precision, nested=False) <= held(pr) + rest + 1
+
+
+def test_request_that_only_fits_as_a_block_factor_is_admitted():
+    p = _sized(64, 64)
+    block, most = request_bytes(p, "fp64", nested=False), request_bytes(p, "fp64")
+    assert block < most
+    eng = ServingEngine("cpu", precision="fp64", slots=2, memory_budget=(block + most) // 2, serve_fn=FakeDevice())
+    res = eng.run([Request(0, p, 0.0), Request(1, p, 0.0)])
+    assert all(not r.error for r in res) and eng.max_bytes_in_flight == block
 
 
 def test_factor_cache_lru():
