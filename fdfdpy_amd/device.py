@@ -222,12 +222,17 @@ class DeviceOperator:
             if not refresh or (ver == self.version and piv == pivot and not blocks):
                 return fac
         g = ctypes.byref(self.grid)
+        kinds = [L.PREC[precision] | (L.FACTOR_PIVOT if pivot else 0) | (L.FACTOR_STEPWISE if stepwise else 0)]
         if self.nested(precision) and not pivot and not stepwise:
-            p = L.PREC[precision] | L.FACTOR_ND
-        else:
-            p = L.PREC[precision] | (L.FACTOR_PIVOT if pivot else 0) | (L.FACTOR_STEPWISE if stepwise else 0)
-        fac = torch.empty(self.lib.fdfd_factor_bytes(g, p), dtype=torch.uint8, device=self.device)
-        work = torch.empty(self.lib.fdfd_factor_workspace_bytes(g, p), dtype=torch.uint8, device=self.device)
+            kinds.insert(0, L.PREC[precision] | L.FACTOR_ND)
+        for p in kinds:
+            try:
+                fac, work = [torch.empty(n, dtype=torch.uint8, device=self.device) for n in
+                             (self.lib.fdfd_factor_bytes(g, p), self.lib.fdfd_factor_workspace_bytes(g, p))]
+                break
+            except torch.cuda.OutOfMemoryError:   # on small and long grids the block factor is the smaller one
+                if p == kinds[-1]:
+                    raise
         s = _stream(self.device)
         t0 = time.perf_counter()
         if self.engine is not None:

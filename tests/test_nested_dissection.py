@@ -331,6 +331,29 @@ def test_solves_are_as_exact_as_the_block_factors(n, seed, precision, tol):
 
 
 @pytest.mark.gpu
+def test_memory_for_a_block_factor_alone_gets_one(monkeypatch):
+    """Where the device has no room for the nested-dissection factor and its
+    workspace (an allocation over the block factor's size fails here), the
+    block factor solves."""
+    N = (64, 64)
+    rng = np.random.default_rng(5)
+    eps = _eps(rng, N)
+    op = _device(N, [8, 8], "Ez", eps, "fp64")
+    most, real = op.lib.fdfd_factor_bytes(ctypes.byref(op.grid), 0), torch.empty
+
+    def limited(*a, **k):
+        if k.get("dtype") is torch.uint8 and a[0] > most:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return real(*a, **k)
+    monkeypatch.setattr(torch, "empty", limited)
+    b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    x, rep = op.solve(torch.tensor(b, device=DEV), precision="fp64", tol=1e-12)
+    assert rep.converged and not rep.fell_back and op.factors["fp64"][0].numel() == most < op.nd_bytes["fp64"]
+    A, _ = construct_A(OMEGA, [0, N[0] * 0.02], [0, N[1] * 0.02], eps, [8, 8], "Ez", 1e-6)
+    assert relerr(x.cpu().numpy(), solver_direct(A, b.reshape(-1)).reshape(N)) < 1e-10
+
+
+@pytest.mark.gpu
 def test_stall_without_fallback_takes_the_block_factor(monkeypatch):
     """fallback=False keeps the precision: when the nested-dissection factor
     does not refine (its report forced here), the block factor does."""
