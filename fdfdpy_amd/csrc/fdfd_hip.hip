@@ -26,6 +26,7 @@
 #include <condition_variable>
 #include <thread>
 #include <deque>
+#include <initializer_list>
 #include <map>
 #include <memory>
 
@@ -65,6 +66,28 @@ int fail(int code, const char *fmt, ...) {
     if (e_ != hipSuccess)                                                      \
       return fail(FDFD_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_));       \
   } while (0)
+
+// Dynamic LDS beyond the default of 64 KB is granted per kernel and device:
+// to each device whose stream runs the kernels, the first time (done: a bit
+// per device, one word for the kernels of a call).
+constexpr size_t LDS_DEFAULT = 64 << 10;
+int grant_lds(std::atomic<uint64_t> &done, std::initializer_list<const void *> kernels, size_t bytes, hipStream_t s) {
+  int cur = 0, dev = 0;
+  HIP_TRY(hipGetDevice(&cur));
+  dev = cur;
+  if (s && s != hipStreamPerThread) HIP_TRY(hipStreamGetDevice(s, &dev));
+  const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+  if (done.load() & bit) return 0;
+  if (dev != cur) HIP_TRY(hipSetDevice(dev));
+  hipError_t e = hipSuccess;
+  for (const void *k : kernels)
+    if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (dev != cur) (void)hipSetDevice(cur);
+  if (e != hipSuccess)
+    return fail(FDFD_ERR_HIP, "%zu bytes of dynamic LDS on device %d: %s", bytes, dev, hipGetErrorString(e));
+  done |= bit;
+  return 0;
+}
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 inline int pad_n(int n) { return (n + TB - 1) / TB * TB; }
@@ -3105,24 +3128,24 @@ int factor_batch_impl(const fdfd_grid *g, const double *const *ops, void *const 
 }
 
 template <typename T>
-void sweep_block_attr() {
-  static std::once_flag lds_attr;
-  std::call_once(lds_attr, [] {
-    const int most = (int)(2 * MAXR * pad_n(MAX_BLOCK_N) * sizeof(T));
-    (void)hipFuncSetAttribute((const void *)k_sweep_fwd<T>, hipFuncAttributeMaxDynamicSharedMemorySize, most);
-    (void)hipFuncSetAttribute((const void *)k_sweep_bwd<T>, hipFuncAttributeMaxDynamicSharedMemorySize, most);
-  });
+int sweep_block_lds(hipStream_t s) {
+  constexpr size_t most = (size_t)2 * MAXR * MAX_BLOCK_N * sizeof(T);
+  static std::atomic<uint64_t> done{0};
+  if constexpr (most > LDS_DEFAULT)
+    return grant_lds(done, {(const void *)k_sweep_fwd<T>, (const void *)k_sweep_bwd<T>}, most, s);
+  return FDFD_OK;
 }
 
 // y_c and x_c += y_c of the twist block, between the forward chains and the
 // backward chains of a twisted sweep
 template <typename T>
-void launch_twist_block(const fdfd_grid *g, const T *G, const double *op, const double *r, T *y, double *x,
+int launch_twist_block(const fdfd_grid *g, const T *G, const double *op, const double *r, T *y, double *x,
                         int nrhs, int c, hipStream_t s) {
   const int np = pad_n(g->ny);
-  sweep_block_attr<T>();
+  if (int rc = sweep_block_lds<T>(s)) return rc;
   hipLaunchKernelGGL(k_sweep_fwd<T>, dim3((np + 3) / 4), dim3(NT), (size_t)2 * MAXR * np * sizeof(T), s, G, op, r,
                      y, x, g->nx, g->ny, np, c, nrhs, c - 1, (int)FDFD_OP_XM, c + 1, (int)FDFD_OP_XP);
+  return FDFD_OK;
 }
 
 template <typename T>
@@ -3133,7 +3156,7 @@ int sweep_blockwise(const fdfd_grid *g, const double *op, const void *factor, co
   const size_t lds = (size_t)2 * MAXR * np * sizeof(T);
   const T *G = (const T *)factor;
   T *yt = (T *)y;
-  sweep_block_attr<T>();
+  if (int rc = sweep_block_lds<T>(s)) return rc;
   auto fwd = [&](int k, int nb, int pl) {
     hipLaunchKernelGGL(k_sweep_fwd<T>, grid, dim3(NT), lds, s, G, op, r, yt, (double *)nullptr, nx, ny, np, k,
                        nrhs, nb, pl, -1, 0);
@@ -3147,7 +3170,7 @@ int sweep_blockwise(const fdfd_grid *g, const double *op, const void *factor, co
   } else {
     for (int k = 0; k < c; ++k) fwd(k, k > 0 ? k - 1 : -1, FDFD_OP_XM);
     for (int k = nx - 1; k > c; --k) fwd(k, k + 1 < nx ? k + 1 : -1, FDFD_OP_XP);
-    launch_twist_block<T>(g, G, op, r, yt, x, nrhs, c, s);
+    if (int rc = launch_twist_block<T>(g, G, op, r, yt, x, nrhs, c, s)) return rc;
     for (int k = c - 1; k >= 0; --k) bwd(k, k + 1, FDFD_OP_XP);
     for (int k = c + 1; k < nx; ++k) bwd(k, k - 1, FDFD_OP_XM);
   }
@@ -3333,15 +3356,7 @@ template <typename T, int RP>
 void launch_psweep(int W, size_t lds, hipStream_t s, const T *G, const double *op, const double *r, T *y,
                    double *x, int nx, int ny, int np, int nr, int dir, const SweepChains &chs, SweepSync *sy,
                    unsigned tag0) {
-  static std::once_flag lds_attr;
-  std::call_once(lds_attr, [] {
-    if constexpr (RP <= LL_MAXRHS)
-      (void)hipFuncSetAttribute((const void *)k_psweep_ll<T, RP>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(2 * RP * PSWEEP_MAX_N * sizeof(T)));
-    else
-      (void)hipFuncSetAttribute((const void *)k_psweep<T, RP>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(2 * RP * PSWEEP_MAX_N * sizeof(T)));
-  });
+  static_assert(2 * RP * PSWEEP_MAX_N * sizeof(T) <= LDS_DEFAULT, "no grant needed");
   if constexpr (RP <= LL_MAXRHS)
     hipLaunchKernelGGL((k_psweep_ll<T, RP>), dim3(W * chs.nch), dim3(NT), lds, s, G, op, r, y, x, nx, ny, np, nr,
                        dir, chs, sy, g_spin_cap.load(), tag0);
@@ -3414,7 +3429,7 @@ int sweep_impl(const fdfd_grid *g, const double *op, const void *factor, const d
       }
       // twisted: the twist block between the two passes
       if (dir == 0 && c < nx - 1)
-        launch_twist_block<T>(g, G, op, r + 2 * M * q0, yq, x + 2 * M * q0, nr, c, s);
+        if (int rc = launch_twist_block<T>(g, G, op, r + 2 * M * q0, yq, x + 2 * M * q0, nr, c, s)) return rc;
     }
   }
   HIP_TRY(hipGetLastError());

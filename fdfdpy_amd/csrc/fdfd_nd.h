@@ -1459,11 +1459,11 @@ int nd_factor(const fdfd_grid *g, const double *op, void *factor, void *work, hi
   T *C[2] = {(T *)(base + w.C[0]), (T *)(base + w.C[1])};
   T *S[2] = {(T *)(base + w.S[0]), (T *)(base + w.S[1])}, *Bf[2] = {(T *)(base + w.B[0]), (T *)(base + w.B[1])};
   T *pv[2] = {(T *)(base + w.pinv[0]), (T *)(base + w.pinv[1])};
-  static std::once_flag lds_attr;
-  std::call_once(lds_attr, [] {
-    (void)hipFuncSetAttribute((const void *)k_nd_merge<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)(sizeof(NdLds2<T>) + nd_merge_tiles(sizeof(T)) * 2 * TB * TBP * sizeof(T)));
-  });
+  constexpr size_t lds = sizeof(NdLds2<T>) + nd_merge_tiles(sizeof(T)) * 2 * TB * TBP * sizeof(T);
+  if constexpr (lds > LDS_DEFAULT) {   // FP64: 67.6 KB
+    static std::atomic<uint64_t> done{0};
+    if (int rc = grant_lds(done, {(const void *)k_nd_merge<T>}, lds, s)) return rc;
+  }
   hipLaunchKernelGGL(k_nd_tables, dim3((std::max(P.nx + P.ny, 512) + NT - 1) / NT), dim3(NT), 0, s, *g,
                      (unsigned long long *)factor, tab, status, ND_HEADER + 32 * (size_t)(P.nx + P.ny),
                      nd_data_off(P), nd_data_off(P) + P.elems * sizeof(T), nd_factor_bytes(g, P, prec));
