@@ -22,6 +22,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
+from .configs import Problem
 from .device import DeviceOperator, FactorEngine, choose_transpose
 
 
@@ -83,6 +84,15 @@ def request_bytes(p, precision, nrhs=None, nested=True):
     return int(lib.fdfd_op_bytes(gp) * 1.2 + 16 * Nx * Ny * (3 * k + 2)
                + max(lib.fdfd_factor_bytes(gp, f) + lib.fdfd_factor_workspace_bytes(gp, f)
                      + lib.fdfd_solve_workspace_bytes(gp, f, k) for f in kinds))
+
+
+def device_rhs(p, device):
+    """p.rhs() on the device; that of a plain Problem is formed there, its
+    sources travel as reals."""
+    own = getattr(p, "rhs", None)
+    if own is not None and getattr(own, "__func__", None) is not Problem.rhs:
+        return torch.as_tensor(own(), device=device)
+    return torch.as_tensor(p.srcs, device=device).to(torch.complex128) * (1j * p.omega)
 
 
 class FactorCache:
@@ -181,8 +191,7 @@ class ServingEngine:
                 if not op.nested(self.precision):   # block factorizations share step launches
                     op.engine = self._engine_for(stream)
                 op.set_eps(p.eps)
-            # Problem.rhs() on the device: the sources travel as reals
-            b = torch.as_tensor(p.srcs, device=self.device).to(torch.complex128) * (1j * p.omega)
+            b = device_rhs(p, self.device)
             x, rep = op.solve(b, precision=self.precision, tol=self.tol, max_iter=self.max_iter)
             stream.synchronize()
         if self.cache.capacity and not reused:

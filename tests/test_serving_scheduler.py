@@ -10,7 +10,7 @@ import pytest
 from fdfdpy_amd import _lib as L
 from fdfdpy_amd import configs as C
 from fdfdpy_amd.device import SolveReport, choose_transpose
-from fdfdpy_amd.serving import FactorCache, Request, ServingEngine, request_bytes, summarize
+from fdfdpy_amd.serving import FactorCache, Request, ServingEngine, device_rhs, request_bytes, summarize
 
 
 class FakeDevice:
@@ -117,6 +117,19 @@ def test_request_that_only_fits_as_a_block_factor_is_admitted():
     eng = ServingEngine("cpu", precision="fp64", slots=2, memory_budget=(block + most) // 2, serve_fn=FakeDevice())
     res = eng.run([Request(0, p, 0.0), Request(1, p, 0.0)])
     assert all(not r.error for r in res) and eng.max_bytes_in_flight == block
+
+
+def test_right_hand_sides_are_the_problems_own():
+    class Shifted(C.Problem):
+        def rhs(self):
+            return super().rhs() + 2.0
+
+    rng = np.random.default_rng(0)
+    for srcs in (rng.random((2, 4, 5)), rng.integers(0, 3, (2, 4, 5)), rng.random((2, 4, 5)) * (1 + 2j)):
+        for kind in (C.Problem, Shifted):
+            p = kind("p", "Ez", C.omega_of(1.55e-6), np.ones((4, 5)), [0, 0], srcs)
+            b = device_rhs(p, "cpu").numpy()
+            assert b.dtype == np.complex128 and np.allclose(b, p.rhs(), rtol=1e-15, atol=0)
 
 
 def test_factor_cache_lru():
