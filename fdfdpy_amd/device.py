@@ -285,7 +285,7 @@ class DeviceOperator:
             plan.append((precision, False, True, True))
         rep, failed, spent = None, [], [0.0, 0.0, 0]
         for prec, piv, refresh, blocks in plan:
-            if rep is not None and rep.converged:
+            if rep is not None and (rep.converged or blocks and self._resident_block(prec)):
                 break
             try:
                 if refresh:
@@ -313,6 +313,11 @@ class DeviceOperator:
                                  f"after {rep.iterations} refinement steps ({rep.precision})")
         out = self.to_user(x)
         return (out[0] if squeeze else out), rep
+
+    def _resident_block(self, precision):
+        """The resident factor is an unpivoted block factor of the current operator."""
+        fac, ver, piv = self.factors.get(precision, (None, None, None))
+        return fac is not None and ver == self.version and not piv and fac.numel() != self.nd_bytes[precision]
 
     def _solve_one(self, bs, x, nrhs, precision, tol, max_iter, transpose):
         t0 = time.perf_counter()

@@ -354,6 +354,24 @@ def test_memory_for_a_block_factor_alone_gets_one(monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("stepwise,tries", [(False, 2), (True, 1)])
+def test_no_factor_is_tried_twice(monkeypatch, stepwise, tries):
+    """fallback=False and a tolerance out of reach: the nested-dissection and
+    the block factor once each, a resident block factor once."""
+    from fdfdpy_amd.device import DeviceOperator
+    N = (80, 72)
+    rng = np.random.default_rng(3)
+    op = _device(N, [9, 9], "Ez", _eps(rng, N), "c64")
+    op.factor("c64", stepwise=stepwise)
+    real, calls = DeviceOperator._solve_one, []
+    monkeypatch.setattr(DeviceOperator, "_solve_one", lambda self, *a: calls.append(1) or real(self, *a))
+    b = torch.tensor(rng.standard_normal(N) + 0j, device=DEV)
+    with pytest.raises(L.NotConverged):
+        op.solve(b, precision="c64", tol=1e-15, max_iter=1, fallback=False)
+    assert len(calls) == tries
+
+
+@pytest.mark.gpu
 def test_stall_without_fallback_takes_the_block_factor(monkeypatch):
     """fallback=False keeps the precision: when the nested-dissection factor
     does not refine (its report forced here), the block factor does."""
