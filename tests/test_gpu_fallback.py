@@ -1,5 +1,5 @@
 """The solve's fallback order on the GPU: complex64 factor -> FP64 factor ->
-FP64 factor with partial pivoting inside the 32x32 pivot tiles.
+FP64 block factor with partial pivoting inside the 32x32 pivot tiles.
 
 The reference's solver_direct (fdfdpy/linalg.py:122-149) factors with
 Pardiso's own pivoting and always returns a solution; here the default
@@ -59,9 +59,9 @@ def test_c64_stall_falls_back_to_fp64():
 
 def test_singular_pivot_block_leaves_complex64_for_fp64():
     """eps[0, 0] is set so that the leading 2 x 2 block of the first pivot
-    tile is singular to rounding while A is not. The complex64 factor cannot
-    refine it; the FP64 factor, whose 2 x 2 pivot amplifies rounding by about
-    1e13 (still below 1 / eps), refines to the tolerance."""
+    tile is singular to rounding while A is not. The complex64 block factor
+    cannot refine it; the FP64 factor has that cell in its root separator and
+    does."""
     omega, eps, src, npml = _problem()
     Nx, Ny = eps.shape
     A, _ = construct_A(omega, [0, Nx * 0.02], [0, Ny * 0.02], eps, npml, 'Ez', 1e-6)
@@ -78,6 +78,41 @@ def test_singular_pivot_block_leaves_complex64_for_fp64():
     assert rep.converged and rep.fell_back and rep.precision == 'fp64'
     xh = x.cpu().numpy()
     assert np.linalg.norm(xh - xr) / np.linalg.norm(xr) <= 1e-10
+
+
+def test_design_beyond_complex64_nested_dissection():
+    """A design with a box of the tree near resonance: the complex64
+    nested-dissection factor does not refine. With fallback the FP64 one
+    solves, without it the complex64 block factor."""
+    p = C.c3_request(146, n=128)
+    A, _ = construct_A(p.omega, [0, 128 * p.dl], [0, 128 * p.dl], p.eps, p.npml, p.pol, p.L0)
+    b = p.rhs()
+    for fallback, precision in ((True, "fp64"), (False, "c64")):
+        op = DeviceOperator(p.shape, p.omega, p.dl, p.npml, p.pol, p.L0, DEV)
+        op.set_eps(p.eps)
+        assert op.factor("c64").numel() == op.nd_bytes["c64"]
+        x, rep = op.solve(torch.tensor(b, device=DEV), precision="c64", tol=1e-10, fallback=fallback)
+        assert rep.converged and rep.precision == precision and rep.fell_back == fallback
+        assert (op.factors[precision][0].numel() == op.nd_bytes[precision]) == fallback
+        for q in range(b.shape[0]):
+            res = A @ x[q].cpu().numpy().reshape(-1) - b[q].reshape(-1)
+            assert np.linalg.norm(res) <= 1.5e-10 * np.linalg.norm(b[q])
+
+
+@pytest.mark.parametrize("cell", [(40, 50), (64, 64), (0, 30)])
+def test_singular_nested_dissection_front_is_reported(cell):
+    """The diagonal entry of one cell (of a leaf, a separator, the root) is
+    not a number: the status of the nested-dissection factor says so, as does
+    every factor after it, and the solve raises."""
+    p = C.c3_request(3, n=128)
+    op = DeviceOperator(p.shape, p.omega, p.dl, p.npml, p.pol, p.L0, DEV)
+    op.set_eps(p.eps)
+    op.op.view(5, *op.eps.shape, 2)[0][cell] = float("nan")
+    with pytest.raises(L.FdfdError) as e:
+        op.factor("fp64")
+    assert e.value.code == L.FDFD_ERR_NUMERIC
+    with pytest.raises(L.FdfdError, match="every factor in the fallback order"):
+        op.solve(torch.tensor(p.rhs(), device=DEV), precision="c64", tol=1e-10)
 
 
 def test_zero_pivot_falls_back_to_pivoted_factor(monkeypatch):

@@ -77,8 +77,10 @@ def test_block_beyond_persistent_sweep_limit(precision):
     op = DeviceOperator(prob.shape, prob.omega, prob.dl, prob.npml, prob.pol, prob.L0, DEV)
     assert not op.transposed and op.grid.ny == 784
     op.set_eps(prob.eps)
+    op.factor(precision, stepwise=True)
     b = prob.rhs()
     x, rep = op.solve(torch.tensor(b, device=DEV), precision=precision, tol=1e-10)
+    assert op.factors[precision][0].numel() != op.nd_bytes[precision]
     print(f"784-cell blocks, {precision}: {rep.iterations} refinement steps, residual {rep.max_rel_residual:.2e}")
     assert rep.converged and not rep.fell_back
     assert max(residuals(oracle_A(prob), x.cpu().numpy(), b)) <= 1.5e-10

@@ -128,8 +128,8 @@ def test_engine_batches_of_more_than_eight_jobs():
 
 
 def test_large_requests_alone_equal_in_mix():
-    """The stream's 384 and 512 grids in a mix with smaller ones (two
-    factorization engines, c64 factors): each field is bit-identical to the
+    """The stream's 384 and 512 grids in a mix with smaller ones (c64
+    nested-dissection factors): each field is bit-identical to the
     same request served alone, and its residual on the oracle's CSR operator
     is within the tolerance."""
     sizes = [384, 512, 128, 256, 384]

@@ -17,11 +17,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def _solve_both(n, precision, nrhs, transpose=0):
+def _solve_both(n, precision, nrhs, blocks, transpose=0):
     p = C.c3_request(300 + n, n=n)
     op = DeviceOperator(p.shape, p.omega, p.dl, p.npml, p.pol, p.L0, DEV)
     op.set_eps(p.eps)
-    fac = op.factor(precision)
+    fac = op.factor(precision, stepwise=blocks)
+    assert (fac.numel() != op.nd_bytes[precision]) == blocks
     lib = L.lib()
     g = ctypes.byref(op.grid)
     pr = L.PREC[precision]
@@ -45,12 +46,13 @@ def _solve_both(n, precision, nrhs, transpose=0):
 
 
 @pytest.mark.parametrize("precision", ["c64", "fp64"])
-def test_static_solve_equals_workspace_solve(precision):
+@pytest.mark.parametrize("blocks", [False, True])
+def test_static_solve_equals_workspace_solve(precision, blocks):
     # two calls in a row on the shared static workspace, the second smaller
     for n, nrhs in ((256, 3), (128, 1)):
-        a, b = _solve_both(n, precision, nrhs)
+        a, b = _solve_both(n, precision, nrhs, blocks)
         assert np.array_equal(a, b), f"{precision} n={n}: max difference {np.abs(a - b).max()}"
-    a, b = _solve_both(192, precision, 2, transpose=1)
+    a, b = _solve_both(192, precision, 2, blocks, transpose=1)
     assert np.array_equal(a, b)
 
 
