@@ -16,10 +16,10 @@ value) and for the FP64-factor path on the same trace.
 Three loads: the throughput leg offers the stream at --rate (Poisson
 arrivals) and gives the headline solves/s, which that rate bounds once the
 service is faster; the capacity leg has the whole stream queued at the start
-("saturated": the service's own rate); the latency leg replays the first
---latency-requests requests at --latency-load (0.25) x the request rate of the
-FP64 path's throughput leg, below both paths' capacity at that load, and its
-p50/p99 are the headline latencies.
+("saturated": either path's own rate, mixed_over_fp64 their ratio); the latency
+leg replays the first --latency-requests requests at --latency-load (0.25) x
+the request rate of the FP64 path's throughput leg, below both paths' capacity
+at that load, and its p50/p99 are the headline latencies.
 
 Also reported: the roofline of the dominant work (the complex64
 nested-dissection factor, timed with HIP events on its stream; HBM bytes per
@@ -569,13 +569,19 @@ def main():
                                                 "the FP64-factor path's result of the same request and RHS")
         del res_f, ref
     del res_m
-    capacity, _ = run_stream([Request(i, p, 0.0) for i, p in enumerate(problems[:n_req])], "c64", args.slots, args.tol,
-                             args.engines)
+    # capacity leg: the whole stream queued at the start, both paths
+    queued = [Request(i, p, 0.0) for i, p in enumerate(problems[:n_req])]
+    capacity, _ = run_stream(queued, "c64", args.slots, args.tol, args.engines)
     log(f"capacity: {json.dumps(capacity)}")
+    capacity_f = None
+    if not args.no_fp64:
+        capacity_f, _ = run_stream(queued, "fp64", args.slots, args.tol, args.engines)
+        log(f"capacity fp64: {json.dumps(capacity_f)}")
     if errors:
         log(f"errors: {json.dumps({k_: {a: b for a, b in v.items() if a != 'per_result'} for k_, v in errors.items() if v})}")
     if args.stream_only:
-        print(json.dumps({"stream_c64": mixed, "stream_fp64": fp64, "capacity_c64": capacity}), flush=True)
+        print(json.dumps({"stream_c64": mixed, "stream_fp64": fp64, "capacity_c64": capacity,
+                          "capacity_fp64": capacity_f}), flush=True)
         return
     # latency leg: a prefix of the stream at latency_load x the FP64 path's request rate
     cap = (fp64 or mixed)["requests_per_s"]
@@ -626,9 +632,9 @@ def main():
         "cpu_baseline": cpu,
     }
     if fp64:
-        out["fp64_path"] = {"saturated": _path_summary(fp64),
+        out["fp64_path"] = {"saturated": _path_summary(capacity_f), "throughput_leg": _path_summary(fp64),
                             "latency_leg": _path_summary(lat_f) if lat_f else None}
-        out["mixed_over_fp64"] = round(mixed["solves_per_s"] / fp64["solves_per_s"], 4)
+        out["mixed_over_fp64"] = round(capacity["solves_per_s"] / capacity_f["solves_per_s"], 4)
     print(json.dumps(out), flush=True)
 
 

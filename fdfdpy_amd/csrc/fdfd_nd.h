@@ -8,8 +8,8 @@
 // for the lower levels and one per level above, and O(n^3) flops. 512^2
 // complex64: factor 65.7 -> 1.87 ms, a sweep 2.1 -> 0.33 ms; 768^2 FP64: 222 ->
 // 6.0 ms. The block path keeps what asks for it by kind (pivoted, stepwise and
-// batched factors) and the grids with a side under ND_MIN_SIDE cells, complex64
-// under ND_MIN_SIDE_C64.
+// batched factors), the grids with a side under ND_MIN_SIDE cells, complex64
+// under ND_MIN_SIDE_C64, and very long ones (nd_long).
 //
 // Tree. Cell column 0 and cell row 0 (the cross) are the root separator, so
 // what is left, cells 1..nx-1 x 1..ny-1, is not periodic. A box is split by
@@ -305,8 +305,9 @@ __device__ inline cd nd_sqrt(cd s) {
   return {re, s.i / (2 * re)};
 }
 // The factor's tag and tables; clears the status word and the bytes [gap0,
-// data) and [gap1, end) of the factor that hold nothing (its bits are a
-// function of the operator).
+// data) and [gap1, end) between and after the factor's parts. (The padding
+// rows of leaves and merged boxes hold what the buffer held: nothing reads
+// them into a result.)
 __global__ void __launch_bounds__(NT) k_nd_tables(fdfd_grid g, unsigned long long *head, double *tab, int *status,
                                                   size_t gap0, size_t data, size_t gap1, size_t end) {
   const int t = blockIdx.x * NT + threadIdx.x, nx = g.nx, ny = g.ny;
@@ -1856,10 +1857,10 @@ __global__ void __launch_bounds__(64 * ND_TREE_WAVES) k_nd_down_tree(NdTree t, N
 // their loads go out before f is gathered, so a batch of 2 NW UN rows costs one
 // trip to memory. Bound by the latencies of one launch: 512^2 complex64 with 4
 // right-hand sides, the root's 1023 rows 20.6 -> 15 us, the levels below it
-// 12.5 .. 7 -> 10 .. 6 us against rows loaded four at a time after f; the solve
-// 1.05 -> 0.99 ms, of 512^2 FP64 with one 0.42 -> 0.35 ms. The caller's NW and
-// UN make one batch of a separator up to 512 rows; larger batches than the
-// separator needs would load rows for nothing.
+// 12.5 .. 7 -> 10 .. 6 us against rows loaded four at a time after f; a solve of
+// three sweeps 1.05 -> 0.99 ms, of one (512^2 FP64, one right-hand side) 0.42 ->
+// 0.35 ms. The caller's NW and UN make one batch of a separator up to 512
+// rows; larger batches than the separator needs would load rows for nothing.
 template <typename T, int R, int NW, int UN>
 __global__ void __launch_bounds__(64 * NW) k_nd_up(NdLevel L, NdVec<T> A, const T *__restrict__ uin,
                                                    T *__restrict__ uout, int nq, int add) {
@@ -2105,7 +2106,9 @@ __global__ void __launch_bounds__(NT) k_nd_residual(fdfd_grid g, double alpha, N
 }
 
 // The subtrees of a plan: the levels whose separators fit a tile, as far up as
-// leaves ND_TREE_BOXES of them (two workgroups of eight waves per CU). 512^2
+// leaves ND_TREE_BOXES of them (two workgroups of eight waves per CU), a number
+// measured on one grid and taken for all: smaller ones, with fewer boxes a
+// level, have more of their levels above the subtrees. 512^2
 // complex64, a solve of 4 / 8 right-hand sides in three sweeps: 1469 / 2259 us
 // with 128 subtrees (half of the CUs idle), 1164 / 1735 with 256, 1042 / 1552
 // with 512, 1146 / 1683 with 1024 and 1311 / 1945 with 2048 (more launches
@@ -2217,14 +2220,14 @@ int nd_sweep(const NdPlan &P, const void *factor, double *x, int nrhs, int add, 
 // workspace, which fdfd_solve_static is limited by (except the kept iterate,
 // which that call does without where it has no room). FP64,
 // new permittivity and solve / resident solve through Simulation, block path
-// against tree: 16 x 16 1.16 / 0.63 against 0.56 / 0.26 ms, 32 x 32 1.46 /
-// 0.85 against 0.61 / 0.26, 48 x 40 2.52 / 0.98 against 0.65 / 0.23, 63 x 63
-// 3.21 / 1.13 against 0.72 / 0.25; below 16 cells a tree has hardly a level.
+// against tree: 16 x 16 1.13 / 0.60 against 0.52 / 0.29 ms, 32 x 32 1.26 /
+// 0.60 against 0.64 / 0.32, 48 x 40 2.27 / 0.70 against 0.71 / 0.32, 63 x 63
+// 3.21 / 1.13 against 0.80 / 0.35; below 16 cells a tree has hardly a level.
 // Complex64 factors of grids with a side below 64 cells stay block factors:
 // how far their refinement gets in a given number of steps, and that a
 // singular leading pivot sends them to FP64, is what the fallback order is
-// tested on (a new permittivity and solve of 48 x 40 cells takes 2.17 ms
-// there; 0.94 as a tree).
+// tested on. No measurement draws that line: a new permittivity and solve of
+// 48 x 40 cells takes 2.15 ms there, 0.94 as a tree.
 constexpr int ND_MIN_SIDE_C64 = 64;
 inline bool nd_fits(const fdfd_grid *g, int precision, NdPlan *P) {
   const int prec = base_prec(precision);
@@ -2239,7 +2242,7 @@ inline bool nd_fits(const fdfd_grid *g, int precision, NdPlan *P) {
 // cross, of order nx + ny - 1 and eliminated whole: the factor's time grows
 // with the cube of the long side and its memory with the square, the block
 // chain's with the side itself. FP64 factor, tree against block path: 6144 x 16
-// 36 against 58 ms, 8192 x 16 81 / 78 (5.8 GB against 0.13), 12288 x 16 266 /
+// 36 against 58 ms, 8192 x 16 81 / 78 (5.7 GB against 0.13), 12288 x 16 266 /
 // 117, 11584 x 64 230 / 326, 16384 x 64 632 / 462, 16384 x 128 645 / 776;
 // complex64 11584 x 64 116 / 254, 16384 x 64 317 / 359. A chain's step costs
 // about its block's tiles: the lines cross near a^2 = 2^21 b for a long side a
