@@ -75,7 +75,7 @@ int grant_lds(std::atomic<uint64_t> &done, std::initializer_list<const void *> k
   int cur = 0, dev = 0;
   HIP_TRY(hipGetDevice(&cur));
   dev = cur;
-  if (s && s != hipStreamPerThread) HIP_TRY(hipStreamGetDevice(s, &dev));
+  if ((uintptr_t)s > 2) HIP_TRY(hipStreamGetDevice(s, &dev));   // not the null, legacy or per-thread stream
   const uint64_t bit = dev < 64 ? 1ull << dev : 0;
   if (done.load() & bit) return 0;
   if (dev != cur) HIP_TRY(hipSetDevice(dev));

@@ -15,7 +15,7 @@ COUNTED = r"""
 static int current, grants[8], launches, refused = -1;
 int hipGetDevice(int *d) { *d = current; return 0; }
 int hipSetDevice(int d) { current = d; return 0; }
-int hipStreamGetDevice(void *s, int *d) { *d = (int)((size_t)s >> 12); return 0; }
+int hipStreamGetDevice(void *s, int *d) { *d = (int)((size_t)s >> 12); return (size_t)s < 4096; }
 int hipFuncSetAttribute(const void *f, int a, int v) { if (current == refused) return 1; ++grants[current]; return 0; }
 int hipLaunchKernel() { ++launches; return 0; }
 int hipGetLastError(void) { return 0; }
@@ -49,6 +49,7 @@ for call, kernels in ((factor, 1), (sweep, 2)):
     new = lambda: [c.seen_grants(d) - before[d] for d in range(5)]
     assert call(0) == 0 and call(0) == 0 and new() == [kernels, 0, 0, 0, 0], new()
     assert call(1) == 0 and new() == [kernels, kernels, 0, 0, 0], new()
+    assert call(1, 1) == 0 and call(1, 2) == 0 and new() == [kernels, kernels, 0, 0, 0], new()   # legacy, per thread
     assert call(0, 2 << 12) == 0 and new() == [kernels, kernels, kernels, 0, 0], new()   # a stream of device 2
     c.refuse(3)
     n = c.seen_launches()
